@@ -457,7 +457,12 @@ int ltpg_tpcc_gen_next(ltpg_tpcc_gen *g, uint32_t n_txns, uint32_t tid_base, uin
 
 /* ---- launch shape of the key-value kernels (replaces the fixed warp-role
  *      and grid constants, YCSB/0/Predefine.h:27-35) ------------------------ */
-/* EXEC_PER_OP: EXECUTE runs one lane per op instead of one lane per
+/* A context starts without a chosen shape: batch and table sizes pick the
+ * EXECUTE form (PARTITIONED for large epochs of point operations, EXEC_PER_OP
+ * for small ones; its buffers, 4 bytes per possible op slot and about 2 bytes
+ * per 16, are then allocated with the context).  ltpg_kv_set_tuning fixes the
+ * shape from then on: 0 is none of the flags below.
+ * EXEC_PER_OP: EXECUTE runs one lane per op instead of one lane per
  *   transaction.
  * SPLIT_REGISTERS: a row's R and W registers live in two arrays instead of
  *   one 16-byte pair.
@@ -477,15 +482,16 @@ int ltpg_tpcc_gen_next(ltpg_tpcc_gen *g, uint32_t n_txns, uint32_t tid_base, uin
  *   autotuner's combinations (LTPG_TUNE_ALL).  The served form runs its
  *   small key-value epochs this way whatever the context's flags.
  * PARTITIONED: EXECUTE of the fast form (no LTPG_FLAG_CONFLICT_COUNTS) bins
- *   the epoch's register operations by row range (8192 rows per bucket) and
- *   keeps each range's W minima in LDS, instead of probing and updating the
- *   per-row registers in HBM at random (EXEC_PER_OP then has no effect).
- *   Two streaming passes over the ops and one over the binned operations
- *   (12 bytes each); the autotuner tries it with SPLIT_REGISTERS,
- *   SMALL_CHUNKS and LANE_COPY.
+ *   the epoch's register operations by row and finds each row's minimum
+ *   writer in LDS, instead of probing and updating the per-row registers in
+ *   HBM at random (EXEC_PER_OP and SPLIT_REGISTERS then have no effect on
+ *   point operations).  Contexts with kv_max_scan <= 1: at most 16384 rows per
+ *   bucket, one pass over the batch and 4 bytes per binned operation.  With
+ *   scans: 8192 rows per bucket, two passes and 12 bytes each.  The autotuner
+ *   tries it with SPLIT_REGISTERS, SMALL_CHUNKS and LANE_COPY.
  *   Needs kv_rows <= 8192 * 16384 and kv_max_slots * max_txns *
  *   max(1, kv_max_scan) < 2^32 (else LTPG_ERR_UNSUPPORTED); the first
- *   selection allocates its buffers, 12 bytes per possible operation.
+ *   selection allocates its buffers.
  * MORE_ITEMS: items per thread -- the per-op EXECUTE (EXEC_PER_OP) takes 4
  *   ops per lane instead of 2 (its LDS fold spans 1024 ops), and the read
  *   marking 2 instead of 1; no effect with PARTITIONED.

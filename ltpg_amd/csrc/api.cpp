@@ -47,6 +47,36 @@ void free_kv(KvState &kv)
     dev_free(kv.part.slices);
     dev_free(kv.part.ent_me);
     dev_free(kv.part.ent_key);
+    dev_free(kv.bin.ent);
+    dev_free(kv.bin.off);
+    dev_free(kv.bin.unsorted);
+}
+
+// Buffers of the binned EXECUTE for every batch the context accepts.
+int kv_bin_prepare(ltpg_ctx *ctx)
+{
+    KvState &kv = ctx->kv;
+    if (kv.bin.ent) return LTPG_OK;
+    const uint64_t ops = (uint64_t)kv.max_slots * ctx->cfg.max_txns;
+    KvState::Bin p;
+    // the largest batch, and the largest of the smaller tiles' shape
+    for (uint64_t n : {ops, std::min(ops, kBinLargeOps - 1)}) {
+        const BinShape f = kv_bin_shape(kv.rows, n);
+        p.cap_ent = std::max(p.cap_ent, (uint64_t)f.tiles << f.tile_bits);
+        p.cap_off = std::max(p.cap_off, (uint64_t)f.tiles * (f.buckets + 1));
+    }
+    int rc;
+    if ((rc = dev_alloc(&p.ent, p.cap_ent, "binned operations")) || (rc = dev_alloc(&p.off, p.cap_off, "bin starts")) ||
+        (rc = dev_alloc(&p.unsorted, 1, "TID order flag"))) {
+        dev_free(p.ent);
+        dev_free(p.off);
+        dev_free(p.unsorted);
+        return rc;
+    }
+    kv.bin = p;  // freed with the context
+    // epoch 0 is never current
+    LTPG_HIP_TRY(launch_fill_u8(reinterpret_cast<uint8_t *>(p.unsorted), 4, 0, ctx->stream));
+    return LTPG_OK;
 }
 
 int init_kv(ltpg_ctx *ctx)
@@ -89,6 +119,11 @@ int init_kv(ltpg_ctx *ctx)
         if ((rc = dev_alloc(&kv.hot_acc, (uint64_t)kCounterStripes * kv.fields, "hot-row accumulators"))) return rc;
         LTPG_HIP_TRY(hipMemsetAsync(kv.hot_acc, 0, (uint64_t)kCounterStripes * kv.fields * 4, ctx->stream));
     }
+    // the default shape of large epochs; without memory for it they take the
+    // register path
+    if (kv.max_scan <= 1 && !(c.flags & LTPG_FLAG_CONFLICT_COUNTS) && kv_bin_auto(kv.rows, S * B) &&
+        kv_bin_prepare(ctx) == LTPG_ERR_NOMEM)
+        (void)hipGetLastError();  // dealt with
     // Registers start as all-ones: tag ~0 belongs to epoch 0, which is never
     // current (epochs start at 1), so every row reads as "no registrant".
     LTPG_HIP_TRY(launch_fill_u64(kv.regs, kv.rows * 2, ~0ull, ctx->stream));
@@ -208,10 +243,12 @@ int kv_part_prepare(ltpg_ctx *ctx)
 {
     KvState &kv = ctx->kv;
     if (kv.part.ent_me) return LTPG_OK;
+    if (kv.max_scan <= 1 && kv.bin.ent) return LTPG_OK;
     const uint64_t nb = (kv.rows + (1ull << kPartShift) - 1) >> kPartShift;
     const uint64_t cap = (uint64_t)kv.max_slots * ctx->cfg.max_txns * kv.read_slot;
     if (nb > kPartMaxBuckets || cap >= (1ull << 32))
         LTPG_FAIL(LTPG_ERR_UNSUPPORTED, "row-partitioned EXECUTE: too many rows or operations per epoch");
+    if (kv.max_scan <= 1) return kv_bin_prepare(ctx);  // point operations
     KvState::Part p;
     p.n_buckets = (uint32_t)nb;
     p.cap_entries = cap;
@@ -836,6 +873,18 @@ int ltpg_kv_table_fill_reference(ltpg_ctx *ctx)
     return LTPG_OK;
 }
 
+}  // extern "C"
+
+void ltpg::kv_default_shape(ltpg_ctx *ctx)
+{
+    KvState &kv = ctx->kv;
+    kv.partitioned = kv.exec_per_op = kv.split_regs = kv.small_chunks = kv.lane_copy = kv.small_epoch = 0;
+    kv.more_items = 0;
+    kv.auto_shape = true;
+}
+
+extern "C" {
+
 int ltpg_kv_set_tuning(ltpg_ctx *ctx, uint32_t flags)
 {
     int rc = check_ctx(ctx);
@@ -851,6 +900,7 @@ int ltpg_kv_set_tuning(ltpg_ctx *ctx, uint32_t flags)
     ctx->kv.lane_copy = (flags & LTPG_TUNE_LANE_COPY) ? 1 : 0;
     ctx->kv.small_epoch = (flags & LTPG_TUNE_SMALL_EPOCH) ? 1 : 0;
     ctx->kv.more_items = (flags & LTPG_TUNE_MORE_ITEMS) ? 1 : 0;
+    ctx->kv.auto_shape = false;
     return LTPG_OK;
 }
 

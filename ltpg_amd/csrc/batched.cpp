@@ -41,6 +41,7 @@ struct ltpg_batched {
     hipGraphExec_t exec[2] = {nullptr, nullptr};
     uint32_t final_epoch[2] = {0, 0};       // host epoch counter after a replay
     std::vector<uint8_t> tune;              // batch i: its LTPG_TUNE_* flags (key-value or order-entry)
+    bool tuned = false;                     // false: key-value batches take the default shape
     unsigned long long *stamps = nullptr;   // graph runs: device clock after batch i; [n + k] start of graph k
     std::vector<double> plain_ms;           // plain runs: host ms from the run's start to batch i's readback
     // key-value pipelining: side stream for EXECUTE, second register / flag set
@@ -58,6 +59,14 @@ uint64_t words(uint64_t n) { return (n + 63) / 64; }
 
 int slot_of(uint32_t workload) { return workload == LTPG_WORKLOAD_KV ? 0 : 1; }
 
+// The launch shape of key-value batch i.
+int set_kv_shape(ltpg_batched *b, ltpg_ctx *ctx, uint32_t i)
+{
+    if (b->tuned) return ltpg_kv_set_tuning(ctx, b->tune[i]);
+    kv_default_shape(ctx);
+    return LTPG_OK;
+}
+
 // One epoch of batch i on its context: submit (device-resident), all
 // phases, archive copy of the commit bitmap(s), and (captured runs) a device
 // clock stamp.  No synchronisation, so it can be captured -- unless
@@ -69,7 +78,7 @@ int enqueue_batch(ltpg_batched *b, uint32_t i, bool stamp, bool stepwise = false
     ltpg_ctx *ctx = b->ctx[slot_of(d.workload)];
     int rc;
     if (d.workload == LTPG_WORKLOAD_KV) {
-        if ((rc = ltpg_kv_set_tuning(ctx, b->tune[i]))) return rc;
+        if ((rc = set_kv_shape(b, ctx, i))) return rc;
         if ((rc = ltpg_kv_submit(ctx, &d.kv, LTPG_MEM_DEVICE))) return rc;
     } else {
         if ((rc = ltpg_tpcc_set_tuning(ctx, b->tune[i]))) return rc;
@@ -151,7 +160,7 @@ int enqueue_kv_pipelined(ltpg_batched *b)
     for (uint32_t i = 0; i < b->d.size(); i++) {
         const ltpg_batch_desc &d = b->d[i];
         if (d.workload != LTPG_WORKLOAD_KV) continue;
-        if ((rc = ltpg_kv_set_tuning(ctx, b->tune[i]))) return rc;
+        if ((rc = set_kv_shape(b, ctx, i))) return rc;
         if (ctx->epoch >= 255) {
             // the submit below wraps the epoch and refills the first set on
             // main: nothing may be in flight on side, and the second set
@@ -392,6 +401,7 @@ int ltpg_batched_autotune(ltpg_batched *b, uint32_t reps, ltpg_tuning_entry *out
             if (rep[c] < 0) rep[c] = (int)i;
         }
         if (k == 0) ctx->kv.regs_clean = false;
+        b->tuned = true;
         const uint32_t values = ctx->cfg.values;
         ctx->cfg.values = LTPG_VALUES_COPYBACK;  // timing runs leave the tables as they are
         const bool timing = ctx->timing;
@@ -483,6 +493,7 @@ int ltpg_batched_set_tuning(ltpg_batched *b, uint32_t flags)
         LTPG_FAIL(LTPG_ERR_INVALID, "unknown tuning flag");
     const uint32_t kv_flags = flags & ~LTPG_TUNE_TPCC_SMALL_BLOCKS, tp_flags = flags & LTPG_TUNE_TPCC_SMALL_BLOCKS;
     int rc;
+    b->tuned = true;
     // validates the flags and prepares their buffers outside any capture
     if (b->ctx[0] && ((rc = check_ctx(b->ctx[0])) || (rc = ltpg_kv_set_tuning(b->ctx[0], kv_flags)))) return rc;
     if (b->ctx[1] && ((rc = check_ctx(b->ctx[1])) || (rc = ltpg_tpcc_set_tuning(b->ctx[1], tp_flags)))) return rc;

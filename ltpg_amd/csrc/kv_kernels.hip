@@ -546,7 +546,8 @@ __global__ __launch_bounds__(kBlock) void kv_execute_dedup_kernel(
     if (bad) atomicAdd(&ctr->range_errors, bad);
 }
 
-// ---- row-partitioned EXECUTE (LTPG_TUNE_PARTITIONED, fast form) -----------
+// ---- row-partitioned EXECUTE with scans (LTPG_TUNE_PARTITIONED, fast form) --
+// ---- (batches of point operations only are binned below) ------------------
 //
 // The register phase touches one random register line per operation; the
 // lines of a 10M-row table overflow the L2s, so each 8-byte probe or atomic
@@ -769,18 +770,6 @@ __global__ __launch_bounds__(kPartBlock) void kv_part_scatter_kernel(PartArgs a)
     }
 }
 
-// Binning of point operations (no scans) through LDS: a block takes
-// P ops per thread, ranks each in its bucket with an LDS counter, turns the
-// counts into block-local starts, reserves one run per bucket in the global
-// bucket with one atomic, places the entries bucket by bucket in LDS and
-// writes them out in that order -- consecutive lanes write consecutive
-// entries of a run, so the stores coalesce instead of scattering 8- and
-// 4-byte writes over every bucket.  MaxB bounds the buckets.  Runs are as
-// long as the block's share of a bucket, so a block takes as many ops as
-// its LDS holds: 8 per thread (122 KB) with at most kPartFewBuckets
-// buckets, 4 per thread beside the 64 KB of counters for 16384.
-constexpr uint32_t kPartFewBuckets = 2048;
-
 // Exclusive prefix sum over the block of one value per thread; *total gets
 // the sum.  Wave scans by shuffles, then the 16 wave totals through LDS.
 __device__ __forceinline__ uint32_t block_exclusive_sum(uint32_t v, uint32_t *s_wt, uint32_t *total)
@@ -804,86 +793,6 @@ __device__ __forceinline__ uint32_t block_exclusive_sum(uint32_t v, uint32_t *s_
     }
     *total = all;
     return before + inc - v;
-}
-
-template <uint32_t MaxB, uint32_t P>
-__global__ __launch_bounds__(kPartBlock) void kv_part_scatter_staged_kernel(PartArgs a)
-{
-    constexpr uint32_t kPer = (MaxB + kPartBlock - 1) / kPartBlock;  // buckets per thread at most
-    __shared__ uint32_t s_at[MaxB];              // counts, then local starts, then global - local
-    __shared__ unsigned long long st_me[P * kPartBlock];
-    __shared__ uint32_t st_key[P * kPartBlock];
-    __shared__ uint16_t st_b[P * kPartBlock];
-    __shared__ uint32_t s_wt[kPartBlock / 64];
-    for (uint32_t b = threadIdx.x; b < a.nb; b += kPartBlock) s_at[b] = 0;
-    __syncthreads();
-    const uint64_t n_ops = (uint64_t)a.S * a.B;
-    const uint64_t base = (uint64_t)blockIdx.x * (P * kPartBlock) + threadIdx.x;
-    Op o[P];
-    part_load(a, base, o);
-    uint32_t bk[P], rank[P];
-    bool use[P];
-    unsigned long long me[P];
-#pragma unroll
-    for (uint32_t u = 0; u < P; ++u) {
-        use[u] = o[u].valid && o[u].len <= 1 && o[u].row != a.hot;
-        bk[u] = (uint32_t)(o[u].row >> kPartShift);
-        const uint64_t i = base + (uint64_t)u * kPartBlock;
-        const uint32_t i32 = i < n_ops ? (uint32_t)i : 0u;
-        const uint32_t t = a.rm ? i32 / a.S : i32 % a.B;
-        me[u] = priority(a.tag, a.tids[t], t);
-    }
-#pragma unroll
-    for (uint32_t u = 0; u < P; ++u)
-        rank[u] = use[u] ? atomicAdd(&s_at[bk[u]], 1u) : 0u;
-    __syncthreads();
-    // thread j owns buckets [j * per, (j + 1) * per): their counts, then
-    // their local starts from the block-wide exclusive sum
-    const uint32_t per = (a.nb + kPartBlock - 1) / kPartBlock;
-    const uint32_t b0 = threadIdx.x * per;
-    uint32_t cnt[kPer], st[kPer];
-    uint32_t sum = 0;
-#pragma unroll
-    for (uint32_t j = 0; j < kPer; ++j) {
-        cnt[j] = (j < per && b0 + j < a.nb) ? s_at[b0 + j] : 0u;
-        sum += cnt[j];
-    }
-    uint32_t total;
-    uint32_t run = block_exclusive_sum(sum, s_wt, &total);
-#pragma unroll
-    for (uint32_t j = 0; j < kPer; ++j) {
-        st[j] = run;
-        run += cnt[j];
-    }
-#pragma unroll
-    for (uint32_t j = 0; j < kPer; ++j)
-        if (cnt[j]) s_at[b0 + j] = st[j];
-    __syncthreads();
-    // this thread's entries go to their bucket's local run
-    uint32_t slot[P];
-#pragma unroll
-    for (uint32_t u = 0; u < P; ++u) slot[u] = use[u] ? s_at[bk[u]] + rank[u] : 0u;
-    // one global run per non-empty bucket; s_at[b] becomes global - local
-    uint32_t delta[kPer];
-#pragma unroll
-    for (uint32_t j = 0; j < kPer; ++j) delta[j] = cnt[j] ? atomicAdd(&a.cursor[b0 + j], cnt[j]) - st[j] : 0u;
-#pragma unroll
-    for (uint32_t u = 0; u < P; ++u) {
-        if (!use[u]) continue;
-        st_me[slot[u]] = me[u];
-        st_key[slot[u]] = ((uint32_t)(o[u].row & (kPartRows - 1)) << 1) | (o[u].kind == LTPG_KV_WRITE ? 1u : 0u);
-        st_b[slot[u]] = (uint16_t)bk[u];
-    }
-    __syncthreads();
-#pragma unroll
-    for (uint32_t j = 0; j < kPer; ++j)
-        if (cnt[j]) s_at[b0 + j] = delta[j];
-    __syncthreads();
-    for (uint32_t j = threadIdx.x; j < total; j += kPartBlock) {
-        const uint32_t at = j + s_at[st_b[j]];
-        a.ent_me[at] = st_me[j];
-        a.ent_key[at] = st_key[j];
-    }
 }
 
 // The fast form's flags of one operation against its row's minimum W
@@ -980,6 +889,303 @@ __global__ __launch_bounds__(kPartBlock) void kv_part_flags_kernel(PartArgs a)
         for (uint32_t u = 0; u < kPartGroup; ++u)
             if (e0 + u * kPartBlock < end) part_flag(a, key[u], me[u], s_w[key[u] >> 1]);
     }
+}
+
+// ---- binned EXECUTE of point operations (LTPG_TUNE_PARTITIONED, or the
+// ---- default shape of a large epoch; fast form, no scans) -----------------
+//
+// The register path touches one random 128-byte register line per operation.
+// Here the operations are binned by row first and every row's minimum writer
+// is found in LDS; the per-row registers in HBM are not touched:
+//   order    are the TIDs non-decreasing in batch position (the usual batch)?
+//            Then position alone is the priority;
+//   bin      one pass over the batch.  A 1024-thread block takes a tile of
+//            P * 1024 consecutive op slots, drops operations that a writer in
+//            the same tile already decides (below), ranks the others per
+//            bucket with LDS counters, places them bucket by bucket in LDS and
+//            writes the tile out in that order, with the start of each
+//            bucket's run (16 bits) in a table;
+//   flags    one block per bucket: reads the bucket's run of every tile twice,
+//            first into the W minima of its rows in LDS, then setting the
+//            fast form's flags from them (part_flag).
+// A row's bucket is the top bits of row * odd mod 2^K (a bijection), so ranges
+// of hot rows spread over the buckets.  An entry is 4 bytes -- row within the
+// bucket, is-write, slot within the tile; the tile gives the rest -- so no
+// TID, position or counting pass goes through memory: the batch is read once,
+// and 4 bytes per operation written once and read twice (the second time
+// mostly from the L2).
+//
+// The in-tile filter: writers enter (position, row) into a direct-mapped LDS
+// table with a 64-bit minimum.  An operation that finds its own row there
+// under a lower position is behind a writer: a write has waw, a read raw, and
+// neither can matter to any other transaction (it is not its row's minimum
+// writer, and as a reader it is behind that minimum, so gives no war).  It is
+// flagged at once and leaves the batch, which keeps a skewed epoch's hot rows
+// from filling one bucket.  Only with ordered TIDs.
+//
+// 2^20 transactions x 16 ops on 10M rows: 486 us on the registers (285
+// registration, 202 read marking) -> 200 us at Zipf 0.6 (order 5, bin 62,
+// flags 130), 515 -> 170 us at Zipf 0.99.  The bin kernel moves 268 MB at 4.3
+// TB/s; the flags kernel is bound by instruction issue (1M runs of 16 entries,
+// half of the lanes idle) and, at Zipf 0.6, by its 6M scattered flag bytes
+// (63 us without them).
+constexpr uint32_t kBinBlock = 1024;
+constexpr uint32_t kBinRows = 1u << kBinRowBits;
+constexpr uint32_t kBinMul = 0x9E3779B1u;  // odd
+
+// i mod d and i / d for i < 2^32 by one high multiply: with m = floor(2^32 /
+// d) (2^32 - 1 for d = 1) the quotient is exact or one too small.
+struct FastMod {
+    uint32_t d, m;
+};
+
+__device__ __forceinline__ uint32_t fast_div(const FastMod &f, uint32_t i, uint32_t *rem)
+{
+    uint32_t q = __umulhi(i, f.m);
+    uint32_t r = i - q * f.d;
+    if (r >= f.d) {
+        r -= f.d;
+        ++q;
+    }
+    *rem = r;
+    return q;
+}
+
+struct BinArgs {
+    const uint64_t *keys;
+    const uint32_t *meta;
+    const uint32_t *tids;
+    uint32_t B, n_ops;
+    uint64_t rows;
+    uint32_t fields, max_scan;
+    uint64_t hot;
+    uint32_t mask, row_bits, nb, tiles, tile_bits;  // 2^K - 1; log2 rows per bucket; buckets; tiles; log2 slots per tile
+    FastMod per;                                    // n_slots (request-major) or n_txns
+    bool rm;
+    uint8_t epoch;
+    uint32_t *ent;         // [tiles << tile_bits]
+    uint16_t *off;         // [tiles][nb + 1] start of each bucket's run in the tile
+    uint32_t *unsorted;    // epoch number of the last epoch whose TIDs were out of order
+    uint8_t *doomed, *raw_flag, *war_flag;
+    DeviceCounters *ctr;
+};
+
+__device__ __forceinline__ uint32_t bin_txn(const BinArgs &a, uint32_t i)
+{
+    uint32_t r;
+    const uint32_t q = fast_div(a.per, i, &r);
+    return a.rm ? q : r;
+}
+
+__global__ __launch_bounds__(kBlock) void kv_bin_order_kernel(BinArgs a, bool zero_counts)
+{
+    if (zero_counts && blockIdx.x == 0)
+        for (uint32_t c = threadIdx.x; c < kCounterStripes * kCountedTypes; c += kBlock)
+            a.ctr->commits[c / kCountedTypes][c % kCountedTypes] = 0;
+    // four pairs per thread, all loads in flight together
+    const uint32_t first = blockIdx.x * (4 * kBlock) + threadIdx.x, last = a.B - 1;
+    uint32_t lo[4], hi[4];
+#pragma unroll
+    for (uint32_t u = 0; u < 4; ++u) {
+        const uint32_t t = first + u * kBlock;
+        lo[u] = a.tids[t < last ? t : last];
+        hi[u] = a.tids[t < last ? t + 1 : last];
+    }
+    bool out = false;
+#pragma unroll
+    for (uint32_t u = 0; u < 4; ++u) out |= lo[u] > hi[u];
+    // a stale equal number (255 epochs ago) only costs the slower path
+    if (out) *a.unsorted = a.epoch;
+}
+
+template <uint32_t P, uint32_t MaxB>
+__global__ __launch_bounds__(kBinBlock, MaxB <= kBinBlock ? 8 : 4) void kv_bin_kernel(BinArgs a)
+{
+    constexpr uint32_t T = P * kBinBlock, kFilter = T / 2;
+    constexpr uint32_t kPer = MaxB / kBinBlock;  // buckets per thread at most
+    constexpr uint32_t G = 4;                    // loads in flight per thread
+    __shared__ __align__(16) uint32_t s_ent[T];  // the filter first, then the tile in bucket order
+    __shared__ uint32_t s_at[MaxB];              // counts, then starts
+    __shared__ uint32_t s_wt[kBinBlock / 64];
+    unsigned long long *s_min = reinterpret_cast<unsigned long long *>(s_ent);
+    const uint32_t base = blockIdx.x * T + threadIdx.x;
+    const bool fold = *a.unsorted != a.epoch;
+    for (uint32_t k = threadIdx.x; k < kFilter; k += kBinBlock) s_min[k] = ~0ull;
+    for (uint32_t b = threadIdx.x; b < a.nb; b += kBinBlock) s_at[b] = 0;
+    __syncthreads();
+    uint32_t hw[P];  // hashed row << 1 | is-write, or all-ones: nothing to register
+    uint32_t bad = 0;
+#pragma unroll
+    for (uint32_t g = 0; g < P; g += G) {
+        uint64_t r[G];
+        uint32_t m[G];
+#pragma unroll
+        for (uint32_t u = 0; u < G; ++u) {
+            const uint32_t i = base + (g + u) * kBinBlock;
+            r[u] = a.keys[i < a.n_ops ? i : 0u];
+            m[u] = a.meta[i < a.n_ops ? i : 0u];
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < G; ++u) {
+            const uint32_t i = base + (g + u) * kBinBlock;
+            const Op o = decode_op(r[u], i < a.n_ops ? m[u] : 0u, a.rows, a.fields, a.max_scan);
+            bad += (o.kind != LTPG_KV_NONE && !o.valid) ? 1u : 0u;
+            const uint32_t w = o.kind == LTPG_KV_WRITE ? 1u : 0u;
+            const uint32_t h = ((uint32_t)o.row * kBinMul) & a.mask;
+            const bool use = o.valid && o.row != a.hot;
+            hw[g + u] = use ? h << 1 | w : ~0u;
+            if (fold && use && w)
+                atomicMin(&s_min[(h ^ (h >> 12)) & (kFilter - 1)], (unsigned long long)bin_txn(a, i) << 32 | h);
+        }
+    }
+    if (bad) atomicAdd(&a.ctr->range_errors, bad);
+    __syncthreads();
+    uint32_t rank[P];
+#pragma unroll
+    for (uint32_t u = 0; u < P; ++u) {
+        const uint32_t h = hw[u] >> 1;
+        if (fold && hw[u] != ~0u) {
+            const unsigned long long v = s_min[(h ^ (h >> 12)) & (kFilter - 1)];
+            if ((uint32_t)v == h) {
+                const uint32_t t = bin_txn(a, base + u * kBinBlock);
+                if ((uint32_t)(v >> 32) < t) {
+                    if (hw[u] & 1u)
+                        a.doomed[t] = a.epoch;
+                    else
+                        a.raw_flag[t] = a.epoch;
+                    hw[u] = ~0u;
+                }
+            }
+        }
+        rank[u] = hw[u] != ~0u ? atomicAdd(&s_at[h >> a.row_bits], 1u) : 0u;
+    }
+    __syncthreads();
+    // thread j owns buckets [j * per, (j + 1) * per)
+    const uint32_t per = (a.nb + kBinBlock - 1) / kBinBlock, b0 = threadIdx.x * per;
+    uint32_t cnt[kPer], sum = 0, total;
+#pragma unroll
+    for (uint32_t j = 0; j < kPer; ++j) {
+        cnt[j] = (j < per && b0 + j < a.nb) ? s_at[b0 + j] : 0u;
+        sum += cnt[j];
+    }
+    uint32_t run = block_exclusive_sum(sum, s_wt, &total);
+    uint16_t *off = a.off + (uint64_t)blockIdx.x * (a.nb + 1);
+#pragma unroll
+    for (uint32_t j = 0; j < kPer; ++j) {
+        if (j < per && b0 + j < a.nb) {
+            s_at[b0 + j] = run;
+            off[b0 + j] = (uint16_t)run;
+        }
+        run += cnt[j];
+    }
+    if (threadIdx.x == 0) off[a.nb] = (uint16_t)total;
+    __syncthreads();
+    const uint32_t inner = (1u << a.row_bits) - 1u;
+#pragma unroll
+    for (uint32_t u = 0; u < P; ++u) {
+        if (hw[u] == ~0u) continue;
+        const uint32_t h = hw[u] >> 1;
+        s_ent[s_at[h >> a.row_bits] + rank[u]] =
+            (h & inner) << (kBinSlotBits + 1) | (hw[u] & 1u) << kBinSlotBits | (u * kBinBlock + threadIdx.x);
+    }
+    __syncthreads();
+    // whole 16-byte vectors: the last one may carry stale words, which stay
+    // inside the tile's own part of ent
+    uint4 *dst = reinterpret_cast<uint4 *>(a.ent + (uint64_t)blockIdx.x * T);
+    const uint4 *src = reinterpret_cast<const uint4 *>(s_ent);
+    for (uint32_t j = threadIdx.x; j < (total + 3) / 4; j += kBinBlock) dst[j] = src[j];
+}
+
+// One pass over bucket b's entries: 16 lanes per tile run, four runs' first
+// 32 entries in flight per group.  MARK false: the W minima of the rows
+// [lo, lo + n) of the bucket into s_w; MARK true: the flags from them.  The
+// priority is the position (u32) or, with TIDs out of order, TID << 24 |
+// position (u64); all-ones: no writer.
+template <typename W, bool MARK>
+__device__ __forceinline__ void bin_pass(const BinArgs &a, uint32_t b, W *s_w, uint32_t lo, uint32_t n)
+{
+    constexpr uint32_t kRun = 16, kGroups = kBinBlock / kRun, U = 4;
+    const uint32_t g = threadIdx.x / kRun, l = threadIdx.x % kRun;
+    const int base_lane = lane_id() & ~(int)(kRun - 1);
+    auto one = [&](uint32_t x, uint32_t tile) {
+        const uint32_t r = (x >> (kBinSlotBits + 1)) - lo;
+        const bool wr = (x >> kBinSlotBits) & 1u;
+        if ((!MARK && !wr) || r >= n) return;
+        const uint32_t t = bin_txn(a, (tile << a.tile_bits) + (x & ((1u << kBinSlotBits) - 1u)));
+        const W me = sizeof(W) == 4 ? (W)t : (W)((unsigned long long)a.tids[t] << kTidShift | t);
+        if (!MARK) {
+            atomicMin(&s_w[r], me);
+            return;
+        }
+        const W w = s_w[r];
+        if (wr) {
+            if (w < me) a.doomed[t] = a.epoch;
+        } else if (w < me) {
+            a.raw_flag[t] = a.epoch;
+        } else if (w > me && w != (W)~(W)0) {
+            a.war_flag[w & (W)kPosMask] = a.epoch;
+        }
+    };
+    for (uint32_t c0 = 0; c0 < a.tiles; c0 += kBinBlock) {
+        // lane l of group g holds the run of tile c0 + l * kGroups + g
+        const uint32_t mine = c0 + l * kGroups + g;
+        uint32_t st = 0, ln = 0;
+        if (mine < a.tiles) {
+            const uint16_t *o = a.off + (uint64_t)mine * (a.nb + 1) + b;
+            st = o[0];
+            ln = o[1] - st;
+        }
+        const uint32_t left = a.tiles - c0;
+        const uint32_t nj = left >= kBinBlock ? kRun : (left + kGroups - 1) / kGroups;
+        for (uint32_t j0 = 0; j0 < nj; j0 += U) {
+            uint32_t s[U], len[U], x[U][2];
+#pragma unroll
+            for (uint32_t u = 0; u < U; ++u) {
+                s[u] = __shfl(st, base_lane + (int)(j0 + u));
+                len[u] = __shfl(ln, base_lane + (int)(j0 + u));
+                const uint32_t tile = c0 + (j0 + u) * kGroups + g;
+                const uint32_t *p = a.ent + (len[u] ? ((uint64_t)tile << a.tile_bits) + s[u] : 0ull);
+                // unconditional loads (a run's first entry, or entry 0, when idle)
+                x[u][0] = p[l < len[u] ? l : 0u];
+                x[u][1] = p[l + kRun < len[u] ? l + kRun : 0u];
+            }
+#pragma unroll
+            for (uint32_t u = 0; u < U; ++u) {
+                const uint32_t tile = c0 + (j0 + u) * kGroups + g;
+                if (l < len[u]) one(x[u][0], tile);
+                if (l + kRun < len[u]) one(x[u][1], tile);
+                for (uint32_t e = l + 2 * kRun; e < len[u]; e += kRun)
+                    one(a.ent[((uint64_t)tile << a.tile_bits) + s[u] + e], tile);
+            }
+        }
+    }
+}
+
+template <typename W>
+__device__ __forceinline__ void bin_flags(const BinArgs &a, uint32_t b, W *s_w, uint32_t cap)
+{
+    for (uint32_t lo = 0; lo < (1u << a.row_bits); lo += cap) {
+        const uint32_t n = min(1u << a.row_bits, cap);
+        for (uint32_t r = threadIdx.x; r < n; r += kBinBlock) s_w[r] = (W)~(W)0;
+        __syncthreads();
+        bin_pass<W, false>(a, b, s_w, lo, n);
+        __syncthreads();
+        bin_pass<W, true>(a, b, s_w, lo, n);
+        __syncthreads();
+    }
+}
+
+__global__ __launch_bounds__(kBinBlock, 8) void kv_bin_flags_kernel(BinArgs a)
+{
+    __shared__ unsigned long long s_w[kBinRows / 2];
+    // blocks of one XCD take neighbouring buckets, whose runs and table
+    // entries share cache lines
+    const uint32_t x = blockIdx.x;
+    const uint32_t b = a.nb >= 8 ? (x & 7u) * (a.nb / 8) + (x >> 3) : x;
+    if (*a.unsorted != a.epoch)
+        bin_flags<uint32_t>(a, b, reinterpret_cast<uint32_t *>(s_w), kBinRows);
+    else
+        bin_flags<unsigned long long>(a, b, s_w, kBinRows / 2);
 }
 
 // Read marking (fast form), one lane per op after every write has
@@ -2877,6 +3083,111 @@ RegLayout reg_layout(const KvState &kv)
     return rl;
 }
 
+// Shape of the binned EXECUTE: 2^K >= rows; large epochs take 1024 buckets
+// and 16 ops per thread, smaller ones 256 buckets and 4 ops per thread (more
+// blocks), and more buckets where a bucket would exceed 2^kBinRowBits rows.
+BinShape kv_bin_shape(uint64_t rows, uint64_t ops)
+{
+    BinShape f;
+    uint32_t K = 0;
+    while (K < 27 && (1ull << K) < rows) ++K;
+    const bool large = ops >= kBinLargeOps;
+    const int rb = (int)K - (large ? 10 : 8);
+    f.row_bits = rb < 8 ? 8u : rb > (int)kBinRowBits ? kBinRowBits : (uint32_t)rb;
+    f.buckets = K > f.row_bits ? 1u << (K - f.row_bits) : 1u;
+    f.mask = (1u << (K > f.row_bits ? K : f.row_bits)) - 1u;
+    f.tile_bits = large || f.buckets >= 1024 ? kBinSlotBits : kBinSlotBits - 2;
+    f.tiles = (uint32_t)((ops + (1ull << f.tile_bits) - 1) >> f.tile_bits);
+    return f;
+}
+
+// Default EXECUTE shapes, from a sweep of rows x ops x (Zipf 0, 0.9, 0.99;
+// 50 and 90 % reads); times in us are register path (one lane per
+// transaction) / per-op register path / binned.
+//
+// Binned: its cost besides streaming is one short run per tile and bucket, so
+// it needs about 1024 ops per bucket.
+//   1M rows (256 buckets):    160K ops 22 / 16 / 16, 320K 28 / 27 / 17,
+//                             1.3M 77 / 60 / 29, 16M 396 / 294 / 166
+//   10M rows (1024 buckets):  650K ops 42 / 45 / 36, 1.3M 69 / 63 / 38,
+//                             4M 168 / 116 / 48, 16M 440 / 374 / 160
+//   100M rows (8192 buckets): 4M ops 180 / 143 / 131, 16M 504 / 447 / 425;
+//                             at Zipf 0.99, 334 / 328 / 409
+// Below 32K rows there are too few buckets to fill the chip (20K rows, 16M
+// ops, Zipf 0: 186 / 191 / 212).
+bool kv_bin_auto(uint64_t rows, uint64_t ops)
+{
+    if (rows <= (1ull << 15) || rows > (1ull << 25) || ops >= (1ull << 31)) return false;
+    const uint64_t per = 1024ull * kv_bin_shape(rows, ops).buckets;
+    return ops >= (1ull << 18) && ops >= per;
+}
+
+namespace {
+
+// Per-op registration where the binned path is not taken: small epochs are a
+// chain of dependent misses per transaction otherwise (80K ops on 1M rows 19
+// / 10 us, 160K 22 / 16), and the largest ones gain from its row folding
+// (100M rows: 4M ops 180 / 143, 16M 504 / 447); in between it loses where
+// most rows are distinct (1.3M ops on 10M rows, Zipf 0: 48 / 53).
+inline bool kv_per_op_auto(uint64_t ops) { return ops < (1ull << 18) || ops >= (1ull << 21); }
+
+bool bin_wanted(const KvState &kv, const KvBatchDev &b)
+{
+    const uint64_t ops = (uint64_t)b.n_txns * b.n_slots;
+    if (!kv.bin.ent || kv.max_scan > 1 || !(kv.partitioned || (kv.auto_shape && kv_bin_auto(kv.rows, ops))) ||
+        ops >= 0xFFFF0000ull)
+        return false;
+    const BinShape f = kv_bin_shape(kv.rows, ops);
+    return ((uint64_t)f.tiles << f.tile_bits) <= kv.bin.cap_ent &&
+           (uint64_t)f.tiles * (f.buckets + 1) <= kv.bin.cap_off;
+}
+
+hipError_t launch_kv_bin(const KvState &kv, const KvBatchDev &b, const EpochTag &e, DeviceCounters *ctr,
+                         hipStream_t s, bool zero_counts)
+{
+    const uint64_t ops = (uint64_t)b.n_txns * b.n_slots;
+    const BinShape f = kv_bin_shape(kv.rows, ops);
+    BinArgs a;
+    a.keys = b.keys;
+    a.meta = b.meta;
+    a.tids = b.tids;
+    a.B = b.n_txns;
+    a.n_ops = (uint32_t)ops;
+    a.rows = kv.rows;
+    a.fields = kv.fields;
+    a.max_scan = kv.max_scan;
+    a.hot = kv.hot_row;
+    a.mask = f.mask;
+    a.row_bits = f.row_bits;
+    a.nb = f.buckets;
+    a.tiles = f.tiles;
+    a.tile_bits = f.tile_bits;
+    a.per.d = b.request_major ? b.n_slots : b.n_txns;
+    a.per.m = a.per.d > 1 ? (uint32_t)((1ull << 32) / a.per.d) : ~0u;
+    a.rm = b.request_major;
+    a.epoch = e.epoch;
+    a.ent = kv.bin.ent;
+    a.off = kv.bin.off;
+    a.unsorted = kv.bin.unsorted;
+    a.doomed = kv.doomed;
+    a.raw_flag = kv.raw_flag;
+    a.war_flag = kv.war_flag;
+    a.ctr = ctr;
+    hipLaunchKernelGGL(kv_bin_order_kernel, dim3((b.n_txns + 4 * kBlock - 1) / (4 * kBlock)), dim3(kBlock), 0, s, a,
+                       zero_counts);
+    const dim3 tiles(f.tiles), blk(kBinBlock);
+    if (f.tile_bits == kBinSlotBits && f.buckets <= 1024)
+        hipLaunchKernelGGL((kv_bin_kernel<16, 1024>), tiles, blk, 0, s, a);
+    else if (f.tile_bits == kBinSlotBits)
+        hipLaunchKernelGGL((kv_bin_kernel<16, 8192>), tiles, blk, 0, s, a);
+    else
+        hipLaunchKernelGGL((kv_bin_kernel<4, 1024>), tiles, blk, 0, s, a);
+    hipLaunchKernelGGL(kv_bin_flags_kernel, dim3(f.buckets), blk, 0, s, a);
+    return hipGetLastError();
+}
+
+}  // namespace
+
 hipError_t launch_kv_execute(const KvState &kv, const KvBatchDev &b, const EpochTag &e, bool counts,
                              DeviceCounters *ctr, hipStream_t s, bool zero_counts)
 {
@@ -2884,6 +3195,7 @@ hipError_t launch_kv_execute(const KvState &kv, const KvBatchDev &b, const Epoch
     if (b.n_txns == 0) return zero_counts ? launch_reset_epoch_counters(ctr, s) : hipSuccess;
     const uint64_t ops = (uint64_t)b.n_txns * b.n_slots;
     const dim3 op_grid((unsigned)((ops + kBlock - 1) / kBlock));
+    if (!counts && bin_wanted(kv, b)) return launch_kv_bin(kv, b, e, ctr, s, zero_counts);
     if (kv.partitioned && !counts && kv.part.ent_me) {
         PartArgs a;
         a.keys = b.keys;
@@ -2919,21 +3231,13 @@ hipError_t launch_kv_execute(const KvState &kv, const KvBatchDev &b, const Epoch
         if (slices > kv.part.cap_slices) slices = kv.part.cap_slices;
         hipLaunchKernelGGL(kv_part_count_kernel, chunks, dim3(kPartBlock), 0, s, a, zero_counts);
         hipLaunchKernelGGL(kv_part_scan_kernel, dim3(1), dim3(kPartBlock), 0, s, a);
-        if (kv.max_scan > 1)
-            hipLaunchKernelGGL(kv_part_scatter_kernel, chunks, dim3(kPartBlock), 0, s, a);
-        else if (a.nb <= kPartFewBuckets)
-            hipLaunchKernelGGL((kv_part_scatter_staged_kernel<kPartFewBuckets, 8>),
-                               dim3((unsigned)((ops + 8 * kPartBlock - 1) / (8 * kPartBlock))), dim3(kPartBlock), 0, s,
-                               a);
-        else
-            hipLaunchKernelGGL((kv_part_scatter_staged_kernel<kPartMaxBuckets, 4>),
-                               dim3((unsigned)((ops + 4 * kPartBlock - 1) / (4 * kPartBlock))), dim3(kPartBlock), 0, s,
-                               a);
+        hipLaunchKernelGGL(kv_part_scatter_kernel, chunks, dim3(kPartBlock), 0, s, a);
         hipLaunchKernelGGL(kv_part_process_kernel, dim3((unsigned)slices), dim3(kPartBlock), 0, s, a);
         hipLaunchKernelGGL(kv_part_flags_kernel, dim3((unsigned)slices), dim3(kPartBlock), 0, s, a);
         return hipGetLastError();
     }
-    if (kv.exec_per_op && !counts) {
+    const bool per_op = kv.exec_per_op || (kv.auto_shape && !counts && kv_per_op_auto(ops));
+    if (per_op && !counts) {
         if (kv.more_items)
             hipLaunchKernelGGL(kv_execute_dedup_kernel<4>, dim3((unsigned)((ops + 4 * kBlock - 1) / (4 * kBlock))),
                                dim3(kBlock), 0, s, b.keys, b.meta, b.tids, b.n_txns, b.n_slots, kv.rows, kv.fields,
@@ -2944,7 +3248,7 @@ hipError_t launch_kv_execute(const KvState &kv, const KvBatchDev &b, const Epoch
                                dim3(kBlock), 0, s, b.keys, b.meta, b.tids, b.n_txns, b.n_slots, kv.rows, kv.fields,
                                kv.regs, reg_layout(kv), kv.hot_row, e.tag, kv.doomed, e.epoch, zero_counts,
                                kv.max_scan, ctr, b.request_major);
-    } else if (kv.exec_per_op) {
+    } else if (per_op) {
         hipLaunchKernelGGL(kv_execute_ops_kernel, op_grid, dim3(kBlock), 0, s, b.keys, b.meta, b.tids, b.n_txns,
                            b.n_slots, kv.rows, kv.fields, kv.regs, reg_layout(kv), kv.hot_row, e.tag, kv.doomed,
                            e.epoch, counts, zero_counts, kv.max_scan, ctr, b.request_major);

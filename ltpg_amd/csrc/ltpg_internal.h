@@ -113,6 +113,16 @@ struct KvState {
         unsigned long long *ent_me = nullptr; // [cap_entries] priority of each binned operation
         uint32_t *ent_key = nullptr;          // [cap_entries] row within its bucket << 1 | is-write
     } part;
+    // binned EXECUTE of point operations: buffers of an epoch's entries
+    struct Bin {
+        uint64_t cap_ent = 0, cap_off = 0;
+        uint32_t *ent = nullptr;              // [cap_ent] binned operations, tile by tile
+        uint16_t *off = nullptr;              // [cap_off] starts of each bucket's run in each tile
+        uint32_t *unsorted = nullptr;         // epoch number of the last epoch whose TIDs were out of order
+    } bin;
+    // no launch shape was asked for (ltpg_kv_set_tuning): sizes decide
+    // (kv_bin_auto, kv_per_op_auto)
+    bool auto_shape = true;
     // no kernel has written regs / doomed / raw_flag / war_flag since the
     // last refill ran (the next epoch-tag wrap may skip the refill)
     bool regs_clean = false;
@@ -306,6 +316,8 @@ hipError_t launch_stamp(unsigned long long *out, hipStream_t s);
 // start of a captured batch sequence use it.
 int refill_registers(ltpg_ctx *ctx);
 int kv_part_prepare(ltpg_ctx *ctx);
+// The key-value launch shape a context starts with: no flag, sizes decide.
+void kv_default_shape(ltpg_ctx *ctx);
 hipError_t launch_kv_fill_reference(const KvState &kv, hipStream_t s);
 // rows idx[0 .. n-1] (device, each < kv.rows) of every field, packed, to out (device)
 hipError_t launch_kv_gather_rows(const KvState &kv, const uint64_t *idx, uint64_t n, uint32_t *out, hipStream_t s);
@@ -318,6 +330,17 @@ hipError_t launch_kv_transpose(const uint32_t *src, uint32_t *dst, uint64_t rows
 constexpr uint32_t kPartShift = 13;
 constexpr uint32_t kPartMaxBuckets = 16384;
 constexpr uint32_t kPartSlice = 32768;
+// Binned EXECUTE: at most 2^kBinRowBits rows per bucket and 2^kBinSlotBits op
+// slots per tile (an entry packs both and a bit); "large" epochs.
+constexpr uint32_t kBinRowBits = 14;
+constexpr uint32_t kBinSlotBits = 14;
+constexpr uint64_t kBinLargeOps = 1ull << 22;
+struct BinShape {
+    uint32_t row_bits, buckets, mask, tile_bits, tiles;
+};
+BinShape kv_bin_shape(uint64_t rows, uint64_t ops);
+// Where the binned EXECUTE is the default (kv_kernels.hip).
+bool kv_bin_auto(uint64_t rows, uint64_t ops);
 hipError_t launch_kv_execute(const KvState &kv, const KvBatchDev &b, const EpochTag &e, bool counts,
                              DeviceCounters *ctr, hipStream_t s, bool zero_counts = true);
 hipError_t launch_kv_check(const KvState &kv, const KvBatchDev &b, const EpochTag &e, bool counts,

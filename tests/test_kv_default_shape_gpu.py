@@ -1,0 +1,59 @@
+"""The key-value launch shape a context picks by size, against the oracle at
+the sizes where the pick or its tiles change: the binned EXECUTE (tiles of
+4096 and 16384 op slots) just above its lower bound, with whole and partial
+last tiles, batches narrower and wider than a tile, TIDs in and out of order
+and equal, a hot row, both batch layouts, invalid ops; and the per-op register
+path below it."""
+import numpy as np
+import pytest
+
+import ltpg_amd as L
+from oracle import oracle
+from tests import kvcases as kc
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rows,B,S", [
+    (40_000, 4096, 63),          # below the binned path's 2^18 ops: per-op registers
+    (40_000, 4096, 64),          # exactly 2^18 ops, whole tiles
+    (32_769, 20_003, 14),        # fewest rows, odd batch, partial last tile
+    (70_000, 1_000_001 // 3, 1), # one slot
+    (300_000, 65_539, 64),       # 2^22 ops and more: tiles of 16384
+    (9_000_000, 66_000, 16),     # 1024 buckets of 16384 rows
+], ids=lambda v: str(v))
+@pytest.mark.parametrize("tids", ["ordered", "shuffled", "equal"])
+def test_default_shape_matches_oracle(gpu, rows, B, S, tids):
+    fields, fw = 2, 1
+    rng = np.random.default_rng(B + S)
+    hot = 0 if tids == "equal" else L.NO_HOT_ROW
+    keys, meta, t = L.kv_generate(seed=B, rows=rows, fields=fields, n_txns=B, n_slots=S, min_ops=1, max_ops=S,
+                                  theta=0.9, read_pct=40, distinct_keys=False)
+    if tids == "shuffled":
+        t = rng.permutation(t).astype(np.uint32)
+    elif tids == "equal":
+        t = (t // 5).astype(np.uint32)
+    bad = rng.choice(keys.size, 7, replace=False)
+    keys[bad[:4]] = rows + bad[:4].astype(np.uint64) * (1 << 31)
+    meta[bad[4:]] = L.kv_meta(L.KV_WRITE, fields)
+    table = kc.initial_table(rows, fields, fw)
+    with L.Context(workload=L.WORKLOAD_KV, kv_rows=rows, kv_fields=fields, kv_field_bytes=4 * fw, max_txns=B,
+                   kv_max_slots=S, kv_hot_row=hot) as ctx:
+        ctx.kv_table_load(table)
+        # the first epoch slot-major, the second request-major
+        for request_major in (False, True):
+            k, m = keys, meta
+            if request_major:
+                k, m = (np.ascontiguousarray(a.reshape(S, B).T).reshape(-1) for a in (keys, meta))
+            ctx.kv_submit(k, m, t, S, request_major=request_major)
+            ctx.epoch_run()
+            with pytest.raises(L.LtpgError) as e:
+                ctx.sync()
+            assert e.value.code == L.ERR_RANGE
+            ora = oracle.kv_epoch(table, rows, fields, fw, keys, meta, t, S, inplace=True, hot_row=hot)
+            np.testing.assert_array_equal(ctx.commit_bitmap(), ora.bitmap)
+            com = np.unpackbits(ora.bitmap.view(np.uint8), bitorder="little")[:B].astype(bool)
+            ok = (keys < rows) & (((meta >> 8) & 0xffff) < fields) & ((meta & 3) == L.KV_READ)
+            read = (ok.reshape(S, B) & com).reshape(-1)
+            np.testing.assert_array_equal(ctx.kv_read_values()[read], ora.read_values[read])
+        np.testing.assert_array_equal(ctx.kv_table_read(), table)
