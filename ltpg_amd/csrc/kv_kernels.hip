@@ -36,12 +36,12 @@
 // field_words rounded up to 16 words = 64 bytes for fields of 64 bytes or
 // more, so a 100-byte field touches exactly two 64-byte segments).  A wave
 // moves the fields of its ops cooperatively, each op's addresses fetched from
-// its owner lane by __shfl: in CHECK's read-out and in WRITEBACK, fields of
-// up to 32 words two per instruction (32 lanes per field, wave_copy_pairs)
-// and wider ones G lanes per field (group_copy), or, with the LANE_COPY
-// shape, one lane per field with 16-byte loads (lane_copy); the counting
-// form's read-out LP lanes per op (LP = next power of two >= field_words,
-// at most 64).
+// its owner lane: in CHECK's read-out and in WRITEBACK through a list in LDS,
+// 16 bytes per lane and as many lanes per field as it has 16-byte pieces
+// (stage_flush; fields of less than 16 bytes one lane each), or, with the
+// LANE_COPY shape, one lane per field (lane_copy); in the counting form's
+// read-out LP lanes per op (LP = next power of two >= field_words, at most
+// 64), fetched by __shfl.
 #include "device_common.h"
 #include "ltpg_internal.h"
 
@@ -1340,86 +1340,15 @@ __device__ __forceinline__ uint32_t list_build(bool pick, uint32_t t, uint32_t *
     return n;
 }
 
-// Position of the j-th set bit of m (j < popcount(m)), by halving.
-__device__ __forceinline__ uint32_t nth_set_bit(unsigned long long m, uint32_t j)
-{
-    uint32_t pos = 0;
-#pragma unroll
-    for (uint32_t width = 32; width >= 1; width >>= 1) {
-        const unsigned long long lo = m & ((1ull << width) - 1ull);
-        const uint32_t c = (uint32_t)__popcll(lo);
-        if (j >= c) {
-            j -= c;
-            m >>= width;
-            pos += width;
-        } else {
-            m = lo;
-        }
-    }
-    return pos;
-}
-
-// Field copies of the wave's flagged lanes, fields of at most 32 words, two
-// fields per instruction: lanes 0-31 copy the field of one flagged lane and
-// lanes 32-63 the next, one word per lane, so a 100-byte field is a single
-// coalesced access.  Flagged lane k: src[src_off + w] (+ delta) ->
-// dst[dst_off + w], w < fw.  Up to 32 fields' loads are issued before their
-// stores, which requires that no two flagged fields of one call write the
-// same word (callers guarantee it).
-__device__ __forceinline__ void wave_copy_pairs(unsigned long long mask, uint64_t src_off, uint64_t dst_off,
-                                                uint32_t delta, const uint32_t *src, uint32_t *dst, uint32_t fw)
-{
-    const uint32_t n = (uint32_t)__popcll(mask);
-    const uint32_t half = (uint32_t)lane_id() >> 5, wl = (uint32_t)lane_id() & 31u;
-    for (uint32_t b = 0; b < n; b += 32) {
-        uint32_t v[16], dl[16];
-        uint64_t d[16];
-        bool ok[16];
-#pragma unroll
-        for (uint32_t u = 0; u < 16; ++u) {
-            const uint32_t j = b + 2 * u + half;
-            const bool has = j < n;
-            const int owner = has ? (int)nth_set_bit(mask, j) : 0;
-            const uint64_t so = __shfl(src_off, owner);
-            d[u] = __shfl(dst_off, owner);
-            dl[u] = __shfl(delta, owner);
-            ok[u] = has && wl < fw;
-            // unconditional load (word 0 when idle), so all 16 are in flight
-            v[u] = src[ok[u] ? so + wl : 0ull];
-        }
-#pragma unroll
-        for (uint32_t u = 0; u < 16; ++u)
-            if (ok[u]) dst[d[u] + wl] = v[u] + dl[u];
-    }
-}
-
-// Random-gather ceiling: n fields of fw words, each from a random slot
-// (stride_w words apart) of src, copied to dst[i * fw ..] -- the access
-// pattern of CHECK's read-out -- with wave_copy_pairs, 64 fields per wave
-// step.
-__global__ __launch_bounds__(kBlock) void calib_gather_kernel(const uint32_t *__restrict__ src, uint64_t slots,
-                                                             uint32_t stride_w, uint32_t fw,
-                                                             uint32_t *__restrict__ dst, uint64_t n, uint32_t per)
-{
-    const uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / 64;
-    for (uint32_t k = 0; k < per; ++k) {
-        const uint64_t i = (wave * per + k) * 64 + (uint64_t)lane_id();
-        const bool has = i < n;
-        const uint64_t so = has ? calib_index(i, slots) * stride_w : 0ull;
-        wave_copy_pairs(__ballot(has), so, has ? i * fw : 0ull, 0u, src, dst, fw);
-    }
-}
-
 // Per-wave staging of field copies.  A wave walks its transactions in
 // rounds of 64 / G; a round of a low-contention batch flags only a few
 // fields, and copying them right away leaves a wave with one round's fields
 // in flight.  Instead each round appends its flagged fields (source,
 // destination, delta) to the wave's own LDS list, and the list is copied
-// once it holds 64 or more (or at the end): wave_copy_pairs then has up to 32
-// fields in flight per step, and rounds of op loads run back to back.  The
-// list holds a round's worth more than the flush threshold.  Only the wave
-// that owns a list touches it, so a wavefront-scope fence orders its lanes'
-// LDS accesses.
+// once it holds 64 or more (or at the end), while rounds of op loads run back
+// to back.  The list holds a round's worth more than the flush threshold.
+// Only the wave that owns a list touches it, so a wavefront-scope fence
+// orders its lanes' LDS accesses.
 constexpr uint32_t kStage = 128;
 
 struct StageList {
@@ -1449,20 +1378,90 @@ __device__ __forceinline__ uint32_t stage_push(StageList &l, uint32_t n, bool fl
     return n + (uint32_t)__popcll(m);
 }
 
-// Copy the wave's n staged fields (fw <= 32) and empty the list.  The
-// staged fields never overlap: callers stage distinct destinations.
-__device__ __forceinline__ void stage_flush(StageList &l, uint32_t n, const uint32_t *src, uint32_t *dst,
-                                            uint32_t fw)
+// Four words at any word boundary: one 16-byte access.
+struct __attribute__((packed, aligned(4))) Words4 {
+    uint32_t w[4];
+};
+
+// How a wave copies fields of fw >= 4 words: 2^log_lanes adjacent lanes per
+// field, lane k the words from 4k -- the last one the field's last four words,
+// which overlap its neighbour's (both load them before either stores, and
+// store equal values), so that no access leaves the field.
+struct FieldLanes {
+    uint32_t log_lanes, off;
+    bool on;
+    __device__ explicit FieldLanes(uint32_t fw)
+    {
+        const uint32_t need = (fw + 3) / 4;
+        log_lanes = need <= 1 ? 0u : 32u - (uint32_t)__clz((int)(need - 1));
+        const uint32_t k = (uint32_t)lane_id() & ((1u << log_lanes) - 1u);
+        on = k < need;
+        off = on ? min(4 * k, fw - 4) : 0u;
+    }
+};
+
+// Copy the wave's n staged fields (fw >= 4): src[src_off + w] + delta ->
+// dst[dst_off + w].  The staged fields never overlap: callers stage distinct
+// destinations.  A 100-byte field takes 7 lanes of 8, so an instruction moves
+// eight fields and four steps are in flight.  Bound by the random lines it
+// touches; with 32 lanes of 4 bytes per field and each field's addresses
+// looked up by ballot it was bound by instruction issue (318M vector
+// instructions for the 7M reads of 2^20 transactions of 9 reads and a write).
+__device__ __forceinline__ void stage_flush(StageList &l, uint32_t n, const FieldLanes &f, const uint32_t *src,
+                                            uint32_t *dst)
 {
+    constexpr uint32_t U = 4;
     wave_lds_fence();
-    for (uint32_t b = 0; b < n; b += 64) {
-        const uint32_t e = b + (uint32_t)lane_id();
-        const bool has = e < n;
-        const uint64_t so = has ? l.src[e] : 0ull, d = has ? l.dst[e] : 0ull;
-        const uint32_t dl = has ? l.delta[e] : 0u;
-        wave_copy_pairs(__ballot(has), so, d, dl, src, dst, fw);
+    const uint32_t mine = (uint32_t)lane_id() >> f.log_lanes, per = 64u >> f.log_lanes;
+    for (uint32_t b = 0; b < n; b += U * per) {
+        Words4 v[U];
+        uint64_t d[U];
+        uint32_t dl[U];
+        bool ok[U];
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            const uint32_t e = b + u * per + mine;
+            ok[u] = f.on && e < n;
+            const uint32_t at = ok[u] ? e : 0u;  // idle lanes load the first field, so no load is conditional
+            d[u] = l.dst[at] + f.off;
+            dl[u] = l.delta[at];
+            v[u] = *reinterpret_cast<const Words4 *>(src + l.src[at] + f.off);
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            if (!ok[u]) continue;
+            Words4 w;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) w.w[k] = v[u].w[k] + dl[u];
+            *reinterpret_cast<Words4 *>(dst + d[u]) = w;
+        }
     }
     wave_lds_fence();
+}
+
+// Random-gather ceiling: n fields of fw words, each from a random slot
+// (stride_w words apart) of src, copied to dst[i * fw ..] -- the access
+// pattern of CHECK's read-out -- the way it copies them, 64 fields per wave
+// step.
+__global__ __launch_bounds__(kBlock) void calib_gather_kernel(const uint32_t *__restrict__ src, uint64_t slots,
+                                                             uint32_t stride_w, uint32_t fw,
+                                                             uint32_t *__restrict__ dst, uint64_t n, uint32_t per)
+{
+    __shared__ StageList s_stage[kBlock / 64];
+    StageList &list = s_stage[threadIdx.x / 64];
+    const FieldLanes lanes(fw);
+    const uint64_t wave = ((uint64_t)blockIdx.x * blockDim.x + threadIdx.x) / 64;
+    for (uint32_t k = 0; k < per; ++k) {
+        const uint64_t i = (wave * per + k) * 64 + (uint64_t)lane_id();
+        const bool has = i < n;
+        const uint64_t so = has ? calib_index(i, slots) * stride_w : 0ull;
+        if (fw >= 4) {
+            const uint32_t pending = stage_push(list, 0, has, so, i * fw, 0u);
+            if (pending) stage_flush(list, pending, lanes, src, dst);
+        } else if (has) {
+            for (uint32_t w = 0; w < fw; ++w) dst[i * fw + w] = src[so + w];
+        }
+    }
 }
 
 // One lane copies one field of fw <= 32 words (src_off a multiple of 4
@@ -1495,45 +1494,39 @@ __device__ __forceinline__ void lane_copy(bool active, uint64_t src_off, uint64_
     }
 }
 
-// Field copies of a group's flagged slots.  The op of slot k lives in lane
-// grp * G + k; its field is src[src_off + w] -> dst[dst_off + w] (+ delta),
-// w < fw, and lane gl of the group handles words gl, gl + G, ...  Loads of
-// KB slots are issued before their stores, which requires that no two
-// flagged slots of one call write the same word (callers guarantee it).
-template <int G, int KB>
-__device__ __forceinline__ void group_copy(unsigned long long flags, uint64_t src_off,
-                                           uint64_t dst_off, uint32_t delta, const uint32_t *src,
-                                           uint32_t *dst, uint32_t fw, uint32_t S, uint32_t grp,
-                                           uint32_t gl)
+// Read-out of one op per lane (its rows' fields to the read values of slot
+// position i): fields of 16 bytes and more through the wave's list, whose
+// length it returns; narrower ones each lane its own, four rows' loads in
+// flight.  Every lane of the wave calls it.
+__device__ __forceinline__ uint32_t read_out(const Op &o, uint64_t i, StageList &list, uint32_t pending,
+                                             const FieldLanes &lanes, const uint32_t *table, uint32_t *read_values,
+                                             uint32_t fields, uint32_t fw, uint32_t fsw, uint32_t L)
 {
-    for (uint32_t k0 = 0; k0 < S; k0 += KB) {
-        uint64_t so[KB], dd[KB];
-        uint32_t dl[KB];
-        bool a[KB];
+    const uint64_t src0 = (o.row * fields + o.field) * fsw, step = (uint64_t)fields * fsw, dst0 = i * L * fw;
+    if (fw < 4) {
+        for (uint32_t k0 = 0; k0 < o.len; k0 += 4) {
+            uint32_t v[4][3];
 #pragma unroll
-        for (int u = 0; u < KB; ++u) {
-            const uint32_t k = k0 + u;
-            const int from = (int)(grp * G + (k < (uint32_t)G ? k : 0u));
-            so[u] = __shfl(src_off, from);
-            dd[u] = __shfl(dst_off, from);
-            dl[u] = __shfl(delta, from);
-            a[u] = k < S && ((flags >> from) & 1ull);
+            for (uint32_t u = 0; u < 4; ++u)
+#pragma unroll
+                for (uint32_t w = 0; w < 3; ++w)
+                    v[u][w] = table[(k0 + u < o.len && w < fw) ? src0 + (k0 + u) * step + w : 0ull];
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u)
+#pragma unroll
+                for (uint32_t w = 0; w < 3; ++w)
+                    if (k0 + u < o.len && w < fw) read_values[dst0 + (k0 + u) * fw + w] = v[u][w];
         }
-        bool any = false;
-#pragma unroll
-        for (int u = 0; u < KB; ++u) any |= a[u];
-        if (!__ballot(any)) continue;
-        for (uint32_t w = gl; w < fw; w += G) {
-            uint32_t v[KB];
-            // unconditional loads (inactive slots read word 0) so that all KB
-            // misses are in flight together; only active slots store
-#pragma unroll
-            for (int u = 0; u < KB; ++u) v[u] = src[a[u] ? so[u] + w : 0ull];
-#pragma unroll
-            for (int u = 0; u < KB; ++u)
-                if (a[u]) dst[dd[u] + w] = v[u] + dl[u];
+        return 0;
+    }
+    for (uint32_t k = 0; __ballot(k < o.len); ++k) {  // row k of each read / scan: its own destination
+        pending = stage_push(list, pending, k < o.len, src0 + k * step, dst0 + k * fw, 0u);
+        if (pending >= 64) {
+            stage_flush(list, pending, lanes, table, read_values);
+            pending = 0;
         }
     }
+    return pending;
 }
 
 // CHECK + COMMIT + read-out, fast form (rules as kv_check_counting_kernel).
@@ -1567,7 +1560,8 @@ __global__ __launch_bounds__(kBlock) void kv_check_fast_kernel(
     const uint32_t n = list_build(commit, t0, s_list, s_cnt);
     constexpr uint32_t PER = 64 / G;  // transactions per wave per round
     const uint32_t grp = (uint32_t)lane / G, gl = (uint32_t)lane % G;
-    const bool staged = !per_lane && fw <= 32 && L == 1;
+    StageList &list = s_stage[threadIdx.x / 64];
+    const FieldLanes lanes(fw);
     uint32_t pending = 0;
     for (uint32_t j0 = (blockIdx.y * (kBlock / 64) + threadIdx.x / 64) * PER; j0 < n;
          j0 += gridDim.y * (kBlock / 64) * PER) {
@@ -1576,50 +1570,16 @@ __global__ __launch_bounds__(kBlock) void kv_check_fast_kernel(
         const uint32_t t = has ? s_list[j] : 0u;
         const uint64_t i = (uint64_t)gl * B + t;  // slot-major: where its reads go
         const Op o = load_op(keys, meta, op_at(gl, t, B, S, rm), has && gl < S, rows, fields, max_scan);
-        if (staged) {
-            // every read slot has its own destination
-            pending = stage_push(s_stage[threadIdx.x / 64], pending, o.len != 0, (o.row * fields + o.field) * fsw,
-                                 i * fw, 0u);
-            if (pending >= 64) {
-                stage_flush(s_stage[threadIdx.x / 64], pending, table, read_values, fw);
-                pending = 0;
-            }
-        } else if (per_lane) {
+        if (per_lane) {
             // one lane per read op: all fields of a round in flight at once
             for (uint32_t k = 0; k < o.len; ++k)
                 lane_copy(true, ((o.row + k) * fields + o.field) * fsw, (i * L + k) * fw, 0u, table,
                           read_values, fw);
-        } else if (fw <= 2 && L > 1) {
-            // narrow fields of scans: each lane copies its own rows, four
-            // loads in flight at a time
-            const uint64_t src0 = (o.row * fields + o.field) * fsw, step = (uint64_t)fields * fsw;
-            for (uint32_t k0 = 0; k0 < o.len; k0 += 4) {
-                uint32_t v[4][2];
-#pragma unroll
-                for (uint32_t u = 0; u < 4; ++u)
-#pragma unroll
-                    for (uint32_t w = 0; w < 2; ++w)
-                        v[u][w] = table[(k0 + u < o.len && w < fw) ? src0 + (k0 + u) * step + w : 0ull];
-#pragma unroll
-                for (uint32_t u = 0; u < 4; ++u)
-#pragma unroll
-                    for (uint32_t w = 0; w < 2; ++w)
-                        if (k0 + u < o.len && w < fw) read_values[(i * L + k0 + u) * fw + w] = v[u][w];
-            }
         } else {
-            for (uint32_t k = 0;; ++k) {  // row k of each read / scan
-                const unsigned long long rd = __ballot(k < o.len);
-                if (!rd) break;
-                if (fw <= 32)
-                    wave_copy_pairs(rd, ((o.row + k) * fields + o.field) * fsw, (i * L + k) * fw, 0u, table,
-                                    read_values, fw);
-                else
-                    group_copy<G, 8>(rd, ((o.row + k) * fields + o.field) * fsw, (i * L + k) * fw, 0u, table,
-                                     read_values, fw, S, grp, gl);
-            }
+            pending = read_out(o, i, list, pending, lanes, table, read_values, fields, fw, fsw, L);
         }
     }
-    if (pending) stage_flush(s_stage[threadIdx.x / 64], pending, table, read_values, fw);
+    if (pending) stage_flush(list, pending, lanes, table, read_values);
     if (blockIdx.y != 0) return;  // the chunk's other blocks only read out
     const uint32_t nwords = (B + 63) / 64;
     if (threadIdx.x < CH / 64 && chunk0 / 64 + threadIdx.x < nwords)
@@ -1658,6 +1618,8 @@ __global__ __launch_bounds__(kBlock) void kv_writeback_kernel(
                                   s_list, s_cnt);
     constexpr uint32_t PER = 64 / G;
     const uint32_t grp = (uint32_t)lane / G, gl = (uint32_t)lane % G;
+    StageList &list = s_stage[threadIdx.x / 64];
+    const FieldLanes lanes(fw);
     uint32_t pending = 0;
     for (uint32_t j0 = (blockIdx.y * (kBlock / 64) + threadIdx.x / 64) * PER; j0 < n;
          j0 += gridDim.y * (kBlock / 64) * PER) {
@@ -1686,19 +1648,20 @@ __global__ __launch_bounds__(kBlock) void kv_writeback_kernel(
             lane_copy(wr && first, off, off, step * count, table, table, fw);
             continue;
         }
-        if (fw <= 32) {
-            // a row's committed writer is unique and its duplicate writes
-            // are folded: staged fields never overlap
-            pending = stage_push(s_stage[threadIdx.x / 64], pending, wr && first, off, off, step * count);
-            if (pending >= 64) {
-                stage_flush(s_stage[threadIdx.x / 64], pending, table, table, fw);
-                pending = 0;
-            }
+        if (fw < 4) {
+            if (wr && first)
+                for (uint32_t w = 0; w < fw; ++w) table[off + w] += step * count;
             continue;
         }
-        group_copy<G, 8>(__ballot(wr && first), off, off, step * count, table, table, fw, S, grp, gl);
+        // a row's committed writer is unique and its duplicate writes are
+        // folded: staged fields never overlap
+        pending = stage_push(list, pending, wr && first, off, off, step * count);
+        if (pending >= 64) {
+            stage_flush(list, pending, lanes, table, table);
+            pending = 0;
+        }
     }
-    if (pending) stage_flush(s_stage[threadIdx.x / 64], pending, table, table, fw);
+    if (pending) stage_flush(list, pending, lanes, table, table);
 }
 
 // One small epoch in one workgroup (LTPG_TUNE_SMALL_EPOCH, and the served
