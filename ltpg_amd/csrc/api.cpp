@@ -33,8 +33,10 @@ void free_kv(KvState &kv)
     dev_free(kv.raw_flag);
     dev_free(kv.war_flag);
     dev_free(kv.read_values);
+    dev_free(kv.read_stage);
     dev_free(kv.bitmap);
     dev_free(kv.conflicts);
+    dev_free(kv.commit_list);
     for (int k = 0; k < 2; k++) {
         dev_free(kv.keys_buf[k]);
         dev_free(kv.meta_buf[k]);
@@ -109,9 +111,10 @@ int init_kv(ltpg_ctx *ctx)
     if ((rc = dev_alloc(&kv.doomed, B, "kv doomed flags"))) return rc;
     if ((rc = dev_alloc(&kv.raw_flag, B, "kv raw flags"))) return rc;
     if ((rc = dev_alloc(&kv.war_flag, B, "kv war flags"))) return rc;
-    if ((rc = dev_alloc(&kv.read_values, S * B * kv.read_slot * kv.field_words, "kv read values"))) return rc;
+    if ((rc = dev_alloc(&kv.read_values, S * B * kv.read_slot * kv.field_stride, "kv read values"))) return rc;
     if ((rc = dev_alloc(&kv.bitmap, (B + 63) / 64, "kv bitmap"))) return rc;
     if ((rc = dev_alloc(&kv.conflicts, B, "kv conflicts"))) return rc;
+    if ((rc = dev_alloc(&kv.commit_list, B, "kv commit list"))) return rc;
     if ((rc = dev_alloc(&kv.keys_buf[0], S * B, "kv keys"))) return rc;
     if ((rc = dev_alloc(&kv.meta_buf[0], S * B, "kv meta"))) return rc;
     if ((rc = dev_alloc(&kv.tids_buf[0], B, "kv tids"))) return rc;
@@ -1094,6 +1097,7 @@ int ltpg_epoch_run(ltpg_ctx *ctx, uint32_t phase_mask)
     hipStream_t s = ctx->stream;
     if (kv.small_epoch && phase_mask == LTPG_PHASE_ALL && !ctx->timing &&
         !(ctx->cfg.flags & LTPG_FLAG_CONFLICT_COUNTS) && kv_small_epoch_ok(kv, kv.cur)) {
+        kv.list_valid = false;
         LTPG_HIP_TRY(launch_kv_small_epoch(kv, kv.cur, ctx->cfg.values, ctx->counters, nullptr, nullptr, 0, s));
         return LTPG_OK;
     }
@@ -1105,14 +1109,22 @@ int ltpg_epoch_run(ltpg_ctx *ctx, uint32_t phase_mask)
     }
     // CID has no key-value work: its bracket is empty.
     if (ev) LTPG_HIP_TRY(hipEventRecord(ev[1], s));
-    if (phase_mask & LTPG_PHASE_EXECUTE)
+    if (phase_mask & LTPG_PHASE_EXECUTE) {
+        kv.list_valid = false;  // its length starts over with the counts
         LTPG_HIP_TRY(launch_kv_execute(kv, kv.cur, e, (ctx->cfg.flags & LTPG_FLAG_CONFLICT_COUNTS) != 0,
                                        ctx->counters, s));
+    }
     if (ev) LTPG_HIP_TRY(hipEventRecord(ev[2], s));
     if (phase_mask & LTPG_PHASE_CHECK) {
-        if (!(phase_mask & LTPG_PHASE_EXECUTE)) LTPG_HIP_TRY(launch_reset_epoch_counters(ctx->counters, s));
+        if (!(phase_mask & LTPG_PHASE_EXECUTE)) {
+            kv.list_valid = false;
+            LTPG_HIP_TRY(launch_reset_epoch_counters(ctx->counters, s));
+        }
         LTPG_HIP_TRY(launch_kv_check(kv, kv.cur, e, (ctx->cfg.flags & LTPG_FLAG_CONFLICT_COUNTS) != 0,
                                      ctx->counters, s));
+        // an empty batch's CHECK leaves the bitmap and the list as they were
+        if (kv.cur.n_txns)
+            kv.list_valid = !(ctx->cfg.flags & LTPG_FLAG_CONFLICT_COUNTS) && kv_check_lists(kv, kv.cur);
     }
     if (ev) LTPG_HIP_TRY(hipEventRecord(ev[3], s));
     // Committed reads see the snapshot, so they are delivered before any
@@ -1121,7 +1133,7 @@ int ltpg_epoch_run(ltpg_ctx *ctx, uint32_t phase_mask)
     if ((phase_mask & LTPG_PHASE_WRITEBACK) && (ctx->cfg.flags & LTPG_FLAG_CONFLICT_COUNTS))
         LTPG_HIP_TRY(launch_kv_readout(kv, kv.cur, s));
     if (ev) LTPG_HIP_TRY(hipEventRecord(ev[4], s));
-    if (phase_mask & LTPG_PHASE_WRITEBACK) LTPG_HIP_TRY(launch_kv_writeback(kv, kv.cur, ctx->cfg.values, s));
+    if (phase_mask & LTPG_PHASE_WRITEBACK) LTPG_HIP_TRY(launch_kv_writeback(kv, kv.cur, ctx->cfg.values, ctx->counters, s));
     if (ev) LTPG_HIP_TRY(hipEventRecord(ev[5], s));
     return LTPG_OK;
 }
@@ -1246,7 +1258,24 @@ int ltpg_kv_read_values(ltpg_ctx *ctx, uint32_t *out, uint64_t n_words)
     const uint64_t have = (uint64_t)kv.cur.n_slots * kv.cur.n_txns * kv.read_slot * kv.field_words;
     if (n_words > have) LTPG_FAIL(LTPG_ERR_INVALID, "n_words exceeds the staged read values");
     LTPG_HIP_TRY(hipStreamSynchronize(ctx->stream));
-    if (n_words) LTPG_HIP_TRY(hipMemcpy(out, kv.read_values, n_words * 4, hipMemcpyDeviceToHost));
+    const uint64_t fw = kv.field_words, fsw = kv.field_stride;
+    if (fw == fsw) {
+        if (n_words) LTPG_HIP_TRY(hipMemcpy(out, kv.read_values, n_words * 4, hipMemcpyDeviceToHost));
+        return LTPG_OK;
+    }
+    // packed on the device, part by part
+    const uint64_t n_fields = (n_words + fw - 1) / fw;
+    const uint64_t part = std::min(kReadStageWords / fw,
+                                   (uint64_t)kv.max_slots * ctx->cfg.max_txns * kv.read_slot);
+    if (n_words && !kv.read_stage && (rc = dev_alloc(&kv.read_stage, part * fw, "read value staging"))) return rc;
+    for (uint64_t f = 0; f < n_fields; f += part) {
+        const uint64_t n = std::min(part, n_fields - f);
+        LTPG_HIP_TRY(launch_repack(kv.read_values + f * fsw, kv.read_stage, n, (uint32_t)fw, (uint32_t)fsw, 0,
+                                   ctx->stream));
+        LTPG_HIP_TRY(hipMemcpyAsync(out + f * fw, kv.read_stage, std::min(n * fw, n_words - f * fw) * 4,
+                                    hipMemcpyDeviceToHost, ctx->stream));
+        LTPG_HIP_TRY(hipStreamSynchronize(ctx->stream));
+    }
     return LTPG_OK;
 }
 

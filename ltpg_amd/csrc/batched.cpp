@@ -195,7 +195,8 @@ int enqueue_kv_pipelined(ltpg_batched *b)
         LTPG_HIP_TRY(new_event(b, &done));
         LTPG_HIP_TRY(hipEventRecord(done, main));
         checked.push_back(done);
-        LTPG_HIP_TRY(launch_kv_writeback(st, st.cur, ctx->cfg.values, main));
+        st.list_valid = true;  // of the CHECK above
+        LTPG_HIP_TRY(launch_kv_writeback(st, st.cur, ctx->cfg.values, ctx->counters, main));
         LTPG_HIP_TRY(launch_copy_u64(b->archive + b->off[i], ctx->kv.bitmap, words(d.kv.n_txns), main));
         LTPG_HIP_TRY(launch_stamp(b->stamps + i, main));
         j++;
@@ -228,6 +229,7 @@ int capture(ltpg_batched *b, int k)
     b->final_epoch[k] = ctx->epoch;
     ctx->epoch = epoch;
     ctx->timing = timing;
+    ctx->kv.list_valid = false;  // the capture ran nothing
     if (rc) {
         if (g) (void)hipGraphDestroy(g);
         return rc;
@@ -360,6 +362,7 @@ int ltpg_batched_run(ltpg_batched *b, uint32_t mode)
         // the registers now carry the captured sequence's epoch tags
         b->ctx[k]->epoch = b->final_epoch[k];
         b->ctx[k]->kv.regs_clean = false;
+        b->ctx[k]->kv.list_valid = false;
     }
     int first = LTPG_OK;
     for (int k = 0; k < 2; k++) {

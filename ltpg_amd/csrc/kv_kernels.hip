@@ -42,6 +42,8 @@
 // LANE_COPY shape, one lane per field (lane_copy); in the counting form's
 // read-out LP lanes per op (LP = next power of two >= field_words, at most
 // 64), fetched by __shfl.
+#include <algorithm>
+
 #include "device_common.h"
 #include "ltpg_internal.h"
 
@@ -132,6 +134,14 @@ __device__ __forceinline__ void add_counts(DeviceCounters *ctr, uint32_t stripe,
     if (attempts) atomicAdd(&ctr->totals[stripe][kAttempts + type], (unsigned long long)attempts);
 }
 
+// An epoch's commit counts start at zero (one block calls it).
+__device__ __forceinline__ void zero_epoch_counts(DeviceCounters *ctr, uint32_t threads)
+{
+    for (uint32_t c = threadIdx.x; c < kCounterStripes * kCountedTypes; c += threads)
+        ctr->commits[c / kCountedTypes][c % kCountedTypes] = 0;
+    if (threadIdx.x == 0) ctr->kv_list_n = 0;
+}
+
 // Per-op decode shared by every phase.
 struct Op {
     uint64_t row;
@@ -192,8 +202,7 @@ __device__ __forceinline__ uint32_t txn_of(uint64_t i, uint32_t B, uint32_t S, b
 // epoch can be captured in a graph).
 __global__ void reset_epoch_counters_kernel(DeviceCounters *ctr)
 {
-    for (uint32_t i = threadIdx.x; i < kCounterStripes * kCountedTypes; i += blockDim.x)
-        ctr->commits[i / kCountedTypes][i % kCountedTypes] = 0;
+    zero_epoch_counts(ctr, blockDim.x);
 }
 
 // Streaming 16-byte copy, grid-stride.
@@ -399,9 +408,7 @@ __global__ __launch_bounds__(kBlock) void kv_execute_kernel(
     const uint32_t t = blockIdx.x * kBlock + threadIdx.x;
     const bool live = t < B;
     // the epoch's commit counts start at zero (CHECK adds to them)
-    if (zero_counts && blockIdx.x == 0)
-        for (uint32_t c = threadIdx.x; c < kCounterStripes * kCountedTypes; c += kBlock)
-            ctr->commits[c / kCountedTypes][c % kCountedTypes] = 0;
+    if (zero_counts && blockIdx.x == 0) zero_epoch_counts(ctr, kBlock);
     const unsigned long long me = live ? priority(tag, tids[t], t) : 0ull;
     bool waw = false;
     uint32_t bad = 0;
@@ -431,9 +438,7 @@ __global__ __launch_bounds__(kBlock) void kv_execute_ops_kernel(
     uint8_t *__restrict__ doomed, uint8_t epoch, bool reg_reads, bool zero_counts, uint32_t max_scan,
     DeviceCounters *__restrict__ ctr, bool rm)
 {
-    if (zero_counts && blockIdx.x == 0)
-        for (uint32_t c = threadIdx.x; c < kCounterStripes * kCountedTypes; c += kBlock)
-            ctr->commits[c / kCountedTypes][c % kCountedTypes] = 0;
+    if (zero_counts && blockIdx.x == 0) zero_epoch_counts(ctr, kBlock);
     const uint64_t i = (uint64_t)blockIdx.x * kBlock + threadIdx.x;
     const bool live = i < (uint64_t)S * B;
     const uint32_t t = live ? txn_of(i, B, S, rm) : 0u;
@@ -473,9 +478,7 @@ __global__ __launch_bounds__(kBlock) void kv_execute_dedup_kernel(
     constexpr uint32_t kDedupSlots = 2 * kDedupOps;  // load factor <= 1/2: probing always ends
     __shared__ unsigned long long s_key[kDedupSlots];  // row + 1, 0 = empty
     __shared__ unsigned long long s_min[kDedupSlots];
-    if (zero_counts && blockIdx.x == 0)
-        for (uint32_t c = threadIdx.x; c < kCounterStripes * kCountedTypes; c += kBlock)
-            ctr->commits[c / kCountedTypes][c % kCountedTypes] = 0;
+    if (zero_counts && blockIdx.x == 0) zero_epoch_counts(ctr, kBlock);
     for (uint32_t k = threadIdx.x; k < kDedupSlots; k += kBlock) {
         s_key[k] = 0ull;
         s_min[k] = ~0ull;
@@ -624,9 +627,7 @@ __device__ __forceinline__ void part_load(const PartArgs &a, uint64_t first, Op 
 __global__ __launch_bounds__(kPartBlock) void kv_part_count_kernel(PartArgs a, bool zero_counts)
 {
     __shared__ uint32_t s_hist[kPartMaxBuckets];
-    if (zero_counts && blockIdx.x == 0)
-        for (uint32_t c = threadIdx.x; c < kCounterStripes * kCountedTypes; c += kPartBlock)
-            a.ctr->commits[c / kCountedTypes][c % kCountedTypes] = 0;
+    if (zero_counts && blockIdx.x == 0) zero_epoch_counts(a.ctr, kPartBlock);
     for (uint32_t b = threadIdx.x; b < a.nb; b += kPartBlock) s_hist[b] = 0;
     __syncthreads();
     const uint64_t base = (uint64_t)blockIdx.x * kPartChunk + threadIdx.x;
@@ -979,9 +980,7 @@ __device__ __forceinline__ uint32_t bin_txn(const BinArgs &a, uint32_t i)
 
 __global__ __launch_bounds__(kBlock) void kv_bin_order_kernel(BinArgs a, bool zero_counts)
 {
-    if (zero_counts && blockIdx.x == 0)
-        for (uint32_t c = threadIdx.x; c < kCounterStripes * kCountedTypes; c += kBlock)
-            a.ctr->commits[c / kCountedTypes][c % kCountedTypes] = 0;
+    if (zero_counts && blockIdx.x == 0) zero_epoch_counts(a.ctr, kBlock);
     // four pairs per thread, all loads in flight together
     const uint32_t first = blockIdx.x * (4 * kBlock) + threadIdx.x, last = a.B - 1;
     uint32_t lo[4], hi[4];
@@ -1599,69 +1598,198 @@ __global__ __launch_bounds__(kBlock) void kv_check_fast_kernel(
 // in slot order writes word + count * delta, the others nothing -- the same
 // result as applying them one by one, and it lets every store of a round go
 // out without ordering between them.
+struct WriteArgs {
+    const uint64_t *keys;
+    const uint32_t *meta;
+    const uint32_t *tids;
+    uint32_t B, S;
+    uint64_t rows;
+    uint32_t fields, fw, fsw;
+    uint32_t *table;
+    uint32_t values;
+    uint64_t hot;
+    uint32_t per_lane;
+    bool rm;
+};
+
+// One round of 64 / G transactions, t the lane group's (if has).
+template <int G>
+__device__ __forceinline__ uint32_t write_round(const WriteArgs &a, bool has, uint32_t t, StageList &list,
+                                                uint32_t pending, const FieldLanes &lanes)
+{
+    const uint32_t grp = (uint32_t)lane_id() / G, gl = (uint32_t)lane_id() % G;
+    const uint32_t step = (has && a.values == LTPG_VALUES_RMW) ? (a.tids[t] | 1u) : 0u;
+    const Op o = load_op(a.keys, a.meta, op_at(gl, t, a.B, a.S, a.rm), has && gl < a.S, a.rows, a.fields);
+    // writes to the hot row go through kv_hot_sum_kernel
+    const bool wr = o.valid && o.kind == LTPG_KV_WRITE && o.row != a.hot;
+    const unsigned long long wm = __ballot(wr);
+    if (!wm) return pending;
+    const uint64_t off = (o.row * a.fields + o.field) * a.fsw;
+    // fold duplicates: count this field among the group's write slots
+    uint32_t count = 0;
+    bool first = true;
+    for (uint32_t k = 0; k < a.S && k < (uint32_t)G; ++k) {
+        const int from = (int)(grp * G + k);
+        const uint64_t ok = __shfl(off, from);
+        if (((wm >> from) & 1ull) && ok == off) {
+            ++count;
+            first &= k >= gl;
+        }
+    }
+    if (a.per_lane) {
+        lane_copy(wr && first, off, off, step * count, a.table, a.table, a.fw);
+        return pending;
+    }
+    if (a.fw < 4) {
+        if (wr && first)
+            for (uint32_t w = 0; w < a.fw; ++w) a.table[off + w] += step * count;
+        return pending;
+    }
+    // a row's committed writer is unique and its duplicate writes are
+    // folded: staged fields never overlap
+    pending = stage_push(list, pending, wr && first, off, off, step * count);
+    if (pending >= 64) {
+        stage_flush(list, pending, lanes, a.table, a.table);
+        pending = 0;
+    }
+    return pending;
+}
+
 template <int G, int CH>
-__global__ __launch_bounds__(kBlock) void kv_writeback_kernel(
-    const uint64_t *__restrict__ keys, const uint32_t *__restrict__ meta,
-    const uint32_t *__restrict__ tids, uint32_t B, uint32_t S, uint64_t rows, uint32_t fields,
-    uint32_t fw, uint32_t fsw, uint32_t *__restrict__ table, const uint64_t *__restrict__ bitmap,
-    uint32_t values, uint64_t hot, uint32_t per_lane, bool rm)
+__global__ __launch_bounds__(kBlock) void kv_writeback_kernel(WriteArgs a, const uint64_t *__restrict__ bitmap)
 {
     __shared__ uint32_t s_list[CH];
     __shared__ uint32_t s_cnt[kBlock / 64];
     __shared__ StageList s_stage[kBlock / 64];
-    const int lane = lane_id();
-    const uint32_t chunk0 = blockIdx.x * CH;
-    const uint32_t t0 = chunk0 + threadIdx.x;
+    const uint32_t t0 = blockIdx.x * CH + threadIdx.x;
     // t0 < B also guards a bitmap word left by an earlier, larger batch
     // when this phase runs without a fresh CHECK
-    const uint32_t n = list_build(threadIdx.x < CH && t0 < B && ((bitmap[t0 / 64] >> (t0 % 64)) & 1ull), t0,
+    const uint32_t n = list_build(threadIdx.x < CH && t0 < a.B && ((bitmap[t0 / 64] >> (t0 % 64)) & 1ull), t0,
                                   s_list, s_cnt);
     constexpr uint32_t PER = 64 / G;
-    const uint32_t grp = (uint32_t)lane / G, gl = (uint32_t)lane % G;
+    const uint32_t grp = (uint32_t)lane_id() / G;
     StageList &list = s_stage[threadIdx.x / 64];
-    const FieldLanes lanes(fw);
+    const FieldLanes lanes(a.fw);
     uint32_t pending = 0;
     for (uint32_t j0 = (blockIdx.y * (kBlock / 64) + threadIdx.x / 64) * PER; j0 < n;
          j0 += gridDim.y * (kBlock / 64) * PER) {
-        const uint32_t j = j0 + grp;
-        const bool has = j < n;
-        const uint32_t t = has ? s_list[j] : 0u;
-        const uint32_t step = (has && values == LTPG_VALUES_RMW) ? (tids[t] | 1u) : 0u;
-        const Op o = load_op(keys, meta, op_at(gl, t, B, S, rm), has && gl < S, rows, fields);
-        // writes to the hot row go through kv_hot_sum_kernel
-        const bool wr = o.valid && o.kind == LTPG_KV_WRITE && o.row != hot;
-        const unsigned long long wm = __ballot(wr);
-        if (!wm) continue;
-        const uint64_t off = (o.row * fields + o.field) * fsw;
-        // fold duplicates: count this field among the group's write slots
-        uint32_t count = 0;
-        bool first = true;
-        for (uint32_t k = 0; k < S && k < (uint32_t)G; ++k) {
-            const int from = (int)(grp * G + k);
-            const uint64_t ok = __shfl(off, from);
-            if (((wm >> from) & 1ull) && ok == off) {
-                ++count;
-                first &= k >= gl;
-            }
+        const bool has = j0 + grp < n;
+        pending = write_round<G>(a, has, has ? s_list[j0 + grp] : 0u, list, pending, lanes);
+    }
+    if (pending) stage_flush(list, pending, lanes, a.table, a.table);
+}
+
+// ---- the committed transactions of a large batch as one list ---------------
+//
+// Commits crowd among the lowest priorities, so with a block per 256
+// transactions a few blocks do nearly all of an epoch's field copies.  For
+// batches of kListTxns transactions and more CHECK decides every transaction
+// first and lists the committed ones (kv_commit_list_kernel); the read-out and
+// WRITEBACK then share that list evenly over the whole chip.  2^20
+// transactions x 16 ops on 100-byte fields, 3.5 % committed: CHECK 64 -> 7 + 29
+// us, WRITEBACK 74 -> 27 us.  With 81 % committed (9 reads, 1 write): CHECK 662
+// -> 7 + 441 us, which is the rate of random 128-byte reads and whole writes
+// (3.6 TB/s; the gather alone reaches 4.2), WRITEBACK 148 -> 176 us.
+constexpr uint32_t kListBlock = 1024, kListPer = 4;  // transactions per block and thread
+
+__global__ __launch_bounds__(kListBlock) void kv_commit_list_kernel(
+    uint32_t B, const uint8_t *__restrict__ doomed, const uint8_t *__restrict__ raw_flag,
+    const uint8_t *__restrict__ war_flag, uint8_t epoch, uint64_t *__restrict__ bitmap, uint32_t *__restrict__ list,
+    DeviceCounters *__restrict__ ctr)
+{
+    constexpr uint32_t kWaves = kListBlock / 64;
+    __shared__ uint32_t s_cnt[kListPer * kWaves], s_base;
+    const uint32_t first = blockIdx.x * (kListPer * kListBlock), wave = threadIdx.x / 64;
+    unsigned long long m[kListPer];
+#pragma unroll
+    for (uint32_t r = 0; r < kListPer; ++r) {
+        const uint32_t t = first + r * kListBlock + threadIdx.x, j = t < B ? t : 0u;
+        const uint8_t d = doomed[j], ra = raw_flag[j], wa = war_flag[j];
+        m[r] = __ballot(t < B && d != epoch && !(ra == epoch && wa == epoch));
+    }
+#pragma unroll
+    for (uint32_t r = 0; r < kListPer; ++r) {
+        if (lane_id() != 0) continue;
+        const uint32_t t = first + r * kListBlock + wave * 64;
+        if (t < B) bitmap[t / 64] = m[r];
+        s_cnt[r * kWaves + wave] = (uint32_t)__popcll(m[r]);
+    }
+    __syncthreads();
+    if (wave == 0) {
+        const uint32_t c = s_cnt[lane_id()];
+        uint32_t inc = c;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t x = __shfl_up(inc, d);
+            if (lane_id() >= d) inc += x;
         }
-        if (per_lane) {
-            lane_copy(wr && first, off, off, step * count, table, table, fw);
-            continue;
-        }
-        if (fw < 4) {
-            if (wr && first)
-                for (uint32_t w = 0; w < fw; ++w) table[off + w] += step * count;
-            continue;
-        }
-        // a row's committed writer is unique and its duplicate writes are
-        // folded: staged fields never overlap
-        pending = stage_push(list, pending, wr && first, off, off, step * count);
-        if (pending >= 64) {
-            stage_flush(list, pending, lanes, table, table);
-            pending = 0;
+        s_cnt[lane_id()] = inc - c;
+        if (lane_id() == 63) {
+            const uint32_t left = B - first, live = left < kListPer * kListBlock ? left : kListPer * kListBlock;
+            s_base = inc ? atomicAdd(&ctr->kv_list_n, inc) : 0u;
+            add_counts(ctr, blockIdx.x % kCounterStripes, LTPG_TYPE_KV, inc, live);
         }
     }
-    if (pending) stage_flush(list, pending, lanes, table, table);
+    __syncthreads();
+#pragma unroll
+    for (uint32_t r = 0; r < kListPer; ++r)
+        if ((m[r] >> lane_id()) & 1ull)
+            list[s_base + s_cnt[r * kWaves + wave] + (uint32_t)__popcll(m[r] & ((1ull << lane_id()) - 1ull))] =
+                first + r * kListBlock + threadIdx.x;
+}
+static_assert(kListPer * kListBlock / 64 == 64, "one wave scans the counts");
+
+// Read-out of the listed transactions.  Slot-major batches: a wave takes one
+// slot of 64 consecutive entries, whose op loads and read values are nearly
+// consecutive; request-major ones: 64 consecutive op slots.
+__global__ __launch_bounds__(kBlock) void kv_readout_list_kernel(
+    const uint64_t *__restrict__ keys, const uint32_t *__restrict__ meta, uint32_t B, uint32_t S, uint64_t rows,
+    uint32_t fields, uint32_t fw, uint32_t fsw, const uint32_t *__restrict__ table, uint32_t *__restrict__ read_values,
+    const uint32_t *__restrict__ commits, const DeviceCounters *__restrict__ ctr, uint32_t max_scan, uint32_t L, bool rm)
+{
+    __shared__ StageList s_stage[kBlock / 64];
+    StageList &list = s_stage[threadIdx.x / 64];
+    const FieldLanes lanes(fw);
+    const uint32_t n = ctr->kv_list_n;
+    const uint32_t chunks = (n + 63) / 64;
+    const uint32_t units = rm ? (n * S + 63) / 64 : chunks * S;  // n * S <= 2^30
+    uint32_t pending = 0;
+    for (uint32_t u = blockIdx.x * (kBlock / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x / 64); u < units;
+         u += gridDim.x * (kBlock / 64)) {
+        uint32_t j, s;
+        if (rm) {
+            const uint32_t f = u * 64 + (uint32_t)lane_id();
+            j = f / S;
+            s = f - j * S;
+        } else {
+            s = u / chunks;
+            j = (u - s * chunks) * 64 + (uint32_t)lane_id();
+        }
+        const uint32_t t = commits[j < n ? j : 0u];
+        const Op o = load_op(keys, meta, op_at(s, t, B, S, rm), j < n, rows, fields, max_scan);
+        pending = read_out(o, (uint64_t)s * B + t, list, pending, lanes, table, read_values, fields, fw, fsw, L);
+    }
+    if (pending) stage_flush(list, pending, lanes, table, read_values);
+}
+
+// WRITEBACK of the listed transactions, 64 / G per round; entries beyond a
+// smaller current batch (the phase without a fresh CHECK) are left out.
+template <int G>
+__global__ __launch_bounds__(kBlock) void kv_writeback_list_kernel(WriteArgs a, const uint32_t *__restrict__ commits,
+                                                                  const DeviceCounters *__restrict__ ctr)
+{
+    __shared__ StageList s_stage[kBlock / 64];
+    StageList &list = s_stage[threadIdx.x / 64];
+    const FieldLanes lanes(a.fw);
+    constexpr uint32_t PER = 64 / G;
+    const uint32_t n = ctr->kv_list_n, grp = (uint32_t)lane_id() / G;
+    uint32_t pending = 0;
+    for (uint32_t j0 = (blockIdx.x * (kBlock / 64) + threadIdx.x / 64) * PER; j0 < n;
+         j0 += gridDim.x * (kBlock / 64) * PER) {
+        const uint32_t t = j0 + grp < n ? commits[j0 + grp] : a.B;
+        pending = write_round<G>(a, t < a.B, t < a.B ? t : 0u, list, pending, lanes);
+    }
+    if (pending) stage_flush(list, pending, lanes, a.table, a.table);
 }
 
 // One small epoch in one workgroup (LTPG_TUNE_SMALL_EPOCH, and the served
@@ -1865,7 +1993,7 @@ __global__ __launch_bounds__(kSmallBlock) void kv_small_epoch_kernel(
         const Op o = decode_op(s_row[i], s_meta[i], rows, fields, max_scan);
         const bool ok = q < o.len;
         src = ok ? ((o.row + q) * fields + o.field) * fsw + w : 0ull;
-        dst = ((((uint64_t)sl * B + t) * L) + q) * fw + w;
+        dst = ((((uint64_t)sl * B + t) * L) + q) * fsw + w;
         return ok;
     };
     const auto write_item = [&](uint32_t x, uint64_t &off, uint32_t &add) -> bool {
@@ -3274,6 +3402,21 @@ static uint32_t lane_copy_ok(const KvState &kv)
     return kv.lane_copy && kv.field_stride % 4 == 0 && kv.field_words <= 32 ? 1u : 0u;
 }
 
+// The list costs one more kernel: 10 blocks' worth of short chunks run as fast
+// in one (10,000 transactions: 13 us as one kernel, 5 + 9 as two).
+constexpr uint32_t kListTxns = 1u << 15;
+constexpr uint32_t kListBlocks = 2048;  // 8 per CU: what the copies' registers allow to be resident
+
+bool kv_check_lists(const KvState &kv, const KvBatchDev &b)
+{
+    return kv.commit_list && b.n_txns >= kListTxns && !kv.small_chunks && !kv.lane_copy;
+}
+
+// Read values and written fields are moved whole, padding included: fields of
+// 64 bytes and more then leave as whole 64-byte segments of memory, where a
+// partly written segment costs a read at the memory side (8.1M reads of 100
+// bytes with every seventh slot left out: 597 us packed, 432 us for 7.7M
+// fields of 128 bytes).  Nothing reads the padding.
 hipError_t launch_kv_check(const KvState &kv, const KvBatchDev &b, const EpochTag &e, bool counts,
                            DeviceCounters *ctr, hipStream_t s)
 {
@@ -3284,9 +3427,20 @@ hipError_t launch_kv_check(const KvState &kv, const KvBatchDev &b, const EpochTa
                            kv.hot_row, e.tag, kv.bitmap, kv.conflicts, kv.max_scan, ctr, b.request_major);
         return hipGetLastError();
     }
+    if (kv_check_lists(kv, b)) {
+        hipLaunchKernelGGL(kv_commit_list_kernel,
+                           dim3((b.n_txns + kListPer * kListBlock - 1) / (kListPer * kListBlock)), dim3(kListBlock), 0,
+                           s, b.n_txns, kv.doomed, kv.raw_flag, kv.war_flag, e.epoch, kv.bitmap, kv.commit_list, ctr);
+        const uint64_t units = ((uint64_t)b.n_txns + 63) / 64 * b.n_slots, per = kBlock / 64;
+        const uint64_t blocks = std::min<uint64_t>(kListBlocks, (units + per - 1) / per);
+        hipLaunchKernelGGL(kv_readout_list_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, s, b.keys, b.meta, b.n_txns,
+                           b.n_slots, kv.rows, kv.fields, kv.field_stride, kv.field_stride, kv.table, kv.read_values,
+                           kv.commit_list, ctr, kv.max_scan, kv.read_slot, b.request_major);
+        return hipGetLastError();
+    }
 #define CALL1(GV, CHV)                                                                               \
     hipLaunchKernelGGL((kv_check_fast_kernel<GV, CHV>), grid_chunks(b.n_txns, CHV, GV), dim3(kBlock), 0, s, b.keys, \
-                       b.meta, b.n_txns, b.n_slots, kv.rows, kv.fields, kv.field_words, kv.field_stride,   \
+                       b.meta, b.n_txns, b.n_slots, kv.rows, kv.fields, kv.field_stride, kv.field_stride,   \
                        kv.doomed, kv.raw_flag, kv.war_flag, e.epoch, kv.table, kv.read_values, kv.bitmap,  \
                        kv.max_scan, kv.read_slot, lane_copy_ok(kv), ctr, b.request_major)
 #define CALL(GV)                    \
@@ -3303,33 +3457,43 @@ hipError_t launch_kv_check(const KvState &kv, const KvBatchDev &b, const EpochTa
 hipError_t launch_kv_readout(const KvState &kv, const KvBatchDev &b, hipStream_t s)
 {
     if (b.n_txns == 0) return hipSuccess;
-    const int lp = lanes_for(kv.field_words);
+    const int lp = lanes_for(kv.field_stride);
 #define CALL(LPV)                                                                          \
     hipLaunchKernelGGL(kv_readout_kernel<LPV>, grid_for(b.n_txns), dim3(kBlock), 0, s,    \
                        b.keys, b.meta, b.n_txns, b.n_slots, kv.rows, kv.fields,           \
-                       kv.field_words, kv.field_stride, kv.table, kv.bitmap, kv.read_values, kv.max_scan, \
+                       kv.field_stride, kv.field_stride, kv.table, kv.bitmap, kv.read_values, kv.max_scan, \
                        kv.read_slot, b.request_major)
     LTPG_LP_SWITCH(lp, CALL)
 #undef CALL
     return hipGetLastError();
 }
 
-hipError_t launch_kv_writeback(const KvState &kv, const KvBatchDev &b, uint32_t values,
+hipError_t launch_kv_writeback(const KvState &kv, const KvBatchDev &b, uint32_t values, DeviceCounters *ctr,
                                hipStream_t s)
 {
     if (b.n_txns == 0) return hipSuccess;
+    const WriteArgs a = {b.keys,          b.meta,          b.tids,   b.n_txns,   b.n_slots, kv.rows,
+                         kv.fields,       kv.field_stride, kv.field_stride, kv.table,   values,    kv.hot_row,
+                         lane_copy_ok(kv), b.request_major};
+    const int g = group_for(b.n_slots);
+    if (kv.list_valid && kv_check_lists(kv, b)) {
+        const uint64_t per = (kBlock / 64) * (64 / g);  // transactions per block and round
+        const dim3 grid((unsigned)std::min<uint64_t>(kListBlocks, (b.n_txns + per - 1) / per));
+#define CALL(GV) hipLaunchKernelGGL(kv_writeback_list_kernel<GV>, grid, dim3(kBlock), 0, s, a, kv.commit_list, ctr)
+        LTPG_G_SWITCH(g, CALL)
+#undef CALL
+    } else {
 #define CALL1(GV, CHV)                                                                                      \
-    hipLaunchKernelGGL((kv_writeback_kernel<GV, CHV>), grid_chunks(b.n_txns, CHV, GV), dim3(kBlock), 0, s, b.keys, \
-                       b.meta, b.tids, b.n_txns, b.n_slots, kv.rows, kv.fields, kv.field_words,             \
-                       kv.field_stride, kv.table, kv.bitmap, values, kv.hot_row, lane_copy_ok(kv), b.request_major)
+    hipLaunchKernelGGL((kv_writeback_kernel<GV, CHV>), grid_chunks(b.n_txns, CHV, GV), dim3(kBlock), 0, s, a, kv.bitmap)
 #define CALL(GV)         \
     if (kv.small_chunks) \
         CALL1(GV, 64);   \
     else                 \
         CALL1(GV, kChunk)
-    LTPG_G_SWITCH(group_for(b.n_slots), CALL)
+        LTPG_G_SWITCH(g, CALL)
 #undef CALL
 #undef CALL1
+    }
     if (kv.hot_row != LTPG_NO_HOT_ROW && values == LTPG_VALUES_RMW) {
         hipLaunchKernelGGL(kv_hot_sum_kernel, grid_for(b.n_txns), dim3(kBlock), 0, s, b.keys, b.meta, b.tids,
                            b.n_txns, b.n_slots, kv.rows, kv.fields, kv.hot_row, kv.bitmap, kv.hot_acc,

@@ -40,7 +40,8 @@ constexpr uint32_t kCountedTypes = 6;  // LTPG_TYPE_KV .. LTPG_TYPE_DELIVERY
 
 struct DeviceCounters {
     uint32_t range_errors;                            // ops outside their table
-    uint32_t pad0[63];
+    uint32_t kv_list_n;                               // length of KvState::commit_list
+    uint32_t pad0[62];
     uint32_t commits[kCounterStripes][64];            // [stripe][type]: last epoch
     unsigned long long totals[kCounterStripes][32];   // [stripe][type]: commits,
                                                       // [stripe][kAttempts + type]: attempts
@@ -78,9 +79,12 @@ struct KvState {
     uint8_t *doomed = nullptr;          // max_txns: epoch number if waw > 0
     uint8_t *raw_flag = nullptr;        // max_txns: epoch number if a read found a lower W (fast form)
     uint8_t *war_flag = nullptr;        // max_txns: epoch number if a lower reader hit its W (fast form)
-    uint32_t *read_values = nullptr;    // max_slots * max_txns * field_words
+    uint32_t *read_values = nullptr;    // max_slots * max_txns * read_slot fields, field_stride words each
+    uint32_t *read_stage = nullptr;     // packed part of the read values on its way to the host
     uint64_t *bitmap = nullptr;         // ceil(max_txns / 64)
     uint32_t *conflicts = nullptr;      // max_txns
+    uint32_t *commit_list = nullptr;    // max_txns: the committed transactions of the last list CHECK
+    bool list_valid = false;            // commit_list lists the same transactions as bitmap
     // library-owned copies of host-submitted batches: two slots, so that
     // the next batch's copy overlaps the current epoch (slot 1 allocated at
     // its first use)
@@ -325,6 +329,8 @@ hipError_t launch_repack(const uint32_t *src, uint32_t *dst, uint64_t n_fields, 
                          uint32_t fsw, int to_strided, hipStream_t s);
 hipError_t launch_kv_transpose(const uint32_t *src, uint32_t *dst, uint64_t rows, uint32_t cols,
                                int to_row_major, hipStream_t s);
+// Words of KvState::read_stage at most.
+constexpr uint64_t kReadStageWords = 8ull << 20;
 // Row-partitioned EXECUTE limits: rows per bucket (1 << kPartShift), buckets,
 // and operations per slice (one workgroup).
 constexpr uint32_t kPartShift = 13;
@@ -345,8 +351,12 @@ hipError_t launch_kv_execute(const KvState &kv, const KvBatchDev &b, const Epoch
                              DeviceCounters *ctr, hipStream_t s, bool zero_counts = true);
 hipError_t launch_kv_check(const KvState &kv, const KvBatchDev &b, const EpochTag &e, bool counts,
                            DeviceCounters *ctr, hipStream_t s);
+// Whether the fast CHECK of this batch lists its committed transactions.
+bool kv_check_lists(const KvState &kv, const KvBatchDev &b);
 hipError_t launch_kv_readout(const KvState &kv, const KvBatchDev &b, hipStream_t s);
-hipError_t launch_kv_writeback(const KvState &kv, const KvBatchDev &b, uint32_t values,
+// Takes the committed transactions from commit_list if kv.list_valid, else
+// from the bitmap.
+hipError_t launch_kv_writeback(const KvState &kv, const KvBatchDev &b, uint32_t values, DeviceCounters *ctr,
                                hipStream_t s);
 // A whole fast-form epoch of at most LTPG_SMALL_EPOCH_OPS op slots in one
 // single-workgroup kernel (a hot row only with at most 1024 fields; rows <

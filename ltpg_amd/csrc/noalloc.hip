@@ -118,7 +118,7 @@ extern "C" int ltpg_kv_epoch_noalloc(uint32_t *table, uint64_t rows, uint32_t fi
         e.tag = 254;
         LTPG_HIP_TRY(launch_kv_execute(kv, b, e, false, ctr, s));
         LTPG_HIP_TRY(launch_kv_check(kv, b, e, false, ctr, s));
-        LTPG_HIP_TRY(launch_kv_writeback(kv, b, values, s));
+        LTPG_HIP_TRY(launch_kv_writeback(kv, b, values, ctr, s));
     }
     if (result) {
         hipLaunchKernelGGL(noalloc_result_kernel, dim3(1), dim3(64), 0, s, ctr, result);

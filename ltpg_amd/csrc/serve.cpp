@@ -598,6 +598,7 @@ int launch(ltpg_server *sv, int w, Flight &f)
             if ((rc = ltpg_kv_submit(ctx, &b, LTPG_MEM_DEVICE | LTPG_BATCH_REQUEST_MAJOR))) return rc;
             published = !sv->cfg.keep_reads;
             const uint64_t seq = published ? ++f.seq : 0;
+            ctx->kv.list_valid = false;
             LTPG_HIP_TRY(launch_kv_small_epoch(ctx->kv, ctx->kv.cur, ctx->cfg.values, ctx->counters,
                                                published ? f.h_bits : nullptr, published ? f.h_seq : nullptr, seq,
                                                ctx->stream));
@@ -611,10 +612,15 @@ int launch(ltpg_server *sv, int w, Flight &f)
             if ((rc = ltpg_kv_submit(ctx, &b, LTPG_MEM_DEVICE | LTPG_BATCH_REQUEST_MAJOR))) return rc;
             if ((rc = ltpg_epoch_run(ctx, LTPG_PHASE_ALL))) return rc;
         }
-        if (sv->cfg.keep_reads)
-            LTPG_HIP_TRY(hipMemcpyAsync(f.h_reads, ctx->kv.read_values,
-                                        (uint64_t)S * B * ctx->kv.read_slot * ctx->kv.field_words * 4,
-                                        hipMemcpyDeviceToHost, ctx->stream));
+        if (sv->cfg.keep_reads) {
+            const uint64_t n = (uint64_t)S * B * ctx->kv.read_slot;
+            const uint32_t fw = ctx->kv.field_words, fsw = ctx->kv.field_stride;
+            if (fw == fsw)
+                LTPG_HIP_TRY(hipMemcpyAsync(f.h_reads, ctx->kv.read_values, n * fw * 4, hipMemcpyDeviceToHost,
+                                            ctx->stream));
+            else  // packed into the pinned staging by a kernel
+                LTPG_HIP_TRY(launch_repack(ctx->kv.read_values, f.h_reads, n, fw, fsw, 0, ctx->stream));
+        }
         if (!published) {
             PublishSet ps{{ctx->kv.bitmap, nullptr, nullptr, nullptr}, {f.h_bits, nullptr, nullptr, nullptr},
                           {(uint32_t)words(B), 0, 0, 0}};

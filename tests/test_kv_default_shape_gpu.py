@@ -57,3 +57,48 @@ def test_default_shape_matches_oracle(gpu, rows, B, S, tids):
             read = (ok.reshape(S, B) & com).reshape(-1)
             np.testing.assert_array_equal(ctx.kv_read_values()[read], ora.read_values[read])
         np.testing.assert_array_equal(ctx.kv_table_read(), table)
+
+
+@pytest.mark.parametrize("B", [32_767, 32_768, 36_865])
+@pytest.mark.parametrize("fw,scan", [(3, 0), (4, 0), (5, 3), (17, 0), (25, 0), (33, 3)])
+def test_commit_list_matches_oracle(gpu, B, fw, scan):
+    """CHECK's list of committed transactions (batches of 32,768 and more) and
+    the field copies from it: list blocks of 4096 with a remainder of one,
+    fields of one lane, whole and overlapping 16-byte pieces, padded and
+    unpadded rows, scans; the phases in one call and one by one; read values
+    read back in whole and cut inside a field."""
+    rows, fields, S = 50_000, 2, 4
+    keys, meta, t = L.kv_generate(seed=B + fw, rows=rows, fields=fields, n_txns=B, n_slots=S, min_ops=1, max_ops=S,
+                                  theta=0.3, read_pct=60, scan_len=scan, distinct_keys=False)
+    if scan:
+        keys[::97] = rows - 2  # clipped at the end of the table
+    table = kc.initial_table(rows, fields, fw)
+    with L.Context(workload=L.WORKLOAD_KV, kv_rows=rows, kv_fields=fields, kv_field_bytes=4 * fw, max_txns=B,
+                   kv_max_slots=S, kv_max_scan=scan) as ctx:
+        ctx.kv_table_load(table)
+        for ep, steps in enumerate([[L.PHASE_ALL], [L.PHASE_EXECUTE, L.PHASE_CHECK, L.PHASE_WRITEBACK],
+                                    [L.PHASE_EXECUTE | L.PHASE_CHECK, L.PHASE_WRITEBACK]]):
+            k, m = keys, meta
+            if ep == 1:
+                k, m = (np.ascontiguousarray(a.reshape(S, B).T).reshape(-1) for a in (keys, meta))
+            ctx.kv_submit(k, m, t, S, request_major=ep == 1)
+            for phases in steps:
+                ctx.epoch_run(phases)
+            ctx.sync()
+            ora = oracle.kv_epoch(table, rows, fields, fw, keys, meta, t, S, inplace=True, max_scan=scan)
+            np.testing.assert_array_equal(ctx.commit_bitmap(), ora.bitmap)
+            assert ctx.commit_count() == ora.commit_count
+            com = np.unpackbits(ora.bitmap.view(np.uint8), bitorder="little")[:B].astype(bool)
+            n = max(1, scan)
+            kinds = (meta & 3).astype(np.int64)
+            lens = np.where(kinds == 3, (meta >> 24).astype(np.int64) + 1, (kinds == 1).astype(np.int64))
+            row = np.arange(n)[None, :]
+            read = (row < lens[:, None]) & ((keys.astype(np.int64)[:, None] + row) < rows)
+            read &= np.tile(com, S)[:, None]
+            got = ctx.kv_read_values()
+            np.testing.assert_array_equal(got.reshape(-1, fw)[read.reshape(-1)],
+                                          ora.read_values.reshape(-1, fw)[read.reshape(-1)])
+            part = np.zeros(7 * fw + 1, np.uint32)
+            assert L.lib.ltpg_kv_read_values(ctx.handle, part.ctypes.data_as(L._lib.c_u32p), part.size) == L.OK
+            np.testing.assert_array_equal(part, got[:part.size])
+        np.testing.assert_array_equal(ctx.kv_table_read(), table)
