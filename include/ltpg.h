@@ -794,7 +794,7 @@ int ltpg_serve_cancel(ltpg_server *sv, uint64_t *dropped);
  * caller-owned device table, with the same kernels and results as
  * ltpg_epoch_run on a context.  It calls no allocator: the per-row registers,
  * per-transaction flags and counters live in a fixed device array of the
- * library (about 19 MB, held by each GPU it runs on until the process ends).
+ * library (about 93 MB, held by each GPU it runs on until the process ends).
  *   table        device, rows x fields x field_bytes, row-major, packed;
  *                updated in place (RMW: a write adds TID | 1 to each word)
  *   batch        device arrays, slot-major (slot s of txn t at s*B + t)

@@ -978,9 +978,19 @@ __device__ __forceinline__ uint32_t bin_txn(const BinArgs &a, uint32_t i)
     return a.rm ? q : r;
 }
 
-__global__ __launch_bounds__(kBlock) void kv_bin_order_kernel(BinArgs a, bool zero_counts)
+// With `clear` (the epoch that keeps no state between calls) also the flags of
+// the block's transactions and the range errors start over.
+__global__ __launch_bounds__(kBlock) void kv_bin_order_kernel(BinArgs a, bool zero_counts, bool clear)
 {
     if (zero_counts && blockIdx.x == 0) zero_epoch_counts(a.ctr, kBlock);
+    if (clear) {
+        if (blockIdx.x == 0 && threadIdx.x == 0) a.ctr->range_errors = 0;
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) {
+            const uint32_t t = blockIdx.x * (4 * kBlock) + u * kBlock + threadIdx.x;
+            if (t < a.B) a.doomed[t] = a.raw_flag[t] = a.war_flag[t] = 0;
+        }
+    }
     // four pairs per thread, all loads in flight together
     const uint32_t first = blockIdx.x * (4 * kBlock) + threadIdx.x, last = a.B - 1;
     uint32_t lo[4], hi[4];
@@ -1803,7 +1813,8 @@ __global__ __launch_bounds__(kBlock) void kv_writeback_list_kernel(WriteArgs a, 
 // which this path never touches.  The batch may sit in pinned host memory
 // (read once).  With seq_out the commit bitmap is also written to host_bits
 // and then seq is stored there with a system-scope release, as
-// publish_kernel does after a multi-kernel epoch.  A hot row (at most
+// publish_kernel does after a multi-kernel epoch.  With result the commit count
+// and the range errors go there instead of the counters.  A hot row (at most
 // kSmallHotFields fields) never registers or conflicts, and its committed
 // deltas are summed per field in LDS and added to the row with the other
 // writes; rows < 2^32 - 1.
@@ -1836,7 +1847,7 @@ __global__ __launch_bounds__(kSmallBlock) void kv_small_epoch_kernel(
     uint32_t B, uint32_t S, bool rm, uint64_t rows, uint32_t fields, uint32_t fw, uint32_t fsw, uint32_t max_scan,
     uint32_t L, uint32_t values, uint64_t hot, uint32_t *__restrict__ table, uint32_t *__restrict__ read_values,
     uint64_t *__restrict__ bitmap, uint64_t *__restrict__ host_bits, uint64_t *seq_out, uint64_t seq,
-    DeviceCounters *__restrict__ ctr)
+    uint32_t *__restrict__ result, DeviceCounters *__restrict__ ctr)
 {
     __shared__ uint64_t s_row[kSmallOps];
     __shared__ uint32_t s_meta[kSmallOps];
@@ -1868,8 +1879,9 @@ __global__ __launch_bounds__(kSmallBlock) void kv_small_epoch_kernel(
     if (has_hot)
         for (uint32_t f = threadIdx.x; f < fields; f += kSmallBlock) s_hot[f] = 0u;
     // the epoch's commit counts start at zero (thread 0 adds to them last)
-    for (uint32_t c = threadIdx.x; c < kCounterStripes * kCountedTypes; c += kSmallBlock)
-        ctr->commits[c / kCountedTypes][c % kCountedTypes] = 0;
+    if (!result)
+        for (uint32_t c = threadIdx.x; c < kCounterStripes * kCountedTypes; c += kSmallBlock)
+            ctr->commits[c / kCountedTypes][c % kCountedTypes] = 0;
     if (threadIdx.x == 0) {
         s_n = 0;
         s_bad = 0;
@@ -2076,7 +2088,10 @@ __global__ __launch_bounds__(kSmallBlock) void kv_small_epoch_kernel(
                 if (ok[u]) table[off[u]] = v[u] + add[u];
         }
     }
-    if (threadIdx.x == 0) {
+    if (threadIdx.x == 0 && result) {
+        result[0] = nc;
+        result[1] = s_bad;
+    } else if (threadIdx.x == 0) {
         add_counts(ctr, 0, LTPG_TYPE_KV, nc, B);
         if (s_bad) atomicAdd(&ctr->range_errors, s_bad);
     }
@@ -3213,16 +3228,7 @@ bool kv_bin_auto(uint64_t rows, uint64_t ops)
     return ops >= (1ull << 18) && ops >= per;
 }
 
-namespace {
-
-// Per-op registration where the binned path is not taken: small epochs are a
-// chain of dependent misses per transaction otherwise (80K ops on 1M rows 19
-// / 10 us, 160K 22 / 16), and the largest ones gain from its row folding
-// (100M rows: 4M ops 180 / 143, 16M 504 / 447); in between it loses where
-// most rows are distinct (1.3M ops on 10M rows, Zipf 0: 48 / 53).
-inline bool kv_per_op_auto(uint64_t ops) { return ops < (1ull << 18) || ops >= (1ull << 21); }
-
-bool bin_wanted(const KvState &kv, const KvBatchDev &b)
+bool kv_execute_bins(const KvState &kv, const KvBatchDev &b)
 {
     const uint64_t ops = (uint64_t)b.n_txns * b.n_slots;
     if (!kv.bin.ent || kv.max_scan > 1 || !(kv.partitioned || (kv.auto_shape && kv_bin_auto(kv.rows, ops))) ||
@@ -3232,6 +3238,15 @@ bool bin_wanted(const KvState &kv, const KvBatchDev &b)
     return ((uint64_t)f.tiles << f.tile_bits) <= kv.bin.cap_ent &&
            (uint64_t)f.tiles * (f.buckets + 1) <= kv.bin.cap_off;
 }
+
+namespace {
+
+// Per-op registration where the binned path is not taken: small epochs are a
+// chain of dependent misses per transaction otherwise (80K ops on 1M rows 19
+// / 10 us, 160K 22 / 16), and the largest ones gain from its row folding
+// (100M rows: 4M ops 180 / 143, 16M 504 / 447); in between it loses where
+// most rows are distinct (1.3M ops on 10M rows, Zipf 0: 48 / 53).
+inline bool kv_per_op_auto(uint64_t ops) { return ops < (1ull << 18) || ops >= (1ull << 21); }
 
 hipError_t launch_kv_bin(const KvState &kv, const KvBatchDev &b, const EpochTag &e, DeviceCounters *ctr,
                          hipStream_t s, bool zero_counts)
@@ -3265,7 +3280,7 @@ hipError_t launch_kv_bin(const KvState &kv, const KvBatchDev &b, const EpochTag 
     a.war_flag = kv.war_flag;
     a.ctr = ctr;
     hipLaunchKernelGGL(kv_bin_order_kernel, dim3((b.n_txns + 4 * kBlock - 1) / (4 * kBlock)), dim3(kBlock), 0, s, a,
-                       zero_counts);
+                       zero_counts, kv.clear_flags);
     const dim3 tiles(f.tiles), blk(kBinBlock);
     if (f.tile_bits == kBinSlotBits && f.buckets <= 1024)
         hipLaunchKernelGGL((kv_bin_kernel<16, 1024>), tiles, blk, 0, s, a);
@@ -3286,7 +3301,7 @@ hipError_t launch_kv_execute(const KvState &kv, const KvBatchDev &b, const Epoch
     if (b.n_txns == 0) return zero_counts ? launch_reset_epoch_counters(ctr, s) : hipSuccess;
     const uint64_t ops = (uint64_t)b.n_txns * b.n_slots;
     const dim3 op_grid((unsigned)((ops + kBlock - 1) / kBlock));
-    if (!counts && bin_wanted(kv, b)) return launch_kv_bin(kv, b, e, ctr, s, zero_counts);
+    if (!counts && kv_execute_bins(kv, b)) return launch_kv_bin(kv, b, e, ctr, s, zero_counts);
     if (kv.partitioned && !counts && kv.part.ent_me) {
         PartArgs a;
         a.keys = b.keys;
@@ -3511,13 +3526,14 @@ bool kv_small_epoch_ok(const KvState &kv, const KvBatchDev &b)
 }
 
 hipError_t launch_kv_small_epoch(const KvState &kv, const KvBatchDev &b, uint32_t values, DeviceCounters *ctr,
-                                 uint64_t *host_bits, uint64_t *seq_out, uint64_t seq, hipStream_t s)
+                                 uint64_t *host_bits, uint64_t *seq_out, uint64_t seq, hipStream_t s,
+                                 uint32_t *result)
 {
     if (!kv_small_epoch_ok(kv, b)) return hipErrorInvalidValue;
     hipLaunchKernelGGL(kv_small_epoch_kernel, dim3(1), dim3(kSmallBlock), 0, s, b.keys, b.meta, b.tids, b.n_txns,
                        b.n_slots, b.request_major, kv.rows, kv.fields, kv.field_words, kv.field_stride, kv.max_scan,
                        kv.read_slot, values, kv.hot_row, kv.table, kv.read_values, kv.bitmap, host_bits, seq_out, seq,
-                       ctr);
+                       result, ctr);
     return hipGetLastError();
 }
 

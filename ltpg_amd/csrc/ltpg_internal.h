@@ -127,6 +127,9 @@ struct KvState {
     // no launch shape was asked for (ltpg_kv_set_tuning): sizes decide
     // (kv_bin_auto, kv_per_op_auto)
     bool auto_shape = true;
+    // the binned EXECUTE clears the batch's flags first (no epochs to tell
+    // them apart)
+    bool clear_flags = false;
     // no kernel has written regs / doomed / raw_flag / war_flag since the
     // last refill ran (the next epoch-tag wrap may skip the refill)
     bool regs_clean = false;
@@ -345,6 +348,8 @@ struct BinShape {
     uint32_t row_bits, buckets, mask, tile_bits, tiles;
 };
 BinShape kv_bin_shape(uint64_t rows, uint64_t ops);
+// Whether EXECUTE (fast form) of this batch takes the binned path.
+bool kv_execute_bins(const KvState &kv, const KvBatchDev &b);
 // Where the binned EXECUTE is the default (kv_kernels.hip).
 bool kv_bin_auto(uint64_t rows, uint64_t ops);
 hipError_t launch_kv_execute(const KvState &kv, const KvBatchDev &b, const EpochTag &e, bool counts,
@@ -364,7 +369,8 @@ hipError_t launch_kv_writeback(const KvState &kv, const KvBatchDev &b, uint32_t 
 // also publishes: the bitmap to host_bits, then seq with a release.
 bool kv_small_epoch_ok(const KvState &kv, const KvBatchDev &b);
 hipError_t launch_kv_small_epoch(const KvState &kv, const KvBatchDev &b, uint32_t values, DeviceCounters *ctr,
-                                 uint64_t *host_bits, uint64_t *seq_out, uint64_t seq, hipStream_t s);
+                                 uint64_t *host_bits, uint64_t *seq_out, uint64_t seq, hipStream_t s,
+                                 uint32_t *result = nullptr);
 // The current batch's epoch phase by phase, a stream synchronisation after
 // each (the reference's driver loop), then ltpg_sync.
 int run_epoch_stepwise(ltpg_ctx *ctx);

@@ -2,8 +2,8 @@
 //
 // ltpg_kv_epoch_noalloc runs the same EXECUTE / CHECK / WRITEBACK kernels as
 // ltpg_epoch_run on a key-value context, but over a table and batch the
-// caller owns, with every per-row register, per-transaction flag and counter
-// in `scratch`: a file-scope device array of fixed size that each GPU holds
+// caller owns, with every per-row register, per-transaction flag, binned
+// operation and counter in `scratch`: a file-scope device array of fixed size that each GPU holds
 // from module load to process end.  For callers that cannot call hipMalloc
 // (code under graph capture, tight serving loops).
 //
@@ -13,6 +13,7 @@
 // current, and every later call on the device uses that address.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -25,18 +26,46 @@ namespace {
 constexpr uint64_t kRegsBytes = 2ull * LTPG_NOALLOC_MAX_ROWS * 8;  // interleaved R / W per row
 constexpr uint64_t kFlagsAt = kRegsBytes;                         // doomed, raw, war: one byte per txn each
 constexpr uint64_t kCountersAt = kFlagsAt + 3ull * LTPG_NOALLOC_MAX_TXNS;
-constexpr uint64_t kScratchBytes = kCountersAt + (sizeof(DeviceCounters) + 255) / 256 * 256;
+constexpr uint64_t kListAt = kCountersAt + (sizeof(DeviceCounters) + 255) / 256 * 256;
+// Binned EXECUTE of up to kBinOps op slots: at most 1024 buckets (2^20 rows)
+// and one tile per 2^kBinSlotBits slots (larger batches use the registers).
+constexpr uint64_t kBinOps = 1ull << 24;
+constexpr uint64_t kBinEnts = kBinOps + (1ull << kBinSlotBits);
+constexpr uint64_t kBinOffs = (kBinOps >> kBinSlotBits) * 1025 + 1025;
+constexpr uint64_t kUnsortedAt = kListAt + 4ull * LTPG_NOALLOC_MAX_TXNS;
+constexpr uint64_t kEntsAt = kUnsortedAt + 256;
+constexpr uint64_t kOffsAt = kEntsAt + 4 * kBinEnts;
+constexpr uint64_t kScratchBytes = kOffsAt + (2 * kBinOffs + 255) / 256 * 256;
 
 static __device__ __align__(256) uint8_t scratch[kScratchBytes];
 
-// The epoch's commit count and range errors (result[0], result[1]).
-__global__ void noalloc_result_kernel(const DeviceCounters *ctr, uint32_t *result)
+// The last call's contents are still there: registers back to "no
+// registrant", the batch's flags and the counters to zero.
+__global__ void noalloc_init_kernel(unsigned long long *regs, uint64_t n_regs, uint8_t *flags, uint32_t B,
+                                    DeviceCounters *ctr)
 {
-    if (threadIdx.x != 0) return;
-    uint32_t c = 0;
-    for (int k = 0; k < kCounterStripes; ++k) c += ctr->commits[k][LTPG_TYPE_KV];
-    result[0] = c;
-    result[1] = ctr->range_errors;
+    const uint64_t first = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x, step = (uint64_t)gridDim.x * blockDim.x;
+    ulonglong2 *r2 = reinterpret_cast<ulonglong2 *>(regs);
+    for (uint64_t i = first; i < n_regs / 2; i += step) r2[i] = make_ulonglong2(~0ull, ~0ull);
+    for (uint64_t i = first; i < B; i += step)
+        flags[i] = flags[LTPG_NOALLOC_MAX_TXNS + i] = flags[2ull * LTPG_NOALLOC_MAX_TXNS + i] = 0;
+    uint32_t *c = reinterpret_cast<uint32_t *>(ctr);
+    for (uint64_t i = first; i < sizeof(DeviceCounters) / 4; i += step) c[i] = 0;
+}
+
+// The epoch's commit count and range errors (result[0], result[1]; zero for
+// an empty epoch), one wave; the TID order flag starts over.
+__global__ void noalloc_result_kernel(const DeviceCounters *ctr, uint32_t *unsorted, uint32_t *result, bool empty)
+{
+    static_assert(kCounterStripes == 64, "one lane per stripe");
+    if (threadIdx.x == 0) *unsorted = 0;
+    if (!result) return;
+    uint32_t c = empty ? 0u : ctr->commits[threadIdx.x][LTPG_TYPE_KV];
+    for (int d = 32; d > 0; d >>= 1) c += __shfl_xor(c, d);
+    if (threadIdx.x == 0) {
+        result[0] = c;
+        result[1] = empty ? 0u : ctr->range_errors;
+    }
 }
 
 // scratch's device address, per device (looked up once each)
@@ -104,25 +133,43 @@ extern "C" int ltpg_kv_epoch_noalloc(uint32_t *table, uint64_t rows, uint32_t fi
     b.keys = batch->keys;
     b.meta = batch->meta;
     b.tids = batch->tids;
-    // the last call's contents are still there: registers back to "no
-    // registrant", this batch's flags and the counters to zero (fill kernels,
-    // so that a caller may capture the call into a graph)
-    LTPG_HIP_TRY(launch_fill_u64(kv.regs, 2 * rows, ~0ull, s));
-    LTPG_HIP_TRY(launch_fill_u8(p + kCountersAt, sizeof(DeviceCounters), 0, s));
+    uint32_t *unsorted = reinterpret_cast<uint32_t *>(p + kUnsortedAt);
+    if (kv_small_epoch_ok(kv, b)) {
+        // one kernel; the registers and flags stay in its LDS (64 x 4 ops: ten
+        // launches 36 us, this one 8 us, most of it the launch)
+        uint32_t *res = result ? result : reinterpret_cast<uint32_t *>(ctr->pad0);
+        LTPG_HIP_TRY(launch_kv_small_epoch(kv, b, values, ctr, nullptr, nullptr, 0, s, res));
+        return LTPG_OK;
+    }
     if (B) {
-        LTPG_HIP_TRY(launch_fill_u8(kv.doomed, B, 0, s));
-        LTPG_HIP_TRY(launch_fill_u8(kv.raw_flag, B, 0, s));
-        LTPG_HIP_TRY(launch_fill_u8(kv.war_flag, B, 0, s));
+        // kernels only, so that a caller may capture the call into a graph
+        kv.commit_list = reinterpret_cast<uint32_t *>(p + kListAt);
+        kv.bin.ent = reinterpret_cast<uint32_t *>(p + kEntsAt);
+        kv.bin.cap_ent = kBinEnts;
+        kv.bin.off = reinterpret_cast<uint16_t *>(p + kOffsAt);
+        kv.bin.cap_off = kBinOffs;
+        kv.bin.unsorted = unsorted;
+        // binning needs no registers, whose refill costs 16 bytes per row:
+        // taken wherever there are rows enough for its buckets (1M rows: 80K
+        // ops take 13 us binned, 9 on the registers and 9 for their refill;
+        // 65,536 x 10 ops, whole call: 81 -> 33 us)
+        kv.partitioned = rows > (1ull << 15);
+        kv.clear_flags = true;
+        if (!kv_execute_bins(kv, b)) {
+            const uint64_t n = std::max<uint64_t>(rows, B / 4);
+            hipLaunchKernelGGL(noalloc_init_kernel, dim3((unsigned)std::min<uint64_t>(4096, (n + 255) / 256)), dim3(256),
+                               0, s, kv.regs, 2 * rows, kv.doomed, B, ctr);
+            LTPG_HIP_TRY(hipGetLastError());
+        }
         EpochTag e;
         e.epoch = 1;
         e.tag = 254;
         LTPG_HIP_TRY(launch_kv_execute(kv, b, e, false, ctr, s));
         LTPG_HIP_TRY(launch_kv_check(kv, b, e, false, ctr, s));
+        kv.list_valid = true;  // of the CHECK above
         LTPG_HIP_TRY(launch_kv_writeback(kv, b, values, ctr, s));
     }
-    if (result) {
-        hipLaunchKernelGGL(noalloc_result_kernel, dim3(1), dim3(64), 0, s, ctr, result);
-        LTPG_HIP_TRY(hipGetLastError());
-    }
+    hipLaunchKernelGGL(noalloc_result_kernel, dim3(1), dim3(64), 0, s, ctr, unsorted, result, B == 0);
+    LTPG_HIP_TRY(hipGetLastError());
     return LTPG_OK;
 }
