@@ -925,11 +925,11 @@ __global__ __launch_bounds__(kPartBlock) void kv_part_flags_kernel(PartArgs a)
 // from filling one bucket.  Only with ordered TIDs.
 //
 // 2^20 transactions x 16 ops on 10M rows: 486 us on the registers (285
-// registration, 202 read marking) -> 200 us at Zipf 0.6 (order 5, bin 62,
-// flags 130), 515 -> 170 us at Zipf 0.99.  The bin kernel moves 268 MB at 4.3
+// registration, 202 read marking) -> 189 us at Zipf 0.6 (order 5, bin 62,
+// flags 122), 515 -> 160 us at Zipf 0.99.  The bin kernel moves 268 MB at 4.3
 // TB/s; the flags kernel is bound by instruction issue (1M runs of 16 entries,
-// half of the lanes idle) and, at Zipf 0.6, by its 6M scattered flag bytes
-// (63 us without them).
+// half of the lanes idle; 130 us with each entry's transaction by division)
+// and, at Zipf 0.6, by its 9M scattered flag bytes (58 us without them).
 constexpr uint32_t kBinBlock = 1024;
 constexpr uint32_t kBinRows = 1u << kBinRowBits;
 constexpr uint32_t kBinMul = 0x9E3779B1u;  // odd
@@ -1105,22 +1105,53 @@ __global__ __launch_bounds__(kBinBlock, MaxB <= kBinBlock ? 8 : 4) void kv_bin_k
     for (uint32_t j = threadIdx.x; j < (total + 3) / 4; j += kBinBlock) dst[j] = src[j];
 }
 
-// One pass over bucket b's entries: 16 lanes per tile run, four runs' first
-// 32 entries in flight per group.  MARK false: the W minima of the rows
-// [lo, lo + n) of the bucket into s_w; MARK true: the flags from them.  The
-// priority is the position (u32) or, with TIDs out of order, TID << 24 |
-// position (u64); all-ones: no writer.
-template <typename W, bool MARK>
-__device__ __forceinline__ void bin_pass(const BinArgs &a, uint32_t b, W *s_w, uint32_t lo, uint32_t n)
+// A bucket's runs are read by groups of 16 lanes, one run per group at a time;
+// lane l of group g holds the run of tile c0 + l * kRunGroups + g: where it
+// starts, its length, and the transaction of the tile's first slot.
+constexpr uint32_t kRunLanes = 16, kRunGroups = kBinBlock / kRunLanes;
+
+struct BinRun {
+    uint32_t start, len, t0;
+};
+
+__device__ __forceinline__ BinRun bin_run(const BinArgs &a, uint32_t b, uint32_t c0)
 {
-    constexpr uint32_t kRun = 16, kGroups = kBinBlock / kRun, U = 4;
-    const uint32_t g = threadIdx.x / kRun, l = threadIdx.x % kRun;
-    const int base_lane = lane_id() & ~(int)(kRun - 1);
-    auto one = [&](uint32_t x, uint32_t tile) {
+    const uint32_t tile = c0 + (threadIdx.x % kRunLanes) * kRunGroups + threadIdx.x / kRunLanes;
+    BinRun r = {0u, 0u, 0u};
+    if (tile < a.tiles) {
+        const uint16_t *o = a.off + (uint64_t)tile * (a.nb + 1) + b;
+        r.start = (tile << a.tile_bits) + o[0];
+        r.len = (uint32_t)o[1] - o[0];
+        r.t0 = bin_txn(a, tile << a.tile_bits);
+    }
+    return r;
+}
+
+// One pass over bucket b's entries of the tiles [c0, c0 + kBinBlock), four
+// runs' first 32 entries in flight per group.  MARK false: the W minima of the
+// rows [lo, lo + n) of the bucket into s_w; MARK true: the flags from them.
+// The priority is the position (u32) or, with TIDs out of order, TID << 24 |
+// position (u64); all-ones: no writer.  DIRECT: slot-major and no narrower
+// than a tile, so a slot's transaction is its tile's first plus its place,
+// once around at most.
+template <typename W, bool MARK, bool DIRECT>
+__device__ __forceinline__ void bin_pass(const BinArgs &a, const BinRun &mine, uint32_t c0, W *s_w, uint32_t lo,
+                                         uint32_t n)
+{
+    constexpr uint32_t U = 4, kSlot = (1u << kBinSlotBits) - 1u;
+    const uint32_t g = threadIdx.x / kRunLanes, l = threadIdx.x % kRunLanes;
+    const int base_lane = lane_id() & ~(int)(kRunLanes - 1);
+    auto one = [&](uint32_t x, uint32_t t0, uint32_t tile) {
         const uint32_t r = (x >> (kBinSlotBits + 1)) - lo;
         const bool wr = (x >> kBinSlotBits) & 1u;
         if ((!MARK && !wr) || r >= n) return;
-        const uint32_t t = bin_txn(a, (tile << a.tile_bits) + (x & ((1u << kBinSlotBits) - 1u)));
+        uint32_t t;
+        if (DIRECT) {
+            t = t0 + (x & kSlot);
+            t = min(t, t - a.B);  // around: t - B wraps below zero otherwise
+        } else {
+            t = bin_txn(a, (tile << a.tile_bits) + (x & kSlot));
+        }
         const W me = sizeof(W) == 4 ? (W)t : (W)((unsigned long long)a.tids[t] << kTidShift | t);
         if (!MARK) {
             atomicMin(&s_w[r], me);
@@ -1135,51 +1166,42 @@ __device__ __forceinline__ void bin_pass(const BinArgs &a, uint32_t b, W *s_w, u
             a.war_flag[w & (W)kPosMask] = a.epoch;
         }
     };
-    for (uint32_t c0 = 0; c0 < a.tiles; c0 += kBinBlock) {
-        // lane l of group g holds the run of tile c0 + l * kGroups + g
-        const uint32_t mine = c0 + l * kGroups + g;
-        uint32_t st = 0, ln = 0;
-        if (mine < a.tiles) {
-            const uint16_t *o = a.off + (uint64_t)mine * (a.nb + 1) + b;
-            st = o[0];
-            ln = o[1] - st;
+    const uint32_t left = a.tiles - c0;
+    const uint32_t nj = left >= kBinBlock ? kRunLanes : (left + kRunGroups - 1) / kRunGroups;
+    for (uint32_t j0 = 0; j0 < nj; j0 += U) {
+        uint32_t s[U], len[U], t0[U], x[U][2];
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u) {
+            s[u] = __shfl(mine.start, base_lane + (int)(j0 + u));
+            len[u] = __shfl(mine.len, base_lane + (int)(j0 + u));
+            t0[u] = DIRECT ? __shfl(mine.t0, base_lane + (int)(j0 + u)) : 0u;
+            // unconditional loads (a run's first entry, or entry 0, when idle)
+            x[u][0] = a.ent[s[u] + (l < len[u] ? l : 0u)];
+            x[u][1] = a.ent[s[u] + (l + kRunLanes < len[u] ? l + kRunLanes : 0u)];
         }
-        const uint32_t left = a.tiles - c0;
-        const uint32_t nj = left >= kBinBlock ? kRun : (left + kGroups - 1) / kGroups;
-        for (uint32_t j0 = 0; j0 < nj; j0 += U) {
-            uint32_t s[U], len[U], x[U][2];
 #pragma unroll
-            for (uint32_t u = 0; u < U; ++u) {
-                s[u] = __shfl(st, base_lane + (int)(j0 + u));
-                len[u] = __shfl(ln, base_lane + (int)(j0 + u));
-                const uint32_t tile = c0 + (j0 + u) * kGroups + g;
-                const uint32_t *p = a.ent + (len[u] ? ((uint64_t)tile << a.tile_bits) + s[u] : 0ull);
-                // unconditional loads (a run's first entry, or entry 0, when idle)
-                x[u][0] = p[l < len[u] ? l : 0u];
-                x[u][1] = p[l + kRun < len[u] ? l + kRun : 0u];
-            }
-#pragma unroll
-            for (uint32_t u = 0; u < U; ++u) {
-                const uint32_t tile = c0 + (j0 + u) * kGroups + g;
-                if (l < len[u]) one(x[u][0], tile);
-                if (l + kRun < len[u]) one(x[u][1], tile);
-                for (uint32_t e = l + 2 * kRun; e < len[u]; e += kRun)
-                    one(a.ent[((uint64_t)tile << a.tile_bits) + s[u] + e], tile);
-            }
+        for (uint32_t u = 0; u < U; ++u) {
+            const uint32_t tile = c0 + (j0 + u) * kRunGroups + g;
+            if (l < len[u]) one(x[u][0], t0[u], tile);
+            if (l + kRunLanes < len[u]) one(x[u][1], t0[u], tile);
+            for (uint32_t e = l + 2 * kRunLanes; e < len[u]; e += kRunLanes) one(a.ent[s[u] + e], t0[u], tile);
         }
     }
 }
 
-template <typename W>
+template <typename W, bool DIRECT>
 __device__ __forceinline__ void bin_flags(const BinArgs &a, uint32_t b, W *s_w, uint32_t cap)
 {
+    const BinRun first = bin_run(a, b, 0);
     for (uint32_t lo = 0; lo < (1u << a.row_bits); lo += cap) {
         const uint32_t n = min(1u << a.row_bits, cap);
         for (uint32_t r = threadIdx.x; r < n; r += kBinBlock) s_w[r] = (W)~(W)0;
         __syncthreads();
-        bin_pass<W, false>(a, b, s_w, lo, n);
+        for (uint32_t c0 = 0; c0 < a.tiles; c0 += kBinBlock)
+            bin_pass<W, false, DIRECT>(a, c0 ? bin_run(a, b, c0) : first, c0, s_w, lo, n);
         __syncthreads();
-        bin_pass<W, true>(a, b, s_w, lo, n);
+        for (uint32_t c0 = 0; c0 < a.tiles; c0 += kBinBlock)
+            bin_pass<W, true, DIRECT>(a, c0 ? bin_run(a, b, c0) : first, c0, s_w, lo, n);
         __syncthreads();
     }
 }
@@ -1191,10 +1213,12 @@ __global__ __launch_bounds__(kBinBlock, 8) void kv_bin_flags_kernel(BinArgs a)
     // entries share cache lines
     const uint32_t x = blockIdx.x;
     const uint32_t b = a.nb >= 8 ? (x & 7u) * (a.nb / 8) + (x >> 3) : x;
-    if (*a.unsorted != a.epoch)
-        bin_flags<uint32_t>(a, b, reinterpret_cast<uint32_t *>(s_w), kBinRows);
+    if (*a.unsorted == a.epoch)
+        bin_flags<unsigned long long, false>(a, b, s_w, kBinRows / 2);
+    else if (!a.rm && a.B >= (1u << a.tile_bits))
+        bin_flags<uint32_t, true>(a, b, reinterpret_cast<uint32_t *>(s_w), kBinRows);
     else
-        bin_flags<unsigned long long>(a, b, s_w, kBinRows / 2);
+        bin_flags<uint32_t, false>(a, b, reinterpret_cast<uint32_t *>(s_w), kBinRows);
 }
 
 // Read marking (fast form), one lane per op after every write has
