@@ -485,9 +485,9 @@ int ltpg_tpcc_gen_next(ltpg_tpcc_gen *g, uint32_t n_txns, uint32_t tid_base, uin
  *   the epoch's register operations by row and finds each row's minimum
  *   writer in LDS, instead of probing and updating the per-row registers in
  *   HBM at random (EXEC_PER_OP and SPLIT_REGISTERS then have no effect on
- *   point operations).  Contexts with kv_max_scan <= 1: at most 16384 rows per
- *   bucket, one pass over the batch and 4 bytes per binned operation.  With
- *   scans: 8192 rows per bucket, two passes and 12 bytes each.  The autotuner
+ *   point operations).  Contexts with kv_max_scan <= 1: one pass over the batch
+ *   and 4 bytes per binned operation.  With scans: 8192 rows per bucket, two
+ *   passes and 12 bytes each.  The autotuner
  *   tries it with SPLIT_REGISTERS, SMALL_CHUNKS and LANE_COPY.
  *   Needs kv_rows <= 8192 * 16384 and kv_max_slots * max_txns *
  *   max(1, kv_max_scan) < 2^32 (else LTPG_ERR_UNSUPPORTED); the first

@@ -25,6 +25,13 @@ void set_error(const std::string &msg) { g_last_error = msg; }
 
 namespace {
 
+void free_bin(BinBuffers &b)
+{
+    dev_free(b.ent);
+    dev_free(b.off);
+    dev_free(b.unsorted);
+}
+
 void free_kv(KvState &kv)
 {
     dev_free(kv.table);
@@ -49,9 +56,7 @@ void free_kv(KvState &kv)
     dev_free(kv.part.slices);
     dev_free(kv.part.ent_me);
     dev_free(kv.part.ent_key);
-    dev_free(kv.bin.ent);
-    dev_free(kv.bin.off);
-    dev_free(kv.bin.unsorted);
+    free_bin(kv.bin);
 }
 
 // Buffers of the binned EXECUTE for every batch the context accepts.
@@ -59,20 +64,18 @@ int kv_bin_prepare(ltpg_ctx *ctx)
 {
     KvState &kv = ctx->kv;
     if (kv.bin.ent) return LTPG_OK;
-    const uint64_t ops = (uint64_t)kv.max_slots * ctx->cfg.max_txns;
-    KvState::Bin p;
-    // the largest batch, and the largest of the smaller tiles' shape
-    for (uint64_t n : {ops, std::min(ops, kBinLargeOps - 1)}) {
-        const BinShape f = kv_bin_shape(kv.rows, n);
+    BinBuffers p;
+    // buckets and tiles do not grow together: sizes from the largest down, in
+    // steps finer than any change of shape
+    for (uint64_t n = (uint64_t)kv.max_slots * ctx->cfg.max_txns; n; n -= n / 64 + 1) {
+        const BinShape f = bin_shape(kv.rows, n);
         p.cap_ent = std::max(p.cap_ent, (uint64_t)f.tiles << f.tile_bits);
-        p.cap_off = std::max(p.cap_off, (uint64_t)f.tiles * (f.buckets + 1));
+        p.cap_off = std::max(p.cap_off, (uint64_t)f.tiles * (f.buckets + 1) * 66 / 64 + f.buckets + 1);
     }
     int rc;
     if ((rc = dev_alloc(&p.ent, p.cap_ent, "binned operations")) || (rc = dev_alloc(&p.off, p.cap_off, "bin starts")) ||
         (rc = dev_alloc(&p.unsorted, 1, "TID order flag"))) {
-        dev_free(p.ent);
-        dev_free(p.off);
-        dev_free(p.unsorted);
+        free_bin(p);
         return rc;
     }
     kv.bin = p;  // freed with the context

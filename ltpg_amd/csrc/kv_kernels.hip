@@ -44,6 +44,7 @@
 // 64), fetched by __shfl.
 #include <algorithm>
 
+#include "bin_execute.h"
 #include "device_common.h"
 #include "ltpg_internal.h"
 
@@ -132,14 +133,6 @@ __device__ __forceinline__ void add_counts(DeviceCounters *ctr, uint32_t stripe,
         atomicAdd(&ctr->totals[stripe][type], (unsigned long long)commits);
     }
     if (attempts) atomicAdd(&ctr->totals[stripe][kAttempts + type], (unsigned long long)attempts);
-}
-
-// An epoch's commit counts start at zero (one block calls it).
-__device__ __forceinline__ void zero_epoch_counts(DeviceCounters *ctr, uint32_t threads)
-{
-    for (uint32_t c = threadIdx.x; c < kCounterStripes * kCountedTypes; c += threads)
-        ctr->commits[c / kCountedTypes][c % kCountedTypes] = 0;
-    if (threadIdx.x == 0) ctr->kv_list_n = 0;
 }
 
 // Per-op decode shared by every phase.
@@ -771,31 +764,6 @@ __global__ __launch_bounds__(kPartBlock) void kv_part_scatter_kernel(PartArgs a)
     }
 }
 
-// Exclusive prefix sum over the block of one value per thread; *total gets
-// the sum.  Wave scans by shuffles, then the 16 wave totals through LDS.
-__device__ __forceinline__ uint32_t block_exclusive_sum(uint32_t v, uint32_t *s_wt, uint32_t *total)
-{
-    constexpr uint32_t kWaves = kPartBlock / 64;
-    const uint32_t lane = threadIdx.x % 64, wave = threadIdx.x / 64;
-    uint32_t inc = v;
-#pragma unroll
-    for (uint32_t d = 1; d < 64; d <<= 1) {
-        const uint32_t x = __shfl_up(inc, d);
-        if (lane >= d) inc += x;
-    }
-    if (lane == 63) s_wt[wave] = inc;
-    __syncthreads();
-    uint32_t before = 0, all = 0;
-#pragma unroll
-    for (uint32_t w = 0; w < kWaves; ++w) {
-        const uint32_t t = s_wt[w];
-        before += w < wave ? t : 0u;
-        all += t;
-    }
-    *total = all;
-    return before + inc - v;
-}
-
 // The fast form's flags of one operation against its row's minimum W
 // priority w (~0: no writer this epoch).
 __device__ __forceinline__ void part_flag(const PartArgs &a, uint32_t key, unsigned long long me,
@@ -893,333 +861,28 @@ __global__ __launch_bounds__(kPartBlock) void kv_part_flags_kernel(PartArgs a)
 }
 
 // ---- binned EXECUTE of point operations (LTPG_TUNE_PARTITIONED, or the
-// ---- default shape of a large epoch; fast form, no scans) -----------------
-//
-// The register path touches one random 128-byte register line per operation.
-// Here the operations are binned by row first and every row's minimum writer
-// is found in LDS; the per-row registers in HBM are not touched:
-//   order    are the TIDs non-decreasing in batch position (the usual batch)?
-//            Then position alone is the priority;
-//   bin      one pass over the batch.  A 1024-thread block takes a tile of
-//            P * 1024 consecutive op slots, drops operations that a writer in
-//            the same tile already decides (below), ranks the others per
-//            bucket with LDS counters, places them bucket by bucket in LDS and
-//            writes the tile out in that order, with the start of each
-//            bucket's run (16 bits) in a table;
-//   flags    one block per bucket: reads the bucket's run of every tile twice,
-//            first into the W minima of its rows in LDS, then setting the
-//            fast form's flags from them (part_flag).
-// A row's bucket is the top bits of row * odd mod 2^K (a bijection), so ranges
-// of hot rows spread over the buckets.  An entry is 4 bytes -- row within the
-// bucket, is-write, slot within the tile; the tile gives the rest -- so no
-// TID, position or counting pass goes through memory: the batch is read once,
-// and 4 bytes per operation written once and read twice (the second time
-// mostly from the L2).
-//
-// The in-tile filter: writers enter (position, row) into a direct-mapped LDS
-// table with a 64-bit minimum.  An operation that finds its own row there
-// under a lower position is behind a writer: a write has waw, a read raw, and
-// neither can matter to any other transaction (it is not its row's minimum
-// writer, and as a reader it is behind that minimum, so gives no war).  It is
-// flagged at once and leaves the batch, which keeps a skewed epoch's hot rows
-// from filling one bucket.  Only with ordered TIDs.
-//
-// 2^20 transactions x 16 ops on 10M rows: 486 us on the registers (285
-// registration, 202 read marking) -> 189 us at Zipf 0.6 (order 5, bin 62,
-// flags 122), 515 -> 160 us at Zipf 0.99.  The bin kernel moves 268 MB at 4.3
-// TB/s; the flags kernel is bound by instruction issue (1M runs of 16 entries,
-// half of the lanes idle; 130 us with each entry's transaction by division)
-// and, at Zipf 0.6, by its 9M scattered flag bytes (58 us without them).
-constexpr uint32_t kBinBlock = 1024;
-constexpr uint32_t kBinRows = 1u << kBinRowBits;
-constexpr uint32_t kBinMul = 0x9E3779B1u;  // odd
-
-// i mod d and i / d for i < 2^32 by one high multiply: with m = floor(2^32 /
-// d) (2^32 - 1 for d = 1) the quotient is exact or one too small.
-struct FastMod {
-    uint32_t d, m;
-};
-
-__device__ __forceinline__ uint32_t fast_div(const FastMod &f, uint32_t i, uint32_t *rem)
-{
-    uint32_t q = __umulhi(i, f.m);
-    uint32_t r = i - q * f.d;
-    if (r >= f.d) {
-        r -= f.d;
-        ++q;
-    }
-    *rem = r;
-    return q;
-}
-
-struct BinArgs {
+// ---- default shape of a large epoch; fast form, no scans; bin_execute.h) ---
+struct KvBinSource {
     const uint64_t *keys;
     const uint32_t *meta;
-    const uint32_t *tids;
-    uint32_t B, n_ops;
     uint64_t rows;
     uint32_t fields, max_scan;
     uint64_t hot;
-    uint32_t mask, row_bits, nb, tiles, tile_bits;  // 2^K - 1; log2 rows per bucket; buckets; tiles; log2 slots per tile
-    FastMod per;                                    // n_slots (request-major) or n_txns
-    bool rm;
-    uint8_t epoch;
-    uint32_t *ent;         // [tiles << tile_bits]
-    uint16_t *off;         // [tiles][nb + 1] start of each bucket's run in the tile
-    uint32_t *unsorted;    // epoch number of the last epoch whose TIDs were out of order
-    uint8_t *doomed, *raw_flag, *war_flag;
-    DeviceCounters *ctr;
-};
-
-__device__ __forceinline__ uint32_t bin_txn(const BinArgs &a, uint32_t i)
-{
-    uint32_t r;
-    const uint32_t q = fast_div(a.per, i, &r);
-    return a.rm ? q : r;
-}
-
-// With `clear` (the epoch that keeps no state between calls) also the flags of
-// the block's transactions and the range errors start over.
-__global__ __launch_bounds__(kBlock) void kv_bin_order_kernel(BinArgs a, bool zero_counts, bool clear)
-{
-    if (zero_counts && blockIdx.x == 0) zero_epoch_counts(a.ctr, kBlock);
-    if (clear) {
-        if (blockIdx.x == 0 && threadIdx.x == 0) a.ctr->range_errors = 0;
-#pragma unroll
-        for (uint32_t u = 0; u < 4; ++u) {
-            const uint32_t t = blockIdx.x * (4 * kBlock) + u * kBlock + threadIdx.x;
-            if (t < a.B) a.doomed[t] = a.raw_flag[t] = a.war_flag[t] = 0;
-        }
-    }
-    // four pairs per thread, all loads in flight together
-    const uint32_t first = blockIdx.x * (4 * kBlock) + threadIdx.x, last = a.B - 1;
-    uint32_t lo[4], hi[4];
-#pragma unroll
-    for (uint32_t u = 0; u < 4; ++u) {
-        const uint32_t t = first + u * kBlock;
-        lo[u] = a.tids[t < last ? t : last];
-        hi[u] = a.tids[t < last ? t + 1 : last];
-    }
-    bool out = false;
-#pragma unroll
-    for (uint32_t u = 0; u < 4; ++u) out |= lo[u] > hi[u];
-    // a stale equal number (255 epochs ago) only costs the slower path
-    if (out) *a.unsorted = a.epoch;
-}
-
-template <uint32_t P, uint32_t MaxB>
-__global__ __launch_bounds__(kBinBlock, MaxB <= kBinBlock ? 8 : 4) void kv_bin_kernel(BinArgs a)
-{
-    constexpr uint32_t T = P * kBinBlock, kFilter = T / 2;
-    constexpr uint32_t kPer = MaxB / kBinBlock;  // buckets per thread at most
-    constexpr uint32_t G = 4;                    // loads in flight per thread
-    __shared__ __align__(16) uint32_t s_ent[T];  // the filter first, then the tile in bucket order
-    __shared__ uint32_t s_at[MaxB];              // counts, then starts
-    __shared__ uint32_t s_wt[kBinBlock / 64];
-    unsigned long long *s_min = reinterpret_cast<unsigned long long *>(s_ent);
-    const uint32_t base = blockIdx.x * T + threadIdx.x;
-    const bool fold = *a.unsorted != a.epoch;
-    for (uint32_t k = threadIdx.x; k < kFilter; k += kBinBlock) s_min[k] = ~0ull;
-    for (uint32_t b = threadIdx.x; b < a.nb; b += kBinBlock) s_at[b] = 0;
-    __syncthreads();
-    uint32_t hw[P];  // hashed row << 1 | is-write, or all-ones: nothing to register
-    uint32_t bad = 0;
-#pragma unroll
-    for (uint32_t g = 0; g < P; g += G) {
-        uint64_t r[G];
-        uint32_t m[G];
-#pragma unroll
-        for (uint32_t u = 0; u < G; ++u) {
-            const uint32_t i = base + (g + u) * kBinBlock;
-            r[u] = a.keys[i < a.n_ops ? i : 0u];
-            m[u] = a.meta[i < a.n_ops ? i : 0u];
-        }
-#pragma unroll
-        for (uint32_t u = 0; u < G; ++u) {
-            const uint32_t i = base + (g + u) * kBinBlock;
-            const Op o = decode_op(r[u], i < a.n_ops ? m[u] : 0u, a.rows, a.fields, a.max_scan);
-            bad += (o.kind != LTPG_KV_NONE && !o.valid) ? 1u : 0u;
-            const uint32_t w = o.kind == LTPG_KV_WRITE ? 1u : 0u;
-            const uint32_t h = ((uint32_t)o.row * kBinMul) & a.mask;
-            const bool use = o.valid && o.row != a.hot;
-            hw[g + u] = use ? h << 1 | w : ~0u;
-            if (fold && use && w)
-                atomicMin(&s_min[(h ^ (h >> 12)) & (kFilter - 1)], (unsigned long long)bin_txn(a, i) << 32 | h);
-        }
-    }
-    if (bad) atomicAdd(&a.ctr->range_errors, bad);
-    __syncthreads();
-    uint32_t rank[P];
-#pragma unroll
-    for (uint32_t u = 0; u < P; ++u) {
-        const uint32_t h = hw[u] >> 1;
-        if (fold && hw[u] != ~0u) {
-            const unsigned long long v = s_min[(h ^ (h >> 12)) & (kFilter - 1)];
-            if ((uint32_t)v == h) {
-                const uint32_t t = bin_txn(a, base + u * kBinBlock);
-                if ((uint32_t)(v >> 32) < t) {
-                    if (hw[u] & 1u)
-                        a.doomed[t] = a.epoch;
-                    else
-                        a.raw_flag[t] = a.epoch;
-                    hw[u] = ~0u;
-                }
-            }
-        }
-        rank[u] = hw[u] != ~0u ? atomicAdd(&s_at[h >> a.row_bits], 1u) : 0u;
-    }
-    __syncthreads();
-    // thread j owns buckets [j * per, (j + 1) * per)
-    const uint32_t per = (a.nb + kBinBlock - 1) / kBinBlock, b0 = threadIdx.x * per;
-    uint32_t cnt[kPer], sum = 0, total;
-#pragma unroll
-    for (uint32_t j = 0; j < kPer; ++j) {
-        cnt[j] = (j < per && b0 + j < a.nb) ? s_at[b0 + j] : 0u;
-        sum += cnt[j];
-    }
-    uint32_t run = block_exclusive_sum(sum, s_wt, &total);
-    uint16_t *off = a.off + (uint64_t)blockIdx.x * (a.nb + 1);
-#pragma unroll
-    for (uint32_t j = 0; j < kPer; ++j) {
-        if (j < per && b0 + j < a.nb) {
-            s_at[b0 + j] = run;
-            off[b0 + j] = (uint16_t)run;
-        }
-        run += cnt[j];
-    }
-    if (threadIdx.x == 0) off[a.nb] = (uint16_t)total;
-    __syncthreads();
-    const uint32_t inner = (1u << a.row_bits) - 1u;
-#pragma unroll
-    for (uint32_t u = 0; u < P; ++u) {
-        if (hw[u] == ~0u) continue;
-        const uint32_t h = hw[u] >> 1;
-        s_ent[s_at[h >> a.row_bits] + rank[u]] =
-            (h & inner) << (kBinSlotBits + 1) | (hw[u] & 1u) << kBinSlotBits | (u * kBinBlock + threadIdx.x);
-    }
-    __syncthreads();
-    // whole 16-byte vectors: the last one may carry stale words, which stay
-    // inside the tile's own part of ent
-    uint4 *dst = reinterpret_cast<uint4 *>(a.ent + (uint64_t)blockIdx.x * T);
-    const uint4 *src = reinterpret_cast<const uint4 *>(s_ent);
-    for (uint32_t j = threadIdx.x; j < (total + 3) / 4; j += kBinBlock) dst[j] = src[j];
-}
-
-// A bucket's runs are read by groups of 16 lanes, one run per group at a time;
-// lane l of group g holds the run of tile c0 + l * kRunGroups + g: where it
-// starts, its length, and the transaction of the tile's first slot.
-constexpr uint32_t kRunLanes = 16, kRunGroups = kBinBlock / kRunLanes;
-
-struct BinRun {
-    uint32_t start, len, t0;
-};
-
-__device__ __forceinline__ BinRun bin_run(const BinArgs &a, uint32_t b, uint32_t c0)
-{
-    const uint32_t tile = c0 + (threadIdx.x % kRunLanes) * kRunGroups + threadIdx.x / kRunLanes;
-    BinRun r = {0u, 0u, 0u};
-    if (tile < a.tiles) {
-        const uint16_t *o = a.off + (uint64_t)tile * (a.nb + 1) + b;
-        r.start = (tile << a.tile_bits) + o[0];
-        r.len = (uint32_t)o[1] - o[0];
-        r.t0 = bin_txn(a, tile << a.tile_bits);
-    }
-    return r;
-}
-
-// One pass over bucket b's entries of the tiles [c0, c0 + kBinBlock), four
-// runs' first 32 entries in flight per group.  MARK false: the W minima of the
-// rows [lo, lo + n) of the bucket into s_w; MARK true: the flags from them.
-// The priority is the position (u32) or, with TIDs out of order, TID << 24 |
-// position (u64); all-ones: no writer.  DIRECT: slot-major and no narrower
-// than a tile, so a slot's transaction is its tile's first plus its place,
-// once around at most.
-template <typename W, bool MARK, bool DIRECT>
-__device__ __forceinline__ void bin_pass(const BinArgs &a, const BinRun &mine, uint32_t c0, W *s_w, uint32_t lo,
-                                         uint32_t n)
-{
-    constexpr uint32_t U = 4, kSlot = (1u << kBinSlotBits) - 1u;
-    const uint32_t g = threadIdx.x / kRunLanes, l = threadIdx.x % kRunLanes;
-    const int base_lane = lane_id() & ~(int)(kRunLanes - 1);
-    auto one = [&](uint32_t x, uint32_t t0, uint32_t tile) {
-        const uint32_t r = (x >> (kBinSlotBits + 1)) - lo;
-        const bool wr = (x >> kBinSlotBits) & 1u;
-        if ((!MARK && !wr) || r >= n) return;
-        uint32_t t;
-        if (DIRECT) {
-            t = t0 + (x & kSlot);
-            t = min(t, t - a.B);  // around: t - B wraps below zero otherwise
-        } else {
-            t = bin_txn(a, (tile << a.tile_bits) + (x & kSlot));
-        }
-        const W me = sizeof(W) == 4 ? (W)t : (W)((unsigned long long)a.tids[t] << kTidShift | t);
-        if (!MARK) {
-            atomicMin(&s_w[r], me);
-            return;
-        }
-        const W w = s_w[r];
-        if (wr) {
-            if (w < me) a.doomed[t] = a.epoch;
-        } else if (w < me) {
-            a.raw_flag[t] = a.epoch;
-        } else if (w > me && w != (W)~(W)0) {
-            a.war_flag[w & (W)kPosMask] = a.epoch;
-        }
+    struct Raw {
+        uint64_t row;
+        uint32_t meta;
     };
-    const uint32_t left = a.tiles - c0;
-    const uint32_t nj = left >= kBinBlock ? kRunLanes : (left + kRunGroups - 1) / kRunGroups;
-    for (uint32_t j0 = 0; j0 < nj; j0 += U) {
-        uint32_t s[U], len[U], t0[U], x[U][2];
-#pragma unroll
-        for (uint32_t u = 0; u < U; ++u) {
-            s[u] = __shfl(mine.start, base_lane + (int)(j0 + u));
-            len[u] = __shfl(mine.len, base_lane + (int)(j0 + u));
-            t0[u] = DIRECT ? __shfl(mine.t0, base_lane + (int)(j0 + u)) : 0u;
-            // unconditional loads (a run's first entry, or entry 0, when idle)
-            x[u][0] = a.ent[s[u] + (l < len[u] ? l : 0u)];
-            x[u][1] = a.ent[s[u] + (l + kRunLanes < len[u] ? l + kRunLanes : 0u)];
-        }
-#pragma unroll
-        for (uint32_t u = 0; u < U; ++u) {
-            const uint32_t tile = c0 + (j0 + u) * kRunGroups + g;
-            if (l < len[u]) one(x[u][0], t0[u], tile);
-            if (l + kRunLanes < len[u]) one(x[u][1], t0[u], tile);
-            for (uint32_t e = l + 2 * kRunLanes; e < len[u]; e += kRunLanes) one(a.ent[s[u] + e], t0[u], tile);
-        }
+    __device__ __forceinline__ Raw load(const BinArgs &, uint32_t i) const { return Raw{keys[i], meta[i]}; }
+    __device__ __forceinline__ uint32_t decode(const BinArgs &, const Raw &r, uint32_t, bool live, bool *use,
+                                               uint32_t *row, bool *write) const
+    {
+        const Op o = decode_op(r.row, live ? r.meta : 0u, rows, fields, max_scan);
+        *use = o.valid && o.row != hot;
+        *row = (uint32_t)o.row;
+        *write = o.kind == LTPG_KV_WRITE;
+        return (o.kind != LTPG_KV_NONE && !o.valid) ? 1u : 0u;
     }
-}
-
-template <typename W, bool DIRECT>
-__device__ __forceinline__ void bin_flags(const BinArgs &a, uint32_t b, W *s_w, uint32_t cap)
-{
-    const BinRun first = bin_run(a, b, 0);
-    for (uint32_t lo = 0; lo < (1u << a.row_bits); lo += cap) {
-        const uint32_t n = min(1u << a.row_bits, cap);
-        for (uint32_t r = threadIdx.x; r < n; r += kBinBlock) s_w[r] = (W)~(W)0;
-        __syncthreads();
-        for (uint32_t c0 = 0; c0 < a.tiles; c0 += kBinBlock)
-            bin_pass<W, false, DIRECT>(a, c0 ? bin_run(a, b, c0) : first, c0, s_w, lo, n);
-        __syncthreads();
-        for (uint32_t c0 = 0; c0 < a.tiles; c0 += kBinBlock)
-            bin_pass<W, true, DIRECT>(a, c0 ? bin_run(a, b, c0) : first, c0, s_w, lo, n);
-        __syncthreads();
-    }
-}
-
-__global__ __launch_bounds__(kBinBlock, 8) void kv_bin_flags_kernel(BinArgs a)
-{
-    __shared__ unsigned long long s_w[kBinRows / 2];
-    // blocks of one XCD take neighbouring buckets, whose runs and table
-    // entries share cache lines
-    const uint32_t x = blockIdx.x;
-    const uint32_t b = a.nb >= 8 ? (x & 7u) * (a.nb / 8) + (x >> 3) : x;
-    if (*a.unsorted == a.epoch)
-        bin_flags<unsigned long long, false>(a, b, s_w, kBinRows / 2);
-    else if (!a.rm && a.B >= (1u << a.tile_bits))
-        bin_flags<uint32_t, true>(a, b, reinterpret_cast<uint32_t *>(s_w), kBinRows);
-    else
-        bin_flags<uint32_t, false>(a, b, reinterpret_cast<uint32_t *>(s_w), kBinRows);
-}
+};
 
 // Read marking (fast form), one lane per op after every write has
 // registered.  A read of row x by t against w = W[x] of this epoch:
@@ -3213,43 +2876,27 @@ RegLayout reg_layout(const KvState &kv)
     return rl;
 }
 
-// Shape of the binned EXECUTE: 2^K >= rows; large epochs take 1024 buckets
-// and 16 ops per thread, smaller ones 256 buckets and 4 ops per thread (more
-// blocks), and more buckets where a bucket would exceed 2^kBinRowBits rows.
-BinShape kv_bin_shape(uint64_t rows, uint64_t ops)
-{
-    BinShape f;
-    uint32_t K = 0;
-    while (K < 27 && (1ull << K) < rows) ++K;
-    const bool large = ops >= kBinLargeOps;
-    const int rb = (int)K - (large ? 10 : 8);
-    f.row_bits = rb < 8 ? 8u : rb > (int)kBinRowBits ? kBinRowBits : (uint32_t)rb;
-    f.buckets = K > f.row_bits ? 1u << (K - f.row_bits) : 1u;
-    f.mask = (1u << (K > f.row_bits ? K : f.row_bits)) - 1u;
-    f.tile_bits = large || f.buckets >= 1024 ? kBinSlotBits : kBinSlotBits - 2;
-    f.tiles = (uint32_t)((ops + (1ull << f.tile_bits) - 1) >> f.tile_bits);
-    return f;
-}
-
 // Default EXECUTE shapes, from a sweep of rows x ops x (Zipf 0, 0.9, 0.99;
 // 50 and 90 % reads); times in us are register path (one lane per
 // transaction) / per-op register path / binned.
 //
 // Binned: its cost besides streaming is one short run per tile and bucket, so
 // it needs about 1024 ops per bucket.
-//   1M rows (256 buckets):    160K ops 22 / 16 / 16, 320K 28 / 27 / 17,
-//                             1.3M 77 / 60 / 29, 16M 396 / 294 / 166
-//   10M rows (1024 buckets):  650K ops 42 / 45 / 36, 1.3M 69 / 63 / 38,
-//                             4M 168 / 116 / 48, 16M 440 / 374 / 160
-//   100M rows (8192 buckets): 4M ops 180 / 143 / 131, 16M 504 / 447 / 425;
-//                             at Zipf 0.99, 334 / 328 / 409
-// Below 32K rows there are too few buckets to fill the chip (20K rows, 16M
-// ops, Zipf 0: 186 / 191 / 212).
+//   1M rows (256 buckets):    160K ops 23 / 17 / 15, 320K 29 / 27 / 16,
+//                             1.3M 78 / 61 / 27, 16M 407 / 295 / 151
+//   10M rows (64 to 512 hashed, 1024 from 2^22 ops):
+//                             160K ops 21 / 17 / 17, 320K 27 / 27 / 18,
+//                             650K 42 / 46 / 21, 4M 189 / 121 / 60,
+//                             16M 444 / 374 / 146
+//   100M rows (1024, 2048 hashed): 650K ops 40 / 48 / 34, 1.3M 64 / 64 / 38,
+//                             16M 512 / 446 / 338
+// (Zipf 0.9, 50 % reads; with 90 % reads at Zipf 0.99 the line is crossed at
+// about twice the ops.)  Below 32K rows there are too few buckets to fill the
+// chip (20K rows, 16M ops, Zipf 0: 186 / 191 / 212).
 bool kv_bin_auto(uint64_t rows, uint64_t ops)
 {
-    if (rows <= (1ull << 15) || rows > (1ull << 25) || ops >= (1ull << 31)) return false;
-    const uint64_t per = 1024ull * kv_bin_shape(rows, ops).buckets;
-    return ops >= (1ull << 18) && ops >= per;
+    if (rows <= (1ull << 15) || rows > (1ull << 28) || ops >= (1ull << 31)) return false;
+    return ops >= (1ull << 18) && ops >= 1024ull * bin_shape(rows, ops).buckets;
 }
 
 bool kv_execute_bins(const KvState &kv, const KvBatchDev &b)
@@ -3258,9 +2905,7 @@ bool kv_execute_bins(const KvState &kv, const KvBatchDev &b)
     if (!kv.bin.ent || kv.max_scan > 1 || !(kv.partitioned || (kv.auto_shape && kv_bin_auto(kv.rows, ops))) ||
         ops >= 0xFFFF0000ull)
         return false;
-    const BinShape f = kv_bin_shape(kv.rows, ops);
-    return ((uint64_t)f.tiles << f.tile_bits) <= kv.bin.cap_ent &&
-           (uint64_t)f.tiles * (f.buckets + 1) <= kv.bin.cap_off;
+    return bin_fits(kv.bin, bin_shape(kv.rows, ops));
 }
 
 namespace {
@@ -3275,45 +2920,17 @@ inline bool kv_per_op_auto(uint64_t ops) { return ops < (1ull << 18) || ops >= (
 hipError_t launch_kv_bin(const KvState &kv, const KvBatchDev &b, const EpochTag &e, DeviceCounters *ctr,
                          hipStream_t s, bool zero_counts)
 {
-    const uint64_t ops = (uint64_t)b.n_txns * b.n_slots;
-    const BinShape f = kv_bin_shape(kv.rows, ops);
+    const KvBinSource src = {b.keys, b.meta, kv.rows, kv.fields, kv.max_scan, kv.hot_row};
     BinArgs a;
-    a.keys = b.keys;
-    a.meta = b.meta;
+    a.width = b.request_major ? b.n_slots : b.n_txns;
+    a.n_ops = b.n_txns * b.n_slots;
+    a.rm = b.request_major;
     a.tids = b.tids;
     a.B = b.n_txns;
-    a.n_ops = (uint32_t)ops;
-    a.rows = kv.rows;
-    a.fields = kv.fields;
-    a.max_scan = kv.max_scan;
-    a.hot = kv.hot_row;
-    a.mask = f.mask;
-    a.row_bits = f.row_bits;
-    a.nb = f.buckets;
-    a.tiles = f.tiles;
-    a.tile_bits = f.tile_bits;
-    a.per.d = b.request_major ? b.n_slots : b.n_txns;
-    a.per.m = a.per.d > 1 ? (uint32_t)((1ull << 32) / a.per.d) : ~0u;
-    a.rm = b.request_major;
-    a.epoch = e.epoch;
-    a.ent = kv.bin.ent;
-    a.off = kv.bin.off;
-    a.unsorted = kv.bin.unsorted;
     a.doomed = kv.doomed;
     a.raw_flag = kv.raw_flag;
     a.war_flag = kv.war_flag;
-    a.ctr = ctr;
-    hipLaunchKernelGGL(kv_bin_order_kernel, dim3((b.n_txns + 4 * kBlock - 1) / (4 * kBlock)), dim3(kBlock), 0, s, a,
-                       zero_counts, kv.clear_flags);
-    const dim3 tiles(f.tiles), blk(kBinBlock);
-    if (f.tile_bits == kBinSlotBits && f.buckets <= 1024)
-        hipLaunchKernelGGL((kv_bin_kernel<16, 1024>), tiles, blk, 0, s, a);
-    else if (f.tile_bits == kBinSlotBits)
-        hipLaunchKernelGGL((kv_bin_kernel<16, 8192>), tiles, blk, 0, s, a);
-    else
-        hipLaunchKernelGGL((kv_bin_kernel<4, 1024>), tiles, blk, 0, s, a);
-    hipLaunchKernelGGL(kv_bin_flags_kernel, dim3(f.buckets), blk, 0, s, a);
-    return hipGetLastError();
+    return launch_bin(src, a, bin_shape(kv.rows, a.n_ops), kv.bin, e, ctr, zero_counts, kv.clear_flags, s);
 }
 
 }  // namespace

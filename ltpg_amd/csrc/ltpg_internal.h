@@ -66,6 +66,50 @@ struct EpochTag {
     uint8_t epoch;
 };
 
+// Binned EXECUTE (bin_execute.h): an entry packs a row within its bucket (at
+// most 2^kBinHashBits), a bit and a slot within its tile (2^kBinSlotBits);
+// rows up to 2^kBinRowBits per bucket have an array of minima in LDS.
+constexpr uint32_t kBinRowBits = 14;
+constexpr uint32_t kBinHashBits = 17;
+constexpr uint32_t kBinSlotBits = 14;
+struct BinShape {
+    uint32_t row_bits, buckets, mask, tile_bits, tiles;
+};
+struct BinBuffers {
+    uint64_t cap_ent = 0, cap_off = 0;
+    uint32_t *ent = nullptr;              // [cap_ent] binned operations, tile by tile
+    uint16_t *off = nullptr;              // [cap_off] starts of each bucket's run in each tile
+    uint32_t *unsorted = nullptr;         // epoch number of the last epoch whose TIDs were out of order
+};
+// Shape for `ops` operation slots on `rows` rows (2^K >= rows, K <= 30).
+// Large epochs with a row array each: 1024 buckets and 16 slots per thread;
+// smaller ones 256 buckets and 4 slots per thread (more blocks).  Where that
+// would take more rows per bucket than the array has, hashed buckets of at most
+// 5120 slots on average, as many as the rows need at least.
+inline BinShape bin_shape(uint64_t rows, uint64_t ops)
+{
+    BinShape f;
+    uint32_t K = 0;
+    while (K < 30 && (1ull << K) < rows) ++K;
+    const bool large = ops >= (1ull << 22);
+    uint32_t nb_bits = large ? 10 : 8;
+    if (K > nb_bits + kBinRowBits) {
+        nb_bits = 6;
+        while (nb_bits < 11 && (ops >> nb_bits) > 5120) ++nb_bits;
+        if (K > nb_bits + kBinHashBits) nb_bits = K - kBinHashBits;
+    }
+    f.row_bits = K > nb_bits + 8 ? K - nb_bits : 8;
+    f.buckets = K > f.row_bits ? 1u << (K - f.row_bits) : 1u;
+    f.mask = (1u << (K > f.row_bits ? K : f.row_bits)) - 1u;
+    f.tile_bits = large || f.buckets > 256 ? kBinSlotBits : kBinSlotBits - 2;
+    f.tiles = (uint32_t)((ops + (1ull << f.tile_bits) - 1) >> f.tile_bits);
+    return f;
+}
+inline bool bin_fits(const BinBuffers &b, const BinShape &f)
+{
+    return b.ent && ((uint64_t)f.tiles << f.tile_bits) <= b.cap_ent && (uint64_t)f.tiles * (f.buckets + 1) <= b.cap_off;
+}
+
 struct KvState {
     uint64_t rows = 0;
     uint32_t fields = 0;
@@ -117,13 +161,7 @@ struct KvState {
         unsigned long long *ent_me = nullptr; // [cap_entries] priority of each binned operation
         uint32_t *ent_key = nullptr;          // [cap_entries] row within its bucket << 1 | is-write
     } part;
-    // binned EXECUTE of point operations: buffers of an epoch's entries
-    struct Bin {
-        uint64_t cap_ent = 0, cap_off = 0;
-        uint32_t *ent = nullptr;              // [cap_ent] binned operations, tile by tile
-        uint16_t *off = nullptr;              // [cap_off] starts of each bucket's run in each tile
-        uint32_t *unsorted = nullptr;         // epoch number of the last epoch whose TIDs were out of order
-    } bin;
+    BinBuffers bin;                     // binned EXECUTE of point operations
     // no launch shape was asked for (ltpg_kv_set_tuning): sizes decide
     // (kv_bin_auto, kv_per_op_auto)
     bool auto_shape = true;
@@ -339,15 +377,6 @@ constexpr uint64_t kReadStageWords = 8ull << 20;
 constexpr uint32_t kPartShift = 13;
 constexpr uint32_t kPartMaxBuckets = 16384;
 constexpr uint32_t kPartSlice = 32768;
-// Binned EXECUTE: at most 2^kBinRowBits rows per bucket and 2^kBinSlotBits op
-// slots per tile (an entry packs both and a bit); "large" epochs.
-constexpr uint32_t kBinRowBits = 14;
-constexpr uint32_t kBinSlotBits = 14;
-constexpr uint64_t kBinLargeOps = 1ull << 22;
-struct BinShape {
-    uint32_t row_bits, buckets, mask, tile_bits, tiles;
-};
-BinShape kv_bin_shape(uint64_t rows, uint64_t ops);
 // Whether EXECUTE (fast form) of this batch takes the binned path.
 bool kv_execute_bins(const KvState &kv, const KvBatchDev &b);
 // Where the binned EXECUTE is the default (kv_kernels.hip).

@@ -20,7 +20,9 @@ pytestmark = pytest.mark.gpu
     (32_769, 20_003, 14),        # fewest rows, odd batch, partial last tile
     (70_000, 1_000_001 // 3, 1), # one slot
     (300_000, 65_539, 64),       # 2^22 ops and more: tiles of 16384
-    (9_000_000, 66_000, 16),     # 1024 buckets of 16384 rows
+    (9_000_000, 66_000, 64),     # 1024 buckets of 16384 rows
+    (9_000_000, 66_000, 16),     # 256 hashed buckets of 65536 rows
+    (9_000_000, 99_991, 20),     # 512 hashed buckets, tiles of 16384
 ], ids=lambda v: str(v))
 @pytest.mark.parametrize("tids", ["ordered", "shuffled", "equal"])
 def test_default_shape_matches_oracle(gpu, rows, B, S, tids):
@@ -56,6 +58,36 @@ def test_default_shape_matches_oracle(gpu, rows, B, S, tids):
             ok = (keys < rows) & (((meta >> 8) & 0xffff) < fields) & ((meta & 3) == L.KV_READ)
             read = (ok.reshape(S, B) & com).reshape(-1)
             np.testing.assert_array_equal(ctx.kv_read_values()[read], ora.read_values[read])
+        np.testing.assert_array_equal(ctx.kv_table_read(), table)
+
+
+@pytest.mark.parametrize("crowd", [4000, 8191, 8192, 40_000])
+@pytest.mark.parametrize("tids", ["ordered", "shuffled"])
+def test_crowded_hash_bucket_matches_oracle(gpu, crowd, tids):
+    """Binned EXECUTE with hashed buckets, 90 % of the operations in one
+    bucket: as many distinct rows there as its hash table nearly or exactly
+    holds, and more (that bucket then goes through its row arrays part by
+    part)."""
+    rows, B, S = 6_000_000, 20_000, 14  # 2^23 hashed rows, 64 buckets
+    rng = np.random.default_rng(crowd)
+    keys, meta, t = L.kv_generate(seed=crowd, rows=rows, fields=1, n_txns=B, n_slots=S, theta=0.0, read_pct=30)
+    inverse = pow(0x9E3779B1, -1, 1 << 23)
+    bucket = (np.arange(1 << 17, dtype=np.uint64) + np.uint64(5 << 17)) * np.uint64(inverse) % np.uint64(1 << 23)
+    bucket = bucket[bucket < rows][:crowd]
+    assert bucket.size == crowd
+    pick = rng.random(keys.size) < 0.9
+    keys[pick] = bucket[rng.integers(0, crowd, int(pick.sum()))]
+    if tids == "shuffled":
+        t = rng.permutation(t).astype(np.uint32)
+    table = kc.initial_table(rows, 1, 1)
+    with L.Context(workload=L.WORKLOAD_KV, kv_rows=rows, kv_fields=1, kv_field_bytes=4, max_txns=B,
+                   kv_max_slots=S) as ctx:
+        ctx.kv_table_load(table)
+        ctx.kv_submit(keys, meta, t, S)
+        ctx.epoch_run()
+        ctx.sync()
+        ora = oracle.kv_epoch(table, rows, 1, 1, keys, meta, t, S, inplace=True)
+        np.testing.assert_array_equal(ctx.commit_bitmap(), ora.bitmap)
         np.testing.assert_array_equal(ctx.kv_table_read(), table)
 
 
