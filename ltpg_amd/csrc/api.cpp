@@ -59,16 +59,15 @@ void free_kv(KvState &kv)
     free_bin(kv.bin);
 }
 
-// Buffers of the binned EXECUTE for every batch the context accepts.
-int kv_bin_prepare(ltpg_ctx *ctx)
+// Buffers for every batch of at most n: `shape` gives the shape of a size.
+// Buckets and tiles do not grow together, so sizes are taken from the largest
+// down, in steps finer than any change of shape.
+template <class Shape>
+int bin_alloc(BinBuffers *bin, uint64_t n, Shape shape, hipStream_t s)
 {
-    KvState &kv = ctx->kv;
-    if (kv.bin.ent) return LTPG_OK;
     BinBuffers p;
-    // buckets and tiles do not grow together: sizes from the largest down, in
-    // steps finer than any change of shape
-    for (uint64_t n = (uint64_t)kv.max_slots * ctx->cfg.max_txns; n; n -= n / 64 + 1) {
-        const BinShape f = bin_shape(kv.rows, n);
+    for (; n; n -= n / 64 + 1) {
+        const BinShape f = shape(n);
         p.cap_ent = std::max(p.cap_ent, (uint64_t)f.tiles << f.tile_bits);
         p.cap_off = std::max(p.cap_off, (uint64_t)f.tiles * (f.buckets + 1) * 66 / 64 + f.buckets + 1);
     }
@@ -78,10 +77,18 @@ int kv_bin_prepare(ltpg_ctx *ctx)
         free_bin(p);
         return rc;
     }
-    kv.bin = p;  // freed with the context
+    *bin = p;  // freed with the context
     // epoch 0 is never current
-    LTPG_HIP_TRY(launch_fill_u8(reinterpret_cast<uint8_t *>(p.unsorted), 4, 0, ctx->stream));
+    LTPG_HIP_TRY(launch_fill_u8(reinterpret_cast<uint8_t *>(p.unsorted), 4, 0, s));
     return LTPG_OK;
+}
+
+int kv_bin_prepare(ltpg_ctx *ctx)
+{
+    KvState &kv = ctx->kv;
+    if (kv.bin.ent) return LTPG_OK;
+    return bin_alloc(&kv.bin, (uint64_t)kv.max_slots * ctx->cfg.max_txns,
+                     [&](uint64_t ops) { return bin_shape(kv.rows, ops); }, ctx->stream);
 }
 
 int init_kv(ltpg_ctx *ctx)
@@ -153,6 +160,7 @@ uint64_t tpcc_rows(uint32_t W, uint32_t t) { return t == LTPG_TPCC_ITEM ? 100000
 
 void free_tpcc(TpccState &tp)
 {
+    free_bin(tp.bin);
     for (auto &t : tp.d.t) dev_free(t.data);
     dev_free(tp.d.regs);
     dev_free(tp.d.name_index);
@@ -227,6 +235,11 @@ int init_tpcc(ltpg_ctx *ctx)
     if ((rc = dev_alloc(&d.reads_sl, (uint64_t)kSlReads * B, "Stock-Level read values"))) return rc;
     if ((rc = dev_alloc(&d.bitmap_dl, (B + 63) / 64, "Delivery bitmap"))) return rc;
     if ((rc = dev_alloc(&d.reads_dl, (uint64_t)kDlReads * B, "Delivery read values"))) return rc;
+    // without memory for the bins every epoch takes the registers
+    if (!(c.flags & LTPG_FLAG_CONFLICT_COUNTS) && B >= kSplitTxns &&
+        bin_alloc(&tp.bin, B, [&](uint64_t n) { return stock_bin_shape(d.t[LTPG_TPCC_STOCK].rows, (uint32_t)n); },
+                  ctx->stream) == LTPG_ERR_NOMEM)
+        (void)hipGetLastError();  // dealt with
     LTPG_HIP_TRY(launch_fill_u8(d.war, B, 0, ctx->stream));
     LTPG_HIP_TRY(launch_fill_u64(d.regs, d.n_regs, ~0ull, ctx->stream));
     LTPG_HIP_TRY(launch_fill_u8(d.doomed, B, 0, ctx->stream));
@@ -1063,7 +1076,11 @@ static int tpcc_epoch_run(ltpg_ctx *ctx, uint32_t phase_mask)
     const bool ro = tp.ro.n_os + tp.ro.n_sl > 0, dl = tp.dl.n > 0;
     const uint32_t dl_base = tp.no.n + tp.pay.n + tp.ro.n_os + tp.ro.n_sl;
     if (phase_mask & LTPG_PHASE_EXECUTE) {
-        LTPG_HIP_TRY(launch_tpcc_execute(tp.d, tp.no, tp.pay, e, counts, tp.small_blocks, ctx->counters, s));
+        // Stock-Level reads the STOCK registers, which the split form leaves out
+        if (!counts && tp.ro.n_sl == 0 && tpcc_execute_split(tp.d, tp.bin, tp.no, tp.pay))
+            LTPG_HIP_TRY(launch_tpcc_execute_split(tp.d, tp.bin, tp.no, tp.pay, e, tp.small_blocks, ctx->counters, s));
+        else
+            LTPG_HIP_TRY(launch_tpcc_execute(tp.d, tp.no, tp.pay, e, counts, tp.small_blocks, ctx->counters, s));
         // Deliveries register after NewOrders and Payments, then read-only
         // transactions mark war on the registered writers
         if (dl) LTPG_HIP_TRY(launch_tpcc_delivery_execute(tp.d, tp.dl, dl_base, e, ctx->counters, s));

@@ -45,7 +45,8 @@
 //
 // A Source gives the operation of op slot i: load(i) its words (every slot
 // below n_ops may be loaded), decode() whether it registers, its row (< 2^32),
-// whether it is a write, and the slot's range errors.
+// whether it is a write, and the slot's range errors.  kSmallTiles: its shapes
+// are tiles of 4 slots per thread and at most 1024 buckets.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -449,9 +450,10 @@ __global__ __launch_bounds__(kBinBlock, 8) void bin_flags_kernel(BinArgs a)
 }
 
 // a: the caller's part of the arguments; `f` must fit `buf` (bin_fits).
+// check_order false: a kernel before has set *buf.unsorted if need be.
 template <class Source>
 hipError_t launch_bin(const Source &src, BinArgs a, const BinShape &f, const BinBuffers &buf, const EpochTag &e,
-                      DeviceCounters *ctr, bool zero_counts, bool clear, hipStream_t s)
+                      DeviceCounters *ctr, bool zero_counts, bool clear, bool check_order, hipStream_t s)
 {
     a.mask = f.mask;
     a.row_bits = f.row_bits;
@@ -465,15 +467,18 @@ hipError_t launch_bin(const Source &src, BinArgs a, const BinShape &f, const Bin
     a.off = buf.off;
     a.unsorted = buf.unsorted;
     a.ctr = ctr;
-    hipLaunchKernelGGL(bin_order_kernel, dim3((a.B + 4 * kOrderBlock - 1) / (4 * kOrderBlock)), dim3(kOrderBlock), 0, s,
-                       a, zero_counts, clear);
+    if (check_order)
+        hipLaunchKernelGGL(bin_order_kernel, dim3((a.B + 4 * kOrderBlock - 1) / (4 * kOrderBlock)), dim3(kOrderBlock),
+                           0, s, a, zero_counts, clear);
     const dim3 tiles(f.tiles), blk(kBinBlock);
-    if (f.tile_bits == kBinSlotBits && f.buckets <= kBinBlock)
-        hipLaunchKernelGGL((bin_kernel<Source, 16, kBinBlock>), tiles, blk, 0, s, a, src);
-    else if (f.tile_bits == kBinSlotBits)
-        hipLaunchKernelGGL((bin_kernel<Source, 16, 8192>), tiles, blk, 0, s, a, src);
-    else
+    if (f.tile_bits < kBinSlotBits) {
         hipLaunchKernelGGL((bin_kernel<Source, 4, kBinBlock>), tiles, blk, 0, s, a, src);
+    } else if constexpr (!Source::kSmallTiles) {
+        if (f.buckets <= kBinBlock)
+            hipLaunchKernelGGL((bin_kernel<Source, 16, kBinBlock>), tiles, blk, 0, s, a, src);
+        else
+            hipLaunchKernelGGL((bin_kernel<Source, 16, 8192>), tiles, blk, 0, s, a, src);
+    }
     if (f.row_bits > kBinRowBits)
         hipLaunchKernelGGL(bin_flags_kernel<true>, dim3(f.buckets), blk, 0, s, a);
     else

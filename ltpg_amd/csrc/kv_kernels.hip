@@ -863,6 +863,7 @@ __global__ __launch_bounds__(kPartBlock) void kv_part_flags_kernel(PartArgs a)
 // ---- binned EXECUTE of point operations (LTPG_TUNE_PARTITIONED, or the
 // ---- default shape of a large epoch; fast form, no scans; bin_execute.h) ---
 struct KvBinSource {
+    static constexpr bool kSmallTiles = false;
     const uint64_t *keys;
     const uint32_t *meta;
     uint64_t rows;
@@ -2930,7 +2931,7 @@ hipError_t launch_kv_bin(const KvState &kv, const KvBatchDev &b, const EpochTag 
     a.doomed = kv.doomed;
     a.raw_flag = kv.raw_flag;
     a.war_flag = kv.war_flag;
-    return launch_bin(src, a, bin_shape(kv.rows, a.n_ops), kv.bin, e, ctr, zero_counts, kv.clear_flags, s);
+    return launch_bin(src, a, bin_shape(kv.rows, a.n_ops), kv.bin, e, ctr, zero_counts, kv.clear_flags, true, s);
 }
 
 }  // namespace

@@ -35,6 +35,7 @@
 
 #include <algorithm>
 
+#include "bin_execute.h"
 #include "device_common.h"
 #include "ltpg_internal.h"
 
@@ -338,6 +339,187 @@ __global__ __launch_bounds__(BLK) void execute_kernel(TpccDev d, NeworderDev no,
         }
     }
     if (bad) atomicAdd(&ctr->range_errors, bad);
+}
+
+// ---- EXECUTE of a large epoch (kSplitTxns transactions and more, fast form,
+// ---- no Stock-Level) ---------------------------------------------------------
+//
+// execute_kernel is bound by random register accesses: of its 77 us at 2^17
+// NewOrders + 2^17 Payments on 64 warehouses about 49 are the 1.3M probes and
+// 0.7M atomics of the STOCK rows, the rest the atomics of the other rows.
+// STOCK rows are shared: the lines' STOCK writes are binned (bin_execute.h,
+// StockSource), with no register.  The other rows are mostly written once per
+// epoch (an order's ORDER, ORDERLINE, HISTORY and NEWORDER rows are new ones,
+// most customers pay once), which needs no atomic:
+//   claim_kernel   stores each write's priority into its row's register,
+//                  plainly; of several one lands last;
+//   settle_kernel  reads the registers back, and a write that finds another's
+//                  value registers with the atomic.
+// The value that stayed counts as the row's first registration: every other
+// writer of the row sees that it is not its own and lowers the register from
+// there, so the minimum remains and every writer but it is doomed, by
+// displacement or by what it finds.  The registers end as execute_kernel
+// leaves them, for the kernels that read them after (Deliveries, Order-Status).
+// 2^17 + 2^17 on 64 warehouses: claim 10, settle 12, bins 10 + 13 us.
+
+// The lines' STOCK writes (op_6_0): slot s of NewOrder q is line s.
+struct StockSource {
+    static constexpr bool kSmallTiles = true;
+    NeworderDev no;
+    uint64_t stock_rows, item_rows;
+    struct Raw {
+        uint32_t item, w, lines;
+    };
+    __device__ __forceinline__ Raw load(const BinArgs &a, uint32_t i) const
+    {
+        uint32_t q;
+        const uint32_t line = fast_div(a.per, i, &q);
+        const uint64_t at = (uint64_t)line * no.line_stride + q;
+        return Raw{no.OL_I_ID[at], no.OL_SUPPLY_W_ID[at], no.O_OL_CNT[q]};
+    }
+    __device__ __forceinline__ uint32_t decode(const BinArgs &a, const Raw &r, uint32_t i, bool live, bool *use,
+                                               uint32_t *row, bool *write) const
+    {
+        uint32_t q;
+        const bool has = live && fast_div(a.per, i, &q) < r.lines;
+        const uint64_t sr = (uint64_t)r.w * 100000 + r.item;
+        *use = has && sr < stock_rows;
+        *row = (uint32_t)sr;
+        *write = true;
+        return has ? (r.item >= item_rows) + !*use : 0u;  // op_5_0 and op_6_0
+    }
+};
+
+// What the claiming and the settling block share: BLK / 4 orders, whose
+// header words come in along the orders (coalesced) and go to LDS; each
+// order's lines then to 16 adjacent lanes.
+template <uint32_t BLK>
+struct OrderTile {
+    static constexpr uint32_t kOrders = BLK / 4, kPass = kOrders * 16 / BLK;
+    uint32_t w[kOrders], first_line[kOrders], lines[kOrders], tid[kOrders];
+    __device__ __forceinline__ void load(const NeworderDev &no, uint32_t q0)
+    {
+        const uint32_t o = threadIdx.x, q = q0 + o;
+        if (o >= kOrders) return;
+        const bool in = q < no.n;
+        w[o] = in ? no.W_ID[q] : 0u;
+        first_line[o] = in ? no.O_OL_ID[q] : 0u;
+        lines[o] = in ? no_lines(no, q) : 0u;
+        tid[o] = in ? no.TID[q] : 0u;
+    }
+    // pass k of this thread: its order, and its line's ORDERLINE row
+    __device__ __forceinline__ uint32_t order(uint32_t k) const { return k * (BLK / 16) + threadIdx.x / 16; }
+    __device__ __forceinline__ bool line_row(uint32_t k, uint64_t *row) const
+    {
+        const uint32_t o = order(k), j = threadIdx.x % 16;
+        *row = (uint64_t)w[o] * 450000 + first_line[o] + j;
+        return j < lines[o];  // at most 15
+    }
+};
+
+template <uint32_t BLK>
+__global__ __launch_bounds__(BLK) void claim_kernel(TpccDev d, NeworderDev no, PaymentDev pay, uint32_t tag,
+                                                      uint8_t epoch, uint32_t no_blocks, uint32_t *unsorted,
+                                                      DeviceCounters *ctr)
+{
+    __shared__ OrderTile<BLK> s_tile;
+    // the epoch's commit counts start at zero (CHECK adds to them)
+    if (blockIdx.x == 0) zero_epoch_counts(ctr, BLK);
+    uint32_t bad = 0;
+    if (blockIdx.x < no_blocks) {
+        const uint32_t q0 = blockIdx.x * OrderTile<BLK>::kOrders, q = q0 + threadIdx.x;
+        s_tile.load(no, q0);
+        if (threadIdx.x < OrderTile<BLK>::kOrders && q < no.n) {
+            // header slots 0..4
+            const NoRows r = no_rows(no, q);
+            const uint32_t tid = no.TID[q], next = no.TID[q + 1 < no.n ? q + 1 : q];
+            const unsigned long long me = priority(tag, tid, q);
+            if (tid > next) *unsorted = epoch;  // for the binned STOCK writes
+            bad += (r.wh >= d.t[WH].rows) + (r.di >= d.t[DI].rows) + (r.cu >= d.t[CU].rows);
+            // NEWORDER insert: a write (waw) under INTENDED; under REFERENCE
+            // its R register is never consulted
+            if (r.no >= d.t[NO].rows) bad++;
+            else if (d.rules == LTPG_RULES_INTENDED) d.regs[d.off_new + r.no] = me;
+            if (r.od < d.t[OR].rows) d.regs[d.off_order + r.od] = me;
+            else bad++;
+        }
+        __syncthreads();
+#pragma unroll
+        for (uint32_t k = 0; k < OrderTile<BLK>::kPass; k++) {
+            uint64_t lr;
+            if (!s_tile.line_row(k, &lr)) continue;
+            const uint32_t o = s_tile.order(k);
+            if (lr < d.t[OL].rows) d.regs[d.off_line + lr] = priority(tag, s_tile.tid[o], q0 + o);
+            else bad++;
+        }
+    } else {
+        const uint32_t p = (blockIdx.x - no_blocks) * BLK + threadIdx.x;
+        if (p < pay.n) {
+            const unsigned long long me = priority(tag, pay.TID[p], no.n + p);
+            const PayRows r = pay_rows(d, pay, p);
+            const bool cok = r.cu < d.t[CU].rows, hok = r.hi < d.t[HI].rows;
+            // slots 0 to 5 in pairs, and the HISTORY insert
+            bad += 2 * ((r.wh >= d.t[WH].rows) + (r.di >= d.t[DI].rows) + !cok) + !hok;
+            if (cok) *cust_w(d, r.cu) = me;
+            if (hok) d.regs[d.off_hist + r.hi] = me;
+        }
+    }
+    if (bad) atomicAdd(&ctr->range_errors, bad);
+}
+
+// A register that holds another writer's value is contended.  (A value read
+// before a concurrent atomicMin of this kernel is at worst too high.)
+__device__ __forceinline__ bool settle(unsigned long long *r, unsigned long long cur, unsigned long long me,
+                                       uint32_t tag, uint8_t *doomed, uint8_t epoch)
+{
+    return cur != me && finish_write(r, cur, me, tag, doomed, epoch);
+}
+
+template <uint32_t BLK>
+__global__ __launch_bounds__(BLK) void settle_kernel(TpccDev d, NeworderDev no, PaymentDev pay, uint32_t tag,
+                                                       uint8_t epoch, uint32_t no_blocks)
+{
+    __shared__ OrderTile<BLK> s_tile;
+    if (blockIdx.x < no_blocks) {
+        constexpr uint32_t kPass = OrderTile<BLK>::kPass;
+        const uint32_t q0 = blockIdx.x * OrderTile<BLK>::kOrders, q = q0 + threadIdx.x;
+        s_tile.load(no, q0);
+        if (threadIdx.x < OrderTile<BLK>::kOrders && q < no.n) {
+            const NoRows r = no_rows(no, q);
+            const unsigned long long me = priority(tag, no.TID[q], q);
+            unsigned long long *rn = d.regs + d.off_new + r.no, *ro = d.regs + d.off_order + r.od;
+            const bool nok = d.rules == LTPG_RULES_INTENDED && r.no < d.t[NO].rows, ook = r.od < d.t[OR].rows;
+            const unsigned long long cn = nok ? *rn : me, co = ook ? *ro : me;
+            const bool wn = settle(rn, cn, me, tag, d.doomed, epoch), wo = settle(ro, co, me, tag, d.doomed, epoch);
+            if (wn || wo) d.doomed[q] = epoch;
+        }
+        __syncthreads();
+        unsigned long long *rl[kPass], cl[kPass];
+        bool lok[kPass];
+#pragma unroll
+        for (uint32_t k = 0; k < kPass; k++) {
+            uint64_t lr;
+            lok[k] = s_tile.line_row(k, &lr) && lr < d.t[OL].rows;
+            rl[k] = d.regs + d.off_line + (lok[k] ? lr : 0);
+            cl[k] = *rl[k];
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < kPass; k++) {
+            const uint32_t o = s_tile.order(k);
+            if (lok[k] && settle(rl[k], cl[k], priority(tag, s_tile.tid[o], q0 + o), tag, d.doomed, epoch))
+                d.doomed[q0 + o] = epoch;
+        }
+    } else {
+        const uint32_t p = (blockIdx.x - no_blocks) * BLK + threadIdx.x;
+        if (p >= pay.n) return;
+        const unsigned long long me = priority(tag, pay.TID[p], no.n + p);
+        const PayRows r = pay_rows(d, pay, p);
+        const bool cok = r.cu < d.t[CU].rows, hok = r.hi < d.t[HI].rows;
+        unsigned long long *rc = cust_w(d, cok ? r.cu : 0), *rh = d.regs + d.off_hist + (hok ? r.hi : 0);
+        const unsigned long long cc = cok ? *rc : me, ch = hok ? *rh : me;
+        const bool wc = settle(rc, cc, me, tag, d.doomed, epoch), wh = settle(rh, ch, me, tag, d.doomed, epoch);
+        if (wc || wh) d.doomed[no.n + p] = epoch;
+    }
 }
 
 // ---- CHECK + read-out of committed reads -------------------------------------
@@ -943,6 +1125,60 @@ void execute_at(const TpccDev &d, const NeworderDev &no, const PaymentDev &pay, 
     else
         hipLaunchKernelGGL((execute_kernel<false, BLK>), dim3(blocks), dim3(BLK), 0, s, d, no, pay, e.tag, e.epoch,
                            no_blocks, ctr);
+}
+
+// Shape of the binned STOCK writes: small tiles (many blocks for a batch of a
+// few 100K lines) and as many buckets as give each a row array, 256 to 1024;
+// hashed beyond.
+BinShape stock_bin_shape(uint64_t stock_rows, uint32_t n_neworder)
+{
+    BinShape f;
+    uint32_t K = 0;
+    while ((1ull << K) < stock_rows) ++K;
+    const uint32_t nb_bits = std::min(10u, std::max(8u, K > kBinRowBits ? K - kBinRowBits : 0u));
+    f.row_bits = K - nb_bits;
+    f.buckets = 1u << nb_bits;
+    f.mask = (1u << K) - 1u;
+    f.tile_bits = kBinSlotBits - 2;
+    f.tiles = (uint32_t)(((uint64_t)n_neworder * LTPG_TPCC_MAX_LINES + (1u << f.tile_bits) - 1) >> f.tile_bits);
+    return f;
+}
+
+bool tpcc_execute_split(const TpccDev &d, const BinBuffers &bin, const NeworderDev &no, const PaymentDev &pay)
+{
+    if (no.n + pay.n < kSplitTxns) return false;
+    if (no.n == 0) return true;
+    const BinShape f = stock_bin_shape(d.t[ST].rows, no.n);
+    return f.row_bits <= kBinHashBits && bin_fits(bin, f);
+}
+
+template <uint32_t BLK>
+void execute_split_at(const TpccDev &d, const NeworderDev &no, const PaymentDev &pay, const EpochTag &e,
+                      uint32_t *unsorted, DeviceCounters *ctr, hipStream_t s)
+{
+    const uint32_t no_blocks = (no.n + BLK / 4 - 1) / (BLK / 4), blocks = no_blocks + (pay.n + BLK - 1) / BLK;
+    hipLaunchKernelGGL(claim_kernel<BLK>, dim3(blocks), dim3(BLK), 0, s, d, no, pay, e.tag, e.epoch, no_blocks,
+                       unsorted, ctr);
+    hipLaunchKernelGGL(settle_kernel<BLK>, dim3(blocks), dim3(BLK), 0, s, d, no, pay, e.tag, e.epoch, no_blocks);
+}
+
+hipError_t launch_tpcc_execute_split(const TpccDev &d, const BinBuffers &bin, const NeworderDev &no,
+                                     const PaymentDev &pay, const EpochTag &e, bool small, DeviceCounters *ctr,
+                                     hipStream_t s)
+{
+    if (small) execute_split_at<64>(d, no, pay, e, bin.unsorted, ctr, s);
+    else execute_split_at<kBlock>(d, no, pay, e, bin.unsorted, ctr, s);
+    if (no.n == 0) return hipGetLastError();
+    const StockSource src = {no, d.t[ST].rows, d.t[IT].rows};
+    BinArgs a;
+    a.width = no.n;
+    a.n_ops = no.n * LTPG_TPCC_MAX_LINES;
+    a.rm = false;
+    a.tids = no.TID;
+    a.B = no.n;
+    a.doomed = d.doomed;
+    a.raw_flag = a.war_flag = nullptr;  // no reads
+    return launch_bin(src, a, stock_bin_shape(d.t[ST].rows, no.n), bin, e, ctr, false, false, false, s);
 }
 
 hipError_t launch_tpcc_execute(const TpccDev &d, const NeworderDev &no, const PaymentDev &pay, const EpochTag &e,
