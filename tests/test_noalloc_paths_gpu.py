@@ -7,7 +7,6 @@ import ctypes
 
 import numpy as np
 import pytest
-import torch
 
 import ltpg_amd as L
 from oracle import oracle
@@ -16,8 +15,24 @@ from tests import kvcases as kc
 pytestmark = pytest.mark.gpu
 
 
+class Hip:
+    """The runtime's stream and graph calls that the captured replays need."""
+
+    def __init__(self):
+        self.lib = ctypes.CDLL("libamdhip64.so")
+
+    def __call__(self, name, *args):
+        rc = getattr(self.lib, name)(*args)
+        assert rc == 0, (name, rc)
+
+    def new(self, name, *args):
+        out = ctypes.c_void_p()
+        self(name, ctypes.byref(out), *args)
+        return out
+
+
 class Call:
-    def __init__(self, rows, fields, fw, B, S, seed, theta=0.8, shuffled=False, bad=0):
+    def __init__(self, ctx, rows, fields, fw, B, S, seed, theta=0.8, shuffled=False, bad=0):
         self.rows, self.fields, self.fw, self.B, self.S = rows, fields, fw, B, S
         keys, meta, tids = L.kv_generate(seed=seed, rows=rows, fields=fields, n_txns=B, n_slots=S, min_ops=1,
                                          max_ops=S, theta=theta, distinct_keys=False)
@@ -27,36 +42,46 @@ class Call:
         meta[:bad] = L.kv_meta(L.KV_READ, 0)
         self.bad, self.batch = bad, (keys, meta, tids)
         self.table0 = kc.initial_table(rows, fields, fw)
-        dev = [torch.from_numpy(a.view(np.int64 if a.dtype.itemsize == 8 else np.int32)).cuda() for a in self.batch]
-        self.dev = dev
-        self.table = torch.from_numpy(self.table0.view(np.int32)).cuda()
-        self.bitmap = torch.full(((B + 63) // 64,), -1, dtype=torch.int64, device="cuda")
-        self.reads = torch.zeros(B * S * fw, dtype=torch.int32, device="cuda")
-        self.result = torch.full((2,), -1, dtype=torch.int32, device="cuda")
-        self.struct = L.KvBatch(B, S, *(d.data_ptr() for d in dev))
+        self.dev = L.DeviceKvBatch(ctx, keys, meta, tids, S)
+        self.out = [np.full(self.table0.shape, 0, np.uint32), np.full((B + 63) // 64, -1, np.int64).view(np.uint64),
+                    np.zeros(B * S * fw, np.uint32), np.full(2, -1, np.int32).view(np.uint32)]
+        self.bufs = [L.DeviceBuffer(ctx, a.nbytes) for a in self.out]
+        self.reset()
+        for k in (1, 2, 3):
+            self.bufs[k].upload(self.out[k])
+        self.struct = self.dev.struct()
 
-    def run(self, result=True):
-        rc = L.lib.ltpg_kv_epoch_noalloc(self.table.data_ptr(), self.rows, self.fields, 4 * self.fw,
-                                         ctypes.byref(self.struct), L.VALUES_RMW, self.bitmap.data_ptr(),
-                                         self.reads.data_ptr(), self.result.data_ptr() if result else None,
-                                         torch.cuda.current_stream().cuda_stream)
+    def reset(self):
+        self.bufs[0].upload(self.table0)
+
+    def run(self, result=True, stream=None):
+        table, bitmap, reads, res = (ctypes.c_void_p(b.ptr) for b in self.bufs)
+        rc = L.lib.ltpg_kv_epoch_noalloc(table, self.rows, self.fields, 4 * self.fw, ctypes.byref(self.struct),
+                                         L.VALUES_RMW, bitmap, reads, res if result else None, stream)
         assert rc == L.OK, L.lib.ltpg_last_error()
 
+    def free(self):
+        self.dev.free()
+        for b in self.bufs:
+            b.free()
+
     def check(self, epochs=1, result=True):
-        torch.cuda.synchronize()
+        for buf, a in zip(self.bufs, self.out):
+            buf.download(a)
+        table_out, bitmap, reads, res = self.out
         table = self.table0.copy()
         for _ in range(epochs):
             ora = oracle.kv_epoch(table, self.rows, self.fields, self.fw, *self.batch, self.S, inplace=True)
-        np.testing.assert_array_equal(self.bitmap.cpu().numpy().view(np.uint64), ora.bitmap)
-        np.testing.assert_array_equal(self.table.cpu().numpy().view(np.uint32), table)
+        np.testing.assert_array_equal(bitmap, ora.bitmap)
+        np.testing.assert_array_equal(table_out, table)
         com = np.unpackbits(ora.bitmap.view(np.uint8), bitorder="little")[:self.B].astype(bool)
         keys, meta, _ = self.batch
         read = ((meta & 3) == L.KV_READ) & (keys < self.rows) & np.tile(com, self.S)
-        got = self.reads.cpu().numpy().view(np.uint32).reshape(-1, self.fw)
+        got = reads.reshape(-1, self.fw)
         np.testing.assert_array_equal(got[read], ora.read_values.reshape(-1, self.fw)[read])
         assert not got[~read].any(), "only committed reads are written"
         if result:
-            assert self.result.cpu().tolist() == [ora.commit_count, self.bad]
+            assert res.tolist() == [ora.commit_count, self.bad]
 
 
 @pytest.mark.parametrize("rows,fw,B,S", [
@@ -69,30 +94,42 @@ class Call:
     (200_000, 1, 1 << 20, 17),       # more op slots than the binned path holds
 ], ids=lambda v: str(v))
 def test_noalloc_paths_match_oracle(gpu, rows, fw, B, S):
-    for seed, shuffled in ((1, False), (2, True), (3, False)):
-        if B * S > 1 << 24 and seed > 1:
-            break
-        c = Call(rows, 2, fw, B, S, seed, shuffled=shuffled, bad=3 if seed == 1 else 0)
-        c.run(result=seed != 2)
-        c.check(result=seed != 2)
+    hip = Hip()
+    with L.Context(workload=L.WORKLOAD_KV, kv_rows=64, kv_fields=1, max_txns=64, kv_max_slots=1) as ctx:
+        for seed, shuffled in ((1, False), (2, True), (3, False)):
+            if B * S > 1 << 24 and seed > 1:
+                break
+            c = Call(ctx, rows, 2, fw, B, S, seed, shuffled=shuffled, bad=3 if seed == 1 else 0)
+            c.run(result=seed != 2)
+            hip("hipDeviceSynchronize")
+            c.check(result=seed != 2)
+            c.free()
 
 
 @pytest.mark.parametrize("rows,B,S", [(2000, 100, 5), (20_000, 3000, 6), (100_000, 40_000, 6)])
 def test_noalloc_captured_replays_match_oracle(gpu, rows, B, S):
-    c = Call(rows, 2, 3, B, S, 5)
-    other = Call(rows, 2, 3, B, S, 6, shuffled=True)
-    s = torch.cuda.Stream()
-    with torch.cuda.stream(s):
-        c.run()
-        s.synchronize()
-        c.table.copy_(torch.from_numpy(c.table0.view(np.int32)))
-        g = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(g, stream=s):
-            c.run()
+    hip = Hip()
+    with L.Context(workload=L.WORKLOAD_KV, kv_rows=64, kv_fields=1, max_txns=64, kv_max_slots=1) as ctx:
+        c = Call(ctx, rows, 2, 3, B, S, 5)
+        other = Call(ctx, rows, 2, 3, B, S, 6, shuffled=True)
+        s = hip.new("hipStreamCreate")
+        c.run(stream=s)
+        hip("hipStreamSynchronize", s)
+        c.reset()
+        hip("hipStreamBeginCapture", s, 0)
+        c.run(stream=s)
+        graph = ctypes.c_void_p()
+        hip("hipStreamEndCapture", s, ctypes.byref(graph))
+        run = hip.new("hipGraphInstantiate", graph, None, None, ctypes.c_size_t(0))
         for k in range(1, 4):  # an eager call of another batch on the same scratch between replays
-            g.replay()
-            s.synchronize()
+            hip("hipGraphLaunch", run, s)
+            hip("hipStreamSynchronize", s)
             c.check(epochs=k)
-            other.run()
-            s.synchronize()
+            other.run(stream=s)
+            hip("hipStreamSynchronize", s)
             other.check(epochs=k)
+        hip("hipGraphExecDestroy", run)
+        hip("hipGraphDestroy", graph)
+        hip("hipStreamDestroy", s)
+        c.free()
+        other.free()
