@@ -27,10 +27,11 @@
  *   - A context is single-threaded: the caller serialises calls on one
  *     context.  Separate contexts are independent.
  *   - The library owns every device allocation.  Batches given with
- *     LTPG_MEM_HOST are copied to the device before the call returns (the
- *     caller may reuse its buffers then), into one of two device slots on a
- *     copy stream, so the copy overlaps the previous epoch still running on
- *     the device; pinned host memory copies at full PCIe speed.  Batches
+ *     LTPG_MEM_HOST are copied before the call returns (the caller may reuse
+ *     its buffers then), into one of two device slots; the copy overlaps the
+ *     previous epoch if that still runs on the device.  Small batches go
+ *     through pinned memory of the context (4 MB, from the first such batch
+ *     on); large ones in pinned host memory copy at full PCIe speed.  Batches
  *     given with LTPG_MEM_DEVICE are read in place and must stay valid until
  *     ltpg_sync() returns.
  *   - TIDs are u32 priorities; a lower TID wins.  The reference relies on

@@ -32,6 +32,30 @@ void free_bin(BinBuffers &b)
     dev_free(b.unsorted);
 }
 
+constexpr uint64_t kReadbackBytes = 256u << 10;  // the bits of 2^20 transactions are 128 KB
+
+// The context's pinned part for results; without it they are copied directly.
+void alloc_readback(ltpg_ctx *ctx)
+{
+    if (hipHostMalloc(reinterpret_cast<void **>(&ctx->readback), kReadbackBytes + 64,
+                      hipHostMallocCoherent | hipHostMallocMapped) == hipSuccess) {
+        std::memset(ctx->readback + kReadbackBytes, 0, 64);
+    } else {
+        (void)hipGetLastError();
+        ctx->readback = nullptr;
+    }
+}
+
+// The device block of a host batch: each array on a line of its own.
+uint64_t batch_row(uint64_t bytes) { return (bytes + 255) & ~255ull; }
+uint64_t kv_batch_bytes(uint64_t slots, uint64_t txns)
+{
+    return batch_row(slots * txns * 8) + batch_row(slots * txns * 4) + batch_row(txns * 4);
+}
+// max_txns NewOrders and Payments (or Order-Status and Stock-Level) together
+uint64_t np_batch_bytes(uint64_t txns) { return 53 * txns * 4 + 63 * 256; }
+uint64_t ro_batch_bytes(uint64_t txns) { return 6 * txns * 4 + 9 * 256; }
+
 void free_kv(KvState &kv)
 {
     dev_free(kv.table);
@@ -44,11 +68,7 @@ void free_kv(KvState &kv)
     dev_free(kv.bitmap);
     dev_free(kv.conflicts);
     dev_free(kv.commit_list);
-    for (int k = 0; k < 2; k++) {
-        dev_free(kv.keys_buf[k]);
-        dev_free(kv.meta_buf[k]);
-        dev_free(kv.tids_buf[k]);
-    }
+    for (int k = 0; k < 2; k++) dev_free(kv.batch_buf[k]);
     dev_free(kv.hot_acc);
     dev_free(kv.part.count);
     dev_free(kv.part.start);
@@ -125,9 +145,7 @@ int init_kv(ltpg_ctx *ctx)
     if ((rc = dev_alloc(&kv.bitmap, (B + 63) / 64, "kv bitmap"))) return rc;
     if ((rc = dev_alloc(&kv.conflicts, B, "kv conflicts"))) return rc;
     if ((rc = dev_alloc(&kv.commit_list, B, "kv commit list"))) return rc;
-    if ((rc = dev_alloc(&kv.keys_buf[0], S * B, "kv keys"))) return rc;
-    if ((rc = dev_alloc(&kv.meta_buf[0], S * B, "kv meta"))) return rc;
-    if ((rc = dev_alloc(&kv.tids_buf[0], B, "kv tids"))) return rc;
+    if ((rc = dev_alloc(&kv.batch_buf[0], kv_batch_bytes(S, B), "kv batch"))) return rc;
     if (kv.hot_row != LTPG_NO_HOT_ROW) {
         if ((rc = dev_alloc(&kv.hot_acc, (uint64_t)kCounterStripes * kv.fields, "hot-row accumulators"))) return rc;
         LTPG_HIP_TRY(hipMemsetAsync(kv.hot_acc, 0, (uint64_t)kCounterStripes * kv.fields * 4, ctx->stream));
@@ -174,8 +192,7 @@ void free_tpcc(TpccState &tp)
     dev_free(tp.d.reads_pay);
     dev_free(tp.d.cid);
     for (int k = 0; k < 2; k++) {
-        dev_free(tp.no_buf[k]);
-        dev_free(tp.pay_buf[k]);
+        dev_free(tp.np_buf[k]);
         dev_free(tp.ro_buf[k]);
         dev_free(tp.dl_buf[k]);
     }
@@ -225,9 +242,8 @@ int init_tpcc(ltpg_ctx *ctx)
     if ((rc = dev_alloc(&d.reads_no, (uint64_t)kNoReads * B, "NewOrder read values"))) return rc;
     if ((rc = dev_alloc(&d.reads_pay, (uint64_t)kPayReads * B, "Payment read values"))) return rc;
     if ((rc = dev_alloc(&d.cid, B, "Payment C_ID"))) return rc;
-    if ((rc = dev_alloc(&tp.no_buf[0], 53 * B, "NewOrder batch"))) return rc;
-    if ((rc = dev_alloc(&tp.pay_buf[0], 10 * B, "Payment batch"))) return rc;
-    if ((rc = dev_alloc(&tp.ro_buf[0], 9 * B, "read-only batches"))) return rc;
+    if ((rc = dev_alloc(&tp.np_buf[0], np_batch_bytes(B), "NewOrder and Payment batches"))) return rc;
+    if ((rc = dev_alloc(&tp.ro_buf[0], ro_batch_bytes(B), "read-only batches"))) return rc;
     if ((rc = dev_alloc(&d.war, B, "read-only war flags"))) return rc;
     if ((rc = dev_alloc(&d.bitmap_os, (B + 63) / 64, "Order-Status bitmap"))) return rc;
     if ((rc = dev_alloc(&d.bitmap_sl, (B + 63) / 64, "Stock-Level bitmap"))) return rc;
@@ -452,6 +468,7 @@ int ltpg_create(const ltpg_config *cfg, ltpg_ctx **out)
             break;
         }
         ctx->stream = ctx->own_stream;
+        alloc_readback(ctx);
         if ((rc = dev_alloc(&ctx->counters, 1, "counters"))) break;
         e = hipMemsetAsync(ctx->counters, 0, sizeof(DeviceCounters), ctx->stream);
         if (e != hipSuccess) {
@@ -497,6 +514,8 @@ int ltpg_destroy(ltpg_ctx *ctx)
         if (ctx->xfer_copied[k]) (void)hipEventDestroy(ctx->xfer_copied[k]);
         if (ctx->xfer_released[k]) (void)hipEventDestroy(ctx->xfer_released[k]);
     }
+    if (ctx->stage) (void)hipHostFree(ctx->stage);
+    if (ctx->readback) (void)hipHostFree(ctx->readback);
     if (ctx->own_stream) (void)hipStreamDestroy(ctx->own_stream);
     delete ctx;
     return LTPG_OK;
@@ -508,6 +527,7 @@ int ltpg_set_stream(ltpg_ctx *ctx, void *hip_stream)
     if (rc) return rc;
     LTPG_HIP_TRY(hipStreamSynchronize(ctx->stream));
     ctx->stream = hip_stream ? static_cast<hipStream_t>(hip_stream) : ctx->own_stream;
+    ctx->quiet = false;
     return LTPG_OK;
 }
 
@@ -939,16 +959,35 @@ int ltpg_tpcc_set_tuning(ltpg_ctx *ctx, uint32_t flags)
 
 namespace {
 
+// A stream under capture can neither be waited for nor take a host batch.
+int refuse_capture(ltpg_ctx *ctx)
+{
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    LTPG_HIP_TRY(hipStreamIsCapturing(ctx->stream, &status));
+    if (status != hipStreamCaptureStatusNone) LTPG_FAIL(LTPG_ERR_DEVICE, "the context's stream is being captured");
+    return LTPG_OK;
+}
+
 // Transport of host-resident batches.  The reference keeps two device query
 // slots and copies the batch of epoch e+1 into one while epoch e runs on the
 // other (TPCC-allopt-final/Query.h:532-605, Predefine.h:18-19).  Here a host
-// submit takes the slot the epoch before last used, copies into it on the
-// context's copy stream once that epoch is done with it, and makes its own
-// epoch's kernels (on the context stream) wait for the copy: the copy of a
-// batch overlaps the epoch still running on the other slot.  The submit
-// returns once its copy is done, so the caller may reuse its buffers at once
-// (pageable memory is staged by the runtime; pinned memory goes at full
-// PCIe speed), without waiting for the device to go idle.
+// submit takes the slot the epoch before last used.  While the context stream
+// still runs an epoch, the batch is copied on the context's copy stream once
+// the slot's epoch is done with it, and its own epoch's kernels wait for the
+// copy, so that it overlaps the epoch on the other slot.  With the stream idle
+// there is nothing to overlap: the copy goes on the context stream itself,
+// which saves the wait of one stream for the other (1 MB 51 us against 77,
+// 64 KB 33 against 62).
+//
+// A batch of up to kStageBytes is packed into pinned memory and goes to the
+// device as one copy; array by array (63 of a NewOrder and Payment batch) each
+// costs the host a transfer (5,000 NewOrders and 5,000 Payments: a submit of
+// 618 us, packed 37; 16,000 key-value transactions of 8 ops 84 us, packed 33).  The caller's buffers are free at once, and
+// the part of the slot is packed again only after its copy is done.  Larger
+// batches are copied array by array, and the submit returns once that is done
+// (pageable memory is staged by the runtime, whose copy of 8 MB takes 241 us
+// against 278 through the pinned part; caller's pinned memory goes at full
+// PCIe speed).
 int xfer_begin(ltpg_ctx *ctx, int *slot)
 {
     if (!ctx->copy_stream) {
@@ -958,27 +997,92 @@ int xfer_begin(ltpg_ctx *ctx, int *slot)
             LTPG_HIP_TRY(hipEventCreateWithFlags(&ctx->xfer_released[k], hipEventDisableTiming));
         }
     }
+    int rc = refuse_capture(ctx);
+    if (rc) return rc;
+    if (!ctx->quiet) {
+        const hipError_t busy = hipStreamQuery(ctx->stream);
+        if (busy == hipErrorNotReady)
+            (void)hipGetLastError();
+        else
+            LTPG_HIP_TRY(busy);
+        ctx->quiet = busy == hipSuccess;
+    }
     const int k = ctx->xfer_slot ^ 1;
     // everything queued so far -- the epoch on the other slot and all before
     // it -- is what must finish before the other slot is free again
     LTPG_HIP_TRY(hipEventRecord(ctx->xfer_released[k ^ 1], ctx->stream));
     ctx->xfer_released_set[k ^ 1] = true;
-    if (ctx->xfer_released_set[k]) LTPG_HIP_TRY(hipStreamWaitEvent(ctx->copy_stream, ctx->xfer_released[k], 0));
+    ctx->xfer_in_order = ctx->quiet;
+    if (!ctx->xfer_in_order && ctx->xfer_released_set[k])
+        LTPG_HIP_TRY(hipStreamWaitEvent(ctx->copy_stream, ctx->xfer_released[k], 0));
     ctx->xfer_slot = k;
+    ctx->stage_used = 0;
     *slot = k;
     return LTPG_OK;
 }
 
-// The slot's copies are queued on the copy stream: the epoch waits for them,
-// and the caller's buffers are free once they are done.
-int xfer_end(ltpg_ctx *ctx)
-{
-    const int k = ctx->xfer_slot;
-    LTPG_HIP_TRY(hipEventRecord(ctx->xfer_copied[k], ctx->copy_stream));
-    LTPG_HIP_TRY(hipStreamWaitEvent(ctx->stream, ctx->xfer_copied[k], 0));
-    LTPG_HIP_TRY(hipStreamSynchronize(ctx->copy_stream));
-    return LTPG_OK;
-}
+constexpr uint64_t kStageBytes = 2u << 20;
+
+// One submit's arrays on their way into a device block: packed into the
+// slot's pinned part if they fit there, otherwise copied one by one.
+class BatchCopy {
+public:
+    BatchCopy(ltpg_ctx *ctx, uint8_t *dev, uint64_t bytes)
+        : ctx_(ctx), dev_(dev), bytes_(bytes), stream_(ctx->xfer_in_order ? ctx->stream : ctx->copy_stream)
+    {
+    }
+
+    int begin()
+    {
+        if (bytes_ > kStageBytes - ctx_->stage_used || ctx_->stage_failed) return LTPG_OK;
+        if (!ctx_->stage && hipHostMalloc(reinterpret_cast<void **>(&ctx_->stage), 2 * kStageBytes, 0) != hipSuccess) {
+            (void)hipGetLastError();
+            ctx_->stage = nullptr;
+            ctx_->stage_failed = true;
+            return LTPG_OK;
+        }
+        const int k = ctx_->xfer_slot;
+        if (ctx_->stage_used == 0 && ctx_->xfer_copied_set[k]) LTPG_HIP_TRY(hipEventSynchronize(ctx_->xfer_copied[k]));
+        stage_ = ctx_->stage + k * kStageBytes + ctx_->stage_used;
+        ctx_->stage_used += batch_row(bytes_);
+        return LTPG_OK;
+    }
+
+    // n arrays of `bytes`, `from` bytes apart in the caller's memory and `to`
+    // in the block
+    int put(uint64_t at, const void *src, uint64_t bytes, uint32_t n = 1, uint64_t from = 0, uint64_t to = 0)
+    {
+        if (bytes == 0) return LTPG_OK;
+        if (stage_) {
+            for (uint32_t k = 0; k < n; k++)
+                std::memcpy(stage_ + at + k * to, static_cast<const uint8_t *>(src) + k * from, bytes);
+        } else if (n == 1) {
+            LTPG_HIP_TRY(hipMemcpyAsync(dev_ + at, src, bytes, hipMemcpyHostToDevice, stream_));
+        } else {
+            LTPG_HIP_TRY(hipMemcpy2DAsync(dev_ + at, to, src, from, bytes, n, hipMemcpyHostToDevice, stream_));
+        }
+        return LTPG_OK;
+    }
+
+    // The epoch waits for the copies, and the caller's buffers are free.
+    int end()
+    {
+        const int k = ctx_->xfer_slot;
+        if (stage_ && bytes_) LTPG_HIP_TRY(hipMemcpyAsync(dev_, stage_, bytes_, hipMemcpyHostToDevice, stream_));
+        LTPG_HIP_TRY(hipEventRecord(ctx_->xfer_copied[k], stream_));
+        ctx_->xfer_copied_set[k] = true;
+        if (!ctx_->xfer_in_order) LTPG_HIP_TRY(hipStreamWaitEvent(ctx_->stream, ctx_->xfer_copied[k], 0));
+        if (!stage_) LTPG_HIP_TRY(hipStreamSynchronize(stream_));
+        return LTPG_OK;
+    }
+
+private:
+    ltpg_ctx *ctx_;
+    uint8_t *dev_;
+    uint64_t bytes_;
+    hipStream_t stream_;
+    uint8_t *stage_ = nullptr;
+};
 
 template <typename T>
 int slot_buffer(T **buf, uint64_t count, const char *what)
@@ -1015,23 +1119,17 @@ int ltpg_kv_submit(ltpg_ctx *ctx, const ltpg_kv_batch *b, uint32_t mem)
         d.tids = b->tids;
     } else {
         int k = 0;
-        const uint64_t cap = (uint64_t)ctx->cfg.max_txns, n = (uint64_t)b->n_txns * b->n_slots;
+        const uint64_t n = (uint64_t)b->n_txns * b->n_slots;
         if ((rc = xfer_begin(ctx, &k))) return rc;
-        if ((rc = slot_buffer(&kv.keys_buf[k], kv.max_slots * cap, "kv keys")) ||
-            (rc = slot_buffer(&kv.meta_buf[k], kv.max_slots * cap, "kv meta")) ||
-            (rc = slot_buffer(&kv.tids_buf[k], cap, "kv tids")))
+        if ((rc = slot_buffer(&kv.batch_buf[k], kv_batch_bytes(kv.max_slots, ctx->cfg.max_txns), "kv batch"))) return rc;
+        const uint64_t meta_at = batch_row(n * 8), tids_at = meta_at + batch_row(n * 4);
+        BatchCopy copy(ctx, kv.batch_buf[k], tids_at + (uint64_t)b->n_txns * 4);
+        if ((rc = copy.begin()) || (rc = copy.put(0, b->keys, n * 8)) || (rc = copy.put(meta_at, b->meta, n * 4)) ||
+            (rc = copy.put(tids_at, b->tids, (uint64_t)b->n_txns * 4)) || (rc = copy.end()))
             return rc;
-        hipStream_t cs = ctx->copy_stream;
-        if (n) {
-            LTPG_HIP_TRY(hipMemcpyAsync(kv.keys_buf[k], b->keys, n * 8, hipMemcpyHostToDevice, cs));
-            LTPG_HIP_TRY(hipMemcpyAsync(kv.meta_buf[k], b->meta, n * 4, hipMemcpyHostToDevice, cs));
-        }
-        if (b->n_txns)
-            LTPG_HIP_TRY(hipMemcpyAsync(kv.tids_buf[k], b->tids, (uint64_t)b->n_txns * 4, hipMemcpyHostToDevice, cs));
-        if ((rc = xfer_end(ctx))) return rc;
-        d.keys = kv.keys_buf[k];
-        d.meta = kv.meta_buf[k];
-        d.tids = kv.tids_buf[k];
+        d.keys = reinterpret_cast<const uint64_t *>(kv.batch_buf[k]);
+        d.meta = reinterpret_cast<const uint32_t *>(kv.batch_buf[k] + meta_at);
+        d.tids = reinterpret_cast<const uint32_t *>(kv.batch_buf[k] + tids_at);
     }
     kv.cur = d;
     kv.has_batch = true;
@@ -1109,6 +1207,7 @@ int ltpg_epoch_run(ltpg_ctx *ctx, uint32_t phase_mask)
 {
     int rc = check_ctx(ctx);
     if (rc) return rc;
+    ctx->quiet = false;
     if (phase_mask & ~LTPG_PHASE_ALL) LTPG_FAIL(LTPG_ERR_INVALID, "unknown phase bit");
     if (ctx->cfg.workload == LTPG_WORKLOAD_TPCC) return tpcc_epoch_run(ctx, phase_mask);
     KvState &kv = ctx->kv;
@@ -1191,6 +1290,52 @@ int ltpg_epoch_reset(ltpg_ctx *ctx)
 
 // ---- results --------------------------------------------------------------
 
+}  // extern "C"
+
+namespace {
+
+constexpr uint32_t kReadbackPolls = 1u << 12;    // between two looks at the stream
+
+// `bytes` (a multiple of 4) from the device once the stream's work is done: a
+// small result through the pinned part, by a kernel that the host polls.  The
+// wait ends with the stream at the latest, also where an error ended it.
+int read_back(ltpg_ctx *ctx, void *out, const void *src, uint64_t bytes)
+{
+    if (bytes == 0 || bytes > kReadbackBytes || !ctx->readback) {
+        LTPG_HIP_TRY(hipStreamSynchronize(ctx->stream));
+        if (bytes) LTPG_HIP_TRY(hipMemcpy(out, src, bytes, hipMemcpyDeviceToHost));
+        return LTPG_OK;
+    }
+    int rc = refuse_capture(ctx);
+    if (rc) return rc;
+    const uint64_t *seq_at = reinterpret_cast<const uint64_t *>(ctx->readback + kReadbackBytes);
+    const uint64_t seq = ++ctx->readback_seq;
+    LTPG_HIP_TRY(launch_readback(reinterpret_cast<uint32_t *>(ctx->readback), static_cast<const uint32_t *>(src),
+                                 (uint32_t)(bytes / 4), &ctx->counters->readback_blocks,
+                                 const_cast<uint64_t *>(seq_at), seq, ctx->stream));
+    for (uint32_t n = 1; __atomic_load_n(seq_at, __ATOMIC_ACQUIRE) != seq; n++) {
+        if (n % kReadbackPolls) {
+            __builtin_ia32_pause();
+            continue;
+        }
+        hipError_t e = hipStreamQuery(ctx->stream);
+        if (e == hipErrorNotReady) {
+            (void)hipGetLastError();
+            if (n < 64 * kReadbackPolls) continue;
+            e = hipStreamSynchronize(ctx->stream);  // a long epoch: wait without polling
+        }
+        LTPG_HIP_TRY(e);
+        break;
+    }
+    ctx->quiet = true;
+    std::memcpy(out, ctx->readback, bytes);
+    return LTPG_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
 int ltpg_commit_bitmap(ltpg_ctx *ctx, uint32_t type, uint64_t *out, uint64_t n_words)
 {
     int rc = check_ctx(ctx);
@@ -1221,9 +1366,7 @@ int ltpg_commit_bitmap(ltpg_ctx *ctx, uint32_t type, uint64_t *out, uint64_t n_w
     }
     const uint64_t need = (n + 63) / 64;
     if (n_words < need) LTPG_FAIL(LTPG_ERR_INVALID, "bitmap buffer too small");
-    LTPG_HIP_TRY(hipStreamSynchronize(ctx->stream));
-    if (need) LTPG_HIP_TRY(hipMemcpy(out, src, need * 8, hipMemcpyDeviceToHost));
-    return LTPG_OK;
+    return read_back(ctx, out, src, need * 8);
 }
 
 int ltpg_commit_count(ltpg_ctx *ctx, uint32_t type, uint32_t *out)
@@ -1232,9 +1375,8 @@ int ltpg_commit_count(ltpg_ctx *ctx, uint32_t type, uint32_t *out)
     if (rc) return rc;
     if (!out) LTPG_FAIL(LTPG_ERR_INVALID, "null output");
     if (type > LTPG_TYPE_DELIVERY) LTPG_FAIL(LTPG_ERR_INVALID, "unknown transaction type");
-    LTPG_HIP_TRY(hipStreamSynchronize(ctx->stream));
     uint32_t h[kCounterStripes][64];
-    LTPG_HIP_TRY(hipMemcpy(h, ctx->counters->commits, sizeof(h), hipMemcpyDeviceToHost));
+    if ((rc = read_back(ctx, h, ctx->counters->commits, sizeof(h)))) return rc;
     uint32_t sum = 0;
     for (int k = 0; k < kCounterStripes; k++) sum += h[k][type];
     *out = sum;
@@ -1263,9 +1405,7 @@ int ltpg_conflict_counters(ltpg_ctx *ctx, uint32_t type, uint32_t *out, uint32_t
     if (!(ctx->cfg.flags & LTPG_FLAG_CONFLICT_COUNTS))
         LTPG_FAIL(LTPG_ERR_UNSUPPORTED, "conflict counters need LTPG_FLAG_CONFLICT_COUNTS");
     if (n > have) LTPG_FAIL(LTPG_ERR_INVALID, "n exceeds the batch size");
-    LTPG_HIP_TRY(hipStreamSynchronize(ctx->stream));
-    if (n) LTPG_HIP_TRY(hipMemcpy(out, src, (uint64_t)n * 4, hipMemcpyDeviceToHost));
-    return LTPG_OK;
+    return read_back(ctx, out, src, (uint64_t)n * 4);
 }
 
 int ltpg_kv_read_values(ltpg_ctx *ctx, uint32_t *out, uint64_t n_words)
@@ -1277,12 +1417,9 @@ int ltpg_kv_read_values(ltpg_ctx *ctx, uint32_t *out, uint64_t n_words)
     if (!kv.table) LTPG_FAIL(LTPG_ERR_UNSUPPORTED, "context has no key-value table");
     const uint64_t have = (uint64_t)kv.cur.n_slots * kv.cur.n_txns * kv.read_slot * kv.field_words;
     if (n_words > have) LTPG_FAIL(LTPG_ERR_INVALID, "n_words exceeds the staged read values");
-    LTPG_HIP_TRY(hipStreamSynchronize(ctx->stream));
     const uint64_t fw = kv.field_words, fsw = kv.field_stride;
-    if (fw == fsw) {
-        if (n_words) LTPG_HIP_TRY(hipMemcpy(out, kv.read_values, n_words * 4, hipMemcpyDeviceToHost));
-        return LTPG_OK;
-    }
+    if (fw == fsw) return read_back(ctx, out, kv.read_values, n_words * 4);
+    LTPG_HIP_TRY(hipStreamSynchronize(ctx->stream));
     // packed on the device, part by part
     const uint64_t n_fields = (n_words + fw - 1) / fw;
     const uint64_t part = std::min(kReadStageWords / fw,
@@ -1411,42 +1548,47 @@ int ltpg_tpcc_submit(ltpg_ctx *ctx, const ltpg_neworder_batch *nb, const ltpg_pa
             pay.H_ID = pb->H_ID; pay.TID = pb->TID;
         }
     } else {
-        // pack into the library's NEWORDER_QUERY / PAYMENT_QUERY blocks of
-        // the next host slot
-        const uint64_t C = ctx->cfg.max_txns;
+        // pack into the library's block of the next host slot
+        const uint64_t C = ctx->cfg.max_txns, no_row = batch_row((uint64_t)n_no * 4),
+                       pay_row = batch_row((uint64_t)n_pay * 4), pay_at = 53 * no_row;
         int slot = 0;
         if ((rc = xfer_begin(ctx, &slot))) return rc;
-        if ((rc = slot_buffer(&tp.no_buf[slot], 53 * C, "NewOrder batch")) ||
-            (rc = slot_buffer(&tp.pay_buf[slot], 10 * C, "Payment batch")) ||
-            (rc = slot_buffer(&tp.ro_buf[slot], 9 * C, "read-only batches")))
+        if ((rc = slot_buffer(&tp.np_buf[slot], np_batch_bytes(C), "NewOrder and Payment batches")) ||
+            (rc = slot_buffer(&tp.ro_buf[slot], ro_batch_bytes(C), "read-only batches")))
             return rc;
-        hipStream_t s = ctx->copy_stream;
+        uint8_t *dev = tp.np_buf[slot];
+        BatchCopy copy(ctx, dev, pay_at + 10 * pay_row);
+        if ((rc = copy.begin())) return rc;
         if (n_no) {
-            uint32_t *b = tp.no_buf[slot];
+            const uint64_t bytes = (uint64_t)n_no * 4;
             const uint32_t *heads[7] = {nb->W_ID, nb->D_ID, nb->C_ID, nb->O_ID, nb->N_O_ID, nb->O_OL_CNT, nb->O_OL_ID};
             for (int k = 0; k < 7; k++)
-                LTPG_HIP_TRY(hipMemcpyAsync(b + k * C, heads[k], (uint64_t)n_no * 4, hipMemcpyHostToDevice, s));
+                if ((rc = copy.put(k * no_row, heads[k], bytes))) return rc;
             const uint32_t *lines[3] = {nb->OL_I_ID, nb->OL_SUPPLY_W_ID, nb->OL_QUANTITY};
             for (int k = 0; k < 3; k++)
-                LTPG_HIP_TRY(hipMemcpy2DAsync(b + (7 + 15 * k) * C, C * 4, lines[k], (uint64_t)nb->line_stride * 4,
-                                              (uint64_t)n_no * 4, LTPG_TPCC_MAX_LINES, hipMemcpyHostToDevice, s));
-            LTPG_HIP_TRY(hipMemcpyAsync(b + 52 * C, nb->TID, (uint64_t)n_no * 4, hipMemcpyHostToDevice, s));
-            no.line_stride = (uint32_t)C;
-            no.W_ID = b; no.D_ID = b + C; no.C_ID = b + 2 * C; no.O_ID = b + 3 * C; no.N_O_ID = b + 4 * C;
-            no.O_OL_CNT = b + 5 * C; no.O_OL_ID = b + 6 * C; no.OL_I_ID = b + 7 * C; no.OL_SUPPLY_W_ID = b + 22 * C;
-            no.OL_QUANTITY = b + 37 * C; no.TID = b + 52 * C;
+                if ((rc = copy.put((7 + 15 * k) * no_row, lines[k], bytes, LTPG_TPCC_MAX_LINES,
+                                   (uint64_t)nb->line_stride * 4, no_row)))
+                    return rc;
+            if ((rc = copy.put(52 * no_row, nb->TID, bytes))) return rc;
+            const uint32_t *b = reinterpret_cast<const uint32_t *>(dev);
+            const uint64_t R = no_row / 4;
+            no.line_stride = (uint32_t)R;
+            no.W_ID = b; no.D_ID = b + R; no.C_ID = b + 2 * R; no.O_ID = b + 3 * R; no.N_O_ID = b + 4 * R;
+            no.O_OL_CNT = b + 5 * R; no.O_OL_ID = b + 6 * R; no.OL_I_ID = b + 7 * R; no.OL_SUPPLY_W_ID = b + 22 * R;
+            no.OL_QUANTITY = b + 37 * R; no.TID = b + 52 * R;
         }
         if (n_pay) {
-            uint32_t *b = tp.pay_buf[slot];
             const uint32_t *cols[10] = {pb->W_ID, pb->D_ID, pb->C_ID, pb->C_LAST, pb->isName,
                                         pb->C_D_ID, pb->C_W_ID, pb->H_AMOUNT, pb->H_ID, pb->TID};
             for (int k = 0; k < 10; k++)
-                LTPG_HIP_TRY(hipMemcpyAsync(b + k * C, cols[k], (uint64_t)n_pay * 4, hipMemcpyHostToDevice, s));
-            pay.W_ID = b; pay.D_ID = b + C; pay.C_ID = b + 2 * C; pay.C_LAST = b + 3 * C; pay.isName = b + 4 * C;
-            pay.C_D_ID = b + 5 * C; pay.C_W_ID = b + 6 * C; pay.H_AMOUNT = b + 7 * C; pay.H_ID = b + 8 * C;
-            pay.TID = b + 9 * C;
+                if ((rc = copy.put(pay_at + k * pay_row, cols[k], (uint64_t)n_pay * 4))) return rc;
+            const uint32_t *b = reinterpret_cast<const uint32_t *>(dev + pay_at);
+            const uint64_t R = pay_row / 4;
+            pay.W_ID = b; pay.D_ID = b + R; pay.C_ID = b + 2 * R; pay.C_LAST = b + 3 * R; pay.isName = b + 4 * R;
+            pay.C_D_ID = b + 5 * R; pay.C_W_ID = b + 6 * R; pay.H_AMOUNT = b + 7 * R; pay.H_ID = b + 8 * R;
+            pay.TID = b + 9 * R;
         }
-        if ((rc = xfer_end(ctx))) return rc;
+        if ((rc = copy.end())) return rc;
     }
     tp.host_slot = mem == LTPG_MEM_HOST;
     // Until a CID phase runs, each Payment uses its query's C_ID (a copy
@@ -1490,25 +1632,23 @@ int ltpg_tpcc_submit_readonly(ltpg_ctx *ctx, const ltpg_orderstatus_batch *ob, c
     } else {
         // the epoch's host slot (its NewOrders and Payments took it), or, if
         // they were device-resident, the next one
-        const uint64_t C = ctx->cfg.max_txns;
+        const uint64_t os_row = batch_row((uint64_t)n_os * 4), sl_row = batch_row((uint64_t)n_sl * 4);
         int slot = ctx->xfer_slot;
         if (!tp.host_slot && (rc = xfer_begin(ctx, &slot))) return rc;
         tp.host_slot = true;
-        if ((rc = slot_buffer(&tp.ro_buf[slot], 9 * C, "read-only batches"))) return rc;
-        uint32_t *rb = tp.ro_buf[slot];
+        if ((rc = slot_buffer(&tp.ro_buf[slot], ro_batch_bytes(ctx->cfg.max_txns), "read-only batches"))) return rc;
+        uint8_t *dev = tp.ro_buf[slot];
+        BatchCopy copy(ctx, dev, 6 * os_row + 3 * sl_row);
+        if ((rc = copy.begin())) return rc;
         for (int k = 0; k < 6; k++) {
-            os_dev[k] = rb + k * C;
-            if (n_os)
-                LTPG_HIP_TRY(hipMemcpyAsync(rb + k * C, os_src[k], (uint64_t)n_os * 4, hipMemcpyHostToDevice,
-                                            ctx->copy_stream));
+            os_dev[k] = reinterpret_cast<const uint32_t *>(dev + k * os_row);
+            if ((rc = copy.put(k * os_row, os_src[k], (uint64_t)n_os * 4))) return rc;
         }
         for (int k = 0; k < 3; k++) {
-            sl_dev[k] = rb + (6 + k) * C;
-            if (n_sl)
-                LTPG_HIP_TRY(hipMemcpyAsync(rb + (6 + k) * C, sl_src[k], (uint64_t)n_sl * 4, hipMemcpyHostToDevice,
-                                            ctx->copy_stream));
+            sl_dev[k] = reinterpret_cast<const uint32_t *>(dev + 6 * os_row + k * sl_row);
+            if ((rc = copy.put(6 * os_row + k * sl_row, sl_src[k], (uint64_t)n_sl * 4))) return rc;
         }
-        if ((rc = xfer_end(ctx))) return rc;
+        if ((rc = copy.end())) return rc;
     }
     ro.os_W_ID = os_dev[0]; ro.os_D_ID = os_dev[1]; ro.os_C_ID = os_dev[2];
     ro.os_O_ID = os_dev[3]; ro.os_OL_ID = os_dev[4]; ro.os_TID = os_dev[5];
@@ -1537,17 +1677,19 @@ int ltpg_tpcc_submit_delivery(ltpg_ctx *ctx, const ltpg_delivery_batch *db, uint
         for (int k = 0; k < 4; k++) dev[k] = src[k];
     } else {
         // the epoch's host slot, or, if its batch was device-resident, the next one
-        const uint64_t C = ctx->cfg.max_txns;
+        const uint64_t row = batch_row((uint64_t)n * 4);
         int slot = ctx->xfer_slot;
         if (!tp.host_slot && (rc = xfer_begin(ctx, &slot))) return rc;
         tp.host_slot = true;
-        if ((rc = slot_buffer(&tp.dl_buf[slot], 4 * C, "Delivery batches"))) return rc;
-        uint32_t *b = tp.dl_buf[slot];
+        if ((rc = slot_buffer(&tp.dl_buf[slot], 4 * batch_row((uint64_t)ctx->cfg.max_txns * 4), "Delivery batches")))
+            return rc;
+        BatchCopy copy(ctx, tp.dl_buf[slot], 4 * row);
+        if ((rc = copy.begin())) return rc;
         for (int k = 0; k < 4; k++) {
-            dev[k] = b + k * C;
-            LTPG_HIP_TRY(hipMemcpyAsync(b + k * C, src[k], (uint64_t)n * 4, hipMemcpyHostToDevice, ctx->copy_stream));
+            dev[k] = reinterpret_cast<const uint32_t *>(tp.dl_buf[slot] + k * row);
+            if ((rc = copy.put(k * row, src[k], (uint64_t)n * 4))) return rc;
         }
-        if ((rc = xfer_end(ctx))) return rc;
+        if ((rc = copy.end())) return rc;
     }
     DeliveryDev dl;
     dl.n = n;
@@ -1565,9 +1707,7 @@ int ltpg_tpcc_payment_cid(ltpg_ctx *ctx, uint32_t *out, uint32_t n)
     if (rc) return rc;
     if (!out) LTPG_FAIL(LTPG_ERR_INVALID, "null output");
     if (n > ctx->tpcc.pay.n) LTPG_FAIL(LTPG_ERR_INVALID, "n exceeds the Payment batch size");
-    LTPG_HIP_TRY(hipStreamSynchronize(ctx->stream));
-    if (n) LTPG_HIP_TRY(hipMemcpy(out, ctx->tpcc.d.cid, (uint64_t)n * 4, hipMemcpyDeviceToHost));
-    return LTPG_OK;
+    return read_back(ctx, out, ctx->tpcc.d.cid, (uint64_t)n * 4);
 }
 
 int ltpg_tpcc_read_values(ltpg_ctx *ctx, uint32_t type, uint32_t *out, uint64_t n_words)
@@ -1596,9 +1736,7 @@ int ltpg_tpcc_read_values(ltpg_ctx *ctx, uint32_t type, uint32_t *out, uint64_t 
         LTPG_FAIL(LTPG_ERR_INVALID, "type must be an order-entry type");
     }
     if (n_words > have) LTPG_FAIL(LTPG_ERR_INVALID, "n_words exceeds the batch's read values");
-    LTPG_HIP_TRY(hipStreamSynchronize(ctx->stream));
-    if (n_words) LTPG_HIP_TRY(hipMemcpy(out, src, n_words * 4, hipMemcpyDeviceToHost));
-    return LTPG_OK;
+    return read_back(ctx, out, src, n_words * 4);
 }
 
 }  // extern "C"

@@ -23,6 +23,7 @@
 #include <hip/hip_runtime.h>
 
 #include <chrono>
+#include <cstring>
 #include <new>
 #include <string>
 #include <vector>
@@ -36,6 +37,7 @@ struct ltpg_batched {
     std::vector<ltpg_batch_desc> d;
     std::vector<uint64_t> off;              // archive offset (u64 words) of batch i's first bitmap
     uint64_t *archive = nullptr;
+    bool archive_pinned = false;            // in pinned host memory
     uint64_t archive_words = 0;
     hipGraph_t graph[2] = {nullptr, nullptr};
     hipGraphExec_t exec[2] = {nullptr, nullptr};
@@ -57,6 +59,12 @@ namespace {
 
 uint64_t words(uint64_t n) { return (n + 63) / 64; }
 
+// An archive of up to 4 MB (32M transactions) is written over PCIe as the run
+// goes: 24 batches of 40,000 transactions on average are 180 KB, and their 36
+// bitmaps then cost the host a copy each, 130 us together with the calls, where
+// a transfer each took 600.
+constexpr uint64_t kPinnedArchiveWords = 1u << 19;
+
 int slot_of(uint32_t workload) { return workload == LTPG_WORKLOAD_KV ? 0 : 1; }
 
 // The launch shape of key-value batch i.
@@ -65,6 +73,27 @@ int set_kv_shape(ltpg_batched *b, ltpg_ctx *ctx, uint32_t i)
     if (b->tuned) return ltpg_kv_set_tuning(ctx, b->tune[i]);
     kv_default_shape(ctx);
     return LTPG_OK;
+}
+
+// The commit bitmaps of batch i and their places in the archive.
+PublishSet archive_set(const ltpg_batched *b, uint32_t i)
+{
+    const ltpg_batch_desc &d = b->d[i];
+    const bool kv = d.workload == LTPG_WORKLOAD_KV;
+    const TpccDev &t = b->ctx[slot_of(d.workload)]->tpcc.d;
+    const uint64_t *src[5] = {kv ? b->ctx[0]->kv.bitmap : t.bitmap_no, t.bitmap_pay, t.bitmap_os, t.bitmap_sl,
+                              t.bitmap_dl};
+    const uint32_t n[5] = {kv ? d.kv.n_txns : d.neworder.n, d.payment.n, d.orderstatus.n, d.stocklevel.n,
+                           d.delivery.n};
+    PublishSet p = {};
+    uint64_t *at = b->archive + b->off[i];
+    for (int k = 0; k < (kv ? 1 : 5); k++) {
+        p.src[k] = src[k];
+        p.dst[k] = at;
+        p.n[k] = (uint32_t)words(n[k]);
+        at += p.n[k];
+    }
+    return p;
 }
 
 // One epoch of batch i on its context: submit (device-resident), all
@@ -89,21 +118,7 @@ int enqueue_batch(ltpg_batched *b, uint32_t i, bool stamp, bool stepwise = false
         if (d.delivery.n && (rc = ltpg_tpcc_submit_delivery(ctx, &d.delivery, LTPG_MEM_DEVICE))) return rc;
     }
     if ((rc = stepwise ? run_epoch_stepwise(ctx) : ltpg_epoch_run(ctx, LTPG_PHASE_ALL))) return rc;
-    if (d.workload == LTPG_WORKLOAD_KV) {
-        LTPG_HIP_TRY(launch_copy_u64(b->archive + b->off[i], ctx->kv.bitmap, words(d.kv.n_txns), ctx->stream));
-    } else {
-        LTPG_HIP_TRY(launch_copy_u64(b->archive + b->off[i], ctx->tpcc.d.bitmap_no, words(d.neworder.n),
-                                     ctx->stream));
-        uint64_t at = b->off[i] + words(d.neworder.n);
-        LTPG_HIP_TRY(launch_copy_u64(b->archive + at, ctx->tpcc.d.bitmap_pay, words(d.payment.n), ctx->stream));
-        at += words(d.payment.n);
-        LTPG_HIP_TRY(launch_copy_u64(b->archive + at, ctx->tpcc.d.bitmap_os, words(d.orderstatus.n), ctx->stream));
-        at += words(d.orderstatus.n);
-        LTPG_HIP_TRY(launch_copy_u64(b->archive + at, ctx->tpcc.d.bitmap_sl, words(d.stocklevel.n), ctx->stream));
-        at += words(d.stocklevel.n);
-        LTPG_HIP_TRY(launch_copy_u64(b->archive + at, ctx->tpcc.d.bitmap_dl, words(d.delivery.n), ctx->stream));
-    }
-    if (stamp) LTPG_HIP_TRY(launch_stamp(b->stamps + i, ctx->stream));
+    LTPG_HIP_TRY(launch_archive(archive_set(b, i), stamp ? b->stamps + i : nullptr, ctx->stream));
     return LTPG_OK;
 }
 
@@ -197,8 +212,7 @@ int enqueue_kv_pipelined(ltpg_batched *b)
         checked.push_back(done);
         st.list_valid = true;  // of the CHECK above
         LTPG_HIP_TRY(launch_kv_writeback(st, st.cur, ctx->cfg.values, ctx->counters, main));
-        LTPG_HIP_TRY(launch_copy_u64(b->archive + b->off[i], ctx->kv.bitmap, words(d.kv.n_txns), main));
-        LTPG_HIP_TRY(launch_stamp(b->stamps + i, main));
+        LTPG_HIP_TRY(launch_archive(archive_set(b, i), b->stamps + i, main));
         j++;
     }
     return join_side(b, main, side);  // side rejoins main before the capture ends
@@ -259,7 +273,10 @@ int ltpg_batched_destroy(ltpg_batched *b)
     dev_free(b->doomed2);
     dev_free(b->raw2);
     dev_free(b->war2);
-    dev_free(b->archive);
+    if (b->archive_pinned)
+        (void)hipHostFree(b->archive);
+    else
+        dev_free(b->archive);
     dev_free(b->stamps);
     delete b;
     return LTPG_OK;
@@ -299,7 +316,16 @@ int ltpg_batched_create(ltpg_ctx *kv_ctx, ltpg_ctx *tpcc_ctx, const ltpg_batch_d
     }
     b->archive_words = w;
     int rc = check_ctx(kv_ctx ? kv_ctx : tpcc_ctx);
-    if (!rc) rc = dev_alloc(&b->archive, w ? w : 1, "bitmap archive");
+    if (!rc && w <= kPinnedArchiveWords) {
+        if (hipHostMalloc(reinterpret_cast<void **>(&b->archive), (w ? w : 1) * 8,
+                          hipHostMallocCoherent | hipHostMallocMapped) == hipSuccess) {
+            b->archive_pinned = true;
+        } else {
+            (void)hipGetLastError();
+            b->archive = nullptr;
+        }
+    }
+    if (!rc && !b->archive) rc = dev_alloc(&b->archive, w ? w : 1, "bitmap archive");
     if (!rc) rc = dev_alloc(&b->stamps, (uint64_t)n + 2, "batch clock stamps");
     b->plain_ms.assign(n, 0.0);
     bool any_kv = false;
@@ -567,7 +593,10 @@ int ltpg_batched_bitmap(ltpg_batched *b, uint32_t batch, uint32_t type, uint64_t
     if (rc) return rc;
     for (int k = 0; k < 2; k++)
         if (b->ctx[k]) LTPG_HIP_TRY(hipStreamSynchronize(b->ctx[k]->stream));
-    if (n) LTPG_HIP_TRY(hipMemcpy(out, b->archive + off, n * 8, hipMemcpyDeviceToHost));
+    if (b->archive_pinned)
+        std::memcpy(out, b->archive + off, n * 8);
+    else if (n)
+        LTPG_HIP_TRY(hipMemcpy(out, b->archive + off, n * 8, hipMemcpyDeviceToHost));
     return LTPG_OK;
 }
 

@@ -41,7 +41,8 @@ constexpr uint32_t kCountedTypes = 6;  // LTPG_TYPE_KV .. LTPG_TYPE_DELIVERY
 struct DeviceCounters {
     uint32_t range_errors;                            // ops outside their table
     uint32_t kv_list_n;                               // length of KvState::commit_list
-    uint32_t pad0[62];
+    uint32_t readback_blocks;                         // blocks of a read-back kernel that are done
+    uint32_t pad0[61];
     uint32_t commits[kCounterStripes][64];            // [stripe][type]: last epoch
     unsigned long long totals[kCounterStripes][32];   // [stripe][type]: commits,
                                                       // [stripe][kAttempts + type]: attempts
@@ -132,9 +133,7 @@ struct KvState {
     // library-owned copies of host-submitted batches: two slots, so that
     // the next batch's copy overlaps the current epoch (slot 1 allocated at
     // its first use)
-    uint64_t *keys_buf[2] = {nullptr, nullptr};
-    uint32_t *meta_buf[2] = {nullptr, nullptr};
-    uint32_t *tids_buf[2] = {nullptr, nullptr};
+    uint8_t *batch_buf[2] = {nullptr, nullptr};
     KvBatchDev cur;
     bool has_batch = false;
     // tuning (ltpg_kv_set_tuning): EXECUTE one lane per op instead of per
@@ -254,10 +253,9 @@ struct TpccDev {
 struct TpccState {
     TpccDev d;
     // host-submitted batches, two slots as for key-value batches
-    uint32_t *no_buf[2] = {nullptr, nullptr};   // packed NEWORDER_QUERY, capacity max_txns
-    uint32_t *pay_buf[2] = {nullptr, nullptr};  // packed PAYMENT_QUERY, capacity max_txns
-    uint32_t *ro_buf[2] = {nullptr, nullptr};   // read-only batches: 6 + 3 arrays of capacity max_txns
-    uint32_t *dl_buf[2] = {nullptr, nullptr};   // Deliveries: 4 arrays of capacity max_txns
+    uint8_t *np_buf[2] = {nullptr, nullptr};    // packed NEWORDER_QUERY (53 arrays) and PAYMENT_QUERY (10)
+    uint8_t *ro_buf[2] = {nullptr, nullptr};    // read-only batches: 6 + 3 arrays
+    uint8_t *dl_buf[2] = {nullptr, nullptr};    // Deliveries: 4 arrays
     bool host_slot = false;                     // the current epoch's batch went through a host slot
     NeworderDev no;
     PaymentDev pay;
@@ -290,7 +288,18 @@ struct ltpg_ctx {
     hipEvent_t xfer_copied[2] = {nullptr, nullptr};
     hipEvent_t xfer_released[2] = {nullptr, nullptr};  // the epochs that used the slot are done
     bool xfer_released_set[2] = {false, false};
-    int xfer_slot = 1;  // slot of the current host batch (the next one takes the other)
+    bool xfer_copied_set[2] = {false, false};
+    int xfer_slot = 1;          // slot of the current host batch (the next one takes the other)
+    bool xfer_in_order = false; // its copies go on `stream` itself
+    bool quiet = false;         // nothing was queued on `stream` since a wait for it (only a hint)
+    // pinned memory until the context ends: from the first small host batch on
+    // the two slots' parts (kStageBytes each), and one for small results
+    // (kReadbackBytes and a sequence number)
+    uint8_t *stage = nullptr;
+    uint64_t stage_used = 0;    // bytes of the current slot's part
+    bool stage_failed = false;
+    uint8_t *readback = nullptr;
+    uint64_t readback_seq = 0;
 };
 
 namespace ltpg {
@@ -342,18 +351,23 @@ hipError_t launch_calibration(unsigned long long *a, uint64_t len, uint64_t n, i
                               unsigned long long *sink, hipStream_t s);
 hipError_t launch_fill_u64(unsigned long long *p, uint64_t n, unsigned long long v, hipStream_t s);
 hipError_t launch_fill_u8(uint8_t *p, uint64_t n, uint8_t v, hipStream_t s);
-hipError_t launch_copy_u64(uint64_t *dst, const uint64_t *src, uint64_t n, hipStream_t s);
 // n u32 words; src may be pinned host memory
 hipError_t launch_copy_u32(uint32_t *dst, const uint32_t *src, uint64_t n, hipStream_t s);
 // Up to four bitmaps to copy to pinned host memory (n[k] words from src[k]
 // to dst[k]; n[k] = 0 for unused entries).
+// Copy to pinned host memory, then store `seq` to *seq_out; `blocks` is zero
+// before and after.
+hipError_t launch_readback(uint32_t *dst, const uint32_t *src, uint32_t words, uint32_t *blocks, uint64_t *seq_out,
+                           uint64_t seq, hipStream_t s);
 struct PublishSet {
     const uint64_t *src[5];
     uint64_t *dst[5];
     uint32_t n[5];
 };
 // copy the bitmaps of p, then store seq to *seq_out (pinned host memory)
-// with a system-scope release
+// with a system-scope release; or copy them and stamp the device clock (unless
+// null)
+hipError_t launch_archive(const PublishSet &p, unsigned long long *stamp, hipStream_t s);
 hipError_t launch_publish(const PublishSet &p, uint64_t *seq_out, uint64_t seq, hipStream_t s);
 hipError_t launch_stamp(unsigned long long *out, hipStream_t s);
 
