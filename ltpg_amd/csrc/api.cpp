@@ -327,6 +327,17 @@ int refill_registers(ltpg_ctx *ctx)
 
 namespace {
 
+// The current batch's Payments use their queries' C_IDs (a copy kernel rather
+// than a memcpy: a captured submit then holds kernel nodes only).
+int settle_cid(ltpg_ctx *ctx)
+{
+    TpccState &tp = ctx->tpcc;
+    if (!tp.cid_pending) return LTPG_OK;
+    LTPG_HIP_TRY(launch_copy_u32(tp.d.cid, tp.pay.C_ID, tp.pay.n, ctx->stream));
+    tp.cid_pending = false;
+    return LTPG_OK;
+}
+
 // Advance the epoch (1..255).  At wrap-around every register goes back to
 // all-ones (the tag of epoch 0, never current) and the doomed flags to 0 --
 // unless no key-value kernel has written them since the last refill ran
@@ -525,6 +536,7 @@ int ltpg_set_stream(ltpg_ctx *ctx, void *hip_stream)
 {
     int rc = check_ctx(ctx);
     if (rc) return rc;
+    if ((rc = settle_cid(ctx))) return rc;
     LTPG_HIP_TRY(hipStreamSynchronize(ctx->stream));
     ctx->stream = hip_stream ? static_cast<hipStream_t>(hip_stream) : ctx->own_stream;
     ctx->quiet = false;
@@ -535,6 +547,7 @@ int ltpg_sync(ltpg_ctx *ctx)
 {
     int rc = check_ctx(ctx);
     if (rc) return rc;
+    if ((rc = settle_cid(ctx))) return rc;  // the caller may free a device-resident batch after this
     LTPG_HIP_TRY(hipStreamSynchronize(ctx->stream));
     uint32_t errors = 0;
     LTPG_HIP_TRY(hipMemcpy(&errors, &ctx->counters->range_errors, sizeof(errors), hipMemcpyDeviceToHost));
@@ -1169,16 +1182,24 @@ static int tpcc_epoch_run(ltpg_ctx *ctx, uint32_t phase_mask)
         if ((rc = take_events(ctx, &ev))) return rc;
         LTPG_HIP_TRY(hipEventRecord(ev[0], s));
     }
-    if (phase_mask & LTPG_PHASE_CID) LTPG_HIP_TRY(launch_tpcc_cid(tp.d, tp.pay, tp.small_blocks, s));
+    // CID and EXECUTE in one call (and not timed apart) are one kernel
+    const bool cid = (phase_mask & LTPG_PHASE_CID) && (phase_mask & LTPG_PHASE_EXECUTE) && !ev;
+    if (phase_mask & LTPG_PHASE_CID) {
+        if (!cid) LTPG_HIP_TRY(launch_tpcc_cid(tp.d, tp.pay, tp.small_blocks, s));
+        tp.cid_pending = false;
+    } else if ((rc = settle_cid(ctx))) {
+        return rc;
+    }
     if (ev) LTPG_HIP_TRY(hipEventRecord(ev[1], s));
     const bool ro = tp.ro.n_os + tp.ro.n_sl > 0, dl = tp.dl.n > 0;
     const uint32_t dl_base = tp.no.n + tp.pay.n + tp.ro.n_os + tp.ro.n_sl;
     if (phase_mask & LTPG_PHASE_EXECUTE) {
         // Stock-Level reads the STOCK registers, which the split form leaves out
         if (!counts && tp.ro.n_sl == 0 && tpcc_execute_split(tp.d, tp.bin, tp.no, tp.pay))
-            LTPG_HIP_TRY(launch_tpcc_execute_split(tp.d, tp.bin, tp.no, tp.pay, e, tp.small_blocks, ctx->counters, s));
+            LTPG_HIP_TRY(launch_tpcc_execute_split(tp.d, tp.bin, tp.no, tp.pay, e, cid, tp.small_blocks, ctx->counters,
+                                                   s));
         else
-            LTPG_HIP_TRY(launch_tpcc_execute(tp.d, tp.no, tp.pay, e, counts, tp.small_blocks, ctx->counters, s));
+            LTPG_HIP_TRY(launch_tpcc_execute(tp.d, tp.no, tp.pay, e, counts, cid, tp.small_blocks, ctx->counters, s));
         // Deliveries register after NewOrders and Payments, then read-only
         // transactions mark war on the registered writers
         if (dl) LTPG_HIP_TRY(launch_tpcc_delivery_execute(tp.d, tp.dl, dl_base, e, ctx->counters, s));
@@ -1591,12 +1612,14 @@ int ltpg_tpcc_submit(ltpg_ctx *ctx, const ltpg_neworder_batch *nb, const ltpg_pa
         if ((rc = copy.end())) return rc;
     }
     tp.host_slot = mem == LTPG_MEM_HOST;
-    // Until a CID phase runs, each Payment uses its query's C_ID (a copy
-    // kernel rather than a memcpy: a batched run captures this submit into a
-    // graph, which then holds kernel nodes only)
-    if (n_pay) LTPG_HIP_TRY(launch_copy_u32(tp.d.cid, pay.C_ID, n_pay, ctx->stream));
     tp.no = no;
     tp.pay = pay;
+    // Until a CID phase runs, each Payment uses its query's C_ID.  The CID
+    // phase nearly always comes first and finds them all, so the copy waits
+    // for a call that needs it; on a stream of the caller's it is made now
+    // (a capture of the phases there says nothing of when they run).
+    tp.cid_pending = n_pay > 0;
+    if (ctx->stream != ctx->own_stream && (rc = settle_cid(ctx))) return rc;
     tp.ro = ReadOnlyDev();
     tp.dl = DeliveryDev();
     tp.has_batch = true;
@@ -1707,6 +1730,7 @@ int ltpg_tpcc_payment_cid(ltpg_ctx *ctx, uint32_t *out, uint32_t n)
     if (rc) return rc;
     if (!out) LTPG_FAIL(LTPG_ERR_INVALID, "null output");
     if (n > ctx->tpcc.pay.n) LTPG_FAIL(LTPG_ERR_INVALID, "n exceeds the Payment batch size");
+    if ((rc = settle_cid(ctx))) return rc;
     return read_back(ctx, out, ctx->tpcc.d.cid, (uint64_t)n * 4);
 }
 

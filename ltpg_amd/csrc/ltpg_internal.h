@@ -263,6 +263,7 @@ struct TpccState {
     DeliveryDev dl;
     BinBuffers bin;                             // binned STOCK writes
     bool has_batch = false;
+    bool cid_pending = false;                   // d.cid does not hold the batch's C_IDs yet
     bool small_blocks = false;                  // LTPG_TUNE_TPCC_SMALL_BLOCKS
 };
 
@@ -502,9 +503,11 @@ hipError_t launch_tpcc_name_index(const TpccDev &d, hipStream_t s);
 hipError_t launch_tpcc_relayout(const uint32_t *src, uint32_t *dst, uint64_t rows, uint32_t cols,
                                 uint32_t stride, uint32_t layout, int to_device, hipStream_t s);
 // `small`: 64-thread blocks (LTPG_TUNE_TPCC_SMALL_BLOCKS) instead of 256.
+// `cid` in EXECUTE: the CID phase in the same kernel.
 hipError_t launch_tpcc_cid(const TpccDev &d, const PaymentDev &pay, bool small, hipStream_t s);
 hipError_t launch_tpcc_execute(const TpccDev &d, const NeworderDev &no, const PaymentDev &pay,
-                               const EpochTag &e, bool counts, bool small, DeviceCounters *ctr, hipStream_t s);
+                               const EpochTag &e, bool counts, bool cid, bool small, DeviceCounters *ctr,
+                               hipStream_t s);
 // EXECUTE of a large fast-form epoch without Stock-Level: whether it is taken,
 // its launch, and the shape of its binned part.  Four kernels against one:
 // 32,000 transactions 23 us split, 22 in one (16 warehouses), 64,000 24 / 31
@@ -513,8 +516,8 @@ constexpr uint32_t kSplitTxns = 3u << 14;
 bool tpcc_execute_split(const TpccDev &d, const BinBuffers &bin, const NeworderDev &no, const PaymentDev &pay);
 BinShape stock_bin_shape(uint64_t stock_rows, uint32_t n_neworder);
 hipError_t launch_tpcc_execute_split(const TpccDev &d, const BinBuffers &bin, const NeworderDev &no,
-                                     const PaymentDev &pay, const EpochTag &e, bool small, DeviceCounters *ctr,
-                                     hipStream_t s);
+                                     const PaymentDev &pay, const EpochTag &e, bool cid, bool small,
+                                     DeviceCounters *ctr, hipStream_t s);
 hipError_t launch_tpcc_readonly(const TpccDev &d, const ReadOnlyDev &ro, uint32_t base, const EpochTag &e,
                                 DeviceCounters *ctr, hipStream_t s);
 // Deliveries (base = their first batch position): EXECUTE registrations,

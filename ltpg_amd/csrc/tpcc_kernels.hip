@@ -186,33 +186,32 @@ __global__ __launch_bounds__(kBlock) void relayout_kernel(const uint32_t *__rest
 
 // C_ID of the k-th (0-based, k = C_LAST & 0xff) customer of district
 // C_W_ID * 10 + C_D_ID whose C_LAST is C_LAST >> 8; 0 when there is none.
+__device__ __forceinline__ uint32_t payment_cid(const TpccDev &d, const PaymentDev &pay, uint32_t p)
+{
+    if (!pay.isName[p]) return pay.C_ID[p];
+    const uint64_t dist = (uint64_t)pay.C_W_ID[p] * 10 + pay.C_D_ID[p];
+    if (dist >= d.t[DI].rows) return 0;
+    const uint32_t cl = pay.C_LAST[p], name = cl >> 8, k = cl & 0xffu;
+    const unsigned long long *idx = d.name_index + dist * kPerDistrict;
+    const unsigned long long key = (unsigned long long)name << 32;
+    uint32_t lo = 0, hi = kPerDistrict;
+    while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (idx[mid] < key) lo = mid + 1; else hi = mid;
+    }
+    const uint32_t j = lo + k;
+    if (j >= kPerDistrict) return 0;
+    const unsigned long long e = idx[j];
+    return (uint32_t)(e >> 32) == name ? d.t[CU].data[(dist * kPerDistrict + (uint32_t)e) * kStride[CU]] : 0u;
+}
+
+// The phase by itself; an epoch that runs it and EXECUTE in one call has it in
+// EXECUTE's kernel (`cid` there).
 template <uint32_t BLK>
 __global__ __launch_bounds__(BLK) void cid_kernel(TpccDev d, PaymentDev pay)
 {
     const uint32_t p = blockIdx.x * BLK + threadIdx.x;
-    if (p >= pay.n) return;
-    uint32_t c = pay.C_ID[p];
-    if (pay.isName[p]) {
-        c = 0;
-        const uint64_t dist = (uint64_t)pay.C_W_ID[p] * 10 + pay.C_D_ID[p];
-        if (dist < d.t[DI].rows) {
-            const uint32_t cl = pay.C_LAST[p], name = cl >> 8, k = cl & 0xffu;
-            const unsigned long long *idx = d.name_index + dist * kPerDistrict;
-            const unsigned long long key = (unsigned long long)name << 32;
-            uint32_t lo = 0, hi = kPerDistrict;
-            while (lo < hi) {
-                const uint32_t mid = (lo + hi) >> 1;
-                if (idx[mid] < key) lo = mid + 1; else hi = mid;
-            }
-            const uint32_t j = lo + k;
-            if (j < kPerDistrict) {
-                const unsigned long long e = idx[j];
-                if ((uint32_t)(e >> 32) == name)
-                    c = d.t[CU].data[(dist * kPerDistrict + (uint32_t)e) * kStride[CU]];
-            }
-        }
-    }
-    d.cid[p] = c;
+    if (p < pay.n) d.cid[p] = payment_cid(d, pay, p);
 }
 
 // ---- row formulas (u64; the reference's u32 forms, Execute_neworder.h:22-266,
@@ -243,15 +242,29 @@ struct PayRows {
     uint64_t wh, di, cu, hi;
 };
 
-__device__ __forceinline__ PayRows pay_rows(const TpccDev &d, const PaymentDev &pay, uint32_t p)
+__device__ __forceinline__ PayRows pay_rows(const PaymentDev &pay, uint32_t p, uint32_t c_id)
 {
     PayRows r;
     const uint64_t w = pay.W_ID[p];
     r.wh = w;
     r.di = w * 10 + pay.D_ID[p];
-    r.cu = (uint64_t)pay.C_W_ID[p] * 30000 + (uint64_t)pay.C_D_ID[p] * 3000 + d.cid[p];
+    r.cu = (uint64_t)pay.C_W_ID[p] * 30000 + (uint64_t)pay.C_D_ID[p] * 3000 + c_id;
     r.hi = w * 30000 + pay.H_ID[p];
     return r;
+}
+
+__device__ __forceinline__ PayRows pay_rows(const TpccDev &d, const PaymentDev &pay, uint32_t p)
+{
+    return pay_rows(pay, p, d.cid[p]);
+}
+
+// The rows of Payment p in EXECUTE, which with `cid` finds its customer first.
+__device__ __forceinline__ PayRows pay_rows_cid(const TpccDev &d, const PaymentDev &pay, uint32_t p, bool cid)
+{
+    if (!cid) return pay_rows(d, pay, p);
+    const uint32_t c = payment_cid(d, pay, p);
+    d.cid[p] = c;
+    return pay_rows(pay, p, c);
 }
 
 // Register addresses.
@@ -263,20 +276,25 @@ __device__ __forceinline__ unsigned long long *cust_w(const TpccDev &d, uint64_t
 // NewOrders take 16 adjacent lanes each (lane j < 15: line j, lane 15: the
 // header slots), BLK / 16 orders per block: an order's consecutive ORDERLINE
 // registers are touched by adjacent lanes, and all its roles share a CU.
-// Payments take one lane each, in the blocks after the NewOrder blocks.
+// Payments take one lane each, in the blocks before the NewOrder blocks: with
+// `cid` (the CID phase in the same call) a Payment that names its customer by
+// C_LAST first goes through the 12 dependent loads of its district's index,
+// and the NewOrder blocks run meanwhile (as a kernel of its own that takes
+// 9 us for 20,000 Payments, 13 us for 2^17, almost all of it latency).
 // BLK is 256, or 64 for the small-blocks launch shape (LTPG_TUNE_TPCC_SMALL_BLOCKS),
 // which spreads a small batch over four times as many CUs.
 template <bool COUNTS, uint32_t BLK>
 __global__ __launch_bounds__(BLK) void execute_kernel(TpccDev d, NeworderDev no, PaymentDev pay, uint32_t tag,
-                                                        uint8_t epoch, uint32_t no_blocks, DeviceCounters *ctr)
+                                                        uint8_t epoch, uint32_t pay_blocks, bool cid,
+                                                        DeviceCounters *ctr)
 {
     // the epoch's commit counts start at zero (CHECK adds to them)
     if (blockIdx.x == 0)
         for (uint32_t c = threadIdx.x; c < kCounterStripes * kCountedTypes; c += BLK)
             ctr->commits[c / kCountedTypes][c % kCountedTypes] = 0;
     uint32_t bad = 0;
-    if (blockIdx.x < no_blocks) {
-        const uint32_t q = blockIdx.x * (BLK / 16) + threadIdx.x / 16;
+    if (blockIdx.x >= pay_blocks) {
+        const uint32_t q = (blockIdx.x - pay_blocks) * (BLK / 16) + threadIdx.x / 16;
         const uint32_t j = threadIdx.x % 16;
         if (q < no.n) {
             const unsigned long long me = priority(tag, no.TID[q], q);
@@ -319,10 +337,10 @@ __global__ __launch_bounds__(BLK) void execute_kernel(TpccDev d, NeworderDev no,
             if (waw) d.doomed[q] = epoch;
         }
     } else {
-        const uint32_t p = (blockIdx.x - no_blocks) * BLK + threadIdx.x;
+        const uint32_t p = blockIdx.x * BLK + threadIdx.x;
         if (p < pay.n) {
             const unsigned long long me = priority(tag, pay.TID[p], no.n + p);
-            const PayRows r = pay_rows(d, pay, p);
+            const PayRows r = pay_rows_cid(d, pay, p, cid);
             bad += r.wh >= d.t[WH].rows ? 2 : 0;  // slots 0, 1
             bad += r.di >= d.t[DI].rows ? 2 : 0;  // slots 2, 3
             bool waw = false;
@@ -419,15 +437,15 @@ struct OrderTile {
 
 template <uint32_t BLK>
 __global__ __launch_bounds__(BLK) void claim_kernel(TpccDev d, NeworderDev no, PaymentDev pay, uint32_t tag,
-                                                      uint8_t epoch, uint32_t no_blocks, uint32_t *unsorted,
+                                                      uint8_t epoch, uint32_t pay_blocks, bool cid, uint32_t *unsorted,
                                                       DeviceCounters *ctr)
 {
     __shared__ OrderTile<BLK> s_tile;
     // the epoch's commit counts start at zero (CHECK adds to them)
     if (blockIdx.x == 0) zero_epoch_counts(ctr, BLK);
     uint32_t bad = 0;
-    if (blockIdx.x < no_blocks) {
-        const uint32_t q0 = blockIdx.x * OrderTile<BLK>::kOrders, q = q0 + threadIdx.x;
+    if (blockIdx.x >= pay_blocks) {
+        const uint32_t q0 = (blockIdx.x - pay_blocks) * OrderTile<BLK>::kOrders, q = q0 + threadIdx.x;
         s_tile.load(no, q0);
         if (threadIdx.x < OrderTile<BLK>::kOrders && q < no.n) {
             // header slots 0..4
@@ -453,10 +471,10 @@ __global__ __launch_bounds__(BLK) void claim_kernel(TpccDev d, NeworderDev no, P
             else bad++;
         }
     } else {
-        const uint32_t p = (blockIdx.x - no_blocks) * BLK + threadIdx.x;
+        const uint32_t p = blockIdx.x * BLK + threadIdx.x;
         if (p < pay.n) {
             const unsigned long long me = priority(tag, pay.TID[p], no.n + p);
-            const PayRows r = pay_rows(d, pay, p);
+            const PayRows r = pay_rows_cid(d, pay, p, cid);
             const bool cok = r.cu < d.t[CU].rows, hok = r.hi < d.t[HI].rows;
             // slots 0 to 5 in pairs, and the HISTORY insert
             bad += 2 * ((r.wh >= d.t[WH].rows) + (r.di >= d.t[DI].rows) + !cok) + !hok;
@@ -900,6 +918,50 @@ __global__ __launch_bounds__(kBlock) void delivery_writeback_kernel(TpccDev d, D
 
 // ---- WRITEBACK ---------------------------------------------------------------
 
+// W_YTD / D_YTD += H_AMOUNT of committed Payments (the hot-row reduce,
+// Genericfunction.h:431-518, applied to the table).  A block sums Payments
+// [p0, p1) into LDS bins (W warehouse bins, then 10W district bins) and adds
+// each non-zero bin to the table once, so a hot row takes one global atomic
+// per block instead of one per Payment.  More bins than `bins` holds: direct
+// global atomics.
+// Up to kYtdShared bins (372 warehouses) this is done by the first blocks of
+// the WRITEBACK kernel, beside its other work and without taking waves from it
+// (10 blocks of 16 KB fit a CU's LDS); as a kernel of its own behind it, it
+// took 5 us for 5,000 Payments and for 2^17.
+constexpr uint32_t kYtdShared = 4096;
+template <uint32_t BLK>
+__device__ __forceinline__ void ytd_block(const TpccDev &d, const PaymentDev &pay, uint64_t p0, uint64_t p1,
+                                          uint32_t *bins, bool lds)
+{
+    const uint64_t W = d.t[WH].rows, nd = d.t[DI].rows;
+    if (lds)
+        for (uint32_t i = threadIdx.x; i < W + nd; i += BLK) bins[i] = 0;
+    __syncthreads();
+#pragma unroll 4
+    for (uint64_t p = p0 + threadIdx.x; p < p1; p += BLK) {
+        // all loads at once: whether it committed, and what it would add
+        const uint64_t bits = d.bitmap_pay[p / 64], w = pay.W_ID[p], di = w * 10 + pay.D_ID[p];
+        const uint32_t amt = pay.H_AMOUNT[p];
+        if (!((bits >> (p % 64)) & 1ull)) continue;
+        if (w < W) {
+            if (lds) atomicAdd(&bins[w], amt);
+            else atomicAdd(d.t[WH].data + w * kStride[WH] + 2, amt);
+        }
+        if (di < nd) {
+            if (lds) atomicAdd(&bins[W + di], amt);
+            else atomicAdd(d.t[DI].data + di * kStride[DI] + 3, amt);
+        }
+    }
+    __syncthreads();
+    if (!lds) return;
+    for (uint32_t i = threadIdx.x; i < W + nd; i += BLK) {
+        const uint32_t v = bins[i];
+        if (v == 0) continue;
+        if (i < W) atomicAdd(d.t[WH].data + (uint64_t)i * kStride[WH] + 2, v);
+        else atomicAdd(d.t[DI].data + (uint64_t)(i - W) * kStride[DI] + 3, v);
+    }
+}
+
 // Committed transactions write their write slots (write_back dispatch,
 // Execute_neworder.h:698-850, Execute_payment.h:613-736).  RMW values:
 //   NEWORDER <- (O_ID, D_ID, W_ID), by its last committed inserter in
@@ -919,13 +981,21 @@ __global__ __launch_bounds__(kBlock) void delivery_writeback_kernel(TpccDev d, D
 // holds its snapshot value, apart from a NewOrder's own earlier lines.
 template <uint32_t BLK>
 __global__ __launch_bounds__(BLK) void writeback_kernel(TpccDev d, NeworderDev no, PaymentDev pay, uint8_t epoch,
-                                                          uint32_t no_blocks, int rmw)
+                                                          uint32_t ytd_blocks, uint32_t ytd_chunk, uint32_t no_blocks,
+                                                          int rmw)
 {
-    if (blockIdx.x < no_blocks) {
+    extern __shared__ uint32_t s_ytd[];
+    if (blockIdx.x < ytd_blocks) {
+        const uint64_t p0 = (uint64_t)blockIdx.x * ytd_chunk;
+        ytd_block<BLK>(d, pay, p0, min<uint64_t>(pay.n, p0 + ytd_chunk), s_ytd, true);
+        return;
+    }
+    const uint32_t block = blockIdx.x - ytd_blocks;
+    if (block < no_blocks) {
         // 16 lanes per NewOrder, as in EXECUTE: lane j < 15 writes line j,
         // lane 15 the NEWORDER and ORDER rows.  The group of an order is
         // active or idle as a whole, so the shuffles below read live lanes.
-        const uint32_t q = blockIdx.x * (BLK / 16) + threadIdx.x / 16;
+        const uint32_t q = block * (BLK / 16) + threadIdx.x / 16;
         const uint32_t j = threadIdx.x % 16;
         if (q >= no.n || !((d.bitmap_no[q / 64] >> (q % 64)) & 1ull)) return;
         const uint32_t oid = no.O_ID[q], did = no.D_ID[q], wid = no.W_ID[q];
@@ -996,7 +1066,7 @@ __global__ __launch_bounds__(BLK) void writeback_kernel(TpccDev d, NeworderDev n
             }
         }
     } else {
-        const uint32_t p = (blockIdx.x - no_blocks) * BLK + threadIdx.x;
+        const uint32_t p = (block - no_blocks) * BLK + threadIdx.x;
         if (p >= pay.n || !((d.bitmap_pay[p / 64] >> (p % 64)) & 1ull)) return;
         const PayRows r = pay_rows(d, pay, p);
         const uint32_t amt = pay.H_AMOUNT[p];
@@ -1021,12 +1091,7 @@ __global__ __launch_bounds__(BLK) void writeback_kernel(TpccDev d, NeworderDev n
     }
 }
 
-// W_YTD / D_YTD += H_AMOUNT of committed Payments (the hot-row reduce,
-// Genericfunction.h:431-518, applied to the table).  A block sums a chunk of
-// Payments into LDS bins (W warehouse bins, then 10W district bins) and adds
-// each non-zero bin to the table once, so a hot row takes one global atomic
-// per block instead of one per Payment.  More bins than LDS holds: direct
-// global atomics.
+// More warehouses than kYtdShared bins hold: a kernel of its own.
 constexpr uint32_t kYtdBins = 12288;  // 48 KB of LDS
 // 1024 threads per block: the block count is kept small (each block ends
 // with one global atomic per touched bin), so each block is made wide
@@ -1036,34 +1101,9 @@ constexpr uint32_t kYtdBlock = 1024;
 __global__ __launch_bounds__(kYtdBlock) void ytd_kernel(TpccDev d, PaymentDev pay, uint32_t chunk)
 {
     __shared__ uint32_t bins[kYtdBins];
-    const uint64_t W = d.t[WH].rows, nd = d.t[DI].rows;
-    const bool lds = W + nd <= kYtdBins;
-    if (lds)
-        for (uint32_t i = threadIdx.x; i < W + nd; i += kYtdBlock) bins[i] = 0;
-    __syncthreads();
-    const uint64_t p0 = (uint64_t)blockIdx.x * chunk, p1 = min<uint64_t>(pay.n, p0 + chunk);
-    for (uint64_t p = p0 + threadIdx.x; p < p1; p += kYtdBlock) {
-        if (!((d.bitmap_pay[p / 64] >> (p % 64)) & 1ull)) continue;
-        const uint64_t w = pay.W_ID[p], di = w * 10 + pay.D_ID[p];
-        const uint32_t amt = pay.H_AMOUNT[p];
-        if (w < W) {
-            if (lds) atomicAdd(&bins[w], amt);
-            else atomicAdd(d.t[WH].data + w * kStride[WH] + 2, amt);
-        }
-        if (di < nd) {
-            if (lds) atomicAdd(&bins[W + di], amt);
-            else atomicAdd(d.t[DI].data + di * kStride[DI] + 3, amt);
-        }
-    }
-    __syncthreads();
-    if (lds) {
-        for (uint32_t i = threadIdx.x; i < W + nd; i += kYtdBlock) {
-            const uint32_t v = bins[i];
-            if (v == 0) continue;
-            if (i < W) atomicAdd(d.t[WH].data + (uint64_t)i * kStride[WH] + 2, v);
-            else atomicAdd(d.t[DI].data + (uint64_t)(i - W) * kStride[DI] + 3, v);
-        }
-    }
+    const uint64_t p0 = (uint64_t)blockIdx.x * chunk;
+    ytd_block<kYtdBlock>(d, pay, p0, min<uint64_t>(pay.n, p0 + chunk), bins,
+                         d.t[WH].rows + d.t[DI].rows <= kYtdBins);
 }
 
 inline uint32_t grid_for(uint64_t n, uint32_t cap = 65536)
@@ -1115,16 +1155,16 @@ hipError_t launch_tpcc_cid(const TpccDev &d, const PaymentDev &pay, bool small, 
 
 template <uint32_t BLK>
 void execute_at(const TpccDev &d, const NeworderDev &no, const PaymentDev &pay, const EpochTag &e, bool counts,
-                DeviceCounters *ctr, hipStream_t s)
+                bool cid, DeviceCounters *ctr, hipStream_t s)
 {
-    const uint32_t no_blocks = (no.n + BLK / 16 - 1) / (BLK / 16);
-    const uint32_t blocks = std::max(1u, no_blocks + (pay.n + BLK - 1) / BLK);
+    const uint32_t pay_blocks = (pay.n + BLK - 1) / BLK;
+    const uint32_t blocks = std::max(1u, pay_blocks + (no.n + BLK / 16 - 1) / (BLK / 16));
     if (counts)
         hipLaunchKernelGGL((execute_kernel<true, BLK>), dim3(blocks), dim3(BLK), 0, s, d, no, pay, e.tag, e.epoch,
-                           no_blocks, ctr);
+                           pay_blocks, cid, ctr);
     else
         hipLaunchKernelGGL((execute_kernel<false, BLK>), dim3(blocks), dim3(BLK), 0, s, d, no, pay, e.tag, e.epoch,
-                           no_blocks, ctr);
+                           pay_blocks, cid, ctr);
 }
 
 // Shape of the binned STOCK writes: small tiles (many blocks for a batch of a
@@ -1154,20 +1194,21 @@ bool tpcc_execute_split(const TpccDev &d, const BinBuffers &bin, const NeworderD
 
 template <uint32_t BLK>
 void execute_split_at(const TpccDev &d, const NeworderDev &no, const PaymentDev &pay, const EpochTag &e,
-                      uint32_t *unsorted, DeviceCounters *ctr, hipStream_t s)
+                      bool cid, uint32_t *unsorted, DeviceCounters *ctr, hipStream_t s)
 {
-    const uint32_t no_blocks = (no.n + BLK / 4 - 1) / (BLK / 4), blocks = no_blocks + (pay.n + BLK - 1) / BLK;
-    hipLaunchKernelGGL(claim_kernel<BLK>, dim3(blocks), dim3(BLK), 0, s, d, no, pay, e.tag, e.epoch, no_blocks,
+    const uint32_t no_blocks = (no.n + BLK / 4 - 1) / (BLK / 4), pay_blocks = (pay.n + BLK - 1) / BLK;
+    const uint32_t blocks = no_blocks + pay_blocks;
+    hipLaunchKernelGGL(claim_kernel<BLK>, dim3(blocks), dim3(BLK), 0, s, d, no, pay, e.tag, e.epoch, pay_blocks, cid,
                        unsorted, ctr);
     hipLaunchKernelGGL(settle_kernel<BLK>, dim3(blocks), dim3(BLK), 0, s, d, no, pay, e.tag, e.epoch, no_blocks);
 }
 
 hipError_t launch_tpcc_execute_split(const TpccDev &d, const BinBuffers &bin, const NeworderDev &no,
-                                     const PaymentDev &pay, const EpochTag &e, bool small, DeviceCounters *ctr,
-                                     hipStream_t s)
+                                     const PaymentDev &pay, const EpochTag &e, bool cid, bool small,
+                                     DeviceCounters *ctr, hipStream_t s)
 {
-    if (small) execute_split_at<64>(d, no, pay, e, bin.unsorted, ctr, s);
-    else execute_split_at<kBlock>(d, no, pay, e, bin.unsorted, ctr, s);
+    if (small) execute_split_at<64>(d, no, pay, e, cid, bin.unsorted, ctr, s);
+    else execute_split_at<kBlock>(d, no, pay, e, cid, bin.unsorted, ctr, s);
     if (no.n == 0) return hipGetLastError();
     const StockSource src = {no, d.t[ST].rows, d.t[IT].rows};
     BinArgs a;
@@ -1182,10 +1223,10 @@ hipError_t launch_tpcc_execute_split(const TpccDev &d, const BinBuffers &bin, co
 }
 
 hipError_t launch_tpcc_execute(const TpccDev &d, const NeworderDev &no, const PaymentDev &pay, const EpochTag &e,
-                               bool counts, bool small, DeviceCounters *ctr, hipStream_t s)
+                               bool counts, bool cid, bool small, DeviceCounters *ctr, hipStream_t s)
 {
-    if (small) execute_at<64>(d, no, pay, e, counts, ctr, s);
-    else execute_at<kBlock>(d, no, pay, e, counts, ctr, s);
+    if (small) execute_at<64>(d, no, pay, e, counts, cid, ctr, s);
+    else execute_at<kBlock>(d, no, pay, e, counts, cid, ctr, s);
     return hipGetLastError();
 }
 
@@ -1257,12 +1298,18 @@ hipError_t launch_tpcc_writeback(const TpccDev &d, const NeworderDev &no, const 
     const uint32_t blocks = no_blocks + (pay.n + blk - 1) / blk;
     if (blocks == 0) return hipSuccess;
     const int rmw = values == LTPG_VALUES_RMW ? 1 : 0;
+    const uint64_t bins = d.t[WH].rows + d.t[DI].rows;
+    const bool ytd = rmw && pay.n, shared = ytd && bins <= kYtdShared;
+    const uint32_t ytd_chunk = std::max(4 * blk, (pay.n + 63) / 64);
+    const uint32_t ytd_blocks = shared ? (pay.n + ytd_chunk - 1) / ytd_chunk : 0;
+    const uint32_t lds = shared ? (uint32_t)bins * 4 : 0;
     if (small)
-        hipLaunchKernelGGL(writeback_kernel<64>, dim3(blocks), dim3(64), 0, s, d, no, pay, e.epoch, no_blocks, rmw);
+        hipLaunchKernelGGL(writeback_kernel<64>, dim3(ytd_blocks + blocks), dim3(64), lds, s, d, no, pay, e.epoch,
+                           ytd_blocks, ytd_chunk, no_blocks, rmw);
     else
-        hipLaunchKernelGGL(writeback_kernel<kBlock>, dim3(blocks), dim3(kBlock), 0, s, d, no, pay, e.epoch, no_blocks,
-                           rmw);
-    if (rmw && pay.n) {
+        hipLaunchKernelGGL(writeback_kernel<kBlock>, dim3(ytd_blocks + blocks), dim3(kBlock), lds, s, d, no, pay,
+                           e.epoch, ytd_blocks, ytd_chunk, no_blocks, rmw);
+    if (ytd && !shared) {
         const uint32_t chunk = std::max<uint32_t>(4096, (pay.n + 255) / 256);
         hipLaunchKernelGGL(ytd_kernel, dim3((pay.n + chunk - 1) / chunk), dim3(kYtdBlock), 0, s, d, pay, chunk);
     }
