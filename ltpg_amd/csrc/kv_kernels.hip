@@ -1417,7 +1417,7 @@ __global__ __launch_bounds__(kBlock) void kv_writeback_kernel(WriteArgs a, const
 // transactions x 16 ops on 100-byte fields, 3.5 % committed: CHECK 64 -> 7 + 29
 // us, WRITEBACK 74 -> 27 us.  With 81 % committed (9 reads, 1 write): CHECK 662
 // -> 7 + 441 us, which is the rate of random 128-byte reads and whole writes
-// (3.6 TB/s; the gather alone reaches 4.2), WRITEBACK 148 -> 176 us.
+// (3.6 TB/s; the gather alone reaches 4.2), WRITEBACK 148 -> 49 us.
 constexpr uint32_t kListBlock = 1024, kListPer = 4;  // transactions per block and thread
 
 __global__ __launch_bounds__(kListBlock) void kv_commit_list_kernel(
@@ -1500,22 +1500,111 @@ __global__ __launch_bounds__(kBlock) void kv_readout_list_kernel(
     if (pending) stage_flush(list, pending, lanes, table, read_values);
 }
 
-// WRITEBACK of the listed transactions, 64 / G per round; entries beyond a
-// smaller current batch (the phase without a fresh CHECK) are left out.
+// One round of 64 listed transactions, a lane each, whose slots are runs of 64.
+// The meta words of all slots come first and say which keys to load; a lane's
+// write fields wait in LDS, `fields` [slot][lane], to be folded.
+__device__ __forceinline__ uint32_t write_slots(const WriteArgs &a, uint32_t t, uint32_t (*fields)[64],
+                                                StageList &list, uint32_t pending, const FieldLanes &lanes)
+{
+    const uint32_t lane = (uint32_t)lane_id(), at = t < a.B ? t : 0u;
+    uint32_t writes = 0;
+#pragma unroll 4
+    for (uint32_t s = 0; s < a.S; ++s)
+        writes |= (uint32_t)((a.meta[(uint64_t)s * a.B + at] & 3u) == LTPG_KV_WRITE) << s;
+    if (t >= a.B) writes = 0;
+    const uint32_t step = a.values == LTPG_VALUES_RMW ? (a.tids[at] | 1u) : 0u;
+    uint32_t n = 0;
+    while (__ballot(writes != 0)) {
+        Op o[4];
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) {
+            const bool has = writes != 0;
+            const uint32_t s = has ? (uint32_t)__ffs(writes) - 1u : 0u;
+            writes &= writes - 1u;
+            o[u] = load_op(a.keys, a.meta, (uint64_t)s * a.B + at, has, a.rows, a.fields);
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u)  // writes to the hot row go through kv_hot_sum_kernel
+            if (o[u].valid && o[u].row != a.hot) fields[n++][lane] = (uint32_t)(o[u].row * a.fields) + o[u].field;
+    }
+    for (uint32_t k = 0; __ballot(k < n); k += 4) {
+        // fold duplicates: the first write of a field counts them all
+        uint32_t mine[4], count[4] = {0, 0, 0, 0};
+        bool first[4];
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) {
+            first[u] = k + u < n;
+            const uint32_t f = fields[first[u] ? k + u : 0u][lane];
+            mine[u] = first[u] ? f : 0u;  // a lane without one holds a field of the table all the same
+        }
+#pragma unroll 2
+        for (uint32_t i = 0; __ballot(i < n); ++i) {
+            const uint32_t f = fields[i < n ? i : 0u][lane];
+#pragma unroll
+            for (uint32_t u = 0; u < 4; ++u) {
+                const bool same = i < n && f == mine[u];
+                count[u] += same;
+                first[u] &= !(same && i < k + u);
+            }
+        }
+        if (a.fw < 4) {
+            for (uint32_t w = 0; w < a.fw; ++w) {
+                uint32_t v[4];
+#pragma unroll
+                for (uint32_t u = 0; u < 4; ++u) v[u] = a.table[(uint64_t)mine[u] * a.fsw + w];
+#pragma unroll
+                for (uint32_t u = 0; u < 4; ++u)
+                    if (first[u]) a.table[(uint64_t)mine[u] * a.fsw + w] = v[u] + step * count[u];
+            }
+            continue;
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < 4; ++u) {
+            const uint64_t off = (uint64_t)mine[u] * a.fsw;
+            pending = stage_push(list, pending, first[u], off, off, step * count[u]);
+            if (pending >= 64) {
+                stage_flush(list, pending, lanes, a.table, a.table);
+                pending = 0;
+            }
+        }
+    }
+    return pending;
+}
+
+// WRITEBACK of the listed transactions: 64 / G per round, or of a long list 64
+// (write_slots); entries beyond a smaller current batch (the phase without a
+// fresh CHECK) are left out.  Listed transactions lie close together, so their
+// slots come in runs, while lane groups read a line per slot and transaction,
+// and the keys of reads too: 1,013,000 commits of 9 reads and a write 142 us in
+// groups, 45 so (100-byte fields), 131,000 24 / 11; of 1 to 16 ops, half of
+// them writes, 456,000 commits 160 / 112, 203,000 70 / 56, 115,000 40 / 38.  A
+// lane's chain is longer, though, and few waves do not hide it: 62,000 of the
+// latter 24 / 33, 254,000 of one or two writes 21 / 22 (935,000: 89 / 81).
+constexpr uint32_t kSlotCommits = 1u << 17, kSlotOps = 1u << 20;
 template <int G>
 __global__ __launch_bounds__(kBlock) void kv_writeback_list_kernel(WriteArgs a, const uint32_t *__restrict__ commits,
-                                                                  const DeviceCounters *__restrict__ ctr)
+                                                                  const DeviceCounters *__restrict__ ctr, bool slots)
 {
+    constexpr bool kSlots = G <= 16;  // op slots that fit LDS
     __shared__ StageList s_stage[kBlock / 64];
-    StageList &list = s_stage[threadIdx.x / 64];
+    __shared__ uint32_t s_fields[kSlots ? kBlock / 64 : 1][kSlots ? G : 1][64];
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    StageList &list = s_stage[wave];
     const FieldLanes lanes(a.fw);
-    constexpr uint32_t PER = 64 / G;
-    const uint32_t n = ctr->kv_list_n, grp = (uint32_t)lane_id() / G;
+    const uint32_t n = ctr->kv_list_n;
     uint32_t pending = 0;
-    for (uint32_t j0 = (blockIdx.x * (kBlock / 64) + threadIdx.x / 64) * PER; j0 < n;
-         j0 += gridDim.x * (kBlock / 64) * PER) {
-        const uint32_t t = j0 + grp < n ? commits[j0 + grp] : a.B;
-        pending = write_round<G>(a, t < a.B, t < a.B ? t : 0u, list, pending, lanes);
+    if (kSlots && slots && n >= kSlotCommits && n * a.S >= kSlotOps) {
+        for (uint32_t j0 = (blockIdx.x * (kBlock / 64) + wave) * 64; j0 < n; j0 += gridDim.x * kBlock) {
+            const uint32_t j = j0 + (uint32_t)lane_id();
+            pending = write_slots(a, j < n ? commits[j] : a.B, s_fields[kSlots ? wave : 0], list, pending, lanes);
+        }
+    } else {
+        constexpr uint32_t PER = 64 / G;
+        const uint32_t grp = (uint32_t)lane_id() / G;
+        for (uint32_t j0 = (blockIdx.x * (kBlock / 64) + wave) * PER; j0 < n; j0 += gridDim.x * (kBlock / 64) * PER) {
+            const uint32_t t = j0 + grp < n ? commits[j0 + grp] : a.B;
+            pending = write_round<G>(a, t < a.B, t < a.B ? t : 0u, list, pending, lanes);
+        }
     }
     if (pending) stage_flush(list, pending, lanes, a.table, a.table);
 }
@@ -3176,7 +3265,9 @@ hipError_t launch_kv_writeback(const KvState &kv, const KvBatchDev &b, uint32_t 
     if (kv.list_valid && kv_check_lists(kv, b)) {
         const uint64_t per = (kBlock / 64) * (64 / g);  // transactions per block and round
         const dim3 grid((unsigned)std::min<uint64_t>(kListBlocks, (b.n_txns + per - 1) / per));
-#define CALL(GV) hipLaunchKernelGGL(kv_writeback_list_kernel<GV>, grid, dim3(kBlock), 0, s, a, kv.commit_list, ctr)
+        const bool slots = !a.rm && kv.rows * kv.fields <= 1ull << 32;  // a field's index fits 32 bits
+#define CALL(GV) \
+    hipLaunchKernelGGL(kv_writeback_list_kernel<GV>, grid, dim3(kBlock), 0, s, a, kv.commit_list, ctr, slots)
         LTPG_G_SWITCH(g, CALL)
 #undef CALL
     } else {
