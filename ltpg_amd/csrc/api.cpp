@@ -157,10 +157,7 @@ int init_kv(ltpg_ctx *ctx)
         (void)hipGetLastError();  // dealt with
     // Registers start as all-ones: tag ~0 belongs to epoch 0, which is never
     // current (epochs start at 1), so every row reads as "no registrant".
-    LTPG_HIP_TRY(launch_fill_u64(kv.regs, kv.rows * 2, ~0ull, ctx->stream));
-    LTPG_HIP_TRY(launch_fill_u8(kv.doomed, B, 0, ctx->stream));
-    LTPG_HIP_TRY(launch_fill_u8(kv.raw_flag, B, 0, ctx->stream));
-    LTPG_HIP_TRY(launch_fill_u8(kv.war_flag, B, 0, ctx->stream));
+    if ((rc = refill_registers(ctx))) return rc;
     LTPG_HIP_TRY(hipMemsetAsync(kv.table, 0, kv.rows * kv.fields * kv.field_stride * 4, ctx->stream));
     LTPG_HIP_TRY(hipMemsetAsync(kv.bitmap, 0, (B + 63) / 64 * 8, ctx->stream));
     LTPG_HIP_TRY(hipMemsetAsync(kv.conflicts, 0, B * 4, ctx->stream));
@@ -256,10 +253,7 @@ int init_tpcc(ltpg_ctx *ctx)
         bin_alloc(&tp.bin, B, [&](uint64_t n) { return stock_bin_shape(d.t[LTPG_TPCC_STOCK].rows, (uint32_t)n); },
                   ctx->stream) == LTPG_ERR_NOMEM)
         (void)hipGetLastError();  // dealt with
-    LTPG_HIP_TRY(launch_fill_u8(d.war, B, 0, ctx->stream));
-    LTPG_HIP_TRY(launch_fill_u64(d.regs, d.n_regs, ~0ull, ctx->stream));
-    LTPG_HIP_TRY(launch_fill_u8(d.doomed, B, 0, ctx->stream));
-    LTPG_HIP_TRY(launch_fill_u64(d.new_last, d.t[LTPG_TPCC_NEWORDER].rows, 0, ctx->stream));
+    if ((rc = refill_registers(ctx))) return rc;
     LTPG_HIP_TRY(hipMemsetAsync(d.bitmap_no, 0, (B + 63) / 64 * 8, ctx->stream));
     LTPG_HIP_TRY(hipMemsetAsync(d.bitmap_pay, 0, (B + 63) / 64 * 8, ctx->stream));
     LTPG_HIP_TRY(hipMemsetAsync(d.conf_no, 0, B * 4, ctx->stream));
@@ -308,20 +302,30 @@ int kv_part_prepare(ltpg_ctx *ctx)
     return LTPG_OK;
 }
 
+void initial_state(const ltpg_ctx *ctx, FillSet *f)
+{
+    const uint64_t B = ctx->cfg.max_txns;
+    const KvState &kv = ctx->kv;
+    if (kv.regs) {
+        f->add(kv.regs, kv.rows * 2 * 8, true);
+        f->add(kv.doomed, B, false);
+        f->add(kv.raw_flag, B, false);
+        f->add(kv.war_flag, B, false);
+    }
+    const TpccDev &d = ctx->tpcc.d;
+    if (d.regs) {
+        f->add(d.regs, d.n_regs * 8, true);
+        f->add(d.doomed, B, false);
+        f->add(d.war, B, false);
+        f->add(d.new_last, d.t[LTPG_TPCC_NEWORDER].rows * 8, false);
+    }
+}
+
 int refill_registers(ltpg_ctx *ctx)
 {
-    if (ctx->kv.regs) {
-        LTPG_HIP_TRY(launch_fill_u64(ctx->kv.regs, ctx->kv.rows * 2, ~0ull, ctx->stream));
-        LTPG_HIP_TRY(launch_fill_u8(ctx->kv.doomed, ctx->cfg.max_txns, 0, ctx->stream));
-        LTPG_HIP_TRY(launch_fill_u8(ctx->kv.raw_flag, ctx->cfg.max_txns, 0, ctx->stream));
-        LTPG_HIP_TRY(launch_fill_u8(ctx->kv.war_flag, ctx->cfg.max_txns, 0, ctx->stream));
-    }
-    if (ctx->tpcc.d.regs) {
-        LTPG_HIP_TRY(launch_fill_u64(ctx->tpcc.d.regs, ctx->tpcc.d.n_regs, ~0ull, ctx->stream));
-        LTPG_HIP_TRY(launch_fill_u8(ctx->tpcc.d.doomed, ctx->cfg.max_txns, 0, ctx->stream));
-        LTPG_HIP_TRY(launch_fill_u8(ctx->tpcc.d.war, ctx->cfg.max_txns, 0, ctx->stream));
-        LTPG_HIP_TRY(launch_fill_u64(ctx->tpcc.d.new_last, ctx->tpcc.d.t[LTPG_TPCC_NEWORDER].rows, 0, ctx->stream));
-    }
+    FillSet f;
+    initial_state(ctx, &f);
+    LTPG_HIP_TRY(launch_fill_set(f, ctx->stream));
     return LTPG_OK;
 }
 

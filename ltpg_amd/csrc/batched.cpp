@@ -22,6 +22,7 @@
 // own epoch tag, so the result is the plain loop's, bit for bit.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <chrono>
 #include <cstring>
 #include <new>
@@ -118,7 +119,7 @@ int enqueue_batch(ltpg_batched *b, uint32_t i, bool stamp, bool stepwise = false
         if (d.delivery.n && (rc = ltpg_tpcc_submit_delivery(ctx, &d.delivery, LTPG_MEM_DEVICE))) return rc;
     }
     if ((rc = stepwise ? run_epoch_stepwise(ctx) : ltpg_epoch_run(ctx, LTPG_PHASE_ALL))) return rc;
-    LTPG_HIP_TRY(launch_archive(archive_set(b, i), stamp ? b->stamps + i : nullptr, ctx->stream));
+    LTPG_HIP_TRY(launch_archive(archive_set(b, i), stamp ? b->stamps + i : nullptr, nullptr, ctx->stream));
     return LTPG_OK;
 }
 
@@ -130,13 +131,12 @@ hipError_t new_event(ltpg_batched *b, hipEvent_t *e)
 }
 
 // the second register set and its flags back to their initial state
-int refill_second_set(ltpg_batched *b, ltpg_ctx *ctx)
+void second_set(const ltpg_batched *b, const ltpg_ctx *ctx, FillSet *f)
 {
-    LTPG_HIP_TRY(launch_fill_u64(b->regs2, ctx->kv.rows * 2, ~0ull, ctx->stream));
-    LTPG_HIP_TRY(launch_fill_u8(b->doomed2, ctx->cfg.max_txns, 0, ctx->stream));
-    LTPG_HIP_TRY(launch_fill_u8(b->raw2, ctx->cfg.max_txns, 0, ctx->stream));
-    LTPG_HIP_TRY(launch_fill_u8(b->war2, ctx->cfg.max_txns, 0, ctx->stream));
-    return LTPG_OK;
+    f->add(b->regs2, ctx->kv.rows * 2 * 8, true);
+    f->add(b->doomed2, ctx->cfg.max_txns, false);
+    f->add(b->raw2, ctx->cfg.max_txns, false);
+    f->add(b->war2, ctx->cfg.max_txns, false);
 }
 
 // Capture topology: side joins the capture by a fork from main (an event
@@ -168,8 +168,10 @@ int enqueue_kv_pipelined(ltpg_batched *b)
     ltpg_ctx *ctx = b->ctx[0];
     hipStream_t main = ctx->stream, side = b->side;
     int rc;
-    if ((rc = refill_second_set(b, ctx))) return rc;
     if ((rc = fork_side(b, main, side))) return rc;  // side joins the capture after the refills
+    const uint32_t n_kv = (uint32_t)std::count_if(b->d.begin(), b->d.end(), [](const ltpg_batch_desc &d) {
+        return d.workload == LTPG_WORKLOAD_KV;
+    });
     std::vector<hipEvent_t> checked;                 // per key-value batch: its CHECK is done
     uint32_t j = 0;
     for (uint32_t i = 0; i < b->d.size(); i++) {
@@ -181,7 +183,9 @@ int enqueue_kv_pipelined(ltpg_batched *b)
             // main: nothing may be in flight on side, and the second set
             // starts over too
             if ((rc = join_side(b, main, side))) return rc;
-            if ((rc = refill_second_set(b, ctx))) return rc;
+            FillSet f;
+            second_set(b, ctx, &f);
+            LTPG_HIP_TRY(launch_fill_set(f, main));
         }
         const uint32_t before = ctx->epoch;
         if ((rc = ltpg_kv_submit(ctx, &d.kv, LTPG_MEM_DEVICE))) return rc;
@@ -200,20 +204,21 @@ int enqueue_kv_pipelined(ltpg_batched *b)
             st.war_flag = b->war2;
         }
         if (j >= 2 && checked[j - 2]) LTPG_HIP_TRY(hipStreamWaitEvent(side, checked[j - 2], 0));
-        LTPG_HIP_TRY(launch_kv_execute(st, st.cur, e, false, ctx->counters, side, false));
+        // the first EXECUTE starts the commit counts at zero, then each archive
+        // does for the batch after it
+        LTPG_HIP_TRY(launch_kv_execute(st, st.cur, e, false, ctx->counters, side, j == 0));
         hipEvent_t executed, done;
         LTPG_HIP_TRY(new_event(b, &executed));
         LTPG_HIP_TRY(hipEventRecord(executed, side));
         LTPG_HIP_TRY(hipStreamWaitEvent(main, executed, 0));
-        LTPG_HIP_TRY(launch_reset_epoch_counters(ctx->counters, main));
         LTPG_HIP_TRY(launch_kv_check(st, st.cur, e, false, ctx->counters, main));
         LTPG_HIP_TRY(new_event(b, &done));
         LTPG_HIP_TRY(hipEventRecord(done, main));
         checked.push_back(done);
         st.list_valid = true;  // of the CHECK above
         LTPG_HIP_TRY(launch_kv_writeback(st, st.cur, ctx->cfg.values, ctx->counters, main));
-        LTPG_HIP_TRY(launch_archive(archive_set(b, i), b->stamps + i, main));
         j++;
+        LTPG_HIP_TRY(launch_archive(archive_set(b, i), b->stamps + i, j < n_kv ? ctx->counters : nullptr, main));
     }
     return join_side(b, main, side);  // side rejoins main before the capture ends
 }
@@ -230,7 +235,10 @@ int capture(ltpg_batched *b, int k)
     LTPG_HIP_TRY(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
     // every replay starts from all-ones registers and epoch 1
     ctx->epoch = 0;
-    int rc = refill_registers(ctx);
+    FillSet f;
+    initial_state(ctx, &f);
+    if (k == 0 && b->side) second_set(b, ctx, &f);
+    int rc = launch_fill_set(f, ctx->stream) == hipSuccess ? LTPG_OK : LTPG_ERR_DEVICE;
     if (!rc && launch_stamp(b->stamps + b->d.size() + k, ctx->stream) != hipSuccess) rc = LTPG_ERR_DEVICE;
     if (k == 0 && b->side) {
         if (!rc) rc = enqueue_kv_pipelined(b);
@@ -382,7 +390,10 @@ int ltpg_batched_run(ltpg_batched *b, uint32_t mode)
         return LTPG_OK;
     }
     if (mode != LTPG_RUN_GRAPH) LTPG_FAIL(LTPG_ERR_INVALID, "unknown run mode");
-    for (int k = 0; k < 2; k++) {
+    // Order entry first: its graph, one chain, is on its way in 50 us, the
+    // key-value graph of two streams in 280 (24 batches: 963 us the other way
+    // round, 821 so).
+    for (int k = 1; k >= 0; k--) {
         if (!b->exec[k]) continue;
         LTPG_HIP_TRY(hipGraphLaunch(b->exec[k], b->ctx[k]->stream));
         // the registers now carry the captured sequence's epoch tags

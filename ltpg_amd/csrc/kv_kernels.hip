@@ -211,6 +211,22 @@ __global__ void fill_u64_kernel(unsigned long long *p, uint64_t n, unsigned long
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += stride) p[i] = v;
 }
 
+// Registers and flags back to their initial state, all in one kernel with
+// 16-byte stores: a replayed run of both workloads starts with 8 arrays of the
+// key-value context (two register sets of 10M rows, their flags) and 4 of the
+// order-entry one, whose fills took 79 and 29 us one by one.
+__global__ __launch_bounds__(256) void fill_set_kernel(FillSet f)
+{
+    const uint64_t first = (uint64_t)blockIdx.x * 256 + threadIdx.x, step = (uint64_t)gridDim.x * 256;
+    for (uint32_t k = 0; k < f.n; k++) {
+        const uint32_t v = f.ones[k] ? ~0u : 0u;
+        const uint64_t vecs = f.bytes[k] / 16;
+        uint4 *p = static_cast<uint4 *>(f.p[k]);
+        for (uint64_t i = first; i < vecs; i += step) p[i] = make_uint4(v, v, v, v);
+        if (first < f.bytes[k] % 16) reinterpret_cast<uint8_t *>(p + vecs)[first] = (uint8_t)v;
+    }
+}
+
 // u32 copy, grid-stride; the source may be pinned host memory (the served
 // form's staging: a kernel on the epoch's own stream costs one launch, where
 // a copy-engine transfer costs a copy call plus a cross-stream event).
@@ -259,8 +275,11 @@ __global__ __launch_bounds__(256) void readback_kernel(uint32_t *__restrict__ ds
 // A batch's commit bitmaps into the archive of a run, which may sit in pinned
 // host memory, and the device clock into its stamp: one kernel, where a copy
 // for each bitmap and one for the stamp were up to six.
-__global__ void archive_kernel(PublishSet p, unsigned long long *stamp)
+// With `reset` the next batch's commit counts and list start over (a run whose
+// EXECUTE overlaps the batch before cannot do that there).
+__global__ void archive_kernel(PublishSet p, unsigned long long *stamp, DeviceCounters *reset)
 {
+    if (reset && blockIdx.x == 0) zero_epoch_counts(reset, blockDim.x);
     const uint32_t stride = gridDim.x * blockDim.x;
     for (int k = 0; k < 5; k++)
         for (uint32_t w = blockIdx.x * blockDim.x + threadIdx.x; w < p.n[k]; w += stride) p.dst[k][w] = p.src[k][w];
@@ -2889,6 +2908,15 @@ hipError_t launch_copy_u128(void *dst, const void *src, uint64_t n16, hipStream_
     return hipGetLastError();
 }
 
+hipError_t launch_fill_set(const FillSet &f, hipStream_t s)
+{
+    uint64_t most = 1;
+    for (uint32_t k = 0; k < f.n; k++) most = std::max(most, f.bytes[k]);
+    const uint64_t blocks = std::min<uint64_t>((most + 16 * 256 - 1) / (16 * 256), 8192);
+    hipLaunchKernelGGL(fill_set_kernel, dim3((unsigned)blocks), dim3(256), 0, s, f);
+    return hipGetLastError();
+}
+
 hipError_t launch_fill_u64(unsigned long long *p, uint64_t n, unsigned long long v, hipStream_t s)
 {
     hipLaunchKernelGGL(fill_u64_kernel, grid_stride(n), dim3(kBlock), 0, s, p, n, v);
@@ -2916,12 +2944,12 @@ hipError_t launch_publish(const PublishSet &p, uint64_t *seq_out, uint64_t seq, 
     return hipGetLastError();
 }
 
-hipError_t launch_archive(const PublishSet &p, unsigned long long *stamp, hipStream_t s)
+hipError_t launch_archive(const PublishSet &p, unsigned long long *stamp, DeviceCounters *reset, hipStream_t s)
 {
     uint32_t most = 1;
     for (int k = 0; k < 5; k++) most = std::max(most, p.n[k]);
     const uint32_t blocks = std::min((most + kBlock - 1) / kBlock, 64u);
-    hipLaunchKernelGGL(archive_kernel, dim3(blocks), dim3(kBlock), 0, s, p, stamp);
+    hipLaunchKernelGGL(archive_kernel, dim3(blocks), dim3(kBlock), 0, s, p, stamp, reset);
     return hipGetLastError();
 }
 

@@ -350,6 +350,20 @@ hipError_t launch_gather_calibration(const uint32_t *src, uint64_t slots, uint32
                                      uint32_t *dst, uint64_t n, hipStream_t s);
 hipError_t launch_calibration(unsigned long long *a, uint64_t len, uint64_t n, int atomics,
                               unsigned long long *sink, hipStream_t s);
+// Arrays to fill with zero or one bits (16-byte aligned).
+struct FillSet {
+    void *p[10];
+    uint64_t bytes[10];
+    bool ones[10];
+    uint32_t n = 0;
+    void add(void *at, uint64_t size, bool set_bits)
+    {
+        p[n] = at;
+        bytes[n] = size;
+        ones[n++] = set_bits;
+    }
+};
+hipError_t launch_fill_set(const FillSet &f, hipStream_t s);
 hipError_t launch_fill_u64(unsigned long long *p, uint64_t n, unsigned long long v, hipStream_t s);
 hipError_t launch_fill_u8(uint8_t *p, uint64_t n, uint8_t v, hipStream_t s);
 // n u32 words; src may be pinned host memory
@@ -368,13 +382,14 @@ struct PublishSet {
 // copy the bitmaps of p, then store seq to *seq_out (pinned host memory)
 // with a system-scope release; or copy them and stamp the device clock (unless
 // null)
-hipError_t launch_archive(const PublishSet &p, unsigned long long *stamp, hipStream_t s);
+hipError_t launch_archive(const PublishSet &p, unsigned long long *stamp, DeviceCounters *reset, hipStream_t s);
 hipError_t launch_publish(const PublishSet &p, uint64_t *seq_out, uint64_t seq, hipStream_t s);
 hipError_t launch_stamp(unsigned long long *out, hipStream_t s);
 
 // Registers back to "no registrant" (all-ones), doomed flags and NEWORDER
 // inserters to 0, on the context's stream (api.cpp).  Epoch-tag wrap and the
 // start of a captured batch sequence use it.
+void initial_state(const ltpg_ctx *ctx, FillSet *f);
 int refill_registers(ltpg_ctx *ctx);
 int kv_part_prepare(ltpg_ctx *ctx);
 // The key-value launch shape a context starts with: no flag, sizes decide.
