@@ -1239,8 +1239,8 @@ int ltpg_epoch_run(ltpg_ctx *ctx, uint32_t phase_mask)
     if (!kv.has_batch) LTPG_FAIL(LTPG_ERR_STATE, "no batch submitted");
     const EpochTag e = epoch_tag(ctx);
     hipStream_t s = ctx->stream;
-    if (kv.small_epoch && phase_mask == LTPG_PHASE_ALL && !ctx->timing &&
-        !(ctx->cfg.flags & LTPG_FLAG_CONFLICT_COUNTS) && kv_small_epoch_ok(kv, kv.cur)) {
+    if (phase_mask == LTPG_PHASE_ALL && !ctx->timing && !(ctx->cfg.flags & LTPG_FLAG_CONFLICT_COUNTS) &&
+        (kv.small_epoch ? kv_small_epoch_ok(kv, kv.cur) : kv_small_auto(kv, kv.cur))) {
         kv.list_valid = false;
         LTPG_HIP_TRY(launch_kv_small_epoch(kv, kv.cur, ctx->cfg.values, ctx->counters, nullptr, nullptr, 0, s));
         return LTPG_OK;

@@ -1648,9 +1648,10 @@ constexpr uint32_t kSmallBlock = 1024;
 constexpr uint32_t kSmallOps = LTPG_SMALL_EPOCH_OPS;
 constexpr uint32_t kSmallPer = kSmallOps / kSmallBlock;  // op slots per thread
 constexpr uint32_t kSmallSlots = 2 * kSmallOps;          // hash load <= 1/2: probing always ends
-constexpr uint32_t kSmallUnroll = 4;                     // field words in flight per thread
-constexpr uint32_t kSmallMerge = 8;                      // items per thread of the one-round copy
+constexpr uint32_t kSmallUnroll = 4;                     // 16-byte pieces in flight per thread
+constexpr uint32_t kSmallMerge = 8;                      // the same in the one-round copy
 constexpr uint32_t kSmallHotFields = 1024;               // fields of a table with a hot row
+constexpr uint32_t kSmallCopies = kSmallOps + kSmallHotFields;
 
 __device__ __forceinline__ uint32_t small_hash(uint64_t row)
 {
@@ -1682,10 +1683,15 @@ __global__ __launch_bounds__(kSmallBlock) void kv_small_epoch_kernel(
     __shared__ unsigned long long s_min[kSmallSlots];  // its writers' minimum TID << 24 | position
     __shared__ uint8_t s_waw[kSmallOps], s_raw[kSmallOps], s_war[kSmallOps];
     __shared__ uint32_t s_list[kSmallOps];             // committed transactions
-    __shared__ uint32_t s_fold[kSmallOps];             // per committed (txn, slot): folded write count
+    __shared__ uint32_t s_add[kSmallCopies];           // of a copy: a write's delta, a read's rows
     __shared__ unsigned long long s_bits[kSmallOps / 64];  // the commit bitmap
     __shared__ uint32_t s_hot[kSmallHotFields];        // committed hot-row deltas per field
-    __shared__ uint32_t s_n, s_bad;
+    __shared__ uint32_t s_n, s_bad, s_reads, s_writes;
+    // the copies, in the hash's place: committed reads from the front, folded
+    // writes from the back
+    unsigned long long *s_field = s_min;  // the table's field
+    uint32_t *s_slot = s_key;             // a read's op slot
+    static_assert(kSmallCopies <= kSmallSlots, "the copies fit the hash");
     const uint32_t n = B * S;
     // the batch: every load issued before the first use
     uint64_t r[kSmallPer];
@@ -1711,6 +1717,8 @@ __global__ __launch_bounds__(kSmallBlock) void kv_small_epoch_kernel(
     if (threadIdx.x == 0) {
         s_n = 0;
         s_bad = 0;
+        s_reads = 0;
+        s_writes = 0;
     }
 #pragma unroll
     for (uint32_t k = 0; k < kSmallPer; ++k) {
@@ -1792,126 +1800,135 @@ __global__ __launch_bounds__(kSmallBlock) void kv_small_epoch_kernel(
     }
     __syncthreads();
     const uint32_t nc = s_n;
-    // write folding, one wave per committed transaction (lane = slot): the
-    // first write slot of a transaction on a field writes word + count *
-    // delta, the others nothing.  Hot-row writes add their delta to the
-    // field's sum instead (kv_hot_sum_kernel's reduce).
-    for (uint32_t j = threadIdx.x / 64; j < nc; j += kSmallBlock / 64) {
-        const uint32_t t = s_list[j], sl = lane_id();
-        const uint32_t i = sl < S ? (rm ? t * S + sl : sl * B + t) : 0u;
+    // list the copies, G lanes per committed transaction (lane = slot): each
+    // read, and the first write slot of a transaction on a field, which writes
+    // word + count * delta, the others nothing.  Hot-row writes add their
+    // delta to the field's sum instead (kv_hot_sum_kernel's reduce).
+    const bool rmw = values == LTPG_VALUES_RMW;  // copy-back changes nothing
+    const uint32_t G = S <= 1 ? 1u : 1u << (32 - __clz((int)(S - 1)));
+    const uint32_t sl = (uint32_t)lane_id() % G, grp = (uint32_t)lane_id() / G, txns = 64 / G;
+    for (uint32_t j0 = (threadIdx.x / 64) * txns; j0 < nc; j0 += kSmallBlock / G) {
+        const bool has = j0 + grp < nc && sl < S;
+        const uint32_t t = has ? s_list[j0 + grp] : 0u;
+        const uint32_t i = has ? (rm ? t * S + sl : sl * B + t) : 0u;
         const Op o = decode_op(s_row[i], s_meta[i], rows, fields, max_scan);
-        const bool any_wr = sl < S && o.valid && o.kind == LTPG_KV_WRITE;
-        if (any_wr && o.row == hot && values == LTPG_VALUES_RMW) atomicAdd(&s_hot[o.field], s_tid[t] | 1u);
-        const bool wr = any_wr && o.row != hot;
-        const unsigned long long wm = __ballot(wr);
+        const bool any_wr = has && rmw && o.valid && o.kind == LTPG_KV_WRITE;
+        if (any_wr && o.row == hot) atomicAdd(&s_hot[o.field], s_tid[t] | 1u);
+        const bool wr = any_wr && o.row != hot, rd = has && o.valid && o.kind != LTPG_KV_WRITE;
+        const unsigned long long wm = __ballot(wr), rdm = __ballot(rd);
         const uint64_t key = o.row * fields + o.field;
         uint32_t count = 0;
-        bool first = true;
-        for (uint32_t k = 0; k < S; ++k) {
-            const uint64_t kk = __shfl(key, (int)k);
-            if (((wm >> k) & 1ull) && kk == key) {
+        bool first = wr;
+        for (uint32_t k = 0; wm && k < S; ++k) {
+            const uint64_t kk = __shfl(key, (int)(grp * G + k));
+            if (((wm >> (grp * G + k)) & 1ull) && kk == key) {
                 ++count;
                 first &= k >= sl;
             }
         }
-        if (sl < S) s_fold[j * S + sl] = wr && first ? count : 0u;
+        const unsigned long long fm = __ballot(first), below = (1ull << lane_id()) - 1ull;
+        uint32_t r0 = 0, w0 = 0;
+        if (lane_id() == 0) {
+            if (rdm) r0 = atomicAdd(&s_reads, (uint32_t)__popcll(rdm));
+            if (fm) w0 = atomicAdd(&s_writes, (uint32_t)__popcll(fm));
+        }
+        r0 = __shfl(r0, 0);
+        w0 = __shfl(w0, 0);
+        const uint32_t at = rd ? r0 + (uint32_t)__popcll(rdm & below)
+                               : kSmallCopies - 1 - (w0 + (uint32_t)__popcll(fm & below));
+        if (rd || first) {
+            s_field[at] = key;
+            s_slot[at] = sl * B + t;
+            s_add[at] = rd ? o.len : count * (s_tid[t] | 1u);
+        }
     }
     __syncthreads();
+    if (has_hot && rmw) {
+        for (uint32_t f = threadIdx.x; f < fields; f += kSmallBlock) {
+            if (s_hot[f] == 0) continue;
+            const uint32_t at = kSmallCopies - 1 - atomicAdd(&s_writes, 1u);
+            s_field[at] = hot * fields + f;
+            s_add[at] = s_hot[f];
+        }
+        __syncthreads();
+    }
     // read-out of the committed reads and write-back of the committed
-    // writes.  Reads see the snapshot: when all items fit one round, every
-    // load is issued before a barrier and every store after it; otherwise
-    // the read-out runs in rounds, then a barrier, then the write-back.
-    const uint32_t per = L * fw, total_r = nc * S * per;
-    const uint32_t total_w = values == LTPG_VALUES_RMW ? nc * S * fw : 0u;
-    const uint32_t total_h = values == LTPG_VALUES_RMW && has_hot ? fields * fw : 0u;
-    const auto read_item = [&](uint32_t x, uint64_t &src, uint64_t &dst) -> bool {
-        const uint32_t j = x / per, q = (x % per) / fw, w = x % fw;
-        const uint32_t t = s_list[j / S], sl = j % S;
-        const uint32_t i = rm ? t * S + sl : sl * B + t;
-        const Op o = decode_op(s_row[i], s_meta[i], rows, fields, max_scan);
-        const bool ok = q < o.len;
-        src = ok ? ((o.row + q) * fields + o.field) * fsw + w : 0ull;
-        dst = ((((uint64_t)sl * B + t) * L) + q) * fsw + w;
-        return ok;
+    // writes, 16 bytes per lane (FieldLanes).  Reads see the snapshot: when
+    // all fit one round, every load is issued before a barrier and every store
+    // after it; otherwise the read-out runs in rounds, then a barrier, then the
+    // write-back.  1,024 transactions of two ops on 100-byte fields, whole
+    // epoch: 102 us word by word with each word's op decoded again, 33 so;
+    // on 1 KB fields 623 and 165.
+    const uint32_t total_r = s_reads * L, total = total_r + s_writes;
+    const FieldLanes lanes(max(fw, 4u));
+    const uint32_t mine = threadIdx.x >> lanes.log_lanes, per = kSmallBlock >> lanes.log_lanes;
+    struct Copy {
+        uint64_t src, dst;
+        uint32_t add;
+        bool ok, read;
+        Words4 v;
     };
-    const auto write_item = [&](uint32_t x, uint64_t &off, uint32_t &add) -> bool {
-        if (x >= total_w) {  // a word of the hot row: its field's sum
-            const uint32_t f = (x - total_w) / fw, w = (x - total_w) % fw;
-            add = s_hot[f];
-            off = add ? (hot * fields + f) * fsw + w : 0ull;
-            return add != 0u;
+    const auto look = [&](uint32_t x, uint32_t end, Copy &c) {
+        c.ok = lanes.on && x < end;
+        c.read = x < total_r;
+        c.src = c.dst = c.add = 0;
+        if (!c.ok) return;
+        if (c.read) {
+            const uint32_t e = L == 1 ? x : x / L, q = x - e * L;  // row q of a scan
+            c.ok = q < s_add[e];
+            if (c.ok) c.src = (s_field[e] + (uint64_t)q * fields) * fsw;
+            c.dst = ((uint64_t)s_slot[e] * L + q) * fsw;
+        } else {
+            const uint32_t e = kSmallCopies - 1 - (x - total_r);
+            c.src = c.dst = s_field[e] * fsw;
+            c.add = s_add[e];
         }
-        const uint32_t j = x / fw, w = x % fw;
-        const uint32_t count = s_fold[j];
-        const uint32_t t = s_list[j / S], sl = j % S;
-        const uint32_t i = rm ? t * S + sl : sl * B + t;
-        const Op o = decode_op(s_row[i], s_meta[i], rows, fields, max_scan);
-        add = count * (s_tid[t] | 1u);
-        off = count ? (o.row * fields + o.field) * fsw + w : 0ull;
-        return count != 0u;
     };
-    if (total_r + total_w + total_h <= kSmallMerge * kSmallBlock) {
-        uint64_t src[kSmallMerge], dst[kSmallMerge];
-        uint32_t v[kSmallMerge], add[kSmallMerge];
-        bool ok[kSmallMerge], rd[kSmallMerge];
-#pragma unroll
-        for (uint32_t u = 0; u < kSmallMerge; ++u) {
-            const uint32_t x = u * kSmallBlock + threadIdx.x;
-            rd[u] = x < total_r;
-            add[u] = 0u;
-            if (rd[u])
-                ok[u] = read_item(x, src[u], dst[u]);
-            else if (x < total_r + total_w + total_h)
-                ok[u] = write_item(x - total_r, src[u], add[u]);
-            else
-                ok[u] = false;
-            if (!ok[u]) src[u] = 0ull;
-            if (!rd[u]) dst[u] = src[u];
+    const auto load = [&](Copy &c) {  // a lane without a copy loads from field 0
+        const uint32_t *p = table + c.src + lanes.off;
+        if (fw >= 4) {
+            c.v = *reinterpret_cast<const Words4 *>(p);
+            return;
         }
 #pragma unroll
-        for (uint32_t u = 0; u < kSmallMerge; ++u) v[u] = table[src[u]];
+        for (uint32_t w = 0; w < 3; ++w) c.v.w[w] = p[min(w, fw - 1)];
+    };
+    const auto store = [&](const Copy &c) {
+        if (!c.ok) return;
+        uint32_t *p = (c.read ? read_values : table) + c.dst + lanes.off;
+        Words4 v = c.v;
+#pragma unroll
+        for (uint32_t w = 0; w < 4; ++w) v.w[w] += c.add;
+        if (fw >= 4) {
+            *reinterpret_cast<Words4 *>(p) = v;
+            return;
+        }
+#pragma unroll
+        for (uint32_t w = 0; w < 3; ++w)
+            if (w < fw) p[w] = v.w[w];
+    };
+    if (total <= kSmallMerge * per) {
+        Copy c[kSmallMerge];
+#pragma unroll
+        for (uint32_t u = 0; u < kSmallMerge; ++u) look(u * per + mine, total, c[u]);
+#pragma unroll
+        for (uint32_t u = 0; u < kSmallMerge; ++u) load(c[u]);
         __syncthreads();
 #pragma unroll
-        for (uint32_t u = 0; u < kSmallMerge; ++u) {
-            if (!ok[u]) continue;
-            if (rd[u])
-                read_values[dst[u]] = v[u];
-            else
-                table[dst[u]] = v[u] + add[u];
-        }
+        for (uint32_t u = 0; u < kSmallMerge; ++u) store(c[u]);
     } else {
-        for (uint32_t b0 = 0; b0 < total_r; b0 += kSmallUnroll * kSmallBlock) {
-            uint64_t src[kSmallUnroll], dst[kSmallUnroll];
-            bool ok[kSmallUnroll];
-            uint32_t v[kSmallUnroll];
+        for (uint32_t part = 0; part < 2; ++part) {
+            const uint32_t end = part ? total : total_r;
+            for (uint32_t x0 = part ? total_r : 0u; x0 < end; x0 += kSmallUnroll * per) {
+                Copy c[kSmallUnroll];
 #pragma unroll
-            for (uint32_t u = 0; u < kSmallUnroll; ++u) {
-                const uint32_t x = b0 + u * kSmallBlock + threadIdx.x;
-                ok[u] = x < total_r && read_item(x, src[u], dst[u]);
-                if (!ok[u]) src[u] = 0ull;
+                for (uint32_t u = 0; u < kSmallUnroll; ++u) look(x0 + u * per + mine, end, c[u]);
+#pragma unroll
+                for (uint32_t u = 0; u < kSmallUnroll; ++u) load(c[u]);
+#pragma unroll
+                for (uint32_t u = 0; u < kSmallUnroll; ++u) store(c[u]);
             }
-#pragma unroll
-            for (uint32_t u = 0; u < kSmallUnroll; ++u) v[u] = table[src[u]];
-#pragma unroll
-            for (uint32_t u = 0; u < kSmallUnroll; ++u)
-                if (ok[u]) read_values[dst[u]] = v[u];
-        }
-        __syncthreads();
-        for (uint32_t b0 = 0; b0 < total_w + total_h; b0 += kSmallUnroll * kSmallBlock) {
-            uint64_t off[kSmallUnroll];
-            uint32_t add[kSmallUnroll], v[kSmallUnroll];
-            bool ok[kSmallUnroll];
-#pragma unroll
-            for (uint32_t u = 0; u < kSmallUnroll; ++u) {
-                const uint32_t x = b0 + u * kSmallBlock + threadIdx.x;
-                ok[u] = x < total_w + total_h && write_item(x, off[u], add[u]);
-                if (!ok[u]) off[u] = 0ull;
-            }
-#pragma unroll
-            for (uint32_t u = 0; u < kSmallUnroll; ++u) v[u] = table[off[u]];
-#pragma unroll
-            for (uint32_t u = 0; u < kSmallUnroll; ++u)
-                if (ok[u]) table[off[u]] = v[u] + add[u];
+            __syncthreads();
         }
     }
     if (threadIdx.x == 0 && result) {
@@ -3324,6 +3341,24 @@ bool kv_small_epoch_ok(const KvState &kv, const KvBatchDev &b)
 {
     return b.n_txns > 0 && b.n_slots > 0 && (uint64_t)b.n_txns * b.n_slots <= kSmallOps &&
            (kv.hot_row == LTPG_NO_HOT_ROW || kv.fields <= kSmallHotFields) && kv.rows < 0xFFFFFFFFull;
+}
+
+// Words a small epoch copies at most.
+uint64_t kv_small_words(const KvState &kv, const KvBatchDev &b)
+{
+    return (uint64_t)b.n_txns * b.n_slots * kv.read_slot * kv.field_words;
+}
+
+// The single-workgroup epoch by default: one workgroup copies fields at a
+// fraction of the chip's rate, so it is taken while what it saves in launches
+// is more (one kernel against four, back to back, uniform rows: 64 ops on
+// 4-byte fields 7 us against 17, 1,024 12 / 18, of 64 slots each 2,048 26 / 22;
+// 100-byte fields 256 ops 12 / 17, 512 15 / 18, 1,024 20 / 19; 1 KB fields 64
+// ops 15 / 22, 256 30 / 25).
+bool kv_small_auto(const KvState &kv, const KvBatchDev &b)
+{
+    return kv.auto_shape && kv_small_epoch_ok(kv, b) && (uint64_t)b.n_txns * b.n_slots <= kSmallOps / 2 &&
+           kv_small_words(kv, b) <= 1u << 14;
 }
 
 hipError_t launch_kv_small_epoch(const KvState &kv, const KvBatchDev &b, uint32_t values, DeviceCounters *ctr,

@@ -428,6 +428,8 @@ hipError_t launch_kv_writeback(const KvState &kv, const KvBatchDev &b, uint32_t 
 // 2^32 - 1).  With seq_out it
 // also publishes: the bitmap to host_bits, then seq with a release.
 bool kv_small_epoch_ok(const KvState &kv, const KvBatchDev &b);
+uint64_t kv_small_words(const KvState &kv, const KvBatchDev &b);
+bool kv_small_auto(const KvState &kv, const KvBatchDev &b);
 hipError_t launch_kv_small_epoch(const KvState &kv, const KvBatchDev &b, uint32_t values, DeviceCounters *ctr,
                                  uint64_t *host_bits, uint64_t *seq_out, uint64_t seq, hipStream_t s,
                                  uint32_t *result = nullptr);

@@ -87,6 +87,12 @@ int scratch_of(int device, uint8_t **out)
     return LTPG_OK;
 }
 
+// Words of fields that one workgroup may copy before the other path's six
+// kernels are faster (uniform rows, back to back: 1,024 ops on 100-byte fields
+// 18 us against 27, 2,048 34 / 27; on 400-byte fields 512 ops 28 / 30, 1,024
+// 46 / 30; on 1 KB fields 256 ops 29 / 35, 512 48 / 34).
+constexpr uint64_t kAloneWords = 3u << 14;
+
 }  // namespace
 }  // namespace ltpg
 
@@ -134,7 +140,7 @@ extern "C" int ltpg_kv_epoch_noalloc(uint32_t *table, uint64_t rows, uint32_t fi
     b.meta = batch->meta;
     b.tids = batch->tids;
     uint32_t *unsorted = reinterpret_cast<uint32_t *>(p + kUnsortedAt);
-    if (kv_small_epoch_ok(kv, b)) {
+    if (kv_small_epoch_ok(kv, b) && kv_small_words(kv, b) <= kAloneWords) {
         // one kernel; the registers and flags stay in its LDS (64 x 4 ops: ten
         // launches 36 us, this one 8 us, most of it the launch)
         uint32_t *res = result ? result : reinterpret_cast<uint32_t *>(ctr->pad0);

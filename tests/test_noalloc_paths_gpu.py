@@ -85,7 +85,9 @@ class Call:
 
 
 @pytest.mark.parametrize("rows,fw,B,S", [
-    (3000, 25, 512, 4),              # 2048 op slots: one workgroup
+    (3000, 24, 512, 4),              # 2048 op slots, 49,152 words: one workgroup
+    (3000, 25, 512, 4),              # more words
+    (3000, 256, 192, 1),             # 49,152 words in few fields
     (3000, 25, 683, 3),              # 2049: registers
     (32_768, 1, 5000, 10),           # the most rows on the registers
     (32_769, 1, 5000, 10),           # binned, 8 bits of row per bucket
