@@ -968,14 +968,24 @@ __global__ __launch_bounds__(kBlock) void kv_mark_reads_kernel(
         if (o[u].len == 0) continue;  // writes, empty and invalid slots
         const unsigned long long me = priority(tag, tids[t[u]], t[u]);
         bool raw = false;
-        for (uint32_t k = 0; k < o[u].len; ++k) {  // a scan: every row of its range
-            if (o[u].row + k == hot) continue;
-            const unsigned long long w = regs[rl.w(o[u].row + k)];
-            if ((uint32_t)(w >> kTagShift) != tag) continue;  // no writer this epoch
-            if (w < me)
-                raw = true;
-            else if (w > me)
-                war_flag[w & kPosMask] = epoch;
+        constexpr uint32_t R = 8;  // a scan: every row of its range, eight registers in flight
+        for (uint32_t k0 = 0; k0 < o[u].len; k0 += R) {
+            unsigned long long w[R];
+#pragma unroll
+            for (uint32_t r = 0; r < R; ++r) {
+                if (r && max_scan <= 1) break;
+                w[r] = regs[rl.w(o[u].row + (k0 + r < o[u].len ? k0 + r : 0u))];
+            }
+#pragma unroll
+            for (uint32_t r = 0; r < R; ++r) {
+                if (r && max_scan <= 1) break;
+                if (k0 + r >= o[u].len || o[u].row + k0 + r == hot) continue;
+                if ((uint32_t)(w[r] >> kTagShift) != tag) continue;  // no writer this epoch
+                if (w[r] < me)
+                    raw = true;
+                else if (w[r] > me)
+                    war_flag[w[r] & kPosMask] = epoch;
+            }
         }
         if (raw) raw_flag[t[u]] = epoch;
     }
@@ -1240,29 +1250,49 @@ __device__ __forceinline__ void lane_copy(bool active, uint64_t src_off, uint64_
     }
 }
 
+// Read-out of one op per lane on fields of FW < 4 words, each lane its own:
+// one load if the wave has no scan, otherwise eight rows' loads in flight
+// (bound by those random loads).  With four rows of three words each, whatever
+// the fields and the ops, 2^20 transactions of 10 ops on 8-byte fields took 267
+// us per epoch, 256 so; 10,000 of 10 scans of 100 rows 186, with the same in
+// the read marking 134 so.
+template <uint32_t FW>
+__device__ __forceinline__ void read_narrow(const Op &o, uint64_t src, uint64_t step, uint64_t dst,
+                                            const uint32_t *table, uint32_t *read_values)
+{
+    struct __attribute__((packed, aligned(4))) Words {
+        uint32_t w[FW];
+    };
+    if (!__ballot(o.len > 1)) {
+        const Words v = *reinterpret_cast<const Words *>(table + (o.len ? src : 0ull));
+        if (o.len) *reinterpret_cast<Words *>(read_values + dst) = v;
+        return;
+    }
+    constexpr uint32_t U = 8;
+    for (uint32_t k0 = 0; k0 < o.len; k0 += U) {
+        Words v[U];
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u)
+            v[u] = *reinterpret_cast<const Words *>(table + (k0 + u < o.len ? src + (k0 + u) * step : 0ull));
+#pragma unroll
+        for (uint32_t u = 0; u < U; ++u)
+            if (k0 + u < o.len) *reinterpret_cast<Words *>(read_values + dst + (k0 + u) * FW) = v[u];
+    }
+}
+
 // Read-out of one op per lane (its rows' fields to the read values of slot
 // position i): fields of 16 bytes and more through the wave's list, whose
-// length it returns; narrower ones each lane its own, four rows' loads in
-// flight.  Every lane of the wave calls it.
+// length it returns; narrower ones each lane its own.  Every lane of the wave
+// calls it.
 __device__ __forceinline__ uint32_t read_out(const Op &o, uint64_t i, StageList &list, uint32_t pending,
                                              const FieldLanes &lanes, const uint32_t *table, uint32_t *read_values,
                                              uint32_t fields, uint32_t fw, uint32_t fsw, uint32_t L)
 {
     const uint64_t src0 = (o.row * fields + o.field) * fsw, step = (uint64_t)fields * fsw, dst0 = i * L * fw;
     if (fw < 4) {
-        for (uint32_t k0 = 0; k0 < o.len; k0 += 4) {
-            uint32_t v[4][3];
-#pragma unroll
-            for (uint32_t u = 0; u < 4; ++u)
-#pragma unroll
-                for (uint32_t w = 0; w < 3; ++w)
-                    v[u][w] = table[(k0 + u < o.len && w < fw) ? src0 + (k0 + u) * step + w : 0ull];
-#pragma unroll
-            for (uint32_t u = 0; u < 4; ++u)
-#pragma unroll
-                for (uint32_t w = 0; w < 3; ++w)
-                    if (k0 + u < o.len && w < fw) read_values[dst0 + (k0 + u) * fw + w] = v[u][w];
-        }
+        if (fw == 1) read_narrow<1>(o, src0, step, dst0, table, read_values);
+        else if (fw == 2) read_narrow<2>(o, src0, step, dst0, table, read_values);
+        else read_narrow<3>(o, src0, step, dst0, table, read_values);
         return 0;
     }
     for (uint32_t k = 0; __ballot(k < o.len); ++k) {  // row k of each read / scan: its own destination
@@ -1954,7 +1984,10 @@ __global__ __launch_bounds__(kSmallBlock) void kv_small_epoch_kernel(
 // Hot row: committed writes to it add their delta (TID | 1 per word) in any
 // order.  A block sums its transactions' deltas per field in LDS and adds
 // each non-zero sum to one of kCounterStripes accumulator rows; then
-// kv_hot_apply_kernel folds the stripes into the row and clears them.
+// kv_hot_apply_kernel folds the stripes into the row and clears them.  Bound by
+// latency: 16,000 transactions of 8 ops 4.7 + 6.6 us one slot and one stripe
+// after the other, 3.5 + 4.6 with their loads in flight together.  (As one
+// kernel whose last block folds: 9.7 us, and 260 more for 3,000 fields.)
 constexpr uint32_t kHotLdsFields = 1024;
 
 __global__ __launch_bounds__(kBlock) void kv_hot_sum_kernel(
@@ -1972,11 +2005,18 @@ __global__ __launch_bounds__(kBlock) void kv_hot_sum_kernel(
     const bool committed = t < B && ((bitmap[t / 64] >> (t % 64)) & 1ull);
     if (committed) {
         const uint32_t delta = tids[t] | 1u;
-        for (uint32_t s = 0; s < S; ++s) {
-            const Op o = load_op(keys, meta, op_at(s, t, B, S, rm), true, rows, fields);
-            if (!o.valid || o.kind != LTPG_KV_WRITE || o.row != hot) continue;
-            if (lds) atomicAdd(&bins[o.field], delta);
-            else atomicAdd(&stripe[o.field], delta);
+        constexpr uint32_t U = 8;
+        for (uint32_t s0 = 0; s0 < S; s0 += U) {
+            Op o[U];
+#pragma unroll
+            for (uint32_t u = 0; u < U; ++u)
+                o[u] = load_op(keys, meta, op_at(s0 + u, t, B, S, rm), s0 + u < S, rows, fields);
+#pragma unroll
+            for (uint32_t u = 0; u < U; ++u) {
+                if (!o[u].valid || o[u].kind != LTPG_KV_WRITE || o[u].row != hot) continue;
+                if (lds) atomicAdd(&bins[o[u].field], delta);
+                else atomicAdd(&stripe[o[u].field], delta);
+            }
         }
     }
     __syncthreads();
@@ -1991,10 +2031,14 @@ __global__ __launch_bounds__(kBlock) void kv_hot_apply_kernel(uint32_t *__restri
 {
     const uint32_t f = blockIdx.x * kBlock + threadIdx.x;
     if (f >= fields) return;
-    uint32_t total = 0;
+    // every load before the first store, which might be to the next one's place
+    uint32_t v[kCounterStripes], total = 0;
+#pragma unroll
+    for (int k = 0; k < kCounterStripes; ++k) v[k] = acc[(uint64_t)k * fields + f];
+#pragma unroll
     for (int k = 0; k < kCounterStripes; ++k) {
-        total += acc[(uint64_t)k * fields + f];
-        acc[(uint64_t)k * fields + f] = 0;
+        total += v[k];
+        if (v[k]) acc[(uint64_t)k * fields + f] = 0;
     }
     if (total == 0) return;
     uint32_t *w = table + (hot * fields + f) * (uint64_t)fsw;

@@ -76,3 +76,10 @@ def test_small_epochs_with_scans_match_oracle(gpu, B, S, scan):
 
 def test_small_epoch_with_the_widest_hot_row_matches_oracle(gpu):
     check(60, 1024, 1, 2048, 1, tuning=L.TUNE_SMALL_EPOCH, theta=0.0, read_pct=20, hot=True)
+
+
+@pytest.mark.parametrize("fw", [1, 2, 3, 4])
+@pytest.mark.parametrize("scan,hot", [(0, True), (1, False), (8, False), (9, True), (19, False)])
+def test_larger_epochs_with_scans_and_a_hot_row_match_oracle(gpu, fw, scan, hot):
+    # several kernels: reads of narrow fields alone and eight rows at a time
+    check(4000, 3, fw, 1500, 9, theta=0.5, scan=scan, hot=hot)
