@@ -1387,7 +1387,25 @@ struct WriteArgs {
     uint64_t hot;
     uint32_t per_lane;
     bool rm;
+    EpochEnd end;
 };
+
+// The end of an epoch that keeps no state: its commit count and range errors
+// (final before WRITEBACK, whose first wave this is), and the TID order flag
+// starts over.  As a kernel of its own 2 us and a launch.
+__device__ __forceinline__ void end_epoch(const EpochEnd &e)
+{
+    static_assert(kCounterStripes == 64, "one lane per stripe");
+    if (!e.ctr || blockIdx.x != 0 || blockIdx.y != 0 || threadIdx.x >= 64) return;
+    uint32_t c = e.ctr->commits[threadIdx.x][LTPG_TYPE_KV];
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) c += __shfl_xor(c, d);
+    if (threadIdx.x != 0) return;
+    *e.unsorted = 0;
+    if (!e.result) return;
+    e.result[0] = c;
+    e.result[1] = e.ctr->range_errors;
+}
 
 // One round of 64 / G transactions, t the lane group's (if has).
 template <int G>
@@ -1438,6 +1456,7 @@ __global__ __launch_bounds__(kBlock) void kv_writeback_kernel(WriteArgs a, const
     __shared__ uint32_t s_list[CH];
     __shared__ uint32_t s_cnt[kBlock / 64];
     __shared__ StageList s_stage[kBlock / 64];
+    end_epoch(a.end);
     const uint32_t t0 = blockIdx.x * CH + threadIdx.x;
     // t0 < B also guards a bitmap word left by an earlier, larger batch
     // when this phase runs without a fresh CHECK
@@ -1637,6 +1656,7 @@ __global__ __launch_bounds__(kBlock) void kv_writeback_list_kernel(WriteArgs a, 
     constexpr bool kSlots = G <= 16;  // op slots that fit LDS
     __shared__ StageList s_stage[kBlock / 64];
     __shared__ uint32_t s_fields[kSlots ? kBlock / 64 : 1][kSlots ? G : 1][64];
+    end_epoch(a.end);
     const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     StageList &list = s_stage[wave];
     const FieldLanes lanes(a.fw);
@@ -3344,12 +3364,12 @@ hipError_t launch_kv_readout(const KvState &kv, const KvBatchDev &b, hipStream_t
 }
 
 hipError_t launch_kv_writeback(const KvState &kv, const KvBatchDev &b, uint32_t values, DeviceCounters *ctr,
-                               hipStream_t s)
+                               hipStream_t s, const EpochEnd &end)
 {
     if (b.n_txns == 0) return hipSuccess;
     const WriteArgs a = {b.keys,          b.meta,          b.tids,   b.n_txns,   b.n_slots, kv.rows,
                          kv.fields,       kv.field_stride, kv.field_stride, kv.table,   values,    kv.hot_row,
-                         lane_copy_ok(kv), b.request_major};
+                         lane_copy_ok(kv), b.request_major, end};
     const int g = group_for(b.n_slots);
     if (kv.list_valid && kv_check_lists(kv, b)) {
         const uint64_t per = (kBlock / 64) * (64 / g);  // transactions per block and round

@@ -421,8 +421,15 @@ bool kv_check_lists(const KvState &kv, const KvBatchDev &b);
 hipError_t launch_kv_readout(const KvState &kv, const KvBatchDev &b, hipStream_t s);
 // Takes the committed transactions from commit_list if kv.list_valid, else
 // from the bitmap.
+// What WRITEBACK also does for ltpg_kv_epoch_noalloc (null ctr: nothing).
+struct EpochEnd {
+    const DeviceCounters *ctr = nullptr;
+    uint32_t *unsorted = nullptr;
+    uint32_t *result = nullptr;
+};
 hipError_t launch_kv_writeback(const KvState &kv, const KvBatchDev &b, uint32_t values, DeviceCounters *ctr,
-                               hipStream_t s);
+                               hipStream_t s,
+                               const EpochEnd &end = EpochEnd());
 // A whole fast-form epoch of at most LTPG_SMALL_EPOCH_OPS op slots in one
 // single-workgroup kernel (a hot row only with at most 1024 fields; rows <
 // 2^32 - 1).  With seq_out it
@@ -528,7 +535,8 @@ hipError_t launch_tpcc_execute(const TpccDev &d, const NeworderDev &no, const Pa
 // EXECUTE of a large fast-form epoch without Stock-Level: whether it is taken,
 // its launch, and the shape of its binned part.  Four kernels against one:
 // 32,000 transactions 23 us split, 22 in one (16 warehouses), 64,000 24 / 31
-// (64 warehouses 26 / 29), 131,072 30 / 50, 262,144 50 / 77.
+// (64 warehouses 26 / 29), 131,072 30 / 50, 262,144 50 / 77; whole epochs on 64
+// warehouses 40,000 48 / 47, 49,152 48 / 50, 131,072 62 / 78.
 constexpr uint32_t kSplitTxns = 3u << 14;
 bool tpcc_execute_split(const TpccDev &d, const BinBuffers &bin, const NeworderDev &no, const PaymentDev &pay);
 BinShape stock_bin_shape(uint64_t stock_rows, uint32_t n_neworder);

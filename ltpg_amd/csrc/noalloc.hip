@@ -53,20 +53,8 @@ __global__ void noalloc_init_kernel(unsigned long long *regs, uint64_t n_regs, u
     for (uint64_t i = first; i < sizeof(DeviceCounters) / 4; i += step) c[i] = 0;
 }
 
-// The epoch's commit count and range errors (result[0], result[1]; zero for
-// an empty epoch), one wave; the TID order flag starts over.
-__global__ void noalloc_result_kernel(const DeviceCounters *ctr, uint32_t *unsorted, uint32_t *result, bool empty)
-{
-    static_assert(kCounterStripes == 64, "one lane per stripe");
-    if (threadIdx.x == 0) *unsorted = 0;
-    if (!result) return;
-    uint32_t c = empty ? 0u : ctr->commits[threadIdx.x][LTPG_TYPE_KV];
-    for (int d = 32; d > 0; d >>= 1) c += __shfl_xor(c, d);
-    if (threadIdx.x == 0) {
-        result[0] = c;
-        result[1] = empty ? 0u : ctr->range_errors;
-    }
-}
+// The result of an empty epoch.
+__global__ void noalloc_empty_kernel(uint32_t *result) { result[threadIdx.x] = 0; }
 
 // scratch's device address, per device (looked up once each)
 std::mutex g_mu;
@@ -173,9 +161,14 @@ extern "C" int ltpg_kv_epoch_noalloc(uint32_t *table, uint64_t rows, uint32_t fi
         LTPG_HIP_TRY(launch_kv_execute(kv, b, e, false, ctr, s));
         LTPG_HIP_TRY(launch_kv_check(kv, b, e, false, ctr, s));
         kv.list_valid = true;  // of the CHECK above
-        LTPG_HIP_TRY(launch_kv_writeback(kv, b, values, ctr, s));
+        EpochEnd end;
+        end.ctr = ctr;
+        end.unsorted = unsorted;
+        end.result = result;
+        LTPG_HIP_TRY(launch_kv_writeback(kv, b, values, ctr, s, end));
+    } else if (result) {
+        hipLaunchKernelGGL(noalloc_empty_kernel, dim3(1), dim3(2), 0, s, result);
+        LTPG_HIP_TRY(hipGetLastError());
     }
-    hipLaunchKernelGGL(noalloc_result_kernel, dim3(1), dim3(64), 0, s, ctr, unsorted, result, B == 0);
-    LTPG_HIP_TRY(hipGetLastError());
     return LTPG_OK;
 }

@@ -135,3 +135,16 @@ def test_noalloc_captured_replays_match_oracle(gpu, rows, B, S):
         hip("hipStreamDestroy", s)
         c.free()
         other.free()
+
+
+@pytest.mark.parametrize("result", [True, False])
+def test_noalloc_empty_epoch(gpu, result):
+    hip = Hip()
+    with L.Context(workload=L.WORKLOAD_KV, kv_rows=64, kv_fields=1, max_txns=64, kv_max_slots=1) as ctx:
+        c = Call(ctx, 100, 2, 1, 8, 2, 1)
+        c.struct.n_txns = 0
+        c.run(result=result)
+        hip("hipDeviceSynchronize")
+        c.bufs[3].download(c.out[3])
+        assert c.out[3].tolist() == ([0, 0] if result else [0xFFFFFFFF] * 2)
+        c.free()
