@@ -1479,7 +1479,7 @@ __global__ __launch_bounds__(kBlock) void kv_writeback_kernel(WriteArgs a, const
 //
 // Commits crowd among the lowest priorities, so with a block per 256
 // transactions a few blocks do nearly all of an epoch's field copies.  For
-// batches of kListTxns transactions and more CHECK decides every transaction
+// large batches (kv_check_lists) CHECK decides every transaction
 // first and lists the committed ones (kv_commit_list_kernel); the read-out and
 // WRITEBACK then share that list evenly over the whole chip.  2^20
 // transactions x 16 ops on 100-byte fields, 3.5 % committed: CHECK 64 -> 7 + 29
@@ -3297,14 +3297,19 @@ static uint32_t lane_copy_ok(const KvState &kv)
     return kv.lane_copy && kv.field_stride % 4 == 0 && kv.field_words <= 32 ? 1u : 0u;
 }
 
-// The list costs one more kernel: 10 blocks' worth of short chunks run as fast
-// in one (10,000 transactions: 13 us as one kernel, 5 + 9 as two).
-constexpr uint32_t kListTxns = 1u << 15;
+// The list costs one more kernel, which an even share of the copies makes up
+// for in large batches that commit unevenly.  CHECK and WRITEBACK with the list
+// and by chunks, uniform rows (Zipf 0.9 in brackets), 100-byte fields: 10,000
+// transactions of 10 ops 19 us against 15 (17 / 13), 98,304 61 / 60 (36 / 34),
+// 196,608 89 / 100 (61 / 60); 32,768 of 16 22 / 21 (16 / 14), 65,536 23 / 28
+// (16 / 15), 262,144 24 / 56 (17 / 17); of 4 ops 262,144 40 / 37 (24 / 20).
+constexpr uint64_t kListOps = 1u << 20, kListOpsFewSlots = 1u << 21;
 constexpr uint32_t kListBlocks = 2048;  // 8 per CU: what the copies' registers allow to be resident
 
 bool kv_check_lists(const KvState &kv, const KvBatchDev &b)
 {
-    return kv.commit_list && b.n_txns >= kListTxns && !kv.small_chunks && !kv.lane_copy;
+    return kv.commit_list && (uint64_t)b.n_txns * b.n_slots >= (b.n_slots >= 8 ? kListOps : kListOpsFewSlots) &&
+           !kv.small_chunks && !kv.lane_copy;
 }
 
 // Read values and written fields are moved whole, padding included: fields of

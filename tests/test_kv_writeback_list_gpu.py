@@ -17,7 +17,9 @@ pytestmark = pytest.mark.gpu
     (4_000_000, 2, 3, 150_001, 16, 97, {}),                      # a ragged last wave
     (1_000_000, 3, 4, 300_007, 4, 50, {}),
     (1_000_000, 2, 25, 200_000, 8, 95, {}),
-    (3_000_000, 1, 1, 1 << 20, 1, 0, {}),                        # one write each
+    (3_000_000, 1, 1, 1 << 20, 1, 0, {}),                        # one write each: no list
+    (3_000_000, 1, 1, 1 << 20, 2, 30, {}),                       # the fewest ops of few slots that are listed
+    (3_000_000, 1, 1, (1 << 20) - 1, 2, 30, {}),                 # not listed
     (2_000_000, 2, 2, 270_000, 5, 60, dict(hot=3)),
     (2_000_000, 2, 5, 200_000, 7, 80, dict(copyback=True)),
     (4_000_000, 2, 1, 140_000, 16, 90, dict(request_major=True)),

@@ -92,7 +92,8 @@ class Call:
     (32_768, 1, 5000, 10),           # the most rows on the registers
     (32_769, 1, 5000, 10),           # binned, 8 bits of row per bucket
     (1 << 20, 2, 1000, 7),           # binned, one short tile
-    (1_000_003, 5, 40_000, 9),       # commit list
+    (1_000_003, 5, 40_000, 9),       # chunks of transactions
+    (1_000_003, 5, 120_001, 9),      # commit list
     (200_000, 1, 1 << 20, 17),       # more op slots than the binned path holds
 ], ids=lambda v: str(v))
 def test_noalloc_paths_match_oracle(gpu, rows, fw, B, S):
