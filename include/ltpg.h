@@ -459,8 +459,9 @@ int ltpg_tpcc_gen_next(ltpg_tpcc_gen *g, uint32_t n_txns, uint32_t tid_base, uin
 /* ---- launch shape of the key-value kernels (replaces the fixed warp-role
  *      and grid constants, YCSB/0/Predefine.h:27-35) ------------------------ */
 /* A context starts without a chosen shape: batch and table sizes pick the
- * EXECUTE form (PARTITIONED for large epochs of point operations, EXEC_PER_OP
- * for small ones; its buffers, 4 bytes per possible op slot and about 2 bytes
+ * form (PARTITIONED for large epochs of point operations, EXEC_PER_OP for
+ * small ones, SMALL_EPOCH up to half its op slots while those hold at most
+ * 16,384 field words; its buffers, 4 bytes per possible op slot and about 2 bytes
  * per 16, are then allocated with the context).  ltpg_kv_set_tuning fixes the
  * shape from then on: 0 is none of the flags below.
  * EXEC_PER_OP: EXECUTE runs one lane per op instead of one lane per
@@ -589,7 +590,7 @@ typedef struct ltpg_batch_desc {
  *   followed by a stream synchronisation, then the commit-count readback.
  * GRAPH: the batches of each workload, in list order, captured once into a
  *   HIP graph (register refill, then per batch: submit, CID / EXECUTE /
- *   CHECK / WRITEBACK, bitmap archive copy); the key-value and order-entry
+ *   CHECK / WRITEBACK, bitmaps to the archive); the key-value and order-entry
  *   graphs run concurrently on their contexts' streams, with one host
  *   synchronisation at the end.
  * Both produce identical commit sets and tables: batches of one workload run

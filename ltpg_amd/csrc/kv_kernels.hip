@@ -1485,7 +1485,7 @@ __global__ __launch_bounds__(kBlock) void kv_writeback_kernel(WriteArgs a, const
 // transactions x 16 ops on 100-byte fields, 3.5 % committed: CHECK 64 -> 7 + 29
 // us, WRITEBACK 74 -> 27 us.  With 81 % committed (9 reads, 1 write): CHECK 662
 // -> 7 + 441 us, which is the rate of random 128-byte reads and whole writes
-// (3.6 TB/s; the gather alone reaches 4.2), WRITEBACK 148 -> 49 us.
+// (3.6 TB/s; the gather alone reaches 4.2), WRITEBACK 148 -> 76 us.
 constexpr uint32_t kListBlock = 1024, kListPer = 4;  // transactions per block and thread
 
 __global__ __launch_bounds__(kListBlock) void kv_commit_list_kernel(
@@ -1643,8 +1643,8 @@ __device__ __forceinline__ uint32_t write_slots(const WriteArgs &a, uint32_t t, 
 // (write_slots); entries beyond a smaller current batch (the phase without a
 // fresh CHECK) are left out.  Listed transactions lie close together, so their
 // slots come in runs, while lane groups read a line per slot and transaction,
-// and the keys of reads too: 1,013,000 commits of 9 reads and a write 142 us in
-// groups, 45 so (100-byte fields), 131,000 24 / 11; of 1 to 16 ops, half of
+// and the keys of reads too: 1,013,000 commits of 1 to 10 ops, a tenth of them
+// writes, 142 us in groups, 45 so (100-byte fields), 131,000 24 / 11; of 1 to 16 ops, half of
 // them writes, 456,000 commits 160 / 112, 203,000 70 / 56, 115,000 40 / 38.  A
 // lane's chain is longer, though, and few waves do not hide it: 62,000 of the
 // latter 24 / 33, 254,000 of one or two writes 21 / 22 (935,000: 89 / 81).
