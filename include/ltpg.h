@@ -461,9 +461,9 @@ int ltpg_tpcc_gen_next(ltpg_tpcc_gen *g, uint32_t n_txns, uint32_t tid_base, uin
 /* A context starts without a chosen shape: batch and table sizes pick the
  * form (PARTITIONED for large epochs of point operations, EXEC_PER_OP for
  * small ones, SMALL_EPOCH up to half its op slots while those hold at most
- * 16,384 field words; its buffers, 4 bytes per possible op slot and about 2 bytes
- * per 16, are then allocated with the context).  ltpg_kv_set_tuning fixes the
- * shape from then on: 0 is none of the flags below.
+ * 16,384 field words; the buffers of PARTITIONED, 4 bytes per possible op slot
+ * and about 2 bytes per 16, are then allocated with the context).
+ * ltpg_kv_set_tuning fixes the shape from then on: 0 is none of the flags below.
  * EXEC_PER_OP: EXECUTE runs one lane per op instead of one lane per
  *   transaction.
  * SPLIT_REGISTERS: a row's R and W registers live in two arrays instead of

@@ -629,6 +629,7 @@ int ltpg_device_free(ltpg_ctx *ctx, void *dptr)
 {
     int rc = check_ctx(ctx);
     if (rc) return rc;
+    if ((rc = settle_cid(ctx))) return rc;  // which may read the buffer
     if (dptr) {
         LTPG_HIP_TRY(hipStreamSynchronize(ctx->stream));
         LTPG_HIP_TRY(hipFree(dptr));
@@ -1149,6 +1150,7 @@ int ltpg_kv_submit(ltpg_ctx *ctx, const ltpg_kv_batch *b, uint32_t mem)
         d.tids = reinterpret_cast<const uint32_t *>(kv.batch_buf[k] + tids_at);
     }
     kv.cur = d;
+    kv.flags_in_lds = false;
     kv.has_batch = true;
     return LTPG_OK;
 }
@@ -1242,6 +1244,7 @@ int ltpg_epoch_run(ltpg_ctx *ctx, uint32_t phase_mask)
     if (phase_mask == LTPG_PHASE_ALL && !ctx->timing && !(ctx->cfg.flags & LTPG_FLAG_CONFLICT_COUNTS) &&
         (kv.small_epoch ? kv_small_epoch_ok(kv, kv.cur) : kv_small_auto(kv, kv.cur))) {
         kv.list_valid = false;
+        kv.flags_in_lds = true;
         LTPG_HIP_TRY(launch_kv_small_epoch(kv, kv.cur, ctx->cfg.values, ctx->counters, nullptr, nullptr, 0, s));
         return LTPG_OK;
     }
@@ -1253,7 +1256,10 @@ int ltpg_epoch_run(ltpg_ctx *ctx, uint32_t phase_mask)
     }
     // CID has no key-value work: its bracket is empty.
     if (ev) LTPG_HIP_TRY(hipEventRecord(ev[1], s));
+    // CHECK by itself after an epoch in one workgroup needs the flags again
+    if ((phase_mask & LTPG_PHASE_CHECK) && kv.flags_in_lds) phase_mask |= LTPG_PHASE_EXECUTE;
     if (phase_mask & LTPG_PHASE_EXECUTE) {
+        kv.flags_in_lds = false;
         kv.list_valid = false;  // its length starts over with the counts
         LTPG_HIP_TRY(launch_kv_execute(kv, kv.cur, e, (ctx->cfg.flags & LTPG_FLAG_CONFLICT_COUNTS) != 0,
                                        ctx->counters, s));

@@ -130,6 +130,7 @@ struct KvState {
     uint32_t *conflicts = nullptr;      // max_txns
     uint32_t *commit_list = nullptr;    // max_txns: the committed transactions of the last list CHECK
     bool list_valid = false;            // commit_list lists the same transactions as bitmap
+    bool flags_in_lds = false;          // the current epoch ran in one workgroup, which kept its flags
     // library-owned copies of host-submitted batches: two slots, so that
     // the next batch's copy overlaps the current epoch (slot 1 allocated at
     // its first use)

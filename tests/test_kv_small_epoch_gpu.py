@@ -83,3 +83,24 @@ def test_small_epoch_with_the_widest_hot_row_matches_oracle(gpu):
 def test_larger_epochs_with_scans_and_a_hot_row_match_oracle(gpu, fw, scan, hot):
     # several kernels: reads of narrow fields alone and eight rows at a time
     check(4000, 3, fw, 1500, 9, theta=0.5, scan=scan, hot=hot)
+
+
+@pytest.mark.parametrize("tuning", [None, L.TUNE_SMALL_EPOCH])
+def test_check_again_after_a_small_epoch(gpu, tuning):
+    rows, B, S = 300, 200, 4
+    with L.Context(workload=L.WORKLOAD_KV, kv_rows=rows, kv_fields=1, kv_field_bytes=4, max_txns=B,
+                   kv_max_slots=S) as ctx:
+        if tuning is not None:
+            ctx.kv_set_tuning(tuning)
+        table = kc.initial_table(rows, 1, 1)
+        ctx.kv_table_load(table)
+        for e in range(3):
+            k, m, t = L.kv_generate(seed=e, rows=rows, fields=1, n_txns=B, n_slots=S, theta=0.5)
+            ctx.kv_submit(k, m, t, S)
+            ctx.epoch_run()
+            ora = oracle.kv_epoch(table, rows, 1, 1, k, m, t, S, inplace=True, want_reads=False)
+            for _ in range(2):
+                ctx.epoch_run(L.PHASE_CHECK)
+                np.testing.assert_array_equal(ctx.commit_bitmap(), ora.bitmap)
+                assert ctx.commit_count() == ora.commit_count
+        np.testing.assert_array_equal(ctx.kv_table_read(), table)

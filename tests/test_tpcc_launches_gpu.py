@@ -60,3 +60,15 @@ def test_ytd_sums_of_committed_payments(gpu, W, txns, small):
             np.add.at(want[1], w * 10 + d, amount.astype(np.uint32))
         for (t, col, rows), v in zip(tables, want):
             np.testing.assert_array_equal(ctx.tpcc_table_read(t).reshape(-1, rows)[col], v)
+
+
+def test_freed_batch_keeps_its_customers(gpu):
+    # a device batch freed through its context right after the submit
+    with L.Context(workload=L.WORKLOAD_TPCC, tpcc_warehouses=1, max_txns=500) as ctx:
+        ctx.tpcc_populate(1)
+        b = L.TpccGenerator(warehouses=1, seed=2).next(500)
+        dev, bufs = L.upload_tpcc_batch(ctx, b)
+        ctx.tpcc_submit(dev, L.MEM_DEVICE)
+        for x in bufs:
+            x.free()
+        np.testing.assert_array_equal(ctx.tpcc_payment_cid(), b.pf("C_ID"))
