@@ -281,7 +281,7 @@ __device__ __forceinline__ BinRun bin_run(const BinArgs &a, uint32_t b, uint32_t
     BinRun r = {0u, 0u, 0u};
     if (tile < a.tiles) {
         const uint16_t *o = a.off + (uint64_t)tile * (a.nb + 1) + b;
-        r.start = (tile << a.tile_bits) + o[0];
+        r.start = bin_run_start(tile, a.tile_bits, o[0], o[1]);
         r.len = (uint32_t)o[1] - o[0];
         r.t0 = bin_txn(a, tile << a.tile_bits);
     }
@@ -378,7 +378,7 @@ __device__ __forceinline__ void bin_pass(const BinArgs &a, const BinRun &mine, u
             s[u] = __shfl(mine.start, base_lane + (int)(j0 + u));
             len[u] = __shfl(mine.len, base_lane + (int)(j0 + u));
             t0[u] = DIRECT ? __shfl(mine.t0, base_lane + (int)(j0 + u)) : 0u;
-            // unconditional loads (a run's first entry, or entry 0, when idle)
+            // unconditional loads (a run's first entry when idle, entry 0 of an empty run)
             x[u][0] = a.ent[s[u] + (l < len[u] ? l : 0u)];
             x[u][1] = a.ent[s[u] + (l + kRunLanes < len[u] ? l + kRunLanes : 0u)];
         }

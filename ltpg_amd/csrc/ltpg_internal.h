@@ -106,6 +106,14 @@ inline BinShape bin_shape(uint64_t rows, uint64_t ops)
     f.tiles = (uint32_t)((ops + (1ull << f.tile_bits) - 1) >> f.tile_bits);
     return f;
 }
+// Where the entries of a bucket's run in a tile begin, the run being [from, to)
+// within the tile.  An idle lane loads a run's first entry.  An empty run has
+// none -- `from` may be the tile's size, which after the last tile is past the
+// buffer -- so it begins at entry 0.
+inline __host__ __device__ uint32_t bin_run_start(uint32_t tile, uint32_t tile_bits, uint32_t from, uint32_t to)
+{
+    return from < to ? (tile << tile_bits) + from : 0u;
+}
 inline bool bin_fits(const BinBuffers &b, const BinShape &f)
 {
     return b.ent && ((uint64_t)f.tiles << f.tile_bits) <= b.cap_ent && (uint64_t)f.tiles * (f.buckets + 1) <= b.cap_off;
