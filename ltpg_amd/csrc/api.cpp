@@ -1316,6 +1316,8 @@ int ltpg_epoch_reset(ltpg_ctx *ctx)
 {
     int rc = check_ctx(ctx);
     if (rc) return rc;
+    // nor do the flags that an epoch in one workgroup kept count any more
+    ctx->kv.flags_in_lds = false;
     return next_epoch(ctx);
 }
 
