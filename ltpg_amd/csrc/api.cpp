@@ -484,8 +484,8 @@ int ltpg_create(const ltpg_config *cfg, ltpg_ctx **out)
         }
         ctx->stream = ctx->own_stream;
         alloc_readback(ctx);
-        if ((rc = dev_alloc(&ctx->counters, 1, "counters"))) break;
-        e = hipMemsetAsync(ctx->counters, 0, sizeof(DeviceCounters), ctx->stream);
+        if ((rc = dev_alloc(&ctx->counters, 2, "counters"))) break;
+        e = hipMemsetAsync(ctx->counters, 0, 2 * sizeof(DeviceCounters), ctx->stream);
         if (e != hipSuccess) {
             set_error(std::string("hipMemsetAsync: ") + hipGetErrorString(e));
             rc = LTPG_ERR_DEVICE;
@@ -1256,13 +1256,16 @@ int ltpg_epoch_run(ltpg_ctx *ctx, uint32_t phase_mask)
     }
     // CID has no key-value work: its bracket is empty.
     if (ev) LTPG_HIP_TRY(hipEventRecord(ev[1], s));
-    // CHECK by itself after an epoch in one workgroup needs the flags again
-    if ((phase_mask & LTPG_PHASE_CHECK) && kv.flags_in_lds) phase_mask |= LTPG_PHASE_EXECUTE;
     if (phase_mask & LTPG_PHASE_EXECUTE) {
         kv.flags_in_lds = false;
         kv.list_valid = false;  // its length starts over with the counts
         LTPG_HIP_TRY(launch_kv_execute(kv, kv.cur, e, (ctx->cfg.flags & LTPG_FLAG_CONFLICT_COUNTS) != 0,
                                        ctx->counters, s));
+    } else if ((phase_mask & LTPG_PHASE_CHECK) && kv.flags_in_lds) {
+        // CHECK by itself after an epoch in one workgroup needs the flags again;
+        // that epoch counted the range errors, so these go to the spare counters
+        LTPG_HIP_TRY(launch_kv_execute(kv, kv.cur, e, false, ctx->counters + 1, s, false));
+        kv.flags_in_lds = false;
     }
     if (ev) LTPG_HIP_TRY(hipEventRecord(ev[2], s));
     if (phase_mask & LTPG_PHASE_CHECK) {

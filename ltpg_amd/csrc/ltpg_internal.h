@@ -284,7 +284,7 @@ struct ltpg_ctx {
     hipStream_t own_stream = nullptr;
     hipStream_t stream = nullptr;
     uint32_t epoch = 1;  // 1..255; 0 owns the all-ones fill value of the registers
-    ltpg::DeviceCounters *counters = nullptr;
+    ltpg::DeviceCounters *counters = nullptr;  // and, behind them, spare ones that nothing reads
     ltpg::KvState kv;
     ltpg::TpccState tpcc;
     // Per-step timing: each timed epoch takes LTPG_TIMING_SLOTS + 1 events
