@@ -272,12 +272,11 @@ int kv_part_prepare(ltpg_ctx *ctx)
 {
     KvState &kv = ctx->kv;
     if (kv.part.ent_me) return LTPG_OK;
-    if (kv.max_scan <= 1 && kv.bin.ent) return LTPG_OK;
     const uint64_t nb = (kv.rows + (1ull << kPartShift) - 1) >> kPartShift;
     const uint64_t cap = (uint64_t)kv.max_slots * ctx->cfg.max_txns * kv.read_slot;
     if (nb > kPartMaxBuckets || cap >= (1ull << 32))
         LTPG_FAIL(LTPG_ERR_UNSUPPORTED, "row-partitioned EXECUTE: too many rows or operations per epoch");
-    if (kv.max_scan <= 1) return kv_bin_prepare(ctx);  // point operations
+    if (kv.max_scan <= 1) return kv_bin_prepare(ctx);  // point operations: nothing to do if the context has its bins
     KvState::Part p;
     p.n_buckets = (uint32_t)nb;
     p.cap_entries = cap;
