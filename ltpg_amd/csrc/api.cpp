@@ -111,6 +111,36 @@ int kv_bin_prepare(ltpg_ctx *ctx)
                      [&](uint64_t ops) { return bin_shape(kv.rows, ops); }, ctx->stream);
 }
 
+// Whether `bytes` that the context could do without leave room for what it
+// still needs: the second slot of host batches, and small change.
+bool kv_room(const ltpg_ctx *ctx, uint64_t bytes)
+{
+    size_t left = 0, total = 0;
+    if (hipMemGetInfo(&left, &total) != hipSuccess) {
+        (void)hipGetLastError();
+        return false;
+    }
+    return left >= bytes + kv_batch_bytes(ctx->kv.max_slots, ctx->cfg.max_txns) + (64ull << 20);
+}
+
+// The read values, at the fields' stride (ltpg_internal.h) where there is room
+// for it, else packed.
+int alloc_read_values(ltpg_ctx *ctx)
+{
+    KvState &kv = ctx->kv;
+    const uint64_t n = (uint64_t)kv.max_slots * ctx->cfg.max_txns * kv.read_slot;
+    kv.read_stride = kv.field_stride;
+    if (kv.field_stride != kv.field_words) {
+        if (kv_room(ctx, n * kv.field_stride * 4)) {
+            const int rc = dev_alloc(&kv.read_values, n * kv.field_stride, "kv read values");
+            if (rc != LTPG_ERR_NOMEM) return rc;
+            (void)hipGetLastError();  // dealt with
+        }
+        kv.read_stride = kv.field_words;
+    }
+    return dev_alloc(&kv.read_values, n * kv.read_stride, "kv read values");
+}
+
 int init_kv(ltpg_ctx *ctx)
 {
     const ltpg_config &c = ctx->cfg;
@@ -141,20 +171,23 @@ int init_kv(ltpg_ctx *ctx)
     if ((rc = dev_alloc(&kv.doomed, B, "kv doomed flags"))) return rc;
     if ((rc = dev_alloc(&kv.raw_flag, B, "kv raw flags"))) return rc;
     if ((rc = dev_alloc(&kv.war_flag, B, "kv war flags"))) return rc;
-    if ((rc = dev_alloc(&kv.read_values, S * B * kv.read_slot * kv.field_stride, "kv read values"))) return rc;
     if ((rc = dev_alloc(&kv.bitmap, (B + 63) / 64, "kv bitmap"))) return rc;
     if ((rc = dev_alloc(&kv.conflicts, B, "kv conflicts"))) return rc;
-    if ((rc = dev_alloc(&kv.commit_list, B, "kv commit list"))) return rc;
     if ((rc = dev_alloc(&kv.batch_buf[0], kv_batch_bytes(S, B), "kv batch"))) return rc;
     if (kv.hot_row != LTPG_NO_HOT_ROW) {
         if ((rc = dev_alloc(&kv.hot_acc, (uint64_t)kCounterStripes * kv.fields, "hot-row accumulators"))) return rc;
         LTPG_HIP_TRY(hipMemsetAsync(kv.hot_acc, 0, (uint64_t)kCounterStripes * kv.fields * 4, ctx->stream));
     }
-    // the default shape of large epochs; without memory for it they take the
-    // register path
-    if (kv.max_scan <= 1 && !(c.flags & LTPG_FLAG_CONFLICT_COUNTS) && kv_bin_auto(kv.rows, S * B) &&
-        kv_bin_prepare(ctx) == LTPG_ERR_NOMEM)
-        (void)hipGetLastError();  // dealt with
+    if ((rc = alloc_read_values(ctx))) return rc;
+    // for the commit list of large epochs and their default shape; without
+    // memory for them they take the bitmap and the register path
+    if (!(c.flags & LTPG_FLAG_CONFLICT_COUNTS)) {
+        if (kv_room(ctx, B * 4) && dev_alloc(&kv.commit_list, B, "kv commit list") == LTPG_ERR_NOMEM)
+            (void)hipGetLastError();  // dealt with
+        if (kv.max_scan <= 1 && kv_bin_auto(kv.rows, S * B) && kv_room(ctx, S * B * 5) &&
+            kv_bin_prepare(ctx) == LTPG_ERR_NOMEM)
+            (void)hipGetLastError();  // dealt with
+    }
     // Registers start as all-ones: tag ~0 belongs to epoch 0, which is never
     // current (epochs start at 1), so every row reads as "no registrant".
     if ((rc = refill_registers(ctx))) return rc;
@@ -1452,7 +1485,7 @@ int ltpg_kv_read_values(ltpg_ctx *ctx, uint32_t *out, uint64_t n_words)
     if (!kv.table) LTPG_FAIL(LTPG_ERR_UNSUPPORTED, "context has no key-value table");
     const uint64_t have = (uint64_t)kv.cur.n_slots * kv.cur.n_txns * kv.read_slot * kv.field_words;
     if (n_words > have) LTPG_FAIL(LTPG_ERR_INVALID, "n_words exceeds the staged read values");
-    const uint64_t fw = kv.field_words, fsw = kv.field_stride;
+    const uint64_t fw = kv.field_words, fsw = kv.read_stride;
     if (fw == fsw) return read_back(ctx, out, kv.read_values, n_words * 4);
     LTPG_HIP_TRY(hipStreamSynchronize(ctx->stream));
     // packed on the device, part by part

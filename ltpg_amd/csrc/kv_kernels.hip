@@ -1721,10 +1721,10 @@ __device__ __forceinline__ int small_find(const uint32_t *s_key, uint64_t row)
 
 __global__ __launch_bounds__(kSmallBlock) void kv_small_epoch_kernel(
     const uint64_t *__restrict__ keys, const uint32_t *__restrict__ meta, const uint32_t *__restrict__ tids,
-    uint32_t B, uint32_t S, bool rm, uint64_t rows, uint32_t fields, uint32_t fw, uint32_t fsw, uint32_t max_scan,
-    uint32_t L, uint32_t values, uint64_t hot, uint32_t *__restrict__ table, uint32_t *__restrict__ read_values,
-    uint64_t *__restrict__ bitmap, uint64_t *__restrict__ host_bits, uint64_t *seq_out, uint64_t seq,
-    uint32_t *__restrict__ result, DeviceCounters *__restrict__ ctr)
+    uint32_t B, uint32_t S, bool rm, uint64_t rows, uint32_t fields, uint32_t fw, uint32_t fsw, uint32_t rsw,
+    uint32_t max_scan, uint32_t L, uint32_t values, uint64_t hot, uint32_t *__restrict__ table,
+    uint32_t *__restrict__ read_values, uint64_t *__restrict__ bitmap, uint64_t *__restrict__ host_bits,
+    uint64_t *seq_out, uint64_t seq, uint32_t *__restrict__ result, DeviceCounters *__restrict__ ctr)
 {
     __shared__ uint64_t s_row[kSmallOps];
     __shared__ uint32_t s_meta[kSmallOps];
@@ -1927,7 +1927,7 @@ __global__ __launch_bounds__(kSmallBlock) void kv_small_epoch_kernel(
             const uint32_t e = L == 1 ? x : x / L, q = x - e * L;  // row q of a scan
             c.ok = q < s_add[e];
             if (c.ok) c.src = (s_field[e] + (uint64_t)q * fields) * fsw;
-            c.dst = ((uint64_t)s_slot[e] * L + q) * fsw;
+            c.dst = ((uint64_t)s_slot[e] * L + q) * rsw;
         } else {
             const uint32_t e = kSmallCopies - 1 - (x - total_r);
             c.src = c.dst = s_field[e] * fsw;
@@ -3316,7 +3316,8 @@ bool kv_check_lists(const KvState &kv, const KvBatchDev &b)
 // 64 bytes and more then leave as whole 64-byte segments of memory, where a
 // partly written segment costs a read at the memory side (8.1M reads of 100
 // bytes with every seventh slot left out: 597 us packed, 432 us for 7.7M
-// fields of 128 bytes).  Nothing reads the padding.
+// fields of 128 bytes).  Nothing reads the padding.  (Read values of a context
+// short of memory are packed, read_stride = field_words.)
 hipError_t launch_kv_check(const KvState &kv, const KvBatchDev &b, const EpochTag &e, bool counts,
                            DeviceCounters *ctr, hipStream_t s)
 {
@@ -3334,13 +3335,13 @@ hipError_t launch_kv_check(const KvState &kv, const KvBatchDev &b, const EpochTa
         const uint64_t units = ((uint64_t)b.n_txns + 63) / 64 * b.n_slots, per = kBlock / 64;
         const uint64_t blocks = std::min<uint64_t>(kListBlocks, (units + per - 1) / per);
         hipLaunchKernelGGL(kv_readout_list_kernel, dim3((unsigned)blocks), dim3(kBlock), 0, s, b.keys, b.meta, b.n_txns,
-                           b.n_slots, kv.rows, kv.fields, kv.field_stride, kv.field_stride, kv.table, kv.read_values,
+                           b.n_slots, kv.rows, kv.fields, kv.read_stride, kv.field_stride, kv.table, kv.read_values,
                            kv.commit_list, ctr, kv.max_scan, kv.read_slot, b.request_major);
         return hipGetLastError();
     }
 #define CALL1(GV, CHV)                                                                               \
     hipLaunchKernelGGL((kv_check_fast_kernel<GV, CHV>), grid_chunks(b.n_txns, CHV, GV), dim3(kBlock), 0, s, b.keys, \
-                       b.meta, b.n_txns, b.n_slots, kv.rows, kv.fields, kv.field_stride, kv.field_stride,   \
+                       b.meta, b.n_txns, b.n_slots, kv.rows, kv.fields, kv.read_stride, kv.field_stride,    \
                        kv.doomed, kv.raw_flag, kv.war_flag, e.epoch, kv.table, kv.read_values, kv.bitmap,  \
                        kv.max_scan, kv.read_slot, lane_copy_ok(kv), ctr, b.request_major)
 #define CALL(GV)                    \
@@ -3357,11 +3358,11 @@ hipError_t launch_kv_check(const KvState &kv, const KvBatchDev &b, const EpochTa
 hipError_t launch_kv_readout(const KvState &kv, const KvBatchDev &b, hipStream_t s)
 {
     if (b.n_txns == 0) return hipSuccess;
-    const int lp = lanes_for(kv.field_stride);
+    const int lp = lanes_for(kv.read_stride);
 #define CALL(LPV)                                                                          \
     hipLaunchKernelGGL(kv_readout_kernel<LPV>, grid_for(b.n_txns), dim3(kBlock), 0, s,    \
                        b.keys, b.meta, b.n_txns, b.n_slots, kv.rows, kv.fields,           \
-                       kv.field_stride, kv.field_stride, kv.table, kv.bitmap, kv.read_values, kv.max_scan, \
+                       kv.read_stride, kv.field_stride, kv.table, kv.bitmap, kv.read_values, kv.max_scan, \
                        kv.read_slot, b.request_major)
     LTPG_LP_SWITCH(lp, CALL)
 #undef CALL
@@ -3436,8 +3437,8 @@ hipError_t launch_kv_small_epoch(const KvState &kv, const KvBatchDev &b, uint32_
 {
     if (!kv_small_epoch_ok(kv, b)) return hipErrorInvalidValue;
     hipLaunchKernelGGL(kv_small_epoch_kernel, dim3(1), dim3(kSmallBlock), 0, s, b.keys, b.meta, b.tids, b.n_txns,
-                       b.n_slots, b.request_major, kv.rows, kv.fields, kv.field_words, kv.field_stride, kv.max_scan,
-                       kv.read_slot, values, kv.hot_row, kv.table, kv.read_values, kv.bitmap, host_bits, seq_out, seq,
+                       b.n_slots, b.request_major, kv.rows, kv.fields, kv.field_words, kv.field_stride, kv.read_stride,
+                       kv.max_scan, kv.read_slot, values, kv.hot_row, kv.table, kv.read_values, kv.bitmap, host_bits, seq_out, seq,
                        result, ctr);
     return hipGetLastError();
 }

@@ -132,7 +132,9 @@ struct KvState {
     uint8_t *doomed = nullptr;          // max_txns: epoch number if waw > 0
     uint8_t *raw_flag = nullptr;        // max_txns: epoch number if a read found a lower W (fast form)
     uint8_t *war_flag = nullptr;        // max_txns: epoch number if a lower reader hit its W (fast form)
-    uint32_t *read_values = nullptr;    // max_slots * max_txns * read_slot fields, field_stride words each
+    uint32_t read_stride = 0;           // words between fields of the read values: field_stride, or field_words
+                                        // where memory does not allow that
+    uint32_t *read_values = nullptr;    // max_slots * max_txns * read_slot fields
     uint32_t *read_stage = nullptr;     // packed part of the read values on its way to the host
     uint64_t *bitmap = nullptr;         // ceil(max_txns / 64)
     uint32_t *conflicts = nullptr;      // max_txns

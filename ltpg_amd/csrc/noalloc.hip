@@ -111,7 +111,7 @@ extern "C" int ltpg_kv_epoch_noalloc(uint32_t *table, uint64_t rows, uint32_t fi
     kv.rows = rows;
     kv.fields = fields;
     kv.field_words = field_bytes / 4;
-    kv.field_stride = kv.field_words;  // the caller's table is packed
+    kv.field_stride = kv.read_stride = kv.field_words;  // the caller's table and read values are packed
     kv.max_slots = S;
     kv.table = table;
     kv.regs = reinterpret_cast<unsigned long long *>(p);

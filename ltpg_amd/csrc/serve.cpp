@@ -614,7 +614,7 @@ int launch(ltpg_server *sv, int w, Flight &f)
         }
         if (sv->cfg.keep_reads) {
             const uint64_t n = (uint64_t)S * B * ctx->kv.read_slot;
-            const uint32_t fw = ctx->kv.field_words, fsw = ctx->kv.field_stride;
+            const uint32_t fw = ctx->kv.field_words, fsw = ctx->kv.read_stride;
             if (fw == fsw)
                 LTPG_HIP_TRY(hipMemcpyAsync(f.h_reads, ctx->kv.read_values, n * fw * 4, hipMemcpyDeviceToHost,
                                             ctx->stream));
