@@ -124,17 +124,20 @@ bool kv_room(const ltpg_ctx *ctx, uint64_t bytes)
 }
 
 // The read values, at the fields' stride (ltpg_internal.h) where there is room
-// for it, else packed.
+// for it and for the staging that packs them for the host, else packed.
 int alloc_read_values(ltpg_ctx *ctx)
 {
     KvState &kv = ctx->kv;
     const uint64_t n = (uint64_t)kv.max_slots * ctx->cfg.max_txns * kv.read_slot;
     kv.read_stride = kv.field_stride;
     if (kv.field_stride != kv.field_words) {
-        if (kv_room(ctx, n * kv.field_stride * 4)) {
-            const int rc = dev_alloc(&kv.read_values, n * kv.field_stride, "kv read values");
+        kv.read_part = std::min(kReadStageWords / kv.field_words, n);
+        if (kv_room(ctx, (n * kv.field_stride + kv.read_part * kv.field_words) * 4)) {
+            int rc = dev_alloc(&kv.read_values, n * kv.field_stride, "kv read values");
+            if (!rc) rc = dev_alloc(&kv.read_stage, kv.read_part * kv.field_words, "read value staging");
             if (rc != LTPG_ERR_NOMEM) return rc;
             (void)hipGetLastError();  // dealt with
+            dev_free(kv.read_values);
         }
         kv.read_stride = kv.field_words;
     }
@@ -1490,11 +1493,8 @@ int ltpg_kv_read_values(ltpg_ctx *ctx, uint32_t *out, uint64_t n_words)
     LTPG_HIP_TRY(hipStreamSynchronize(ctx->stream));
     // packed on the device, part by part
     const uint64_t n_fields = (n_words + fw - 1) / fw;
-    const uint64_t part = std::min(kReadStageWords / fw,
-                                   (uint64_t)kv.max_slots * ctx->cfg.max_txns * kv.read_slot);
-    if (n_words && !kv.read_stage && (rc = dev_alloc(&kv.read_stage, part * fw, "read value staging"))) return rc;
-    for (uint64_t f = 0; f < n_fields; f += part) {
-        const uint64_t n = std::min(part, n_fields - f);
+    for (uint64_t f = 0; f < n_fields; f += kv.read_part) {
+        const uint64_t n = std::min(kv.read_part, n_fields - f);
         LTPG_HIP_TRY(launch_repack(kv.read_values + f * fsw, kv.read_stage, n, (uint32_t)fw, (uint32_t)fsw, 0,
                                    ctx->stream));
         LTPG_HIP_TRY(hipMemcpyAsync(out + f * fw, kv.read_stage, std::min(n * fw, n_words - f * fw) * 4,

@@ -135,7 +135,8 @@ struct KvState {
     uint32_t read_stride = 0;           // words between fields of the read values: field_stride, or field_words
                                         // where memory does not allow that
     uint32_t *read_values = nullptr;    // max_slots * max_txns * read_slot fields
-    uint32_t *read_stage = nullptr;     // packed part of the read values on its way to the host
+    uint32_t *read_stage = nullptr;     // with read_stride != field_words: a part of them, packed, on its way to
+    uint64_t read_part = 0;             // the host; fields of a part
     uint64_t *bitmap = nullptr;         // ceil(max_txns / 64)
     uint32_t *conflicts = nullptr;      // max_txns
     uint32_t *commit_list = nullptr;    // max_txns: the committed transactions of the last list CHECK
