@@ -285,7 +285,7 @@ int init_tpcc(ltpg_ctx *ctx)
     if ((rc = dev_alloc(&d.bitmap_dl, (B + 63) / 64, "Delivery bitmap"))) return rc;
     if ((rc = dev_alloc(&d.reads_dl, (uint64_t)kDlReads * B, "Delivery read values"))) return rc;
     // without memory for the bins every epoch takes the registers
-    if (!(c.flags & LTPG_FLAG_CONFLICT_COUNTS) && B >= kSplitTxns &&
+    if (!(c.flags & LTPG_FLAG_CONFLICT_COUNTS) && B >= kSplitTxns && stock_bins(d.t[LTPG_TPCC_STOCK].rows) &&
         bin_alloc(&tp.bin, B, [&](uint64_t n) { return stock_bin_shape(d.t[LTPG_TPCC_STOCK].rows, (uint32_t)n); },
                   ctx->stream) == LTPG_ERR_NOMEM)
         (void)hipGetLastError();  // dealt with

@@ -551,6 +551,8 @@ hipError_t launch_tpcc_execute(const TpccDev &d, const NeworderDev &no, const Pa
 // warehouses 40,000 48 / 47, 49,152 48 / 50, 131,072 62 / 78.
 constexpr uint32_t kSplitTxns = 3u << 14;
 bool tpcc_execute_split(const TpccDev &d, const BinBuffers &bin, const NeworderDev &no, const PaymentDev &pay);
+// Whether the bins take a STOCK table of this size at all (1,342 warehouses).
+bool stock_bins(uint64_t stock_rows);
 BinShape stock_bin_shape(uint64_t stock_rows, uint32_t n_neworder);
 hipError_t launch_tpcc_execute_split(const TpccDev &d, const BinBuffers &bin, const NeworderDev &no,
                                      const PaymentDev &pay, const EpochTag &e, bool cid, bool small,

@@ -1170,6 +1170,8 @@ void execute_at(const TpccDev &d, const NeworderDev &no, const PaymentDev &pay, 
 // Shape of the binned STOCK writes: small tiles (many blocks for a batch of a
 // few 100K lines) and as many buckets as give each a row array, 256 to 1024;
 // hashed beyond.
+bool stock_bins(uint64_t stock_rows) { return stock_rows <= 1024ull << kBinHashBits; }
+
 BinShape stock_bin_shape(uint64_t stock_rows, uint32_t n_neworder)
 {
     BinShape f;
@@ -1188,8 +1190,7 @@ bool tpcc_execute_split(const TpccDev &d, const BinBuffers &bin, const NeworderD
 {
     if (no.n + pay.n < kSplitTxns) return false;
     if (no.n == 0) return true;
-    const BinShape f = stock_bin_shape(d.t[ST].rows, no.n);
-    return f.row_bits <= kBinHashBits && bin_fits(bin, f);
+    return stock_bins(d.t[ST].rows) && bin_fits(bin, stock_bin_shape(d.t[ST].rows, no.n));
 }
 
 template <uint32_t BLK>
