@@ -111,6 +111,14 @@ int kv_bin_prepare(ltpg_ctx *ctx)
                      [&](uint64_t ops) { return bin_shape(kv.rows, ops); }, ctx->stream);
 }
 
+// The result of an allocation that the context can do without.
+int optional(int rc)
+{
+    if (rc != LTPG_ERR_NOMEM) return rc;
+    (void)hipGetLastError();  // dealt with
+    return LTPG_OK;
+}
+
 // Whether `bytes` that the context could do without leave room for what it
 // still needs: the second slot of host batches, and small change.
 bool kv_room(const ltpg_ctx *ctx, uint64_t bytes)
@@ -185,11 +193,10 @@ int init_kv(ltpg_ctx *ctx)
     // for the commit list of large epochs and their default shape; without
     // memory for them they take the bitmap and the register path
     if (!(c.flags & LTPG_FLAG_CONFLICT_COUNTS)) {
-        if (kv_room(ctx, B * 4) && dev_alloc(&kv.commit_list, B, "kv commit list") == LTPG_ERR_NOMEM)
-            (void)hipGetLastError();  // dealt with
+        if (kv_room(ctx, B * 4) && (rc = optional(dev_alloc(&kv.commit_list, B, "kv commit list")))) return rc;
         if (kv.max_scan <= 1 && kv_bin_auto(kv.rows, S * B) && kv_room(ctx, S * B * 5) &&
-            kv_bin_prepare(ctx) == LTPG_ERR_NOMEM)
-            (void)hipGetLastError();  // dealt with
+            (rc = optional(kv_bin_prepare(ctx))))
+            return rc;
     }
     // Registers start as all-ones: tag ~0 belongs to epoch 0, which is never
     // current (epochs start at 1), so every row reads as "no registrant".
@@ -285,10 +292,11 @@ int init_tpcc(ltpg_ctx *ctx)
     if ((rc = dev_alloc(&d.bitmap_dl, (B + 63) / 64, "Delivery bitmap"))) return rc;
     if ((rc = dev_alloc(&d.reads_dl, (uint64_t)kDlReads * B, "Delivery read values"))) return rc;
     // without memory for the bins every epoch takes the registers
-    if (!(c.flags & LTPG_FLAG_CONFLICT_COUNTS) && B >= kSplitTxns && stock_bins(d.t[LTPG_TPCC_STOCK].rows) &&
-        bin_alloc(&tp.bin, B, [&](uint64_t n) { return stock_bin_shape(d.t[LTPG_TPCC_STOCK].rows, (uint32_t)n); },
-                  ctx->stream) == LTPG_ERR_NOMEM)
-        (void)hipGetLastError();  // dealt with
+    const uint64_t stock = d.t[LTPG_TPCC_STOCK].rows;
+    if (!(c.flags & LTPG_FLAG_CONFLICT_COUNTS) && B >= kSplitTxns && stock_bins(stock) &&
+        (rc = optional(bin_alloc(
+             &tp.bin, B, [&](uint64_t n) { return stock_bin_shape(stock, (uint32_t)n); }, ctx->stream))))
+        return rc;
     if ((rc = refill_registers(ctx))) return rc;
     LTPG_HIP_TRY(hipMemsetAsync(d.bitmap_no, 0, (B + 63) / 64 * 8, ctx->stream));
     LTPG_HIP_TRY(hipMemsetAsync(d.bitmap_pay, 0, (B + 63) / 64 * 8, ctx->stream));
