@@ -462,7 +462,9 @@ int ltpg_tpcc_gen_next(ltpg_tpcc_gen *g, uint32_t n_txns, uint32_t tid_base, uin
  * form (PARTITIONED for large epochs of point operations, EXEC_PER_OP for
  * small ones, SMALL_EPOCH up to half its op slots while those hold at most
  * 16,384 field words; the buffers of PARTITIONED, 4 bytes per possible op slot
- * and about 2 bytes per 16, are then allocated with the context).
+ * and about 4 bytes per 16, are then allocated with the context).  Large epochs
+ * are fastest with TIDs that do not descend in batch position; in another order
+ * the same form takes about twice the time.
  * ltpg_kv_set_tuning fixes the shape from then on: 0 is none of the flags below.
  * EXEC_PER_OP: EXECUTE runs one lane per op instead of one lane per
  *   transaction.
@@ -796,7 +798,7 @@ int ltpg_serve_cancel(ltpg_server *sv, uint64_t *dropped);
  * caller-owned device table, with the same kernels and results as
  * ltpg_epoch_run on a context.  It calls no allocator: the per-row registers,
  * per-transaction flags and counters live in a fixed device array of the
- * library (about 93 MB, held by each GPU it runs on until the process ends).
+ * library (about 96 MB, held by each GPU it runs on until the process ends).
  *   table        device, rows x fields x field_bytes, row-major, packed;
  *                updated in place (RMW: a write adds TID | 1 to each word)
  *   batch        device arrays, slot-major (slot s of txn t at s*B + t)

@@ -29,7 +29,7 @@ void free_bin(BinBuffers &b)
 {
     dev_free(b.ent);
     dev_free(b.off);
-    dev_free(b.unsorted);
+    dev_free(b.marks);
 }
 
 constexpr uint64_t kReadbackBytes = 256u << 10;  // the bits of 2^20 transactions are 128 KB
@@ -89,17 +89,17 @@ int bin_alloc(BinBuffers *bin, uint64_t n, Shape shape, hipStream_t s)
     for (; n; n -= n / 64 + 1) {
         const BinShape f = shape(n);
         p.cap_ent = std::max(p.cap_ent, (uint64_t)f.tiles << f.tile_bits);
-        p.cap_off = std::max(p.cap_off, (uint64_t)f.tiles * (f.buckets + 1) * 66 / 64 + f.buckets + 1);
+        p.cap_off = std::max(p.cap_off, bin_starts(f) * 66 / 64 + f.buckets + 1);
     }
     int rc;
     if ((rc = dev_alloc(&p.ent, p.cap_ent, "binned operations")) || (rc = dev_alloc(&p.off, p.cap_off, "bin starts")) ||
-        (rc = dev_alloc(&p.unsorted, 1, "TID order flag"))) {
+        (rc = dev_alloc(&p.marks, kBinMarks, "bin marks"))) {
         free_bin(p);
         return rc;
     }
     *bin = p;  // freed with the context
     // epoch 0 is never current
-    LTPG_HIP_TRY(launch_fill_u8(reinterpret_cast<uint8_t *>(p.unsorted), 4, 0, s));
+    LTPG_HIP_TRY(launch_fill_u8(reinterpret_cast<uint8_t *>(p.marks), kBinMarks * 4, 0, s));
     return LTPG_OK;
 }
 

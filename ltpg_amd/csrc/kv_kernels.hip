@@ -1401,7 +1401,7 @@ __device__ __forceinline__ void end_epoch(const EpochEnd &e)
 #pragma unroll
     for (int d = 32; d > 0; d >>= 1) c += __shfl_xor(c, d);
     if (threadIdx.x != 0) return;
-    *e.unsorted = 0;
+    e.marks[kMarkUnsorted] = e.marks[kMarkWritten] = 0;
     if (!e.result) return;
     e.result[0] = c;
     e.result[1] = e.ctr->range_errors;
@@ -3115,23 +3115,37 @@ RegLayout reg_layout(const KvState &kv)
     return rl;
 }
 
-// Default EXECUTE shapes, from a sweep of rows x ops x (Zipf 0, 0.9, 0.99;
-// 50 and 90 % reads); times in us are register path (one lane per
-// transaction) / per-op register path / binned.
+// Default EXECUTE shapes, from a sweep of rows x ops x Zipf x reads; times in
+// us, per-transaction registers / per-op registers / binned.
 //
 // Binned: its cost besides streaming is one short run per tile and bucket, so
-// it needs about 1024 ops per bucket.
-//   1M rows (256 buckets):    160K ops 23 / 17 / 15, 320K 29 / 27 / 16,
-//                             1.3M 78 / 61 / 27, 16M 407 / 295 / 151
+// it needs about 1024 ops per bucket.  TIDs in order, Zipf 0.9, 50 % reads:
+//   1M rows (256 buckets):    160K ops 23 / 17 / 15, 320K 28 / 27 / 17,
+//                             1.3M 76 / 61 / 27, 16M 394 / 295 / 152
 //   10M rows (64 to 512 hashed, 1024 from 2^22 ops):
-//                             160K ops 21 / 17 / 17, 320K 27 / 27 / 18,
-//                             650K 42 / 46 / 21, 4M 189 / 121 / 60,
-//                             16M 444 / 374 / 146
-//   100M rows (1024, 2048 hashed): 650K ops 40 / 48 / 34, 1.3M 64 / 64 / 38,
-//                             16M 512 / 446 / 338
-// (Zipf 0.9, 50 % reads; with 90 % reads at Zipf 0.99 the line is crossed at
-// about twice the ops.)  Below 32K rows there are too few buckets to fill the
-// chip (20K rows, 16M ops, Zipf 0: 186 / 191 / 212).
+//                             160K ops 21 / 17 / 17, 320K 25 / 27 / 19,
+//                             650K 43 / 46 / 24, 4M 191 / 121 / 58,
+//                             16M 442 / 374 / 153
+//   100M rows (1024, 2048 hashed): 1.3M ops 64 / 64 / 38, 16M 505 / 446 / 217
+// (with 90 % reads at Zipf 0.99 the line is crossed at about twice the ops).
+// All reads take the bins without their flags: 10M rows, Zipf 0.99, 320K ops 10
+// / - / 11, 4M 55 / - / 34, 16M 196 / - / 83.
+//
+// Whether TIDs are in order, and what is read, the host does not know.  The
+// same with TIDs shuffled, per-transaction registers / binned (Zipf 0.99, 50 %
+// reads in brackets):
+//   50K rows: 320K ops 31 / 19 (39 / 21), 4M 217 / 78 (293 / 77), 16M 389 / 280
+//   1M rows:  320K ops 28 / 21 (35 / 18), 4M 206 / 85 (299 / 78), 16M 413 / 345
+//   10M rows: 320K ops 26 / 24 (33 / 27), 4M 190 / 105 (280 / 98), 16M 464 / 398
+// The registers are the faster ones, and ltpg_kv_set_tuning(0) keeps a context on
+// them, where the TIDs are shuffled and nearly all operations write rows of their
+// own (10M rows, Zipf 0, 650K ops 33 / 89, 16M on 50K rows 240 / 268), and where
+// a few writes meet reads that crowd on few rows (Zipf 0.99, 99 % reads, in order
+// 50K rows 1.3M ops 24 / 37, 16M 125 / 177; 10M rows 1.3M 33 / 49, 4M 73 / 75,
+// 16M 237 / 168; shuffled 16M 126 / 408 and 238 / 425): there each read has a
+// flag byte to store.
+// Below 32K rows there are too few buckets to fill the chip (20K rows, 16M ops,
+// Zipf 0: 186 / 191 / 212).
 bool kv_bin_auto(uint64_t rows, uint64_t ops)
 {
     if (rows <= (1ull << 15) || rows > (1ull << 28) || ops >= (1ull << 31)) return false;

@@ -76,11 +76,17 @@ constexpr uint32_t kBinSlotBits = 14;
 struct BinShape {
     uint32_t row_bits, buckets, mask, tile_bits, tiles;
 };
+constexpr uint32_t kMarkUnsorted = 0, kMarkWritten = 1, kMarkHot = 2, kMarkLong = 3;
+constexpr uint32_t kBinMarks = kMarkLong + 8192;
+inline uint64_t bin_starts(const BinShape &f) { return (uint64_t)f.tiles * (f.buckets + 1); }
 struct BinBuffers {
     uint64_t cap_ent = 0, cap_off = 0;
     uint32_t *ent = nullptr;              // [cap_ent] binned operations, tile by tile
-    uint16_t *off = nullptr;              // [cap_off] starts of each bucket's run in each tile
-    uint32_t *unsorted = nullptr;         // epoch number of the last epoch whose TIDs were out of order
+    uint32_t *off = nullptr;              // [cap_off] starts of each bucket's writes and reads in each tile
+    // epoch numbers of the last epoch whose TIDs were out of order and of the
+    // last with a write; of this epoch whether a bucket is hot, and bucket b's
+    // entries in runs that are long for a tile ([kMarkLong + b])
+    uint32_t *marks = nullptr;            // [kBinMarks]
 };
 // Shape for `ops` operation slots on `rows` rows (2^K >= rows, K <= 30).
 // Large epochs with a row array each: 1024 buckets and 16 slots per thread;
@@ -116,7 +122,7 @@ inline __host__ __device__ uint32_t bin_run_start(uint32_t tile, uint32_t tile_b
 }
 inline bool bin_fits(const BinBuffers &b, const BinShape &f)
 {
-    return b.ent && ((uint64_t)f.tiles << f.tile_bits) <= b.cap_ent && (uint64_t)f.tiles * (f.buckets + 1) <= b.cap_off;
+    return b.ent && ((uint64_t)f.tiles << f.tile_bits) <= b.cap_ent && bin_starts(f) <= b.cap_off;
 }
 
 struct KvState {
@@ -436,7 +442,7 @@ hipError_t launch_kv_readout(const KvState &kv, const KvBatchDev &b, hipStream_t
 // What WRITEBACK also does for ltpg_kv_epoch_noalloc (null ctr: nothing).
 struct EpochEnd {
     const DeviceCounters *ctr = nullptr;
-    uint32_t *unsorted = nullptr;
+    uint32_t *marks = nullptr;
     uint32_t *result = nullptr;
 };
 hipError_t launch_kv_writeback(const KvState &kv, const KvBatchDev &b, uint32_t values, DeviceCounters *ctr,

@@ -32,10 +32,10 @@ constexpr uint64_t kListAt = kCountersAt + (sizeof(DeviceCounters) + 255) / 256 
 constexpr uint64_t kBinOps = 1ull << 24;
 constexpr uint64_t kBinEnts = kBinOps + (1ull << kBinSlotBits);
 constexpr uint64_t kBinOffs = (kBinOps >> kBinSlotBits) * 1025 + 1025;
-constexpr uint64_t kUnsortedAt = kListAt + 4ull * LTPG_NOALLOC_MAX_TXNS;
-constexpr uint64_t kEntsAt = kUnsortedAt + 256;
+constexpr uint64_t kMarksAt = kListAt + 4ull * LTPG_NOALLOC_MAX_TXNS;
+constexpr uint64_t kEntsAt = kMarksAt + (4 * kBinMarks + 255) / 256 * 256;
 constexpr uint64_t kOffsAt = kEntsAt + 4 * kBinEnts;
-constexpr uint64_t kScratchBytes = kOffsAt + (2 * kBinOffs + 255) / 256 * 256;
+constexpr uint64_t kScratchBytes = kOffsAt + (4 * kBinOffs + 255) / 256 * 256;
 
 static __device__ __align__(256) uint8_t scratch[kScratchBytes];
 
@@ -127,7 +127,7 @@ extern "C" int ltpg_kv_epoch_noalloc(uint32_t *table, uint64_t rows, uint32_t fi
     b.keys = batch->keys;
     b.meta = batch->meta;
     b.tids = batch->tids;
-    uint32_t *unsorted = reinterpret_cast<uint32_t *>(p + kUnsortedAt);
+    uint32_t *marks = reinterpret_cast<uint32_t *>(p + kMarksAt);
     if (kv_small_epoch_ok(kv, b) && kv_small_words(kv, b) <= kAloneWords) {
         // one kernel; the registers and flags stay in its LDS (64 x 4 ops: ten
         // launches 36 us, this one 8 us, most of it the launch)
@@ -140,9 +140,9 @@ extern "C" int ltpg_kv_epoch_noalloc(uint32_t *table, uint64_t rows, uint32_t fi
         kv.commit_list = reinterpret_cast<uint32_t *>(p + kListAt);
         kv.bin.ent = reinterpret_cast<uint32_t *>(p + kEntsAt);
         kv.bin.cap_ent = kBinEnts;
-        kv.bin.off = reinterpret_cast<uint16_t *>(p + kOffsAt);
+        kv.bin.off = reinterpret_cast<uint32_t *>(p + kOffsAt);
         kv.bin.cap_off = kBinOffs;
-        kv.bin.unsorted = unsorted;
+        kv.bin.marks = marks;
         // binning needs no registers, whose refill costs 16 bytes per row:
         // taken wherever there are rows enough for its buckets (1M rows: 80K
         // ops take 13 us binned, 9 on the registers and 9 for their refill;
@@ -163,7 +163,7 @@ extern "C" int ltpg_kv_epoch_noalloc(uint32_t *table, uint64_t rows, uint32_t fi
         kv.list_valid = true;  // of the CHECK above
         EpochEnd end;
         end.ctr = ctr;
-        end.unsorted = unsorted;
+        end.marks = marks;
         end.result = result;
         LTPG_HIP_TRY(launch_kv_writeback(kv, b, values, ctr, s, end));
     } else if (result) {

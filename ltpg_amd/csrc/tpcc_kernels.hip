@@ -437,12 +437,13 @@ struct OrderTile {
 
 template <uint32_t BLK>
 __global__ __launch_bounds__(BLK) void claim_kernel(TpccDev d, NeworderDev no, PaymentDev pay, uint32_t tag,
-                                                      uint8_t epoch, uint32_t pay_blocks, bool cid, uint32_t *unsorted,
+                                                      uint8_t epoch, uint32_t pay_blocks, bool cid, uint32_t *marks,
                                                       DeviceCounters *ctr)
 {
     __shared__ OrderTile<BLK> s_tile;
     // the epoch's commit counts start at zero (CHECK adds to them)
     if (blockIdx.x == 0) zero_epoch_counts(ctr, BLK);
+    if (blockIdx.x == 0 && no.n) bin_no_long_runs(marks, 1024, BLK);  // of the binned STOCK writes
     uint32_t bad = 0;
     if (blockIdx.x >= pay_blocks) {
         const uint32_t q0 = (blockIdx.x - pay_blocks) * OrderTile<BLK>::kOrders, q = q0 + threadIdx.x;
@@ -452,7 +453,7 @@ __global__ __launch_bounds__(BLK) void claim_kernel(TpccDev d, NeworderDev no, P
             const NoRows r = no_rows(no, q);
             const uint32_t tid = no.TID[q], next = no.TID[q + 1 < no.n ? q + 1 : q];
             const unsigned long long me = priority(tag, tid, q);
-            if (tid > next) *unsorted = epoch;  // for the binned STOCK writes
+            if (tid > next) marks[kMarkUnsorted] = epoch;  // for the binned STOCK writes
             bad += (r.wh >= d.t[WH].rows) + (r.di >= d.t[DI].rows) + (r.cu >= d.t[CU].rows);
             // NEWORDER insert: a write (waw) under INTENDED; under REFERENCE
             // its R register is never consulted
@@ -1195,12 +1196,12 @@ bool tpcc_execute_split(const TpccDev &d, const BinBuffers &bin, const NeworderD
 
 template <uint32_t BLK>
 void execute_split_at(const TpccDev &d, const NeworderDev &no, const PaymentDev &pay, const EpochTag &e,
-                      bool cid, uint32_t *unsorted, DeviceCounters *ctr, hipStream_t s)
+                      bool cid, uint32_t *marks, DeviceCounters *ctr, hipStream_t s)
 {
     const uint32_t no_blocks = (no.n + BLK / 4 - 1) / (BLK / 4), pay_blocks = (pay.n + BLK - 1) / BLK;
     const uint32_t blocks = no_blocks + pay_blocks;
     hipLaunchKernelGGL(claim_kernel<BLK>, dim3(blocks), dim3(BLK), 0, s, d, no, pay, e.tag, e.epoch, pay_blocks, cid,
-                       unsorted, ctr);
+                       marks, ctr);
     hipLaunchKernelGGL(settle_kernel<BLK>, dim3(blocks), dim3(BLK), 0, s, d, no, pay, e.tag, e.epoch, no_blocks);
 }
 
@@ -1208,8 +1209,8 @@ hipError_t launch_tpcc_execute_split(const TpccDev &d, const BinBuffers &bin, co
                                      const PaymentDev &pay, const EpochTag &e, bool cid, bool small,
                                      DeviceCounters *ctr, hipStream_t s)
 {
-    if (small) execute_split_at<64>(d, no, pay, e, cid, bin.unsorted, ctr, s);
-    else execute_split_at<kBlock>(d, no, pay, e, cid, bin.unsorted, ctr, s);
+    if (small) execute_split_at<64>(d, no, pay, e, cid, bin.marks, ctr, s);
+    else execute_split_at<kBlock>(d, no, pay, e, cid, bin.marks, ctr, s);
     if (no.n == 0) return hipGetLastError();
     const StockSource src = {no, d.t[ST].rows, d.t[IT].rows};
     BinArgs a;
