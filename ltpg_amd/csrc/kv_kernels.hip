@@ -3318,7 +3318,12 @@ static uint32_t lane_copy_ok(const KvState &kv)
 // 196,608 89 / 100 (61 / 60); 32,768 of 16 22 / 21 (16 / 14), 65,536 23 / 28
 // (16 / 15), 262,144 24 / 56 (17 / 17); of 4 ops 262,144 40 / 37 (24 / 20).
 constexpr uint64_t kListOps = 1u << 20, kListOpsFewSlots = 1u << 21;
-constexpr uint32_t kListBlocks = 2048;  // 8 per CU: what the copies' registers allow to be resident
+// 8 per CU, what the read-out's registers and LDS allow to be resident.  Of
+// WRITEBACK 7 are (with up to 8 slots or more than 16; 1792 blocks take the same
+// time), but with 9 to 16 slots the lanes' fields leave LDS for 6, and the last
+// 512 blocks would be a second round: 2^20 transactions of 16 ops at Zipf 0.6
+// 28.4 us with 2048, 26.2 with 1536 (1792 cost 9 us more at 1.01M commits).
+constexpr uint32_t kListBlocks = 2048, kListBlocks16 = 1536;
 
 bool kv_check_lists(const KvState &kv, const KvBatchDev &b)
 {
@@ -3393,7 +3398,8 @@ hipError_t launch_kv_writeback(const KvState &kv, const KvBatchDev &b, uint32_t 
     const int g = group_for(b.n_slots);
     if (kv.list_valid && kv_check_lists(kv, b)) {
         const uint64_t per = (kBlock / 64) * (64 / g);  // transactions per block and round
-        const dim3 grid((unsigned)std::min<uint64_t>(kListBlocks, (b.n_txns + per - 1) / per));
+        const uint32_t most = g == 16 ? kListBlocks16 : kListBlocks;
+        const dim3 grid((unsigned)std::min<uint64_t>(most, (b.n_txns + per - 1) / per));
         const bool slots = !a.rm && kv.rows * kv.fields <= 1ull << 32;  // a field's index fits 32 bits
 #define CALL(GV) \
     hipLaunchKernelGGL(kv_writeback_list_kernel<GV>, grid, dim3(kBlock), 0, s, a, kv.commit_list, ctr, slots)
