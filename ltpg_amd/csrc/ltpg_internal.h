@@ -386,21 +386,22 @@ hipError_t launch_fill_u64(unsigned long long *p, uint64_t n, unsigned long long
 hipError_t launch_fill_u8(uint8_t *p, uint64_t n, uint8_t v, hipStream_t s);
 // n u32 words; src may be pinned host memory
 hipError_t launch_copy_u32(uint32_t *dst, const uint32_t *src, uint64_t n, hipStream_t s);
-// Up to four bitmaps to copy to pinned host memory (n[k] words from src[k]
-// to dst[k]; n[k] = 0 for unused entries).
 // Copy to pinned host memory, then store `seq` to *seq_out; `blocks` is zero
 // before and after.
 hipError_t launch_readback(uint32_t *dst, const uint32_t *src, uint32_t words, uint32_t *blocks, uint64_t *seq_out,
                            uint64_t seq, hipStream_t s);
+// Up to five bitmaps to copy to pinned host memory or an archive (n[k] words
+// from src[k] to dst[k]; n[k] = 0 for unused entries).
 struct PublishSet {
     const uint64_t *src[5];
     uint64_t *dst[5];
     uint32_t n[5];
 };
-// copy the bitmaps of p, then store seq to *seq_out (pinned host memory)
-// with a system-scope release; or copy them and stamp the device clock (unless
-// null)
+// Copy the bitmaps of p and stamp the device clock (unless null); with `reset`
+// the commit counts start over.
 hipError_t launch_archive(const PublishSet &p, unsigned long long *stamp, DeviceCounters *reset, hipStream_t s);
+// Copy the bitmaps of p, then store seq to *seq_out (pinned host memory) with a
+// system-scope release.
 hipError_t launch_publish(const PublishSet &p, uint64_t *seq_out, uint64_t seq, hipStream_t s);
 hipError_t launch_stamp(unsigned long long *out, hipStream_t s);
 
@@ -437,17 +438,16 @@ hipError_t launch_kv_check(const KvState &kv, const KvBatchDev &b, const EpochTa
 // Whether the fast CHECK of this batch lists its committed transactions.
 bool kv_check_lists(const KvState &kv, const KvBatchDev &b);
 hipError_t launch_kv_readout(const KvState &kv, const KvBatchDev &b, hipStream_t s);
-// Takes the committed transactions from commit_list if kv.list_valid, else
-// from the bitmap.
 // What WRITEBACK also does for ltpg_kv_epoch_noalloc (null ctr: nothing).
 struct EpochEnd {
     const DeviceCounters *ctr = nullptr;
     uint32_t *marks = nullptr;
     uint32_t *result = nullptr;
 };
+// Takes the committed transactions from commit_list if kv.list_valid, else
+// from the bitmap.
 hipError_t launch_kv_writeback(const KvState &kv, const KvBatchDev &b, uint32_t values, DeviceCounters *ctr,
-                               hipStream_t s,
-                               const EpochEnd &end = EpochEnd());
+                               hipStream_t s, const EpochEnd &end = EpochEnd());
 // A whole fast-form epoch of at most LTPG_SMALL_EPOCH_OPS op slots in one
 // single-workgroup kernel (a hot row only with at most 1024 fields; rows <
 // 2^32 - 1).  With seq_out it
