@@ -466,6 +466,8 @@ int ltpg_tpcc_gen_next(ltpg_tpcc_gen *g, uint32_t n_txns, uint32_t tid_base, uin
  * are fastest with TIDs that do not descend in batch position; in another order
  * the same form takes about twice the time.
  * ltpg_kv_set_tuning fixes the shape from then on: 0 is none of the flags below.
+ * (A batched run sets its own, and leaves the context with it: the default, or
+ * what ltpg_batched_set_tuning or ltpg_batched_autotune chose.)
  * EXEC_PER_OP: EXECUTE runs one lane per op instead of one lane per
  *   transaction.
  * SPLIT_REGISTERS: a row's R and W registers live in two arrays instead of
