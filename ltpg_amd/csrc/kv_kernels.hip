@@ -2993,7 +2993,10 @@ hipError_t launch_fill_set(const FillSet &f, hipStream_t s)
 {
     uint64_t most = 1;
     for (uint32_t k = 0; k < f.n; k++) most = std::max(most, f.bytes[k]);
-    const uint64_t blocks = std::min<uint64_t>((most + 16 * 256 - 1) / (16 * 256), 8192);
+    // Few blocks start sooner, many keep the stores of one block together: 160 MB
+    // 26 us with 8192, 28 with 65,536, 1.6 GB 319 and 271.
+    const uint64_t cap = most > (1ull << 29) ? 65536 : 8192;
+    const uint64_t blocks = std::min<uint64_t>((most + 16 * 256 - 1) / (16 * 256), cap);
     hipLaunchKernelGGL(fill_set_kernel, dim3((unsigned)blocks), dim3(256), 0, s, f);
     return hipGetLastError();
 }
