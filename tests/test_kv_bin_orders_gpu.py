@@ -52,6 +52,8 @@ def order(kind, B, seed):
     (9_000_000, 40_000, 16, 1, 0.0, 1.0),    # hashed, one share of distinct writes
     (9_000_000, 81_920, 8, 1, 0.0, 0.97),    # as many writes as the 64-bit table has slots
     (120_000_000, 1_000_003, 16, 1, 0.0, 1.0),  # two shares; 2048 buckets, tiles of 16384
+    (400_000, 1_048_577, 17, 2, 0.3, 0.01),  # more than 1024 tiles, hot
+    (60_000_000, 1_048_577, 17, 2, 0.2, 0.5),  # the same, hashed
 ], ids=lambda v: str(v))
 @pytest.mark.parametrize("tids", ["ordered", "shuffled", "ties"])
 def test_orders_and_crowds_match_oracle(gpu, rows, B, S, hot_rows, hot_share, writes, tids):
