@@ -552,7 +552,10 @@ int ltpg_conflict_counters(ltpg_ctx *ctx, uint32_t type, uint32_t *out, uint32_t
  * at out[(((s * B) + t) * L + i) * field_words + w], taken from the snapshot
  * (the table before the epoch's write-back).  Only read and scan slots of
  * committed transactions are written, and of a scan only the rows inside
- * the table: an aborted transaction's reads are discarded. */
+ * the table: an aborted transaction's reads are discarded.  The device keeps
+ * fields of 64 bytes and more on multiples of 64 bytes (100-byte fields 128
+ * apart), and up to 32 MB to pack them for the host, all allocated with the
+ * context; where the device's memory does not hold that it keeps them packed. */
 int ltpg_kv_read_values(ltpg_ctx *ctx, uint32_t *out, uint64_t n_words);
 /* Running totals since the last reset: committed and attempted (checked)
  * transactions of `type`, kept on the device so a pipelined epoch loop needs
